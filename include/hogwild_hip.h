@@ -355,6 +355,32 @@ typedef struct hw_append {
 
 int hw_rope_append(const hw_append* a, void* stream);
 
+/*
+ * merge_caches (python/hogwild/attention.py:251-257) for all layers of a model: for every layer l, n[l] rows of the source
+ * segment are appended behind the first dst_len[l] rows of the target,
+ *   K_dst[l][h, dst_len[l] + t, :] = rope(K_src[l][h, t, :], cos/sin of `position`),  V_dst[l][h, dst_len[l] + t, :] = V_src[l][h, t, :]
+ * with the tables of hw_build_inputs (cos/sin(float(position) * inv_freq) * attention_scaling, rounded to table_dtype) and
+ * the rotation of hw_rope_append (mode, RotE).  The HOST arrays hold one entry per layer; buffers are [Hkv, cap, E|Ev].
+ * table_dtype is HW_F32 or dtype.
+ */
+typedef struct hw_merge_segments_args {
+    int32_t dtype, table_dtype, mode;
+    int32_t layers, Hkv, E, Ev, RotE;
+    int32_t position;
+    float attention_scaling;
+    const float* inv_freq;           /* device fp32 [RotE/2] */
+    const void* const* k_src;        /* HOST arrays of `layers` device pointers */
+    const void* const* v_src;
+    const int32_t* src_cap;
+    const int32_t* n;
+    void* const* k_dst;
+    void* const* v_dst;
+    const int32_t* dst_cap;
+    const int32_t* dst_len;
+} hw_merge_segments_args;
+
+int hw_merge_segments(const hw_merge_segments_args* a, void* stream);
+
 /* Number of compute units of the current device (0 on failure). */
 int hw_device_cus(void);
 

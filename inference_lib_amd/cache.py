@@ -10,7 +10,8 @@ library: the objects a model's attention layer talks to during a Hogwild! decode
                       CacheStructure, get_queries_buffer / get_att_buffer / get_input_kwargs.  The per-worker Python
                       loop of update (:148-158) is one `hw_rope_append` launch; the layer-0 construction of locations and
                       rotary tables (:164-196) is one `hw_build_inputs` launch.
-  merge_caches ...... attention.py:251-257: re-rotate a segment by the target's length and append it.
+  merge_caches ...... attention.py:251-257: re-rotate a segment by the target's length and append it, all layers in one
+                      launch.
 
 Everything numeric runs in the HIP library; there is no torch fallback.
 """
@@ -22,6 +23,7 @@ from typing import Any, Dict, List, Optional, Sequence
 import torch
 
 from . import _lib
+from .attention import HAVE_TORCH_OPS
 
 
 class _LayerViews:
@@ -333,8 +335,21 @@ def merge_caches(target: SegmentCache, source: SegmentCache, model=None, *, inv_
         return
     dev = source.k[0].device
     tdt = table_dtype if table_dtype is not None else source.k[0].dtype
+    position = target.get_seq_length()
+    if HAVE_TORCH_OPS and dev.type == "cuda" and source.k and len(source.k) >= len(target.k) and len(source.v) >= len(target.v):
+        layers = range(len(target.k))
+        for layer in layers:          # grow like every other append (the reference's merge goes through target.update)
+            if target.lengths[layer] + source.lengths[layer] > target.k[layer].size(1):
+                target.reserve(layer, source.lengths[layer])
+        added = source.lengths[: len(target.k)]
+        if torch.ops.libhogatt.merge_segments(target.k, target.v, target.lengths, source.k[: len(target.k)], source.v[: len(target.k)], added,
+                                              inv_freq.to(dev), attention_scaling, position, tdt, mode):
+            for layer in layers:
+                target.lengths[layer] += added[layer]
+            return
+    # buffers of several forms, or not packed: layer by layer
     # one table row: the position is target's length for every source token (S = 1 and pos_end = length + 1)
-    _, cos, sin = _lib.build_inputs([[target.get_seq_length() + 1]], 1, inv_freq.to(dev), attention_scaling=attention_scaling,
+    _, cos, sin = _lib.build_inputs([[position + 1]], 1, inv_freq.to(dev), attention_scaling=attention_scaling,
                                     table_dtype=None if tdt == torch.float32 else tdt)
     cos = cos.reshape(1, 1, -1).to(tdt)
     sin = sin.reshape(1, 1, -1).to(tdt)

@@ -386,6 +386,58 @@ void copy_to_blocks(const at::Tensor& key_states, const at::Tensor& value_states
     check_status(hw_copy_to_blocks(&c, stream), "hw_copy_to_blocks");
 }
 
+// ---- segments ----------------------------------------------------------------------------------------------------
+
+// hw_merge_segments on lists of per-layer buffers [Hkv, cap, E|Ev] (all layers of one form, packed).  Returns false, with
+// nothing queued, for buffers that are not of that form: the caller then goes layer by layer.
+bool merge_segments(at::TensorList k_dst, at::TensorList v_dst, at::IntArrayRef dst_len, at::TensorList k_src, at::TensorList v_src, at::IntArrayRef n,
+                    const at::Tensor& inv_freq, double scaling, int64_t position, at::ScalarType table_dtype, int64_t mode) {
+    const size_t L = k_dst.size();
+    if (L == 0 || v_dst.size() != L || dst_len.size() != L || k_src.size() != L || v_src.size() != L || n.size() != L) return false;
+    const at::Tensor &kd0 = k_dst[0], &vd0 = v_dst[0];
+    const at::ScalarType dt = kd0.scalar_type();
+    if ((dt != at::kFloat && dt != at::kHalf && dt != at::kBFloat16) || (table_dtype != at::kFloat && table_dtype != dt)) return false;
+    if (kd0.dim() != 3 || vd0.dim() != 3 || inv_freq.dim() != 1 || inv_freq.scalar_type() != at::kFloat || !inv_freq.is_contiguous() ||
+        inv_freq.device() != kd0.device())
+        return false;
+    const int64_t Hkv = kd0.size(0), E = kd0.size(2), Ev = vd0.size(2), RotE = 2 * inv_freq.size(0);
+    if (RotE > E || position < 0 || position >= (1ll << 31)) return false;
+    std::vector<const void*> ks(L), vs(L);
+    std::vector<void*> kd(L), vd(L);
+    std::vector<int32_t> scap(L), dcap(L), nn(L), dl(L);
+    for (size_t l = 0; l < L; ++l) {
+        const at::Tensor* four[4] = {&k_dst[l], &v_dst[l], &k_src[l], &v_src[l]};
+        for (int i = 0; i < 4; ++i)
+            if (four[i]->dim() != 3 || four[i]->size(0) != Hkv || four[i]->size(2) != (i % 2 ? Ev : E) || four[i]->scalar_type() != dt ||
+                four[i]->device() != kd0.device() || !four[i]->is_contiguous() || four[i]->size(1) >= (1ll << 31))
+                return false;
+        if (k_dst[l].size(1) != v_dst[l].size(1) || k_src[l].size(1) != v_src[l].size(1)) return false;
+        if (n[l] < 0 || n[l] > k_src[l].size(1) || dst_len[l] < 0 || dst_len[l] + n[l] > k_dst[l].size(1)) return false;
+        kd[l] = k_dst[l].data_ptr();
+        vd[l] = v_dst[l].data_ptr();
+        ks[l] = k_src[l].const_data_ptr();
+        vs[l] = v_src[l].const_data_ptr();
+        scap[l] = (int32_t)k_src[l].size(1);
+        dcap[l] = (int32_t)k_dst[l].size(1);
+        nn[l] = (int32_t)n[l];
+        dl[l] = (int32_t)dst_len[l];
+    }
+    hw_merge_segments_args a{};
+    a.dtype = dtype_code(kd0);
+    a.table_dtype = table_dtype == at::kFloat ? HW_F32 : a.dtype;
+    a.mode = (int32_t)mode;
+    a.layers = (int32_t)L;
+    a.Hkv = (int32_t)Hkv; a.E = (int32_t)E; a.Ev = (int32_t)Ev; a.RotE = (int32_t)RotE;
+    a.position = (int32_t)position;
+    a.attention_scaling = (float)scaling;
+    a.inv_freq = inv_freq.const_data_ptr<float>();
+    a.k_src = ks.data(); a.v_src = vs.data(); a.src_cap = scap.data(); a.n = nn.data();
+    a.k_dst = kd.data(); a.v_dst = vd.data(); a.dst_cap = dcap.data(); a.dst_len = dl.data();
+    c10::hip::HIPGuardMasqueradingAsCUDA guard(kd0.device());
+    check_status(hw_merge_segments(&a, c10::hip::getCurrentHIPStreamMasqueradingAsCUDA(kd0.device().index()).stream()), "merge_segments");
+    return true;
+}
+
 }  // namespace
 
 // `import hogatt` only has to load this shared object so that the registrations below run.
@@ -415,6 +467,9 @@ TORCH_LIBRARY(libhogatt, m) {
           "Tensor block_table, Tensor seq_lengths) -> ()", tags);
     m.def("hogwild_varlen_paged_sdpa(Tensor(a!) output, float scale, Tensor locations, Tensor queries, "
           "Tensor fragment_lengths, Tensor key_cache, Tensor value_cache, Tensor block_table, Tensor cu_seqlens_q, Tensor cu_seqlens_k) -> ()", tags);
+    // addition: merge_caches (python/hogwild/attention.py:251-257) for all layers of a segment
+    m.def("merge_segments(Tensor(a!)[] k_dst, Tensor(b!)[] v_dst, int[] dst_len, Tensor[] k_src, Tensor[] v_src, int[] n, Tensor inv_freq, "
+          "float scaling, int position, ScalarType table_dtype, int mode) -> bool", tags);
 }
 
 TORCH_LIBRARY_IMPL(libhogatt, CUDA, m) {
@@ -427,4 +482,5 @@ TORCH_LIBRARY_IMPL(libhogatt, CUDA, m) {
     m.impl("hogwild_paged_sdpa", hogwild_paged_sdpa);
     m.impl("copy_to_blocks", copy_to_blocks);
     m.impl("hogwild_varlen_paged_sdpa", hogwild_varlen_paged_sdpa);
+    m.impl("merge_segments", merge_segments);
 }

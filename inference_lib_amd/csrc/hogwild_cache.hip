@@ -5,18 +5,20 @@
 //                           (python/hogwild/attention.py:164-196) with model.rotary_emb.
 //   rope_append_kernel .... rotate the new keys (apply_rotary_pos_emb, python/hogwild/attention.py:84-90, called
 //                           at :313-315) and append keys and values to each worker's segment
-//                           (:148-158), in one pass and in place.  With one source "worker" and a single
-//                           cos/sin row broadcast over its tokens this is also merge_caches (:251-257): re-rotate a
-//                           whole segment by a constant offset and append it to another.
+//                           (:148-158), in one pass and in place.
+//   merge_segments_kernel . merge_caches (:251-257): re-rotate whole segments by a constant offset and append them to
+//                           others, all layers of a model in one launch (bound by memory, not by latency).
 //   advance_lengths_kernel  len_dev[f] += add[f]: segment lengths kept in device memory, so that a decode step captured
 //                           as a graph can be replayed while the segments grow (the first two kernels and the
 //                           attention kernel then read the lengths from there).
 //
-// All are tiny, latency-bound kernels; they exist so that a decode step needs no per-worker Python loop, no
+// The others are tiny, latency-bound kernels; they exist so that a decode step needs no per-worker Python loop, no
 // torch.cat reallocation and no .contiguous() copy of the segments.
 
 #include <hip/hip_runtime.h>
 #include <stdint.h>
+
+#include <type_traits>
 
 #include "hogwild_kernels.h"
 #include "hogwild_device.h"
@@ -178,9 +180,139 @@ __global__ __launch_bounds__(256) void rope_append_kernel(const AppendArgs a) {
     }
 }
 
+// merge_caches for all layers at once: layer l's n source rows per kv head go behind the first dst_len rows of its target,
+// the keys rotated by the angles of ONE position (the target's length), the values as they are.  grid = (row blocks, kv
+// head, layer).  Bound by memory: every byte is read and written once, with four to eight 16-byte loads of a thread in
+// flight, and the one cos / sin row is worked out by every workgroup for itself (RotE / 2 angles, into LDS) instead of by
+// three launches in front.  One launch per layer left the chip idle between launches of 5.5 us that a host call of 23 us
+// each could not keep fed: 16 layers x 2 segments of 1000 and 777 tokens (8 kv heads, D = 128, bf16; 233 MB) 757 -> 51 us
+// (4.6 TB/s; a large copy reaches 4.9).
+constexpr int MERGE_ROWS = 64;     // rows of one kv head per workgroup: 4 value and 2 key chunk pairs per thread at D = 128
+template <class DT, bool EAGER, bool CS16, bool VEC>
+__global__ __launch_bounds__(256) void merge_segments_kernel(const MergeSegmentsArgs a) {
+    typedef typename Elem<DT>::store_t store_t;
+    constexpr int SZ = Elem<DT>::size;
+    constexpr int CH = VEC ? Chunk<DT>::CH : 1;
+    constexpr int ROUND = !CS16 ? 0 : std::is_same<DT, F16>::value ? 1 : 2;
+    constexpr int UN = 4;
+    typedef typename std::conditional<VEC, u32x4, store_t>::type item_t;
+    extern __shared__ float tab[];                    // [cos | sin], RotE / 2 each
+    const int tid = threadIdx.x;
+    const int half = a.RotE >> 1;
+    const int t_begin = (int)blockIdx.x * MERGE_ROWS;
+    const MergeSegmentsArgs::Layer& ly = a.layer[blockIdx.z];
+    const int rows = min(MERGE_ROWS, ly.n - t_begin);
+    if (rows <= 0) return;                            // uniform over the workgroup
+    for (int i = tid; i < half; i += 256) {           // the arithmetic of build_inputs_kernel
+        const float ang = (float)a.position * a.inv_freq[i];
+        tab[i] = round_table<ROUND>(cosf(ang) * a.scaling);
+        tab[half + i] = round_table<ROUND>(sinf(ang) * a.scaling);
+    }
+    const int h = blockIdx.y;
+    const size_t srow = (size_t)h * ly.src_cap + t_begin, drow = (size_t)h * ly.dst_cap + ly.dst_len + t_begin;
+    // values: rows * Ev consecutive elements on both sides
+    {
+        const item_t* src = reinterpret_cast<const item_t*>(reinterpret_cast<const char*>(ly.v_src) + srow * a.Ev * SZ);
+        item_t* dst = reinterpret_cast<item_t*>(reinterpret_cast<char*>(ly.v_dst) + drow * a.Ev * SZ);
+        const int total = rows * (a.Ev / CH);
+        for (int i0 = tid; i0 < total; i0 += 256 * UN) {
+            item_t x[UN];
+#pragma unroll
+            for (int u = 0; u < UN; ++u) x[u] = src[min(i0 + u * 256, total - 1)];
+#pragma unroll
+            for (int u = 0; u < UN; ++u)
+                if (i0 + u * 256 < total) dst[i0 + u * 256] = x[u];
+        }
+    }
+    __syncthreads();
+    // keys: chunk pairs (e, e + RotE/2), then the elements behind the rotary width
+    const char* ksrc = reinterpret_cast<const char*>(ly.k_src) + srow * a.E * SZ;
+    char* kdst = reinterpret_cast<char*>(ly.k_dst) + drow * a.E * SZ;
+    const int n_pair = half / CH;
+    const int pairs = rows * n_pair;
+    for (int i0 = tid; i0 < pairs; i0 += 256 * 2) {
+        item_t p1[2], p2[2];
+        int at[2], e[2];
+#pragma unroll
+        for (int u = 0; u < 2; ++u) {
+            const int i = min(i0 + u * 256, pairs - 1);
+            const int t = i / n_pair;
+            e[u] = (i - t * n_pair) * CH;
+            at[u] = (t * a.E + e[u]) * SZ;            // < 64 rows: fits easily
+            p1[u] = *reinterpret_cast<const item_t*>(ksrc + at[u]);
+            p2[u] = *reinterpret_cast<const item_t*>(ksrc + at[u] + half * SZ);
+        }
+#pragma unroll
+        for (int u = 0; u < 2; ++u) {
+            if (i0 + u * 256 >= pairs) continue;
+            float x1[CH], x2[CH], y1[CH], y2[CH];
+            if constexpr (VEC) {
+                Chunk<DT>::unpack(p1[u], x1);
+                Chunk<DT>::unpack(p2[u], x2);
+            } else {
+                x1[0] = Elem<DT>::to_float(p1[u]);
+                x2[0] = Elem<DT>::to_float(p2[u]);
+            }
+#pragma unroll
+            for (int i = 0; i < CH; ++i) {
+                const float c = tab[e[u] + i], sn = tab[half + e[u] + i];
+                rotate_pair<DT, EAGER, CS16>(x1[i], x2[i], c, sn, c, sn, y1[i], y2[i]);
+            }
+            item_t r1, r2;
+            if constexpr (VEC) {
+                r1 = Chunk<DT>::pack(y1);
+                r2 = Chunk<DT>::pack(y2);
+            } else {
+                r1 = Elem<DT>::from_float(y1[0]);
+                r2 = Elem<DT>::from_float(y2[0]);
+            }
+            *reinterpret_cast<item_t*>(kdst + at[u]) = r1;
+            *reinterpret_cast<item_t*>(kdst + at[u] + half * SZ) = r2;
+        }
+    }
+    const int n_pass = (a.E - a.RotE) / CH;
+    for (int i = tid; i < rows * n_pass; i += 256) {
+        const int t = i / n_pass;
+        const int off = (t * a.E + a.RotE + (i - t * n_pass) * CH) * SZ;
+        *reinterpret_cast<item_t*>(kdst + off) = *reinterpret_cast<const item_t*>(ksrc + off);
+    }
+}
+
 // ------------------------------------------------------------------------------------------------
 // launchers
 // ------------------------------------------------------------------------------------------------
+template <class DT, bool EAGER, bool CS16>
+static hipError_t launch_merge_segments_v(const MergeSegmentsArgs& a, int max_n, hipStream_t stream) {
+    constexpr int CH = Chunk<DT>::CH;
+    bool vec = a.E % CH == 0 && a.Ev % CH == 0 && (a.RotE / 2) % CH == 0;
+    for (int l = 0; l < a.layers; ++l) {
+        const MergeSegmentsArgs::Layer& ly = a.layer[l];
+        vec = vec && ((reinterpret_cast<uintptr_t>(ly.k_src) | reinterpret_cast<uintptr_t>(ly.v_src) | reinterpret_cast<uintptr_t>(ly.k_dst) |
+                       reinterpret_cast<uintptr_t>(ly.v_dst)) & 15u) == 0;
+    }
+    const dim3 grid((unsigned)((max_n + MERGE_ROWS - 1) / MERGE_ROWS), (unsigned)a.Hkv, (unsigned)a.layers);
+    const size_t lds = (size_t)a.RotE * sizeof(float);
+    if (vec) hipLaunchKernelGGL((merge_segments_kernel<DT, EAGER, CS16, true>), grid, dim3(256), lds, stream, a);
+    else hipLaunchKernelGGL((merge_segments_kernel<DT, EAGER, CS16, false>), grid, dim3(256), lds, stream, a);
+    return hipGetLastError();
+}
+
+template <class DT>
+static hipError_t launch_merge_segments_dt(const MergeSegmentsArgs& a, bool eager, bool cs16, int max_n, hipStream_t stream) {
+    if constexpr (Elem<DT>::size == 2) {
+        if (cs16) return eager ? launch_merge_segments_v<DT, true, true>(a, max_n, stream) : launch_merge_segments_v<DT, false, true>(a, max_n, stream);
+    }
+    return eager ? launch_merge_segments_v<DT, true, false>(a, max_n, stream) : launch_merge_segments_v<DT, false, false>(a, max_n, stream);
+}
+
+hipError_t launch_merge_segments(const MergeSegmentsArgs& a, int dtype, bool eager, bool cs16, int max_n, hipStream_t stream) {
+    switch (dtype) {
+        case 0: return launch_merge_segments_dt<F32>(a, eager, false, max_n, stream);
+        case 1: return launch_merge_segments_dt<F16>(a, eager, cs16, max_n, stream);
+        default: return launch_merge_segments_dt<BF16>(a, eager, cs16, max_n, stream);
+    }
+}
+
 hipError_t launch_build_inputs(const BuildInputsArgs& a, int round_dtype, hipStream_t stream) {
     const long long total = (long long)a.F * a.W * a.S * ((a.RotE >> 1) > 0 ? (a.RotE >> 1) : 1);
     if (total <= 0) return hipSuccess;

@@ -368,6 +368,49 @@ int rope_append_run(const hw_append* p, void* stream) {
     return HW_OK;
 }
 
+int merge_segments_run(const hw_merge_segments_args* p, void* stream) {
+    if (p == nullptr) return HW_ERR_NULL;
+    if (p->dtype != HW_F32 && p->dtype != HW_F16 && p->dtype != HW_BF16) return HW_ERR_DTYPE;
+    if (p->table_dtype != HW_F32 && p->table_dtype != p->dtype) return HW_ERR_DTYPE;
+    if (p->mode != HW_ROPE_EAGER && p->mode != HW_ROPE_FUSED) return HW_ERR_SHAPE;
+    if (p->layers < 0 || p->Hkv < 1 || p->Hkv > 65535 || p->E < 1 || p->Ev < 1) return HW_ERR_SHAPE;
+    if (p->E >= (1 << 20) || p->Ev >= (1 << 20)) return HW_ERR_SHAPE;          // 64 rows are addressed with 32-bit offsets
+    if (p->RotE < 0 || p->RotE > p->E || (p->RotE & 1) || p->RotE > 8192) return HW_ERR_SHAPE;   // the table row lies in LDS
+    if (p->layers == 0) return HW_OK;
+    if (p->k_src == nullptr || p->v_src == nullptr || p->src_cap == nullptr || p->n == nullptr || p->k_dst == nullptr || p->v_dst == nullptr ||
+        p->dst_cap == nullptr || p->dst_len == nullptr || (p->RotE > 0 && p->inv_freq == nullptr))
+        return HW_ERR_NULL;
+    for (int l = 0; l < p->layers; ++l) {
+        if (p->n[l] < 0 || p->n[l] > p->src_cap[l] || p->dst_len[l] < 0 || (long long)p->dst_len[l] + p->n[l] > p->dst_cap[l]) return HW_ERR_SHAPE;
+        if (p->n[l] > 0 && (p->k_src[l] == nullptr || p->v_src[l] == nullptr || p->k_dst[l] == nullptr || p->v_dst[l] == nullptr)) return HW_ERR_NULL;
+    }
+    for (int l0 = 0; l0 < p->layers; l0 += hw::MAX_MERGE_LAYERS) {
+        const int nl = p->layers - l0 < hw::MAX_MERGE_LAYERS ? p->layers - l0 : hw::MAX_MERGE_LAYERS;
+        hw::MergeSegmentsArgs a;
+        std::memset(&a, 0, sizeof(a));
+        int max_n = 0;
+        for (int l = 0; l < nl; ++l) {
+            a.layer[l].k_src = p->k_src[l0 + l];
+            a.layer[l].v_src = p->v_src[l0 + l];
+            a.layer[l].k_dst = p->k_dst[l0 + l];
+            a.layer[l].v_dst = p->v_dst[l0 + l];
+            a.layer[l].src_cap = p->src_cap[l0 + l];
+            a.layer[l].dst_cap = p->dst_cap[l0 + l];
+            a.layer[l].n = p->n[l0 + l];
+            a.layer[l].dst_len = p->dst_len[l0 + l];
+            if (p->n[l0 + l] > max_n) max_n = p->n[l0 + l];
+        }
+        if (max_n == 0) continue;
+        a.inv_freq = p->inv_freq;
+        a.scaling = p->attention_scaling;
+        a.position = p->position;
+        a.layers = nl; a.Hkv = p->Hkv; a.E = p->E; a.Ev = p->Ev; a.RotE = p->RotE;
+        const hipError_t e = hw::launch_merge_segments(a, p->dtype, p->mode == HW_ROPE_EAGER, p->table_dtype != HW_F32, max_n, reinterpret_cast<hipStream_t>(stream));
+        if (e != hipSuccess) return (int)e;
+    }
+    return HW_OK;
+}
+
 }  // namespace
 
 extern "C" {
@@ -517,6 +560,8 @@ int hw_build_inputs_dev(int32_t* locations, float* cosines, float* sines, const 
 }
 
 int hw_advance_lengths(int32_t* len_dev, const int32_t* add, int F, void* stream) { return advance_lengths_run(len_dev, add, F, stream); }
+
+int hw_merge_segments(const hw_merge_segments_args* a, void* stream) { return merge_segments_run(a, stream); }
 
 int hw_rope_append(const hw_append* a, void* stream) { return rope_append_run(a, stream); }
 

@@ -160,6 +160,24 @@ struct AppendArgs {
     const int* len_dev;                  // segment lengths in device memory, or null
 };
 
+// Whole segments appended to others, every layer of a model in one launch (see merge_segments_kernel).
+constexpr int MAX_MERGE_LAYERS = 48;    // layers per launch: their table travels in the kernel arguments
+struct MergeSegmentsArgs {
+    struct Layer {
+        const void* k_src;     // [Hkv, src_cap, E], packed rows
+        const void* v_src;     // [Hkv, src_cap, Ev]
+        void* k_dst;           // [Hkv, dst_cap, E]
+        void* v_dst;
+        int src_cap, dst_cap;
+        int n, dst_len;        // n rows are appended behind the first dst_len
+    } layer[MAX_MERGE_LAYERS];
+    const float* inv_freq;     // [RotE / 2]
+    float scaling;
+    int position;              // every key is rotated by the angles of this position
+    int layers, Hkv, E, Ev, RotE;
+};
+hipError_t launch_merge_segments(const MergeSegmentsArgs& a, int dtype, bool eager, bool cs16, int max_n, hipStream_t stream);
+
 hipError_t launch_build_inputs(const BuildInputsArgs& a, int round_dtype, hipStream_t stream);
 hipError_t launch_rope_append(const AppendArgs& a, int dtype, bool eager, bool cs16, hipStream_t stream);
 // len_dev[f] += add[f] for f < F (F <= MAXF): the first node of a captured decode step
