@@ -29,6 +29,7 @@ EXPORTS = [
     "hw_paged_validate", "hw_paged_plan_debug", "hw_paged_workspace_bytes", "hw_paged_sdpa", "hw_varlen_paged_sdpa",
     "hw_paged_sdpa_stages", "hw_copy_to_blocks", "hw_build_inputs", "hw_rope_append",
     "hw_build_inputs_dev", "hw_advance_lengths", "hw_fused_attention_static", "hw_sdpa_workspace_bytes",
+    "hw_merge_segments",
 ]
 
 
