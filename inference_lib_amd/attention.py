@@ -58,6 +58,8 @@ def hogwild_fused(queries: torch.Tensor, locations: torch.Tensor, keys: List[tor
 
 
 def _in_place_or_contiguous(keys: List[torch.Tensor], values: List[torch.Tensor]):
+    if len(keys) == len(values) and all(k.is_contiguous() and v.is_contiguous() for k, v in zip(keys, values)):
+        return keys, values
     ks, vs = [], []
     for k, v in zip(keys, values):
         k3, v3 = (k[0] if k.dim() == 4 else k), (v[0] if v.dim() == 4 else v)

@@ -25,6 +25,9 @@ import torch
 from . import _lib
 from .attention import HAVE_TORCH_OPS
 
+if HAVE_TORCH_OPS:
+    _rope_append = torch.ops.libhogatt.rope_append.default
+    _segment_views = torch.ops.libhogatt.segment_views.default
 
 class _LayerViews:
     """`segment.key_cache[layer]` -> the [1, Hkv, L, D] view of what has been written so far."""
@@ -253,8 +256,11 @@ class HogwildCache:
             end[id(s)] = start + n
         for s in segs:
             s.reserve(layer_idx, end[id(s)] - s.lengths[layer_idx])
-        _lib.rope_append(key_states, value_states, [s.k[layer_idx] for s in segs], [s.v[layer_idx] for s in segs],
-                         dst, cosines=cosines, sines=sines, n_new=n_new, mode=mode)
+        k_dst, v_dst = [s.k[layer_idx] for s in segs], [s.v[layer_idx] for s in segs]
+        # the operator takes the plain forms and returns False for the others, which _lib handles or refuses
+        if not (HAVE_TORCH_OPS and key_states.is_cuda and k_dst and
+                _rope_append(k_dst, v_dst, dst, n_new, key_states, value_states, cosines, sines, mode)):
+            _lib.rope_append(key_states, value_states, k_dst, v_dst, dst, cosines=cosines, sines=sines, n_new=n_new, mode=mode)
         for s in segs:
             s.lengths[layer_idx] = end[id(s)]
 
@@ -275,8 +281,15 @@ class HogwildCache:
                 table_dtype=None if tdt == torch.float32 else tdt)
             self.segments = segments
             self.frags = torch.tensor([cs.get_seq_length(layer_idx) for cs in segments], dtype=torch.int32, device=key_states.device)
-        keys = [cs.key_cache[layer_idx] for cs in self.segments]    # views; no .contiguous() copies (attention.py:160-162,199-203)
-        vals = [cs.value_cache[layer_idx] for cs in self.segments]
+        # views; no .contiguous() copies (attention.py:160-162,199-203)
+        keys, vals = [cs.k[layer_idx] for cs in self.segments], [cs.v[layer_idx] for cs in self.segments]
+        lens = [cs.lengths[layer_idx] for cs in self.segments]
+        if HAVE_TORCH_OPS and keys[0].is_cuda:
+            both = _segment_views(keys + vals, lens + lens)
+            keys, vals = both[: len(lens)], both[len(lens):]
+        else:
+            keys = [b[:, :n, :].unsqueeze(0) for b, n in zip(keys, lens)]
+            vals = [b[:, :n, :].unsqueeze(0) for b, n in zip(vals, lens)]
         return CacheStructure(keys=keys, values=vals, cos=self.cosines, sin=self.sines, loc=self.locations, frags=self.frags)
 
     def update(self, key_states: torch.Tensor, value_states: torch.Tensor, layer_idx: int,

@@ -19,12 +19,15 @@
 //   * `hogwild_fused_devlen` takes the current fragment lengths from `fragment_lengths` in device memory.
 
 #include <ATen/Tensor.h>
+#include <ATen/ops/as_strided.h>
 #include <ATen/ops/empty.h>
 #include <Python.h>
 #include <ATen/hip/impl/HIPGuardImplMasqueradingAsCUDA.h>
 #include <ATen/hip/impl/HIPStreamMasqueradingAsCUDA.h>
 #include <torch/library.h>
 
+#include <algorithm>
+#include <optional>
 #include <string>
 #include <vector>
 
@@ -45,28 +48,34 @@ void check_status(int status, const char* where) {
     TORCH_CHECK(status == 0, "libhogatt::", where, " failed with status ", status, ": ", hw_status_string(status));
 }
 
-// Drops the optional leading batch dimension of 1 of a KV fragment: [1, Hkv, L, D] -> [Hkv, L, D].
-at::Tensor fragment_view(const at::Tensor& t, const char* what, size_t f) {
+// Geometry of a KV fragment [Hkv, L, D], read through the optional leading batch dimension of 1 ([1, Hkv, L, D]).  (Not
+// by a select() per tensor: that is a view to make and to drop for every fragment of every call.)
+struct FragmentDims {
+    int64_t heads, len, width, head_stride, row_stride, elem_stride;
+};
+FragmentDims fragment_dims(const at::Tensor& t, const char* what, size_t f) {
     TORCH_CHECK(t.dim() == 3 || (t.dim() == 4 && t.size(0) == 1), "libhogatt: ", what, " fragment ", f,
                 " must be [Hkv, L, D] or [1, Hkv, L, D], got ", t.sizes());
-    return t.dim() == 4 ? t.select(0, 0) : t;
+    const int64_t o = t.dim() - 3;
+    const at::IntArrayRef n = t.sizes(), st = t.strides();
+    return {n[o], n[o + 1], n[o + 2], st[o], st[o + 1], st[o + 2]};
 }
 
 // Rows between consecutive kv heads of a fragment [Hkv, L, D] whose rows are contiguous, or -1 if the pair of tensors is
 // not of that form (packed fragments give L).
-int64_t row_capacity(const at::Tensor& k, const at::Tensor& v) {
-    const int64_t Hkv = k.size(0), L = k.size(1), E = k.size(2), Ev = v.size(2);
+int64_t row_capacity(const FragmentDims& k, const FragmentDims& v) {
+    const int64_t Hkv = k.heads, L = k.len, E = k.width, Ev = v.width;
     if (L == 0) return 0;
-    if ((E > 1 && k.stride(2) != 1) || (Ev > 1 && v.stride(2) != 1)) return -1;
-    if (L > 1 && (k.stride(1) != E || v.stride(1) != Ev)) return -1;
+    if ((E > 1 && k.elem_stride != 1) || (Ev > 1 && v.elem_stride != 1)) return -1;
+    if (L > 1 && (k.row_stride != E || v.row_stride != Ev)) return -1;
     if (Hkv == 1) return L;
-    if (k.stride(0) % E != 0 || v.stride(0) % Ev != 0 || k.stride(0) / E != v.stride(0) / Ev || k.stride(0) / E < L) return -1;
-    return k.stride(0) / E;
+    if (k.head_stride % E != 0 || v.head_stride % Ev != 0 || k.head_stride / E != v.head_stride / Ev || k.head_stride / E < L) return -1;
+    return k.head_stride / E;
 }
 
 struct Unpacked {
     hw_problem p{};
-    std::vector<at::Tensor> keep;          // contiguous fragment tensors kept alive until the launch is queued
+    std::vector<at::Tensor> keep;          // contiguous copies of fragments, kept alive until the launch is queued
     std::vector<const void*> kptr, vptr;
     std::vector<int32_t> len, cap;
     at::Tensor workspace;
@@ -102,32 +111,32 @@ void unpack_common(Unpacked& u, at::Tensor& out, double scale, const at::Tensor&
     u.cap.resize(F);
     int64_t Hkv = -1;
     for (int64_t f = 0; f < F; ++f) {
-        at::Tensor k = fragment_view(key_fragments[f], "key", f);
-        at::Tensor v = fragment_view(value_fragments[f], "value", f);
-        if (f == 0) Hkv = k.size(0);
-        TORCH_CHECK(k.size(0) == Hkv && v.size(0) == Hkv, "libhogatt: fragment ", f, " has a different number of kv heads");
-        TORCH_CHECK(k.size(1) == v.size(1), "libhogatt: key and value fragment ", f, " differ in length");
-        TORCH_CHECK(k.size(2) == E && v.size(2) == Ev, "libhogatt: fragment ", f, " has the wrong head dimension");
+        const at::Tensor &k = key_fragments[f], &v = value_fragments[f];
+        const FragmentDims kd = fragment_dims(k, "key", f), vd = fragment_dims(v, "value", f);
+        if (f == 0) Hkv = kd.heads;
+        TORCH_CHECK(kd.heads == Hkv && vd.heads == Hkv, "libhogatt: fragment ", f, " has a different number of kv heads");
+        TORCH_CHECK(kd.len == vd.len, "libhogatt: key and value fragment ", f, " differ in length");
+        TORCH_CHECK(kd.width == E && vd.width == Ev, "libhogatt: fragment ", f, " has the wrong head dimension");
         TORCH_CHECK(k.scalar_type() == out.scalar_type() && v.scalar_type() == out.scalar_type(),
                     "libhogatt: fragment ", f, " has a different dtype than the output");
         TORCH_CHECK(k.device() == out.device() && v.device() == out.device(), "libhogatt: fragment ", f, " lives on another device");
         // A fragment may be a view into a [Hkv, cap, D] allocation that grows in place: rows contiguous, kv heads a
         // whole number of rows apart.  Anything else is copied by the fused op (as the reference does,
         // src/binding.cu:330-337) and rejected by hogwild_sdpa.
-        int64_t cap = row_capacity(k, v);
+        int64_t cap = row_capacity(kd, vd);
+        u.kptr[f] = k.const_data_ptr();
+        u.vptr[f] = v.const_data_ptr();
         if (cap < 0 && copy_noncontiguous) {
-            k = k.contiguous();
-            v = v.contiguous();
-            cap = k.size(1);
+            u.keep.push_back(k.contiguous());
+            u.kptr[f] = u.keep.back().const_data_ptr();
+            u.keep.push_back(v.contiguous());
+            u.vptr[f] = u.keep.back().const_data_ptr();
+            cap = kd.len;
         }
         TORCH_CHECK(cap >= 0, "libhogatt: fragment ", f, " must be contiguous (or have contiguous rows and kv heads a whole "
                     "number of rows apart, the same for keys and values)");
-        u.kptr[f] = k.const_data_ptr();
-        u.vptr[f] = v.const_data_ptr();
-        u.len[f] = (int32_t)k.size(1);
+        u.len[f] = (int32_t)kd.len;
         u.cap[f] = (int32_t)cap;
-        u.keep.push_back(k);
-        u.keep.push_back(v);
     }
     TORCH_CHECK(Hkv > 0 && Hq % Hkv == 0, "libhogatt: Hq must be a multiple of Hkv");
     hw_problem& p = u.p;
@@ -438,6 +447,77 @@ bool merge_segments(at::TensorList k_dst, at::TensorList v_dst, at::IntArrayRef 
     return true;
 }
 
+// hw_rope_append on tensors: the append of HogwildCache, whose argument checks and pointer tables took most of a step's host
+// time in Python (12 layers, two workers, three segments: 694 -> 364 us a step with this, segment_views and fragment_dims).  Returns false, with nothing queued, for anything the checks below do not take: the caller's general path then
+// handles it or names what is wrong.
+bool rope_append(at::TensorList k_dst, at::TensorList v_dst, at::IntArrayRef dst_len, at::IntArrayRef n_new, const at::Tensor& key_states,
+                 const at::Tensor& value_states, const std::optional<at::Tensor>& cosines, const std::optional<at::Tensor>& sines, int64_t mode) {
+    const at::Tensor &ks = key_states, &vs = value_states;
+    if (ks.dim() != 4 || vs.dim() != 4) return false;
+    const int64_t W = ks.size(0), Hkv = ks.size(1), S = ks.size(2), E = ks.size(3), Ev = vs.size(3);
+    const at::ScalarType dt = ks.scalar_type();
+    if (vs.size(0) != W || vs.size(1) != Hkv || vs.size(2) != S || vs.scalar_type() != dt || vs.device() != ks.device()) return false;
+    if (dt != at::kFloat && dt != at::kHalf && dt != at::kBFloat16) return false;
+    if (E < 1 || Ev < 1 || (E > 1 && ks.stride(3) != 1) || (Ev > 1 && vs.stride(3) != 1)) return false;
+    if (W < 1 || W >= (1 << 20) || Hkv < 1 || Hkv >= (1 << 20) || S < 1 || S >= (1 << 20) || E >= (1 << 20) || Ev >= (1 << 20)) return false;
+    if ((int64_t)k_dst.size() != W || (int64_t)v_dst.size() != W || (int64_t)dst_len.size() != W || (int64_t)n_new.size() != W) return false;
+    std::vector<void*> kd(W), vd(W);
+    std::vector<int32_t> len(W), cap(W), nn(W);
+    for (int64_t w = 0; w < W; ++w) {
+        const at::Tensor &k = k_dst[w], &v = v_dst[w];
+        if (k.dim() != 3 || v.dim() != 3 || k.size(0) != Hkv || v.size(0) != Hkv || k.size(2) != E || v.size(2) != Ev || k.size(1) != v.size(1) ||
+            k.size(1) >= (1ll << 31) || !k.is_contiguous() || !v.is_contiguous() || k.scalar_type() != dt || v.scalar_type() != dt ||
+            k.device() != ks.device() || v.device() != ks.device())
+            return false;
+        if (n_new[w] < 0 || n_new[w] > S || dst_len[w] < 0 || dst_len[w] + n_new[w] > k.size(1)) return false;
+        kd[w] = k.data_ptr();
+        vd[w] = v.data_ptr();
+        len[w] = (int32_t)dst_len[w];
+        cap[w] = (int32_t)k.size(1);
+        nn[w] = (int32_t)n_new[w];
+    }
+    hw_append a{};
+    a.dtype = dtype_code(ks);
+    a.cs_dtype = HW_F32;
+    a.mode = (int32_t)mode;
+    a.W = (int32_t)W; a.Hkv = (int32_t)Hkv; a.S = (int32_t)S; a.E = (int32_t)E; a.Ev = (int32_t)Ev;
+    a.key_states = ks.const_data_ptr(); a.value_states = vs.const_data_ptr();
+    a.ks_w = ks.stride(0); a.ks_h = ks.stride(1); a.ks_s = ks.stride(2);
+    a.vs_w = vs.stride(0); a.vs_h = vs.stride(1); a.vs_s = vs.stride(2);
+    if (cosines.has_value() != sines.has_value()) return false;
+    if (cosines.has_value()) {
+        const at::Tensor &c = *cosines, &s = *sines;
+        if (c.dim() != 3 || s.sizes() != c.sizes() || c.size(0) != W || (c.size(1) != 1 && c.size(1) != S) || c.scalar_type() != s.scalar_type() ||
+            (c.scalar_type() != at::kFloat && c.scalar_type() != dt) || !c.is_contiguous() || !s.is_contiguous() || c.device() != ks.device() ||
+            s.device() != ks.device())
+            return false;
+        a.RotE = (int32_t)c.size(2);
+        a.cs_dtype = dtype_code(c);
+        a.cosines = c.const_data_ptr(); a.sines = s.const_data_ptr();
+        a.cs_w = c.size(1) * c.size(2);
+        a.cs_s = c.size(1) == 1 ? 0 : c.size(2);
+    }
+    a.k_dst = kd.data(); a.v_dst = vd.data();
+    a.dst_len = len.data(); a.dst_cap = cap.data(); a.n_new = nn.data();
+    c10::hip::HIPGuardMasqueradingAsCUDA guard(ks.device());
+    check_status(hw_rope_append(&a, c10::hip::getCurrentHIPStreamMasqueradingAsCUDA(ks.device().index()).stream()), "rope_append");
+    return true;
+}
+
+// The filled parts of segment buffers [Hkv, cap, D] as fragments: [1, Hkv, len, D] views.
+std::vector<at::Tensor> segment_views(at::TensorList buffers, at::IntArrayRef len) {
+    TORCH_CHECK(buffers.size() == len.size(), "libhogatt: one length per buffer");
+    std::vector<at::Tensor> out;
+    out.reserve(buffers.size());
+    for (size_t i = 0; i < buffers.size(); ++i) {
+        const at::Tensor& b = buffers[i];
+        TORCH_CHECK(b.dim() == 3 && len[i] >= 0, "libhogatt: segment buffers must be [Hkv, cap, D], lengths not negative");
+        const int64_t n = std::min(len[i], b.size(1));           // as slicing does
+        out.push_back(at::as_strided(b, {1, b.size(0), n, b.size(2)}, {b.size(0) * b.stride(0), b.stride(0), b.stride(1), b.stride(2)}));
+    }
+    return out;
+}
+
 }  // namespace
 
 // `import hogatt` only has to load this shared object so that the registrations below run.
@@ -470,6 +550,10 @@ TORCH_LIBRARY(libhogatt, m) {
     // addition: merge_caches (python/hogwild/attention.py:251-257) for all layers of a segment
     m.def("merge_segments(Tensor(a!)[] k_dst, Tensor(b!)[] v_dst, int[] dst_len, Tensor[] k_src, Tensor[] v_src, int[] n, Tensor inv_freq, "
           "float scaling, int position, ScalarType table_dtype, int mode) -> bool", tags);
+    // additions: the append of HogwildCache.update (:148-158) and the fragments it returns (:160-162)
+    m.def("rope_append(Tensor(a!)[] k_dst, Tensor(b!)[] v_dst, int[] dst_len, int[] n_new, Tensor key_states, Tensor value_states, "
+          "Tensor? cosines, Tensor? sines, int mode) -> bool", tags);
+    m.def("segment_views(Tensor(a)[] buffers, int[] len) -> Tensor(a)[]", tags);
 }
 
 TORCH_LIBRARY_IMPL(libhogatt, CUDA, m) {
@@ -483,4 +567,6 @@ TORCH_LIBRARY_IMPL(libhogatt, CUDA, m) {
     m.impl("copy_to_blocks", copy_to_blocks);
     m.impl("hogwild_varlen_paged_sdpa", hogwild_varlen_paged_sdpa);
     m.impl("merge_segments", merge_segments);
+    m.impl("rope_append", rope_append);
+    m.impl("segment_views", segment_views);
 }
