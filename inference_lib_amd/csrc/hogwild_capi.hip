@@ -68,6 +68,9 @@ int run(const hw_problem* p, void* stream_, int fused, int stages = HW_STAGE_ATT
     if (st != HW_OK) return st;
     if (p->workspace == nullptr || p->workspace_bytes < cp.workspace_bytes || !aligned16(p->workspace)) return HW_ERR_WORKSPACE;
     const hw_plan& plan0 = cp.plan[0];
+    // (a workspace sized for CallPlan only, as the static scratch may be, keeps to its launch)
+    StreamPlan sp;
+    const bool stream_runs = stream_plan(p, cus, cp, &sp) && p->workspace_bytes >= sp.workspace_bytes;
     // the VALU logits exist for what they are measured on: the fused entry with full rotary width, one row block, host lengths
     if (p->variant == HW_VARIANT_VALU_QK && (!fused || p->RotE != p->E || plan0.row_blocks != 1 || p->len_dev != nullptr)) return HW_ERR_UNSUPPORTED;
 
@@ -77,7 +80,7 @@ int run(const hw_problem* p, void* stream_, int fused, int stages = HW_STAGE_ATT
     bool prerotated = !fused;
     if (fused && p->RotE != p->E) {
         void* rqbuf = p->rq;
-        if (rqbuf == nullptr) rqbuf = reinterpret_cast<char*>(p->workspace) + cp.partial_bytes;
+        if (rqbuf == nullptr) rqbuf = reinterpret_cast<char*>(p->workspace) + (stream_runs ? sp.workspace_bytes - cp.rope_bytes : cp.partial_bytes);
         if (stages & HW_STAGE_ATTENTION) {
             hipError_t er = hw::launch_rope(rqbuf, p->q, p->cosines, p->sines, p->dtype, p->F, p->W, p->Hq, p->S, p->E, p->RotE, stream);
             if (er != hipSuccess) return (int)er;
@@ -87,7 +90,8 @@ int run(const hw_problem* p, void* stream_, int fused, int stages = HW_STAGE_ATT
     }
     const int rows = plan0.rows;
     float* const part_o = reinterpret_cast<float*>(p->workspace);
-    float* const part_ml = part_o + (size_t)p->Hkv * cp.slots * rows * p->Ev;
+    const size_t part_rows = stream_runs ? (size_t)sp.slots * hw::PLAN_SLOT_ROWS : (size_t)cp.slots * rows;     // per kv head
+    float* const part_ml = part_o + (size_t)p->Hkv * part_rows * p->Ev;
     // One workgroup per kv head and row group holds whole rows: it writes out / lse itself and the merge launch is
     // dropped (the 128-row kernel has an epilogue of its own and always goes through the merge).
     const bool direct = cp.groups == 1 && plan0.wgs_per_head == 1 && stages == (HW_STAGE_ATTENTION | HW_STAGE_MERGE) &&
@@ -109,7 +113,7 @@ int run(const hw_problem* p, void* stream_, int fused, int stages = HW_STAGE_ATT
             ka.frag.lc[f].cap = p->cap != nullptr ? p->cap[f0 + f] : p->len[f0 + f];
         }
         for (int f = 0; f <= HW_MAX_LAUNCH_FRAGMENTS; ++f) ka.frag.tile_begin[f] = plan.tile_begin[f];
-        for (int i = 0; i <= HW_MAX_SPLITS; ++i) ka.wg_tile[i] = plan.wg_tile_begin[i];
+        for (int i = 0; i <= HW_MAX_SPLITS; ++i) ka.wg_tile[i] = stream_runs ? sp.wg_tile_begin[i] : plan.wg_tile_begin[i];
         // everything indexed by fragment starts at this group's first fragment
         ka.h.q = prerotated ? q_in + (size_t)f0 * q_frag : q_in;
         ka.h.loc = p->locations + (size_t)f0 * ws_rows;
@@ -136,6 +140,15 @@ int run(const hw_problem* p, void* stream_, int fused, int stages = HW_STAGE_ATT
         ka.h.magic_s = magic(p->S);
         ka.h.magic_nrg = magic(plan.row_groups);
         ka.h.magic_wg = magic(plan.wgs_per_head);
+        if (stream_runs) {
+            ka.h.nrg = 1;
+            ka.h.magic_nrg = magic(1);
+            ka.h.wgs_per_head = sp.wgs;
+            ka.h.magic_wg = magic(sp.wgs);
+            ka.h.nwg = sp.wgs * p->Hkv;
+            ka.h.slot_stride = sp.slots;
+            ka.h.flags = ((ka.h.nwg % 8 == 0) ? hw::KH_XCD_REMAP : 0) | (prerotated ? hw::KH_PREROTATED : 0) | hw::KH_STREAM;
+        }
         if (plan.row_blocks == hw::WIDE_ROW_BLOCKS)
             e = hw::launch_attention_wide(ka, p->dtype, p->E, stream);
         else
@@ -153,6 +166,12 @@ int run(const hw_problem* p, void* stream_, int fused, int stages = HW_STAGE_ATT
     ma.xcd_local = (cp.groups == 1 && plan0.workgroups % 8 == 0 && p->Hkv % 8 == 0) ? 1 : 0;
     ma.row_tab = nullptr;
     ma.pslots = 0;
+    if (stream_runs) {
+        ma.wgs_per_head = sp.max_pieces;
+        ma.xcd_local = ((sp.wgs * p->Hkv) % 8 == 0 && p->Hkv % 8 == 0) ? 1 : 0;
+        ma.row_tab = reinterpret_cast<const int*>(part_ml + (size_t)p->Hkv * part_rows * 2);
+        ma.pslots = sp.slots;
+    }
     e = hw::launch_merge(ma, p->dtype, p->Ev, stream);
     return (int)e;
 }
@@ -456,7 +475,9 @@ static int workspace_bytes_for(const hw_problem* p, int fused, size_t* bytes) {
     CallPlan cp;
     st = plan_call(p, cus, &cp, fused);
     if (st != HW_OK) return st;
+    StreamPlan sp;
     *bytes = cp.workspace_bytes;
+    if (stream_plan(p, cus, cp, &sp) && sp.workspace_bytes > *bytes) *bytes = sp.workspace_bytes;
     return HW_OK;
 }
 

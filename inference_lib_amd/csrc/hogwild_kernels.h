@@ -46,6 +46,9 @@ static_assert(sizeof(KernelHeader) == 128, "KernelHeader must be 32 dwords");
 constexpr int KH_XCD_REMAP = 1;   // consecutive logical workgroup ids share an XCD (the grid is a multiple of 8)
 constexpr int KH_DIRECT = 2;      // one workgroup per kv head and row group: it normalises its own result and writes out / lse
                                   // itself (part_o then holds the address of out, part_ml that of lse or null); no merge launch
+constexpr int KH_STREAM = 8;      // 128-row workgroups that run across row groups: wg_tile counts the tiles of all row groups one
+                                  // behind the other, slot_stride = slots of PLAN_SLOT_ROWS rows per kv head, the piece of
+                                  // workgroup g in row group rg goes to slot g + rg, a row table for the merge lies behind part_ml
 constexpr int KH_PREROTATED = 4;  // the queries arrive rotated, [F,W,Hq,S,E] (read by the launchers only)
 
 struct KernelArgs {
@@ -61,8 +64,8 @@ struct MergeArgs {
     float* lse;
     int W, Hq, Hkv, S, R, wgs_per_head;
     int xcd_local;      // kv head h was computed on XCD h / (Hkv/8): merge it there
-    // Partials laid out by workgroup slot instead of by row (the paged launch that is planned on the device, see
-    // PagedHeader): row_tab[kv head][r] = {first slot | slots << 16, row within the slot}, a slot holds PLAN_SLOT_ROWS rows, pslots
+    // Partials laid out by workgroup slot instead of by row (KH_STREAM, and the paged launch that is planned on the device,
+    // see PagedHeader): row_tab[kv head][r] = {first slot | slots << 16, row within the slot}, a slot holds PLAN_SLOT_ROWS rows, pslots
     // slots per kv head; wgs_per_head then only bounds the slots of a row (for the choice of the merge kernel's shape).
     const int* row_tab;
     int pslots;

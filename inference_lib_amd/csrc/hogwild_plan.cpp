@@ -213,6 +213,79 @@ int plan_call(const hw_problem* p, int num_cus, CallPlan* cp, int fused) {
     return HW_OK;
 }
 
+// Row groups of 128 rows that do not fill the CUs evenly: 40 row groups of 8 kv heads (1024 prompt tokens at a GQA ratio of
+// 5) are 320 workgroups, so 256 CUs take two rounds of which the second is a quarter full.  Cut into equal runs across the
+// row groups every CU gets 1.25 row groups of work instead of 2.  A run that crosses into the next row group opens it anew
+// (queries, partial sums: about kJobCost tiles), so the runs are taken only where the count below promises a tenth.
+bool stream_plan(const hw_problem* p, int num_cus, const CallPlan& cp, StreamPlan* sp) {
+    const hw_plan& plan = cp.plan[0];
+    if (cp.groups != 1 || p->splits > 0 || plan.row_blocks != hw::WIDE_ROW_BLOCKS || plan.row_groups < 2 || plan.tiles_per_head < 1) return false;
+    constexpr double kJobCost = 6.0, kOpenCost = 2.0;     // in tiles: a row group's prologue and epilogue; one more fragment
+    constexpr int kMinPiece = 4;                          // tiles worth opening a row group for
+    const int nrg = plan.row_groups, T = plan.tiles_per_head;
+    int nf = 0;
+    for (int f = 0; f < p->F; ++f) nf += p->len[f] > 0 ? 1 : 0;
+    const double job = T + kJobCost + kOpenCost * nf;     // a whole row group
+    int wgs = num_cus / p->Hkv;
+    if (wgs > hw::MAX_SPLITS) wgs = hw::MAX_SPLITS;
+    if ((long long)wgs * 2 * kMinPiece > (long long)nrg * T) wgs = (int)((long long)nrg * T / (2 * kMinPiece));
+    if (wgs < 1 || (long long)wgs + nrg >= (1 << 15) || (long long)nrg * T >= (1ll << 30)) return false;
+    const long long launched = plan.workgroups, rounds = (launched + num_cus - 1) / num_cus;
+    const double cost_rounds = rounds * ((double)T / plan.wgs_per_head + kJobCost + kOpenCost * (1.0 + (double)(nf - 1) / plan.wgs_per_head));
+    const double cost_stream = (nrg * job + (wgs - 1) * (kJobCost + kOpenCost)) / wgs;
+    if (cost_stream * 1.1 > cost_rounds) return false;
+    sp->wgs = wgs;
+    double left = nrg * job;            // work not dealt yet, without the re-openings of the workgroups to come
+    int wg = 0;
+    double used = 0.0;
+    sp->wg_tile_begin[0] = 0;
+    for (int rg = 0; rg < nrg; ++rg) {
+        bool open = false;              // the current workgroup holds the row group's queries
+        for (int f = 0; f < p->F; ++f) {
+            const int ft = (int)(((long long)p->len[f] + hw::TILE - 1) / hw::TILE);
+            int t = 0;
+            while (t < ft) {
+                const int wgs_left = wgs - wg;
+                const double target = (left + used + (wgs_left - 1) * (kJobCost + kOpenCost)) / wgs_left;
+                const double opening = kOpenCost + (open ? 0.0 : kJobCost);
+                const double room = target - used - opening;
+                if (used > 0.0 && wgs_left > 1 && room < (open ? 1 : kMinPiece)) {      // not worth opening this here
+                    sp->wg_tile_begin[++wg] = rg * T + plan.tile_begin[f] + t;
+                    used = 0.0;
+                    open = false;
+                    continue;
+                }
+                int take = (int)(room + 0.5);
+                if (take < 1) take = 1;
+                if (take > ft - t || wgs_left == 1) take = ft - t;
+                used += opening + take;
+                left -= take + (t == 0 ? kOpenCost : 0.0) + (t == 0 && plan.tile_begin[f] == 0 ? kJobCost : 0.0);
+                open = true;
+                t += take;
+                if (t < ft) {
+                    sp->wg_tile_begin[++wg] = rg * T + plan.tile_begin[f] + t;
+                    used = 0.0;
+                    open = false;
+                }
+            }
+        }
+    }
+    sp->wgs = wg + 1;
+    for (int i = sp->wgs; i <= HW_MAX_SPLITS; ++i) sp->wg_tile_begin[i] = nrg * T;
+    sp->max_pieces = 1;
+    for (int rg = 0, g = 0; rg < nrg; ++rg) {
+        while (sp->wg_tile_begin[g + 1] <= rg * T) ++g;
+        int last = g;
+        while (sp->wg_tile_begin[last + 1] < (rg + 1) * T) ++last;
+        if (last - g + 1 > sp->max_pieces) sp->max_pieces = last - g + 1;
+    }
+    sp->slots = sp->wgs + nrg - 1;
+    const size_t rows = (size_t)sp->slots * hw::PLAN_SLOT_ROWS;
+    sp->partial_bytes = (size_t)p->Hkv * rows * ((size_t)p->Ev + 2) * sizeof(float);
+    sp->workspace_bytes = ((sp->partial_bytes + (size_t)p->Hkv * plan.rows * 2 * sizeof(int) + 255) & ~(size_t)255) + cp.rope_bytes;
+    return magic_exact((unsigned long long)sp->wgs, (unsigned long long)sp->wgs * p->Hkv);
+}
+
 int paged_validate(const hw_paged_problem* p) {
     if (p == nullptr) return HW_ERR_NULL;
     if (p->dtype != HW_F32 && p->dtype != HW_F16 && p->dtype != HW_BF16) return HW_ERR_DTYPE;

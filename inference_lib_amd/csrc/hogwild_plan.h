@@ -36,6 +36,19 @@ struct CallPlan {
     size_t workspace_bytes;    // partial_bytes + rope_bytes
 };
 int plan_call(const hw_problem* p, int num_cus, CallPlan* cp, int fused);
+// The other way to deal a call of 128-row workgroups, for row groups that do not fill the CUs evenly (see stream_plan in
+// the source): one workgroup per CU takes an equal run of the sequence (row group 0: tiles 0 .. T-1, row group 1: ...) of
+// its kv head, across row groups.  Piece (workgroup g, row group rg) writes its partial sums into slot g + rg.
+struct StreamPlan {
+    int wgs;                             // workgroups per kv head
+    int slots;                           // partial slots of PLAN_SLOT_ROWS rows per kv head
+    int max_pieces;                      // pieces of one row group, at most
+    int wg_tile_begin[HW_MAX_SPLITS + 1];   // first tile of each workgroup, counted through all row groups
+    size_t partial_bytes;                // part_o + part_ml of all slots
+    size_t workspace_bytes;              // partials, the merge's row table, and CallPlan::rope_bytes
+};
+// false: the call is better served by CallPlan's launch
+bool stream_plan(const hw_problem* p, int num_cus, const CallPlan& cp, StreamPlan* sp);
 int paged_validate(const hw_paged_problem* p);
 int paged_plan(const hw_paged_problem* p, int num_cus, hw_paged_plan* plan);
 

@@ -180,7 +180,9 @@ struct WideRotation {
     }
 };
 
-template <class DT, int E, int EV, int NS, bool PRE, int NW, int PAR>
+// STREAM: the workgroup's run of tiles may cross row groups (KH_STREAM): the whole body is then done once per row group.
+// Prompt chunk of 1024 tokens behind 4096 (40 / 8 heads, D = 128, bf16): PREFILL_FIGURES
+template <class DT, int E, int EV, int NS, bool PRE, int NW, int PAR, bool STREAM>
 __global__ __launch_bounds__(NW * 64, 1) void attention_wide_kernel(const KernelArgs args) {
     typedef Geo<DT, E, EV> G;
     constexpr int NT = NW * 64;                 // threads per workgroup
@@ -252,15 +254,6 @@ __global__ __launch_bounds__(NW * 64, 1) void attention_wide_kernel(const Kernel
     const unsigned long long my_image_ptr = k_wave ? my_k : my_v;   // lane f: this wave's image of fragment f
     const int image_row = k_wave ? G::KROW : G::VROW;               // bytes per token in it
     const unsigned my_image = lds_address(ring) + (k_wave ? 0 : KBYTES) + first * 1024;   // in slot 0
-    WaveState<RB, G::NOC> st;
-#pragma unroll
-    for (int rb = 0; rb < RB; ++rb) {
-        st.m[rb] = NEG_BIG;
-        st.l[rb] = 0.f;
-#pragma unroll
-        for (int c = 0; c < G::NOC; ++c) st.o[rb][c] = f32x4{0.f, 0.f, 0.f, 0.f};
-    }
-    st.fresh = true;
     unsigned voff[G::NOC];                             // this lane's positions in a V image (transposed reads)
     vtr_lane_offsets<G::VROW>(voff, lane);
     asm volatile("s_waitcnt lgkmcnt(0)" : "+s"(hb.lo), "+s"(hb.hi) : : "memory");
@@ -281,21 +274,44 @@ __global__ __launch_bounds__(NW * 64, 1) void attention_wide_kernel(const Kernel
             T1 = __builtin_amdgcn_readlane(my_wt1[i], g & 63);
         }
     }
-    const int r0 = rg * WIDE_ROWS;              // first row of the workgroup
-    const int w0 = r0 + rw * WROWS;             // first row of this wave
     const int GQ = a.Hq / a.Hkv;
-    // (worker, token) pairs the rows of this workgroup belong to
-    const int ws_lo = fast_div(r0, a.magic_gq);
-    const int nws = fast_div(min(r0 + WIDE_ROWS, a.R) - 1, a.magic_gq) - ws_lo + 1;
-    const bool staged = !PRE && nws <= WRot::CSMAX;          // uniform over the workgroup
+    [[maybe_unused]] const int tiles_head = STREAM ? __builtin_amdgcn_readlane(my_te, MAXF - 1) : 0;   // tiles of a row group
+    [[maybe_unused]] const int run_begin = T0, run_end = T1;
+    int rgi = STREAM ? run_begin / tiles_head : rg;
+    int r0, w0;                                 // first row of the workgroup, of this wave
+    int ws_lo, nws;                             // (worker, token) pairs the rows of this workgroup belong to
+    bool staged;                                // their tables go through LDS; uniform over the workgroup
+    unsigned long long todo;                    // fragments with tiles of this workgroup
+    WRot wrot;
+    WaveState<RB, G::NOC> st;
     // The queries to rotate are the same for every fragment: they are requested here, before the workgroup's tile range
     // and first fragment are worked out, and are on their way while that happens.
-    WRot wrot;
-    const bool early_queries = staged;
-    if (early_queries) wrot.load_queries(a, hkv, r0, GQ, tid);
+    auto open_rows = [&]() {
+        if constexpr (STREAM) {
+            T0 = max(run_begin - rgi * tiles_head, 0);
+            T1 = min(run_end - rgi * tiles_head, tiles_head);
+        }
+        r0 = rgi * WIDE_ROWS;
+        w0 = r0 + rw * WROWS;
+        ws_lo = fast_div(r0, a.magic_gq);
+        nws = fast_div(min(r0 + WIDE_ROWS, a.R) - 1, a.magic_gq) - ws_lo + 1;
+        staged = !PRE && nws <= WRot::CSMAX;
+        int tids = tid;
+        if constexpr (STREAM) asm volatile("" : "+v"(tids));      // (see open_segment)
+        if (staged) wrot.load_queries(a, hkv, r0, GQ, tids);
+#pragma unroll
+        for (int rb = 0; rb < RB; ++rb) {
+            st.m[rb] = NEG_BIG;
+            st.l[rb] = 0.f;
+#pragma unroll
+            for (int c = 0; c < G::NOC; ++c) st.o[rb][c] = f32x4{0.f, 0.f, 0.f, 0.f};
+        }
+        st.fresh = true;
+        todo = __ballot(lane < a.F && max(T0, my_tb) < min(T1, my_te));
+    };
+    open_rows();
 
     HW_MARK(10);
-    unsigned long long todo = __ballot(lane < a.F && max(T0, my_tb) < min(T1, my_te));
     int f = 0, L = 0, lt0 = 0, lt1 = 0;
     bool opens_fragment = false;
     u32x4 view = {0, 0, 0, 0};                               // this wave's image of the current fragment (K or V slice)
@@ -345,8 +361,89 @@ __global__ __launch_bounds__(NW * 64, 1) void attention_wide_kernel(const Kernel
         // the bound of row tid / TPR (TPR threads per row, all load: keeps the load unconditional)
         lm = a.loc[(size_t)f * a.W * a.S + fast_div(min(r0 + tids / TPR, a.R - 1), a.magic_gq)];
     };
+    // ---- The PAR waves that share their rows hold a partial sum each: block rb of the rows goes to wave rb % PAR of them
+    // through LDS, lane for lane in the accumulator layout, and is added up there.  Then every wave stores the blocks it
+    // owns.  The accumulator layout scatters a row over the lanes in 16-byte pieces; written like that, a partial (17 MB
+    // per launch at 128 rows x 32 workgroups x 8 heads) would reach memory as a million partial-line writes.  So each
+    // 16-row block goes through LDS once more -- all of this in the ring, which no tile needs any more -- and leaves as
+    // whole rows, 1 KB per store. ----
+    auto store_rows = [&]() {
+        // (STREAM: the lane as the compiler cannot see through it, see open_segment)
+        int lane_ = lane;
+        if constexpr (STREAM) asm volatile("" : "+v"(lane_));
+        const int lane = lane_, n = lane & 15, q = lane >> 4;
+        constexpr int OSTR = EV + 4;                                  // floats per staged row (padded against bank conflicts)
+        constexpr int REGION = 16 * OSTR;                             // floats per wave: a staged 16-row block, or a block in accumulator layout
+        static_assert(G::NOC * 64 * 4 <= REGION && (NW * REGION + NW * 64 * 2) * 4 <= NS * SLOT, "the blocks of all waves fit into the ring");
+        HW_MARK(3);
+        __syncthreads();                                              // every wave has left the last tile
+        HW_MARK(4);
+        float* const regions = reinterpret_cast<float*>(ring);
+        float* const mls = regions + NW * REGION;
+        if constexpr (PAR > 1) {
+#pragma unroll
+            for (int rb = 0; rb < RB; ++rb) {
+                const int owner = rw + (rb % PAR) * NRW;
+                if (owner != wv) {
+#pragma unroll
+                    for (int c = 0; c < G::NOC; ++c) *reinterpret_cast<f32x4*>(regions + owner * REGION + (c * 64 + lane) * 4) = st.o[rb][c];
+                    *reinterpret_cast<f32x2*>(mls + (owner * 64 + lane) * 2) = f32x2{st.m[rb], st.l[rb]};
+                }
+            }
+            __syncthreads();
+        }
+        float* stage = regions + wv * REGION;
+#pragma unroll
+        for (int rb = 0; rb < RB; ++rb) {
+            if (rw + (rb % PAR) * NRW != wv) continue;                // uniform over the wave
+            if constexpr (PAR > 1) {
+                const f32x2 oml = *reinterpret_cast<const f32x2*>(mls + (wv * 64 + lane) * 2);
+                const float mnew = fmaxf(st.m[rb], oml.x);
+                const float mine = exp2f(st.m[rb] - mnew), theirs = exp2f(oml.x - mnew);
+#pragma unroll
+                for (int c = 0; c < G::NOC; ++c) {
+                    const f32x4 o2 = *reinterpret_cast<const f32x4*>(stage + (c * 64 + lane) * 4);
+#pragma unroll
+                    for (int i = 0; i < 4; ++i) st.o[rb][c][i] = st.o[rb][c][i] * mine + o2[i] * theirs;
+                }
+                st.l[rb] = st.l[rb] * mine + oml.y * theirs;
+                st.m[rb] = mnew;
+            }
+            const float lsum = quarter_sum(st.l[rb]);
+            const int row0 = w0 + rb * 16;                            // first row of the block
+            const size_t prow0 = STREAM ? (size_t)(hkv * a.slot_stride + g + rgi) * PLAN_SLOT_ROWS + (row0 - r0) : (size_t)(hkv * a.slot_stride + g) * a.R + row0;
+#pragma unroll
+            for (int c = 0; c < G::NOC; ++c)              // block c, accumulator rows 4q .. 4q+3 = elements 16c + 4q ..
+                *reinterpret_cast<f32x4*>(stage + n * OSTR + 16 * c + 4 * q) = st.o[rb][c];
+            if (q == 0 && row0 + n < a.R) *reinterpret_cast<HW_GLOBAL f32x2*>(a.part_ml + (prow0 + n) * 2) = f32x2{st.m[rb], lsum};
+            // (one wave: the LDS writes above are complete before the reads below are issued, in program order, and
+            // the reads before the next block's writes)
+            const int nvalid = min(16, a.R - row0);                   // rows of the block that exist
+            HW_GLOBAL float* dst = a.part_o + prow0 * EV;
+#pragma unroll
+            for (int ps = 0; ps < 16 * EV / 256; ++ps) {              // 64 lanes x 4 floats per pass
+                const int idx = ps * 256 + lane * 4;
+                const int rr = idx / EV, e = idx % EV;
+                if (rr < nvalid) *reinterpret_cast<HW_GLOBAL f32x4*>(dst + idx) = *reinterpret_cast<const f32x4*>(stage + rr * OSTR + e);
+            }
+        }
+    };
+    // STREAM: for the workgroup that holds the row group's first tile, where the merge finds the partial sums of its rows:
+    // slots g + rgi ... of the workgroups up to the one that holds the row group's last tile
+    [[maybe_unused]] auto write_row_table = [&]() {
+        int begun = 0;                           // workgroups that begin before the row group ends
+#pragma unroll
+        for (int i = 0; i < MAX_SPLITS / 64; ++i)
+            begun += __builtin_popcountll(__ballot(lane + 64 * i < a.wgs_per_head && args.wg_tile[lane + 64 * i] < (rgi + 1) * tiles_head));
+        HW_GLOBAL int* row_tab = reinterpret_cast<HW_GLOBAL int*>(a.part_ml + (size_t)a.Hkv * a.slot_stride * PLAN_SLOT_ROWS * 2) + (size_t)hkv * a.R * 2;
+        if (T0 == 0 && tid < min(WIDE_ROWS, a.R - r0)) {
+            row_tab[2 * (r0 + tid)] = (g + rgi) | ((begun - g) << 16);
+            row_tab[2 * (r0 + tid) + 1] = tid;
+        }
+    };
+
     bool more = todo != 0;
-    if (more) open_segment(early_queries);
+    if (more) open_segment(staged);
     HW_MARK(6);
     bool hw_first = true;
 
@@ -456,85 +553,39 @@ __global__ __launch_bounds__(NW * 64, 1) void attention_wide_kernel(const Kernel
         if (more) {
             __syncthreads();   // every wave is done with the ring
             open_segment(false);
-        }
-    }
-
-    // ---- The PAR waves that share their rows hold a partial sum each: block rb of the rows goes to wave rb % PAR of them
-    // through LDS, lane for lane in the accumulator layout, and is added up there.  Then every wave stores the blocks it
-    // owns.  The accumulator layout scatters a row over the lanes in 16-byte pieces; written like that, a partial (17 MB
-    // per launch at 128 rows x 32 workgroups x 8 heads) would reach memory as a million partial-line writes.  So each
-    // 16-row block goes through LDS once more -- all of this in the ring, which no tile needs any more -- and leaves as
-    // whole rows, 1 KB per store. ----
-    {
-        constexpr int OSTR = EV + 4;                                  // floats per staged row (padded against bank conflicts)
-        constexpr int REGION = 16 * OSTR;                             // floats per wave: a staged 16-row block, or a block in accumulator layout
-        static_assert(G::NOC * 64 * 4 <= REGION && (NW * REGION + NW * 64 * 2) * 4 <= NS * SLOT, "the blocks of all waves fit into the ring");
-        HW_MARK(3);
-        __syncthreads();                                              // every wave has left the last tile
-        HW_MARK(4);
-        float* const regions = reinterpret_cast<float*>(ring);
-        float* const mls = regions + NW * REGION;
-        if constexpr (PAR > 1) {
-#pragma unroll
-            for (int rb = 0; rb < RB; ++rb) {
-                const int owner = rw + (rb % PAR) * NRW;
-                if (owner != wv) {
-#pragma unroll
-                    for (int c = 0; c < G::NOC; ++c) *reinterpret_cast<f32x4*>(regions + owner * REGION + (c * 64 + lane) * 4) = st.o[rb][c];
-                    *reinterpret_cast<f32x2*>(mls + (owner * 64 + lane) * 2) = f32x2{st.m[rb], st.l[rb]};
-                }
-            }
-            __syncthreads();
-        }
-        float* stage = regions + wv * REGION;
-#pragma unroll
-        for (int rb = 0; rb < RB; ++rb) {
-            if (rw + (rb % PAR) * NRW != wv) continue;                // uniform over the wave
-            if constexpr (PAR > 1) {
-                const f32x2 oml = *reinterpret_cast<const f32x2*>(mls + (wv * 64 + lane) * 2);
-                const float mnew = fmaxf(st.m[rb], oml.x);
-                const float mine = exp2f(st.m[rb] - mnew), theirs = exp2f(oml.x - mnew);
-#pragma unroll
-                for (int c = 0; c < G::NOC; ++c) {
-                    const f32x4 o2 = *reinterpret_cast<const f32x4*>(stage + (c * 64 + lane) * 4);
-#pragma unroll
-                    for (int i = 0; i < 4; ++i) st.o[rb][c][i] = st.o[rb][c][i] * mine + o2[i] * theirs;
-                }
-                st.l[rb] = st.l[rb] * mine + oml.y * theirs;
-                st.m[rb] = mnew;
-            }
-            const float lsum = quarter_sum(st.l[rb]);
-            const int row0 = w0 + rb * 16;                            // first row of the block
-            const size_t prow0 = (size_t)(hkv * a.slot_stride + g) * a.R + row0;
-#pragma unroll
-            for (int c = 0; c < G::NOC; ++c)              // block c, accumulator rows 4q .. 4q+3 = elements 16c + 4q ..
-                *reinterpret_cast<f32x4*>(stage + n * OSTR + 16 * c + 4 * q) = st.o[rb][c];
-            if (q == 0 && row0 + n < a.R) *reinterpret_cast<HW_GLOBAL f32x2*>(a.part_ml + (prow0 + n) * 2) = f32x2{st.m[rb], lsum};
-            // (one wave: the LDS writes above are complete before the reads below are issued, in program order, and
-            // the reads before the next block's writes)
-            const int nvalid = min(16, a.R - row0);                   // rows of the block that exist
-            HW_GLOBAL float* dst = a.part_o + prow0 * EV;
-#pragma unroll
-            for (int ps = 0; ps < 16 * EV / 256; ++ps) {              // 64 lanes x 4 floats per pass
-                const int idx = ps * 256 + lane * 4;
-                const int rr = idx / EV, e = idx % EV;
-                if (rr < nvalid) *reinterpret_cast<HW_GLOBAL f32x4*>(dst + idx) = *reinterpret_cast<const f32x4*>(stage + rr * OSTR + e);
+        } else if constexpr (STREAM) {
+            store_rows();
+            write_row_table();
+            ++rgi;
+            if (rgi * tiles_head < run_end) {          // the run goes on in the next row group
+                __syncthreads();                       // every wave is done with the ring
+                open_rows();
+                open_segment(staged);
+                more = true;
             }
         }
     }
 
+    if constexpr (!STREAM) store_rows();
     HW_MARK(5);
 
-    // rotated queries of zero-length fragments are still part of the operator's visible output
-    if (!PRE && a.rq != nullptr && g == 0) {
-        unsigned long long empty = __ballot(lane < a.F && my_len == 0);
-        while (empty != 0) {
+    // rotated queries of zero-length fragments are still part of the operator's visible output: for the workgroup that holds
+    // the first tile of a row group (one loop over fragments and row groups)
+    if (!PRE && a.rq != nullptr && (STREAM || g == 0)) {
+        const unsigned long long all_empty = __ballot(lane < a.F && my_len == 0);
+        unsigned long long empty = all_empty;
+        if constexpr (STREAM) rgi = (run_begin + tiles_head - 1) / tiles_head;
+        while (empty != 0 && (!STREAM || rgi * tiles_head < run_end)) {
             f = __builtin_ctzll(empty);
             empty &= empty - 1;
             __syncthreads();
             QueryRotation<DT, E, WIDE_ROWS, G::QSTR, PRE, NT> qempty;
-            qempty.load(a, f, hkv, r0, GQ, tid);
-            qempty.finish(a, q_lds, f, hkv, r0, GQ, true, tid);
+            qempty.load(a, f, hkv, rgi * WIDE_ROWS, GQ, tid);
+            qempty.finish(a, q_lds, f, hkv, rgi * WIDE_ROWS, GQ, true, tid);
+            if (STREAM && empty == 0) {
+                empty = all_empty;
+                ++rgi;
+            }
         }
     }
 }
@@ -1149,13 +1200,21 @@ static hipError_t launch_wide_dt(const KernelArgs& ka, int E, hipStream_t stream
     constexpr int NW = WIDE_WAVES;
     constexpr int PAR = WIDE_PAR;
     if (E != 64 && E != 128) return hipErrorInvalidValue;
-    if (ka.h.flags & KH_PREROTATED) {
-        if (E == 128) hipLaunchKernelGGL((attention_wide_kernel<DT, 128, 128, NS, true, NW, PAR>), dim3(ka.h.nwg), dim3(NW * 64), 0, stream, ka);
-        else hipLaunchKernelGGL((attention_wide_kernel<DT, 64, 64, NS, true, NW, PAR>), dim3(ka.h.nwg), dim3(NW * 64), 0, stream, ka);
-    } else {
-        if (E == 128) hipLaunchKernelGGL((attention_wide_kernel<DT, 128, 128, NS, false, NW, PAR>), dim3(ka.h.nwg), dim3(NW * 64), 0, stream, ka);
-        else hipLaunchKernelGGL((attention_wide_kernel<DT, 64, 64, NS, false, NW, PAR>), dim3(ka.h.nwg), dim3(NW * 64), 0, stream, ka);
-    }
+    auto go = [&](auto head_dim, auto pre, auto stream_runs) {
+        constexpr int HD = decltype(head_dim)::value;
+        hipLaunchKernelGGL((attention_wide_kernel<DT, HD, HD, NS, decltype(pre)::value, NW, PAR, decltype(stream_runs)::value>), dim3(ka.h.nwg),
+                           dim3(NW * 64), 0, stream, ka);
+    };
+    auto by_entry = [&](auto head_dim, auto stream_runs) {
+        if (ka.h.flags & KH_PREROTATED) go(head_dim, std::true_type{}, stream_runs);
+        else go(head_dim, std::false_type{}, stream_runs);
+    };
+    auto by_runs = [&](auto head_dim) {
+        if (ka.h.flags & KH_STREAM) by_entry(head_dim, std::true_type{});
+        else by_entry(head_dim, std::false_type{});
+    };
+    if (E == 128) by_runs(std::integral_constant<int, 128>{});
+    else by_runs(std::integral_constant<int, 64>{});
     return hipGetLastError();
 }
 
