@@ -29,6 +29,7 @@ if HAVE_TORCH_OPS:
     _rope_append = torch.ops.libhogatt.rope_append.default
     _segment_views = torch.ops.libhogatt.segment_views.default
 
+
 class _LayerViews:
     """`segment.key_cache[layer]` -> the [1, Hkv, L, D] view of what has been written so far."""
 
@@ -40,6 +41,18 @@ class _LayerViews:
 
     def __len__(self) -> int:
         return len(self._bufs)
+
+
+def _fragments(keys: list, values: list, layer: int):
+    """keys[f][layer], values[f][layer] of the segments' key_cache / value_cache.  Where all of them are SegmentCache's own the
+    views are made in one native call; a segment of another kind, or one whose members were replaced, is asked for its tensors."""
+    caches = keys + values
+    if HAVE_TORCH_OPS and caches and all(type(c) is _LayerViews for c in caches):
+        bufs = [c._bufs[layer] for c in caches]
+        if bufs[0].is_cuda:
+            views = _segment_views(bufs, [c._seg.lengths[layer] for c in caches])
+            return views[: len(keys)], views[len(keys):]
+    return [c[layer] for c in keys], [c[layer] for c in values]
 
 
 class SegmentCache:
@@ -282,14 +295,7 @@ class HogwildCache:
             self.segments = segments
             self.frags = torch.tensor([cs.get_seq_length(layer_idx) for cs in segments], dtype=torch.int32, device=key_states.device)
         # views; no .contiguous() copies (attention.py:160-162,199-203)
-        keys, vals = [cs.k[layer_idx] for cs in self.segments], [cs.v[layer_idx] for cs in self.segments]
-        lens = [cs.lengths[layer_idx] for cs in self.segments]
-        if HAVE_TORCH_OPS and keys[0].is_cuda:
-            both = _segment_views(keys + vals, lens + lens)
-            keys, vals = both[: len(lens)], both[len(lens):]
-        else:
-            keys = [b[:, :n, :].unsqueeze(0) for b, n in zip(keys, lens)]
-            vals = [b[:, :n, :].unsqueeze(0) for b, n in zip(vals, lens)]
+        keys, vals = _fragments([cs.key_cache for cs in self.segments], [cs.value_cache for cs in self.segments], layer_idx)
         return CacheStructure(keys=keys, values=vals, cos=self.cosines, sin=self.sines, loc=self.locations, frags=self.frags)
 
     def update(self, key_states: torch.Tensor, value_states: torch.Tensor, layer_idx: int,
