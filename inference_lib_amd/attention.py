@@ -9,7 +9,7 @@ C entry points are called through ctypes.
 from __future__ import annotations
 
 import os
-from typing import List, Optional
+from typing import Iterable, List, Optional
 
 import torch
 
@@ -57,11 +57,12 @@ def hogwild_fused(queries: torch.Tensor, locations: torch.Tensor, keys: List[tor
     return out
 
 
-def _in_place_or_contiguous(keys: List[torch.Tensor], values: List[torch.Tensor]):
-    if len(keys) == len(values) and all(k.is_contiguous() and v.is_contiguous() for k, v in zip(keys, values)):
-        return keys, values
+def _in_place_or_contiguous(keys: Iterable[torch.Tensor], values: Iterable[torch.Tensor]):
+    pairs = list(zip(keys, values))
+    if all(k.is_contiguous() and v.is_contiguous() for k, v in pairs):
+        return [k for k, _ in pairs], [v for _, v in pairs]
     ks, vs = [], []
-    for k, v in zip(keys, values):
+    for k, v in pairs:
         k3, v3 = (k[0] if k.dim() == 4 else k), (v[0] if v.dim() == 4 else v)
         if k3.dim() == 3 and v3.dim() == 3 and _lib.fragment_capacity(k3, v3) is not None:
             ks.append(k)
