@@ -448,7 +448,8 @@ bool merge_segments(at::TensorList k_dst, at::TensorList v_dst, at::IntArrayRef 
 }
 
 // hw_rope_append on tensors: the append of HogwildCache, whose argument checks and pointer tables took most of a step's host
-// time in Python (12 layers, two workers, three segments: 694 -> 364 us a step with this, segment_views and fragment_dims).  Returns false, with nothing queued, for anything the checks below do not take: the caller's general path then
+// time in Python (12 layers, two workers, three segments: 694 -> 364 us a step with this, segment_views and fragment_dims).
+// Returns false, with nothing queued, for anything the checks below or the library do not take: the caller's general path then
 // handles it or names what is wrong.
 bool rope_append(at::TensorList k_dst, at::TensorList v_dst, at::IntArrayRef dst_len, at::IntArrayRef n_new, const at::Tensor& key_states,
                  const at::Tensor& value_states, const std::optional<at::Tensor>& cosines, const std::optional<at::Tensor>& sines, int64_t mode) {
@@ -500,7 +501,9 @@ bool rope_append(at::TensorList k_dst, at::TensorList v_dst, at::IntArrayRef dst
     a.k_dst = kd.data(); a.v_dst = vd.data();
     a.dst_len = len.data(); a.dst_cap = cap.data(); a.n_new = nn.data();
     c10::hip::HIPGuardMasqueradingAsCUDA guard(ks.device());
-    check_status(hw_rope_append(&a, c10::hip::getCurrentHIPStreamMasqueradingAsCUDA(ks.device().index()).stream()), "rope_append");
+    const int status = hw_rope_append(&a, c10::hip::getCurrentHIPStreamMasqueradingAsCUDA(ks.device().index()).stream());
+    if (status < 0) return false;          // refused by the library, before anything was queued
+    check_status(status, "rope_append");
     return true;
 }
 

@@ -56,6 +56,22 @@ def test_append_operator_declines_what_does_not_fit():
         _lib.rope_append(k, k, [buf], [buf.clone()], [2], n_new=[4])
 
 
+@pytest.mark.parametrize("what", ["wide_tables", "odd_tables", "mode"])
+def test_refusals_of_the_library_reach_the_caller_as_hogwild_error(what):
+    """What hw_rope_append refuses is declined by the operator too, so that the general path names it, status included."""
+    from inference_lib_amd import cache
+    rot = {"wide_tables": 66, "odd_tables": 33, "mode": 64}[what]
+    mode = 7 if what == "mode" else _lib.HW_ROPE_EAGER
+    k = torch.randn((1, 2, 1, 64), device="cuda", dtype=torch.float16)
+    cos = torch.ones((1, 1, rot), device="cuda", dtype=torch.float16)
+    seg = cache.SegmentCache(1, 2, 64, 8, dtype=torch.float16)
+    c = cache.HogwildCache([[seg]], inv_freq=torch.ones(32, device="cuda"))
+    with pytest.raises(_lib.HogwildError) as e:
+        c.update_fused(k, k, cos, cos, 0, mode=mode)
+    assert e.value.status == -3 and seg.lengths == [0]
+    assert not torch.ops.libhogatt.rope_append(seg.k, seg.v, [0], [1], k, k, cos, cos, mode)
+
+
 @pytest.mark.parametrize("n", [0, 1, 7])
 def test_segment_views_are_slices(n):
     buf = torch.randn((3, 7, 64), device="cuda")
