@@ -355,18 +355,18 @@ def merge_caches(target: SegmentCache, source: SegmentCache, model=None, *, inv_
     dev = source.k[0].device
     tdt = table_dtype if table_dtype is not None else source.k[0].dtype
     position = target.get_seq_length()
-    if HAVE_TORCH_OPS and dev.type == "cuda" and source.k and len(source.k) >= len(target.k) and len(source.v) >= len(target.v):
+    if HAVE_TORCH_OPS and dev.type == "cuda" and len(source.k) >= len(target.k) and len(source.v) >= len(target.v):
         layers = range(len(target.k))
         for layer in layers:          # grow like every other append (the reference's merge goes through target.update)
             if target.lengths[layer] + source.lengths[layer] > target.k[layer].size(1):
                 target.reserve(layer, source.lengths[layer])
-        added = source.lengths[: len(target.k)]
-        if torch.ops.libhogatt.merge_segments(target.k, target.v, target.lengths, source.k[: len(target.k)], source.v[: len(target.k)], added,
-                                              inv_freq.to(dev), attention_scaling, position, tdt, mode):
+        k_dst, v_dst, k_src, v_src, at, added = ([of[layer] for layer in layers] for of in (target.k, target.v, source.k, source.v,
+                                                                                          target.lengths, source.lengths))
+        if torch.ops.libhogatt.merge_segments(k_dst, v_dst, at, k_src, v_src, added, inv_freq.to(dev), attention_scaling, position, tdt, mode):
             for layer in layers:
                 target.lengths[layer] += added[layer]
             return
-    # buffers of several forms, or not packed: layer by layer
+    # buffers of several forms, not packed, or beyond the limits of one launch: layer by layer
     # one table row: the position is target's length for every source token (S = 1 and pos_end = length + 1)
     _, cos, sin = _lib.build_inputs([[position + 1]], 1, inv_freq.to(dev), attention_scaling=attention_scaling,
                                     table_dtype=None if tdt == torch.float32 else tdt)

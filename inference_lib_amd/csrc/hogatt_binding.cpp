@@ -398,7 +398,8 @@ void copy_to_blocks(const at::Tensor& key_states, const at::Tensor& value_states
 // ---- segments ----------------------------------------------------------------------------------------------------
 
 // hw_merge_segments on lists of per-layer buffers [Hkv, cap, E|Ev] (all layers of one form, packed).  Returns false, with
-// nothing queued, for buffers that are not of that form: the caller then goes layer by layer.
+// nothing queued, for buffers that are not of that form and for what the library refuses (one launch has limits that an append
+// does not have): the caller then goes layer by layer.
 bool merge_segments(at::TensorList k_dst, at::TensorList v_dst, at::IntArrayRef dst_len, at::TensorList k_src, at::TensorList v_src, at::IntArrayRef n,
                     const at::Tensor& inv_freq, double scaling, int64_t position, at::ScalarType table_dtype, int64_t mode) {
     const size_t L = k_dst.size();
@@ -443,7 +444,9 @@ bool merge_segments(at::TensorList k_dst, at::TensorList v_dst, at::IntArrayRef 
     a.k_src = ks.data(); a.v_src = vs.data(); a.src_cap = scap.data(); a.n = nn.data();
     a.k_dst = kd.data(); a.v_dst = vd.data(); a.dst_cap = dcap.data(); a.dst_len = dl.data();
     c10::hip::HIPGuardMasqueradingAsCUDA guard(kd0.device());
-    check_status(hw_merge_segments(&a, c10::hip::getCurrentHIPStreamMasqueradingAsCUDA(kd0.device().index()).stream()), "merge_segments");
+    const int status = hw_merge_segments(&a, c10::hip::getCurrentHIPStreamMasqueradingAsCUDA(kd0.device().index()).stream());
+    if (status < 0) return false;          // refused by the library, before anything was queued
+    check_status(status, "merge_segments");
     return true;
 }
 

@@ -81,3 +81,38 @@ def test_layers_of_several_forms_and_a_segment_merged_into_itself():
         for i in range(len(a.k)):
             assert torch.equal(a.k[i][:, : a.lengths[i]], b.k[i][:, : b.lengths[i]])
             assert torch.equal(a.v[i][:, : a.lengths[i]], b.v[i][:, : b.lengths[i]])
+
+
+@pytest.mark.parametrize("Hkv,E,Ev,rot", [(1, 8224, 8, 8200), (65537, 2, 1, 2)])
+def test_what_one_launch_does_not_take_goes_layer_by_layer(Hkv, E, Ev, rot):
+    """A table row that does not fit the LDS, more kv heads than a grid dimension."""
+    from inference_lib_amd import cache
+    inv = (10000.0 ** (-torch.arange(rot // 2, dtype=torch.float64) / (rot // 2))).to(torch.float32).to(DEV)
+    got, want = (segment(2, Hkv, E, Ev, 8, (3, 1), torch.bfloat16, 5) for _ in range(2))
+    source = segment(2, Hkv, E, Ev, 4, (2, 4), torch.bfloat16, 6)
+    cache.merge_caches(got, source, inv_freq=inv)
+    layer_by_layer(want, source, inv, 1.0, torch.bfloat16, 0)
+    assert got.lengths == want.lengths == [5, 5]
+    for i in range(2):
+        assert torch.equal(got.k[i], want.k[i]) and torch.equal(got.v[i], want.v[i])
+
+
+def test_an_unknown_mode_is_refused_as_hogwild_error():
+    from inference_lib_amd import _lib, cache
+    target, source = (segment(2, 2, 64, 64, 8, (2, 2), torch.bfloat16, s) for s in (1, 2))
+    before = [t.clone() for t in target.k + target.v]
+    with pytest.raises(_lib.HogwildError) as e:
+        cache.merge_caches(target, source, inv_freq=torch.ones(32, device=DEV), mode=7)
+    assert e.value.status == -3 and target.lengths == [2, 2] and all(torch.equal(a, b) for a, b in zip(before, target.k + target.v))
+
+
+def test_layers_in_one_tensor():
+    """Anything that yields a layer's buffer by index holds the layers of a segment."""
+    from inference_lib_amd import cache
+    inv = (10000.0 ** (-torch.arange(32, dtype=torch.float64) / 32)).to(torch.float32).to(DEV)
+    got, want = (segment(2, 2, 64, 64, 40, (3, 3), torch.bfloat16, 5) for _ in range(2))
+    source = segment(2, 2, 64, 64, 16, (16, 16), torch.bfloat16, 6)
+    layer_by_layer(want, source, inv, 1.0, torch.bfloat16, 0)
+    source.k, source.v = torch.stack(source.k), torch.stack(source.v)
+    cache.merge_caches(got, source, inv_freq=inv)
+    assert all(torch.equal(a, b) for a, b in zip(got.k + got.v, want.k + want.v))
