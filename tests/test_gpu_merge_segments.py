@@ -4,6 +4,8 @@ same order, so keys and values must be equal bit for bit."""
 import pytest
 import torch
 
+from inference_lib_amd import attention  # noqa: F401  (loads the operators)
+
 pytestmark = pytest.mark.gpu
 
 DEV = "cuda:0"
@@ -34,11 +36,23 @@ def layer_by_layer(target, source, inv, scaling, tdt, mode):
         target.lengths[layer] += m
 
 
+@pytest.fixture
+def taken(monkeypatch):
+    """What the one-launch operator answers: merge_caches falls back silently when it declines."""
+    op, answers = torch.ops.libhogatt.merge_segments, []
+
+    def record(*args):
+        answers.append(op(*args))
+        return answers[-1]
+    monkeypatch.setattr(torch.ops.libhogatt, "merge_segments", record)
+    return answers
+
+
 @pytest.mark.parametrize("dtype,E,Ev,rot,table,mode", [
     ("bf16", 128, 128, 128, None, 0), ("bf16", 128, 128, 128, "f32", 0), ("f16", 64, 64, 64, None, 1), ("f32", 64, 64, 64, None, 0),
     ("bf16", 256, 256, 256, None, 1), ("f16", 128, 64, 96, None, 0), ("bf16", 80, 72, 36, None, 0), ("f32", 7, 5, 6, None, 1),
     ("bf16", 33, 33, 0, None, 0)])
-def test_all_layers_at_once_equal_layer_by_layer(dtype, E, Ev, rot, table, mode):
+def test_all_layers_at_once_equal_layer_by_layer(taken, dtype, E, Ev, rot, table, mode):
     """Layers of different length (0, 1, the edges of a 64-row block, many blocks), more layers than one launch takes, a
     target that has to grow in some layers; chunked and element-wise forms, partial rotary widths."""
     from inference_lib_amd import cache
@@ -52,14 +66,15 @@ def test_all_layers_at_once_equal_layer_by_layer(dtype, E, Ev, rot, table, mode)
     cache.merge_caches(got, source, inv_freq=inv, attention_scaling=1.25, table_dtype=None if table is None else TDT[table], mode=mode)
     layer_by_layer(want, source, inv, 1.25, tdt if table is None else TDT[table], mode)
     torch.cuda.synchronize()
+    assert taken == [True]
     assert got.lengths == want.lengths == [a + b for a, b in zip(dst_lens, src_lens)]
     for i in range(layers):
-        n = got.lengths[i]
+        n = got.lengths[i] if got.k[i].size(1) != 256 else 256        # rows behind the appended ones keep what they held
         assert got.k[i].shape == want.k[i].shape
         assert torch.equal(got.k[i][:, :n], want.k[i][:, :n]) and torch.equal(got.v[i][:, :n], want.v[i][:, :n]), i
 
 
-def test_layers_of_several_forms_and_a_segment_merged_into_itself():
+def test_layers_of_several_forms_and_a_segment_merged_into_itself(taken):
     """Buffers that are not all of one form go layer by layer; a segment may be appended to itself."""
     from inference_lib_amd import cache
     inv = (10000.0 ** (-torch.arange(32, dtype=torch.float64) / 32)).to(torch.float32).to(DEV)
@@ -76,6 +91,7 @@ def test_layers_of_several_forms_and_a_segment_merged_into_itself():
     cache.merge_caches(one, one, inv_freq=inv)
     layer_by_layer(two, two, inv, 1.0, torch.float16, 0)
     torch.cuda.synchronize()
+    assert taken == [False, True]
     for a, b in ((segs[0][0], segs[1][0]), (one, two)):
         assert a.lengths == b.lengths
         for i in range(len(a.k)):
@@ -84,7 +100,7 @@ def test_layers_of_several_forms_and_a_segment_merged_into_itself():
 
 
 @pytest.mark.parametrize("Hkv,E,Ev,rot", [(1, 8224, 8, 8200), (65537, 2, 1, 2)])
-def test_what_one_launch_does_not_take_goes_layer_by_layer(Hkv, E, Ev, rot):
+def test_what_one_launch_does_not_take_goes_layer_by_layer(taken, Hkv, E, Ev, rot):
     """A table row that does not fit the LDS, more kv heads than a grid dimension."""
     from inference_lib_amd import cache
     inv = (10000.0 ** (-torch.arange(rot // 2, dtype=torch.float64) / (rot // 2))).to(torch.float32).to(DEV)
@@ -92,7 +108,7 @@ def test_what_one_launch_does_not_take_goes_layer_by_layer(Hkv, E, Ev, rot):
     source = segment(2, Hkv, E, Ev, 4, (2, 4), torch.bfloat16, 6)
     cache.merge_caches(got, source, inv_freq=inv)
     layer_by_layer(want, source, inv, 1.0, torch.bfloat16, 0)
-    assert got.lengths == want.lengths == [5, 5]
+    assert taken == [False] and got.lengths == want.lengths == [5, 5]
     for i in range(2):
         assert torch.equal(got.k[i], want.k[i]) and torch.equal(got.v[i], want.v[i])
 
