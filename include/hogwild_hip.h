@@ -124,7 +124,11 @@ typedef struct hw_problem {
     int32_t variant;
 } hw_problem;
 
-/* How a problem is cut into workgroups; filled by hw_plan_debug (host only, no device needed). */
+/* How a problem is cut into workgroups; filled by hw_plan_debug (host only, no device needed).  This is the launch of every
+ * call but one kind: with row_blocks = 8, splits = 0 and several row groups that would leave much of the chip idle,
+ * hw_fused_attention and hw_sdpa deal equal runs of tiles across the row groups instead (one workgroup per CU, more workspace)
+ * if the workspace is as large as hw_workspace_bytes / hw_sdpa_workspace_bytes say.  In a workspace of hw_plan.workspace_bytes
+ * such a call runs as described here, somewhat slower. */
 typedef struct hw_plan {
     int32_t rows;             /* W*S*(Hq/Hkv): query rows that share one kv head */
     int32_t row_blocks;       /* 16-row MFMA blocks per workgroup (1, 2 or 8) */
@@ -150,7 +154,8 @@ int hw_validate(const hw_problem* p, int fused);
 int hw_plan_debug(const hw_problem* p, int num_cus, hw_plan* plan);
 
 /* Workspace size for the current device: what hw_fused_attention needs for this problem (if the rotary width is not
-   the head dimension and p->rq is NULL, that includes room for the rotated queries); enough for hw_sdpa as well. */
+   the head dimension and p->rq is NULL, that includes room for the rotated queries); enough for hw_sdpa as well.  For a call
+   that is dealt in runs across row groups (see hw_plan) this is what the runs need, up to a few times hw_plan.workspace_bytes. */
 int hw_workspace_bytes(const hw_problem* p, size_t* bytes);
 /* The same for hw_sdpa alone (pre-rotated queries: RotE, cosines, sines and rq are ignored). */
 int hw_sdpa_workspace_bytes(const hw_problem* p, size_t* bytes);
@@ -163,20 +168,25 @@ int hw_fused_attention(const hw_problem* p, void* stream);
  * loops, harnesses that forbid hipMalloc).  No counterpart in the reference.  Same inputs, outputs and kernels as
  * hw_fused_attention, except that p->workspace / p->workspace_bytes are ignored: the split-K partials go to a
  * device array that is part of the library image (HW_STATIC_SCRATCH_BYTES per GPU, resident until the process ends).
- * The call allocates and frees nothing.  A problem whose hw_workspace_bytes() exceeds HW_STATIC_SCRATCH_BYTES is
- * refused with HW_ERR_STATIC_SCRATCH before anything is queued -- except that with row_blocks = 0 a plan of 128-row
- * workgroups that does not fit is replaced by the 32-row kernel's (fewer partials), and only that one has to fit.  All calls on one GPU share that GPU's array: calls
- * that overlap in time on one GPU (different streams, or graphs replayed concurrently) race on the partials and
- * must be serialised by the caller.  Nothing in the array has to survive between calls or start at zero.
+ * The call allocates and frees nothing.  A problem whose launch as hw_plan describes it needs more than
+ * HW_STATIC_SCRATCH_BYTES is refused with HW_ERR_STATIC_SCRATCH before anything is queued -- except that with row_blocks = 0
+ * a plan of 128-row workgroups that does not fit is replaced by the 32-row kernel's (fewer partials), and only that one has
+ * to fit.  (Runs across row groups, see hw_plan, are used only where they fit as well: the larger hw_workspace_bytes() of
+ * such a call is no reason for a refusal.)  All calls on one GPU share that GPU's array: calls that overlap in time on
+ * one GPU (different streams, or graphs replayed concurrently) race on the partials and must be serialised by the caller.
+ * Nothing in the array has to survive between calls or start at zero.
  */
 #define HW_STATIC_SCRATCH_BYTES (8u << 20)
 int hw_fused_attention_static(const hw_problem* p, void* stream);
 
 /* The two kernels of hw_fused_attention separately.  HW_STAGE_ATTENTION leaves the split-K partials of this
-   device's KV in the workspace (per kv head and workgroup: unnormalised output rows, running max in base-2 units
-   and sum); HW_STAGE_MERGE combines the partials found there into out / lse.  For a caller that holds only part of
-   the fragments and exchanges partials before merging, and for timing the attention kernel alone.  The reference
-   has the same split internally (kernel + reduce kernel, src/kernels/kernel_v21.cuh:985-989). */
+   device's KV in the workspace (per kv head and workgroup of hw_plan: unnormalised output rows fp32
+   [Hkv][wgs_per_head][rows][Ev], then running max in base-2 units and sum [Hkv][wgs_per_head][rows][2]; a call of more than
+   HW_MAX_LAUNCH_FRAGMENTS fragments has the workgroups of its groups side by side); HW_STAGE_MERGE combines the partials
+   found there into out / lse.  A call with one stage always uses the launch of hw_plan, also where hw_fused_attention deals
+   runs across row groups.  For a caller that holds only part of the fragments and exchanges partials before merging, and
+   for timing the attention kernel alone.  The reference has the same split internally (kernel + reduce kernel,
+   src/kernels/kernel_v21.cuh:985-989). */
 #define HW_STAGE_ATTENTION 1
 #define HW_STAGE_MERGE 2
 int hw_fused_attention_stages(const hw_problem* p, void* stream, int stages);

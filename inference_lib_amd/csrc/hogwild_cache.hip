@@ -182,7 +182,7 @@ __global__ __launch_bounds__(256) void rope_append_kernel(const AppendArgs a) {
 
 // merge_caches for all layers at once: layer l's n source rows per kv head go behind the first dst_len rows of its target,
 // the keys rotated by the angles of ONE position (the target's length), the values as they are.  grid = (row blocks, kv
-// head, layer).  Bound by memory: every byte is read and written once, with four to eight 16-byte loads of a thread in
+// head, layer).  Bound by memory: every byte is read and written once, with four 16-byte loads of a thread in
 // flight, and the one cos / sin row is worked out by every workgroup for itself (RotE / 2 angles, into LDS) instead of by
 // three launches in front.  One launch per layer left the chip idle between launches of 5.5 us that a host call of 23 us
 // each could not keep fed: 16 layers x 2 segments of 1000 and 777 tokens (8 kv heads, D = 128, bf16; 233 MB) 757 -> 51 us

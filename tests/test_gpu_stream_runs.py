@@ -128,3 +128,28 @@ def test_partial_rotary_width_with_the_rotated_queries_in_the_workspace(W, S, Hq
         pr.run()
         assert bool(((out.double() - ref).abs() <= bound).all()) and float((lse.double() - ref_lse).abs().max()) <= 1e-4
         assert bool((guard[bytes_:] == 165).all())
+
+
+def test_the_attention_stage_alone_leaves_the_documented_partials():
+    """hw_fused_attention_stages: a caller that reads or exchanges the partials finds [Hkv][workgroup][row][Ev] and behind it
+    [Hkv][workgroup][row][2] (maximum in base-2 units, sum) with the workgroups of hw_plan_debug, also for a call that
+    hw_fused_attention deals in runs."""
+    W, S, Hq, Hkv, D, lens, dtype = CASES[3]
+    scale = D ** -0.5
+    q, loc, cos, sin, keys, values = _inputs(W, S, Hq, Hkv, D, lens, dtype, D)
+    out = torch.empty_like(q)
+    pr = _lib.Problem(q=q, locations=loc, keys=keys, values=values, scale=scale, out=out, cosines=cos, sines=sin)
+    plan = _rounds_plan(pr)
+    ws = torch.zeros(pr.workspace_bytes(), dtype=torch.uint8, device="cuda")
+    pr.set_workspace(ws)
+    pr.run(stages=1)
+    n = Hkv * plan.wgs_per_head * plan.rows
+    part = ws.view(torch.float32)[: n * (D + 2)].double()
+    o, ml = part[: n * D].view(Hkv, plan.wgs_per_head, plan.rows, D), part[n * D:].view(Hkv, plan.wgs_per_head, plan.rows, 2)
+    weight = torch.exp2(ml[..., 0] - ml[..., 0].amax(dim=1, keepdim=True))
+    got = (o * weight[..., None]).sum(1) / (ml[..., 1] * weight).sum(1)[..., None]            # [Hkv][(worker, token, head of group)]
+    got = got.view(Hkv, W, S, Hq // Hkv, D).permute(1, 0, 3, 2, 4).reshape(W, Hq, S, D)
+    ref, _, bound = _reference(ops.hogwild_rope(q, cos, sin), loc, keys, values, scale, Hkv)
+    assert bool(((got - ref).abs() <= bound).all())
+    pr.run(stages=2)
+    assert bool(((out.double() - ref).abs() <= bound).all())
