@@ -216,15 +216,21 @@ int plan_call(const hw_problem* p, int num_cus, CallPlan* cp, int fused) {
 // Row groups of 128 rows that do not fill the CUs evenly: 40 row groups of 8 kv heads (1024 prompt tokens at a GQA ratio of
 // 5) are 320 workgroups, so 256 CUs take two rounds of which the second is a quarter full.  Cut into equal runs across the
 // row groups every CU gets 1.25 row groups of work instead of 2.  A run that crosses into the next row group opens it anew
-// (queries, partial sums: about kJobCost tiles), so the runs are taken only where the count below promises a tenth.  Two
-// layers of that chunk behind 4096 tokens take 276 us in runs and 342 us in rounds, merge launches included.  (Runs dealt by
-// the kernel over the tiles that the locations leave visible were measured at 300 us: a row group's unseen tiles cost next
-// to nothing as it is, and the uneven row groups give some runs a third one to open.)
+// (queries, partial sums), so the runs are dealt by tiles plus openings at kJobCost and kOpenCost tiles.  (Runs dealt by
+// the kernel over the tiles that the locations leave visible were measured slower, 300 against 276 us for two layers of 1024
+// tokens behind 4096: a row group's unseen tiles cost next to nothing as it is, and the uneven row groups give some runs a
+// third one to open.)
+// Where to take them: a price of each launch in tiles, rounds against runs, with kJobPrice and kOpenPrice per opening.  The
+// prices and the line at kWorth were fitted to 1626 calls timed both ways, merge launches included (24 to 1500 new tokens of
+// 1 to 8 workers behind 0 to 16 K, eight head layouts, D = 64 and 128): the 1305 that the rule takes gain 0.994 to 1.66,
+// 1.21 in the median (1024 tokens behind 4096 at 40/8 heads, D = 128: 180 -> 138 us a layer); the 321 that it leaves in rounds
+// would give 0.88 to 1.17, 1.03 in the median (133 tokens of two workers behind 761: 28 -> 32 us).
 bool stream_plan(const hw_problem* p, int num_cus, const CallPlan& cp, StreamPlan* sp) {
     const hw_plan& plan = cp.plan[0];
     if (cp.groups != 1 || p->splits > 0 || plan.row_blocks != hw::WIDE_ROW_BLOCKS || plan.row_groups < 2 || plan.tiles_per_head < 1) return false;
     constexpr double kJobCost = 6.0, kOpenCost = 2.0;     // in tiles: a row group's prologue and epilogue; one more fragment
     constexpr int kMinPiece = 4;                          // tiles worth opening a row group for
+    constexpr double kJobPrice = 12.0, kOpenPrice = 4.0, kWorth = 1.22;   // the choice of runs
     const int nrg = plan.row_groups, T = plan.tiles_per_head;
     int nf = 0;
     for (int f = 0; f < p->F; ++f) nf += p->len[f] > 0 ? 1 : 0;
@@ -234,9 +240,9 @@ bool stream_plan(const hw_problem* p, int num_cus, const CallPlan& cp, StreamPla
     if ((long long)wgs * 2 * kMinPiece > (long long)nrg * T) wgs = (int)((long long)nrg * T / (2 * kMinPiece));
     if (wgs < 1 || (long long)wgs + nrg >= (1 << 15) || (long long)nrg * T >= (1ll << 30)) return false;
     const long long launched = plan.workgroups, rounds = (launched + num_cus - 1) / num_cus;
-    const double cost_rounds = rounds * ((double)T / plan.wgs_per_head + kJobCost + kOpenCost * (1.0 + (double)(nf - 1) / plan.wgs_per_head));
-    const double cost_stream = (nrg * job + (wgs - 1) * (kJobCost + kOpenCost)) / wgs;
-    if (cost_stream * 1.1 > cost_rounds) return false;
+    const double cost_rounds = rounds * ((double)T / plan.wgs_per_head + kJobPrice + kOpenPrice * (1.0 + (double)(nf - 1) / plan.wgs_per_head));
+    const double cost_stream = (nrg * (T + kJobPrice + kOpenPrice * nf) + (wgs - 1) * (kJobPrice + kOpenPrice)) / wgs;
+    if (cost_stream * kWorth > cost_rounds) return false;
     sp->wgs = wgs;
     double left = nrg * job;            // work not dealt yet, without the re-openings of the workgroups to come
     int wg = 0;

@@ -1,5 +1,5 @@
 // stream_plan over random calls of 128-row workgroups: the runs tile the row groups' tiles without gaps, every piece has a
-// slot of its own inside the workspace, and max_pieces bounds the pieces of a row group.
+// slot of its own inside the workspace, and max_pieces bounds the pieces of a row group; and the rule's choice for measured calls.
 #include <cstdio>
 #include <cstdlib>
 #include <random>
@@ -10,7 +10,44 @@
 
 #define CHECK(c) do { if (!(c)) { std::printf("failed: %s (Hkv %d rows %d F %d)\n", #c, p.Hkv, cp.plan[0].rows, p.F); return 1; } } while (0)
 
+// Calls timed in rounds and in runs on an MI355X: rounds / runs.  Below 1 the runs lost time and must not be taken.
+struct Measured { int W, S, Hq, Hkv, D; std::vector<int32_t> len; double gain; };
+static const Measured kMeasured[] = {
+    {2, 133, 40, 8, 128, {761, 133, 133}, 0.88},
+    {6, 22, 64, 8, 128, {66, 2384, 28, 58, 22, 822, 162}, 0.89},
+    {1, 170, 64, 8, 128, {1311, 170}, 0.89},
+    {2, 707, 8, 2, 64, {0, 707, 707}, 0.90},
+    {1, 1031, 12, 3, 128, {979, 1031}, 0.91},
+    {1, 1286, 40, 8, 64, {0, 1286}, 0.92},
+    {1, 693, 32, 8, 128, {176, 693}, 0.93},
+    {6, 43, 40, 8, 128, {635, 647, 63, 260, 43, 43, 43}, 0.94},
+    {1, 1433, 8, 2, 64, {459, 1433}, 0.96},
+    {1, 1177, 40, 8, 64, {1177}, 0.96},
+    {1, 1024, 40, 8, 128, {4096, 1024}, 1.31},
+    {1, 412, 40, 8, 128, {3013, 412}, 1.28},
+    {2, 576, 40, 8, 64, {3073, 576, 576}, 1.25},
+    {4, 1153, 8, 2, 64, {70, 1153, 1153, 1153, 1153}, 1.46},
+};
+
+static int check_measured() {
+    int wrong = 0;
+    for (const Measured& m : kMeasured) {
+        hw_problem p{};
+        p.dtype = HW_BF16;
+        p.F = (int)m.len.size(); p.W = m.W; p.S = m.S; p.Hq = m.Hq; p.Hkv = m.Hkv; p.E = p.Ev = p.RotE = m.D;
+        p.len = m.len.data();
+        hw::host::CallPlan cp;
+        hw::host::StreamPlan sp;
+        if (hw::host::plan_call(&p, 256, &cp, 1) != HW_OK || hw::host::stream_plan(&p, 256, cp, &sp) != (m.gain > 1)) {
+            std::printf("wrong launch: W %d S %d %d/%d D %d first length %d (measured %.2f)\n", m.W, m.S, m.Hq, m.Hkv, m.D, m.len[0], m.gain);
+            ++wrong;
+        }
+    }
+    return wrong;
+}
+
 int main(int argc, char** argv) {
+    if (check_measured() != 0) return 1;
     const int rounds = argc > 1 ? std::atoi(argv[1]) : 20000;
     std::mt19937 rng(11);
     auto pick = [&](int lo, int hi) { return (int)(lo + rng() % (unsigned)(hi - lo + 1)); };

@@ -68,7 +68,7 @@ CASES = [
     (1, 830, 40, 8, 128, (100, 830), torch.bfloat16),            # 33 row groups, the last of 54 rows
     (1, 830, 40, 8, 64, (100, 0, 830), torch.float16),           # an empty fragment
     (1, 1400, 24, 3, 128, (33, 7, 1400), torch.bfloat16),        # 88 row groups of 3 heads: grid not a multiple of 8
-    (2, 640, 16, 8, 64, (64, 640, 640), torch.bfloat16),         # GQA 2: every row loads its own table row; row groups in three
+    (2, 550, 16, 8, 64, (64, 550, 550), torch.bfloat16),         # GQA 2: every row loads its own table row; row groups in three
     (1, 1460, 28, 4, 128, (1, 1460), torch.float16),             # 80 row groups, one-token fragment
     (2, 1300, 8, 8, 64, (200, 1300, 1300), torch.float16),
 ]
