@@ -71,7 +71,8 @@ int run(const hw_problem* p, void* stream_, int fused, int stages = HW_STAGE_ATT
     // (a workspace sized for CallPlan only, as the static scratch may be, keeps to its launch; so do the stages on their own,
     // whose partials are for the caller to read: they are laid out by hw_plan)
     StreamPlan sp;
-    const bool stream_runs = stages == (HW_STAGE_ATTENTION | HW_STAGE_MERGE) && stream_plan(p, cus, cp, &sp) && p->workspace_bytes >= sp.workspace_bytes;
+    const bool stream_runs = stages == (HW_STAGE_ATTENTION | HW_STAGE_MERGE) && stream_size(p, cus, cp, &sp) && p->workspace_bytes >= sp.workspace_bytes;
+    if (stream_runs) stream_deal(p, cp, &sp);
     // the VALU logits exist for what they are measured on: the fused entry with full rotary width, one row block, host lengths
     if (p->variant == HW_VARIANT_VALU_QK && (!fused || p->RotE != p->E || plan0.row_blocks != 1 || p->len_dev != nullptr)) return HW_ERR_UNSUPPORTED;
 
@@ -478,7 +479,7 @@ static int workspace_bytes_for(const hw_problem* p, int fused, size_t* bytes) {
     if (st != HW_OK) return st;
     StreamPlan sp;
     *bytes = cp.workspace_bytes;
-    if (stream_plan(p, cus, cp, &sp) && sp.workspace_bytes > *bytes) *bytes = sp.workspace_bytes;
+    if (stream_size(p, cus, cp, &sp) && sp.workspace_bytes > *bytes) *bytes = sp.workspace_bytes;
     return HW_OK;
 }
 

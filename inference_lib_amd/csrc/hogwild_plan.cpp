@@ -2,6 +2,7 @@
 // call, so that every rejection and every plan can be tested (and fuzzed under sanitizers) on a machine without a GPU.
 #include "hogwild_plan.h"
 
+#include <algorithm>
 #include <cmath>
 #include <cstring>
 
@@ -225,16 +226,14 @@ int plan_call(const hw_problem* p, int num_cus, CallPlan* cp, int fused) {
 // 1 to 8 workers behind 0 to 16 K, eight head layouts, D = 64 and 128): the 1305 that the rule takes gain 0.994 to 1.66,
 // 1.21 in the median (1024 tokens behind 4096 at 40/8 heads, D = 128: 180 -> 138 us a layer); the 321 that it leaves in rounds
 // would give 0.88 to 1.17, 1.03 in the median (133 tokens of two workers behind 761: 28 -> 32 us).
-bool stream_plan(const hw_problem* p, int num_cus, const CallPlan& cp, StreamPlan* sp) {
+constexpr int kMinPiece = 4;      // tiles worth opening a row group for
+bool stream_size(const hw_problem* p, int num_cus, const CallPlan& cp, StreamPlan* sp) {
     const hw_plan& plan = cp.plan[0];
     if (cp.groups != 1 || p->splits > 0 || plan.row_blocks != hw::WIDE_ROW_BLOCKS || plan.row_groups < 2 || plan.tiles_per_head < 1) return false;
-    constexpr double kJobCost = 6.0, kOpenCost = 2.0;     // in tiles: a row group's prologue and epilogue; one more fragment
-    constexpr int kMinPiece = 4;                          // tiles worth opening a row group for
     constexpr double kJobPrice = 12.0, kOpenPrice = 4.0, kWorth = 1.22;   // the choice of runs
     const int nrg = plan.row_groups, T = plan.tiles_per_head;
     int nf = 0;
     for (int f = 0; f < p->F; ++f) nf += p->len[f] > 0 ? 1 : 0;
-    const double job = T + kJobCost + kOpenCost * nf;     // a whole row group
     int wgs = num_cus / p->Hkv;
     if (wgs > hw::MAX_SPLITS) wgs = hw::MAX_SPLITS;
     if ((long long)wgs * 2 * kMinPiece > (long long)nrg * T) wgs = (int)((long long)nrg * T / (2 * kMinPiece));
@@ -243,40 +242,75 @@ bool stream_plan(const hw_problem* p, int num_cus, const CallPlan& cp, StreamPla
     const double cost_rounds = rounds * ((double)T / plan.wgs_per_head + kJobPrice + kOpenPrice * (1.0 + (double)(nf - 1) / plan.wgs_per_head));
     const double cost_stream = (nrg * (T + kJobPrice + kOpenPrice * nf) + (wgs - 1) * (kJobPrice + kOpenPrice)) / wgs;
     if (cost_stream * kWorth > cost_rounds) return false;
+    // the kernel divides (head, workgroup) pairs by the workgroups per head: exact for every count up to wgs (see magic_exact)
+    if ((unsigned long long)wgs * wgs * p->Hkv >= (1ull << 32)) return false;
     sp->wgs = wgs;
-    double left = nrg * job;            // work not dealt yet, without the re-openings of the workgroups to come
+    sp->slots = wgs + nrg - 1;
+    const size_t rows = (size_t)sp->slots * hw::PLAN_SLOT_ROWS;
+    sp->partial_bytes = (size_t)p->Hkv * rows * ((size_t)p->Ev + 2) * sizeof(float);
+    sp->workspace_bytes = ((sp->partial_bytes + (size_t)p->Hkv * plan.rows * 2 * sizeof(int) + 255) & ~(size_t)255) + cp.rope_bytes;
+    return true;
+}
+
+void stream_deal(const hw_problem* p, const CallPlan& cp, StreamPlan* sp) {
+    constexpr double kJobCost = 6.0, kOpenCost = 2.0;     // in tiles: a row group's prologue and epilogue; one more fragment
+    const hw_plan& plan = cp.plan[0];
+    const int nrg = plan.row_groups, T = plan.tiles_per_head, wgs = sp->wgs;
+    // The fragments with tiles.  price[f]: tiles and openings of a row group in front of fragment f; a workgroup that holds the
+    // row group and has r of its share left there takes fragments up to the first whose whole[] exceeds r + price[f].
+    int nf = 0, begin[HW_MAX_LAUNCH_FRAGMENTS], tiles[HW_MAX_LAUNCH_FRAGMENTS];
+    double price[HW_MAX_LAUNCH_FRAGMENTS + 1], whole[HW_MAX_LAUNCH_FRAGMENTS];
+    price[0] = 0.0;
+    for (int f = 0; f < p->F; ++f) {
+        const int n = plan.tile_begin[f + 1] - plan.tile_begin[f];
+        if (n == 0) continue;
+        begin[nf] = plan.tile_begin[f];
+        tiles[nf] = n;
+        whole[nf] = price[nf] + kOpenCost + std::max(n - 0.5, 1.0);
+        price[nf + 1] = price[nf] + kOpenCost + n;
+        ++nf;
+    }
+    double left = nrg * (kJobCost + price[nf]);    // work not dealt yet, without the re-openings of the workgroups to come
     int wg = 0;
-    double used = 0.0;
+    double used = 0.0, target = 0.0;
     sp->wg_tile_begin[0] = 0;
     for (int rg = 0; rg < nrg; ++rg) {
-        bool open = false;              // the current workgroup holds the row group's queries
-        for (int f = 0; f < p->F; ++f) {
-            const int ft = (int)(((long long)p->len[f] + hw::TILE - 1) / hw::TILE);
-            int t = 0;
-            while (t < ft) {
+        int pieces = 0;                 // of the row group, taken by the current workgroup; with the first it holds the queries
+        for (int f = 0; f < nf;) {
+            const int wgs_left = wgs - wg;
+            if (pieces > 1) {           // whole fragments at once
+                const int to = wgs_left == 1 ? nf : (int)(std::upper_bound(whole + f, whole + nf, target - used + price[f]) - whole);
+                used += price[to] - price[f];
+                left -= price[to] - price[f];
+                f = to;
+                if (f == nf) break;
+            }
+            for (int t = 0; t < tiles[f];) {
                 const int wgs_left = wgs - wg;
-                const double target = (left + used + (wgs_left - 1) * (kJobCost + kOpenCost)) / wgs_left;
-                const double opening = kOpenCost + (open ? 0.0 : kJobCost);
+                // this workgroup's fair share; what it takes of a row group that it holds already does not change that
+                if (pieces < 2) target = (left + used + (wgs_left - 1) * (kJobCost + kOpenCost)) / wgs_left;
+                const double opening = kOpenCost + (pieces > 0 ? 0.0 : kJobCost);
                 const double room = target - used - opening;
-                if (used > 0.0 && wgs_left > 1 && room < (open ? 1 : kMinPiece)) {      // not worth opening this here
-                    sp->wg_tile_begin[++wg] = rg * T + plan.tile_begin[f] + t;
+                if (used > 0.0 && wgs_left > 1 && room < (pieces > 0 ? 1 : kMinPiece)) {      // not worth opening this here
+                    sp->wg_tile_begin[++wg] = rg * T + begin[f] + t;
                     used = 0.0;
-                    open = false;
+                    pieces = 0;
                     continue;
                 }
                 int take = (int)(room + 0.5);
                 if (take < 1) take = 1;
-                if (take > ft - t || wgs_left == 1) take = ft - t;
+                if (take > tiles[f] - t || wgs_left == 1) take = tiles[f] - t;
                 used += opening + take;
-                left -= take + (t == 0 ? kOpenCost : 0.0) + (t == 0 && plan.tile_begin[f] == 0 ? kJobCost : 0.0);
-                open = true;
+                left -= take + (t == 0 ? kOpenCost : 0.0) + (t == 0 && f == 0 ? kJobCost : 0.0);
+                ++pieces;
                 t += take;
-                if (t < ft) {
-                    sp->wg_tile_begin[++wg] = rg * T + plan.tile_begin[f] + t;
+                if (t < tiles[f]) {
+                    sp->wg_tile_begin[++wg] = rg * T + begin[f] + t;
                     used = 0.0;
-                    open = false;
+                    pieces = 0;
                 }
             }
+            ++f;
         }
     }
     sp->wgs = wg + 1;
@@ -288,11 +322,6 @@ bool stream_plan(const hw_problem* p, int num_cus, const CallPlan& cp, StreamPla
         while (sp->wg_tile_begin[last + 1] < (rg + 1) * T) ++last;
         if (last - g + 1 > sp->max_pieces) sp->max_pieces = last - g + 1;
     }
-    sp->slots = sp->wgs + nrg - 1;
-    const size_t rows = (size_t)sp->slots * hw::PLAN_SLOT_ROWS;
-    sp->partial_bytes = (size_t)p->Hkv * rows * ((size_t)p->Ev + 2) * sizeof(float);
-    sp->workspace_bytes = ((sp->partial_bytes + (size_t)p->Hkv * plan.rows * 2 * sizeof(int) + 255) & ~(size_t)255) + cp.rope_bytes;
-    return magic_exact((unsigned long long)sp->wgs, (unsigned long long)sp->wgs * p->Hkv);
 }
 
 int paged_validate(const hw_paged_problem* p) {

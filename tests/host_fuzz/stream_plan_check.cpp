@@ -1,5 +1,7 @@
-// stream_plan over random calls of 128-row workgroups: the runs tile the row groups' tiles without gaps, every piece has a
+// stream_size and stream_deal over random calls of 128-row workgroups: the runs tile the row groups' tiles without gaps, every piece has a
 // slot of its own inside the workspace, and max_pieces bounds the pieces of a row group; and the rule's choice for measured calls.
+#include <algorithm>
+#include <chrono>
 #include <cstdio>
 #include <cstdlib>
 #include <random>
@@ -29,6 +31,77 @@ static const Measured kMeasured[] = {
     {4, 1153, 8, 2, 64, {70, 1153, 1153, 1153, 1153}, 1.46},
 };
 
+static bool stream_plan(const hw_problem* p, int cus, const hw::host::CallPlan& cp, hw::host::StreamPlan* sp) {
+    if (!hw::host::stream_size(p, cus, cp, sp)) return false;
+    hw::host::stream_deal(p, cp, sp);
+    return true;
+}
+
+// The deal as a plain loop over row groups and fragments: the boundaries that stream_deal has to give.
+static std::vector<int> plain_deal(const hw_problem* p, const hw_plan& plan, int wgs) {
+    const int nrg = plan.row_groups, T = plan.tiles_per_head;
+    const double kJobCost = 6.0, kOpenCost = 2.0, kMinPiece = 4.0;
+    int nf = 0;
+    for (int f = 0; f < p->F; ++f) nf += p->len[f] > 0;
+    double left = nrg * (T + kJobCost + kOpenCost * nf), used = 0.0;
+    std::vector<int> begin(1, 0);
+    for (int rg = 0; rg < nrg; ++rg) {
+        bool open = false;
+        for (int f = 0; f < p->F; ++f) {
+            const int first = plan.tile_begin[f], n = plan.tile_begin[f + 1] - first;
+            for (int t = 0; t < n;) {
+                const int wgs_left = wgs - (int)begin.size() + 1;
+                const double target = (left + used + (wgs_left - 1) * (kJobCost + kOpenCost)) / wgs_left;
+                const double opening = kOpenCost + (open ? 0.0 : kJobCost), room = target - used - opening;
+                int take = (int)(room + 0.5);
+                const bool cut = used > 0.0 && wgs_left > 1 && room < (open ? 1.0 : kMinPiece);
+                if (cut) take = 0;
+                else if (wgs_left == 1 || take > n - t) take = n - t;
+                else if (take < 1) take = 1;
+                if (!cut) {
+                    used += opening + take;
+                    left -= take + (t == 0 ? kOpenCost + (first == 0 ? kJobCost : 0.0) : 0.0);
+                    open = true;
+                    t += take;
+                }
+                if (cut || t < n) {
+                    begin.push_back(rg * T + first + t);
+                    used = 0.0;
+                    open = false;
+                }
+            }
+        }
+    }
+    begin.push_back(nrg * T);
+    return begin;
+}
+
+// Planning stays small against a launch: a call sizes twice (workspace, launch) and deals once.
+static int check_time() {
+    std::vector<int32_t> len(60, 68);
+    len.back() = 1024;
+    hw_problem p{};
+    p.dtype = HW_BF16;
+    p.F = 60; p.W = 1; p.S = 1024; p.Hq = 40; p.Hkv = 8; p.E = p.Ev = p.RotE = 128;
+    p.len = len.data();
+    hw::host::CallPlan cp;
+    hw::host::StreamPlan sp;
+    auto best = [](auto f) {
+        double t = 1e9;
+        for (int b = 0; b < 20; ++b) {
+            const auto t0 = std::chrono::steady_clock::now();
+            for (int i = 0; i < 50; ++i) f();
+            t = std::min(t, std::chrono::duration<double, std::micro>(std::chrono::steady_clock::now() - t0).count() / 50);
+        }
+        return t;
+    };
+    bool taken = false;
+    const double call = best([&] { hw::host::plan_call(&p, 256, &cp, 1); });
+    const double runs = best([&] { hw::host::stream_size(&p, 256, cp, &sp); taken = stream_plan(&p, 256, cp, &sp); });
+    std::printf("60 fragments, 40 row groups: plan_call %.2f us, runs %.2f us\n", call, runs);
+    return taken && runs < 20 * call ? 0 : 1;
+}
+
 static int check_measured() {
     int wrong = 0;
     for (const Measured& m : kMeasured) {
@@ -38,7 +111,7 @@ static int check_measured() {
         p.len = m.len.data();
         hw::host::CallPlan cp;
         hw::host::StreamPlan sp;
-        if (hw::host::plan_call(&p, 256, &cp, 1) != HW_OK || hw::host::stream_plan(&p, 256, cp, &sp) != (m.gain > 1)) {
+        if (hw::host::plan_call(&p, 256, &cp, 1) != HW_OK || stream_plan(&p, 256, cp, &sp) != (m.gain > 1)) {
             std::printf("wrong launch: W %d S %d %d/%d D %d first length %d (measured %.2f)\n", m.W, m.S, m.Hq, m.Hkv, m.D, m.len[0], m.gain);
             ++wrong;
         }
@@ -47,7 +120,7 @@ static int check_measured() {
 }
 
 int main(int argc, char** argv) {
-    if (check_measured() != 0) return 1;
+    if (check_measured() != 0 || check_time() != 0) return 1;
     const int rounds = argc > 1 ? std::atoi(argv[1]) : 20000;
     std::mt19937 rng(11);
     auto pick = [&](int lo, int hi) { return (int)(lo + rng() % (unsigned)(hi - lo + 1)); };
@@ -69,8 +142,11 @@ int main(int argc, char** argv) {
         hw::host::CallPlan cp;
         if (hw::host::plan_call(&p, cus, &cp, 1) != HW_OK) continue;
         hw::host::StreamPlan sp;
-        if (!hw::host::stream_plan(&p, cus, cp, &sp)) continue;
+        if (!hw::host::stream_size(&p, cus, cp, &sp)) continue;
         ++taken;
+        const std::vector<int> plain = plain_deal(&p, cp.plan[0], sp.wgs);
+        hw::host::stream_deal(&p, cp, &sp);
+        CHECK((int)plain.size() == sp.wgs + 1 && std::equal(plain.begin(), plain.end(), sp.wg_tile_begin));
         const int T = cp.plan[0].tiles_per_head, nrg = cp.plan[0].row_groups, rows = cp.plan[0].rows;
         CHECK(sp.wgs >= 1 && sp.wgs <= HW_MAX_SPLITS && (long long)sp.wgs * p.Hkv <= (cus > p.Hkv ? cus : p.Hkv));
         CHECK(sp.wg_tile_begin[0] == 0 && sp.wg_tile_begin[sp.wgs] == nrg * T);
