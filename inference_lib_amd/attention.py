@@ -58,11 +58,12 @@ def hogwild_fused(queries: torch.Tensor, locations: torch.Tensor, keys: List[tor
 
 
 def _in_place_or_contiguous(keys: Iterable[torch.Tensor], values: Iterable[torch.Tensor]):
-    pairs = list(zip(keys, values))
-    if all(k.is_contiguous() and v.is_contiguous() for k, v in pairs):
-        return [k for k, _ in pairs], [v for _, v in pairs]
+    if type(keys) is not list or type(values) is not list:
+        keys, values = list(keys), list(values)
+    if len(keys) == len(values) and all(k.is_contiguous() and v.is_contiguous() for k, v in zip(keys, values)):
+        return keys, values
     ks, vs = [], []
-    for k, v in pairs:
+    for k, v in zip(keys, values):
         k3, v3 = (k[0] if k.dim() == 4 else k), (v[0] if v.dim() == 4 else v)
         if k3.dim() == 3 and v3.dim() == 3 and _lib.fragment_capacity(k3, v3) is not None:
             ks.append(k)

@@ -43,16 +43,21 @@ class _LayerViews:
         return len(self._bufs)
 
 
-def _fragments(keys: list, values: list, layer: int):
-    """keys[f][layer], values[f][layer] of the segments' key_cache / value_cache.  Where all of them are SegmentCache's own the
-    views are made in one native call; a segment of another kind, or one whose members were replaced, is asked for its tensors."""
-    caches = keys + values
-    if HAVE_TORCH_OPS and caches and all(type(c) is _LayerViews for c in caches):
-        bufs = [c._bufs[layer] for c in caches]
-        if bufs[0].is_cuda:
-            views = _segment_views(bufs, [c._seg.lengths[layer] for c in caches])
-            return views[: len(keys)], views[len(keys):]
-    return [c[layer] for c in keys], [c[layer] for c in values]
+def _fragments(segments: list, layer: int):
+    """(key_cache[layer], value_cache[layer]) of every segment.  Where all of them are SegmentCache's own the views are made in one
+    native call; a segment of another kind, or one whose members were replaced, is asked for its tensors."""
+    bufs, lens = [], []
+    for seg in segments if HAVE_TORCH_OPS else ():
+        k, v = seg.key_cache, seg.value_cache
+        if type(k) is not _LayerViews or type(v) is not _LayerViews:
+            break
+        bufs += k._bufs[layer], v._bufs[layer]
+        lens += k._seg.lengths[layer], v._seg.lengths[layer]
+    else:
+        if bufs and bufs[0].is_cuda:
+            views = _segment_views(bufs, lens)
+            return views[0::2], views[1::2]
+    return [seg.key_cache[layer] for seg in segments], [seg.value_cache[layer] for seg in segments]
 
 
 class SegmentCache:
@@ -295,7 +300,7 @@ class HogwildCache:
             self.segments = segments
             self.frags = torch.tensor([cs.get_seq_length(layer_idx) for cs in segments], dtype=torch.int32, device=key_states.device)
         # views; no .contiguous() copies (attention.py:160-162,199-203)
-        keys, vals = _fragments([cs.key_cache for cs in self.segments], [cs.value_cache for cs in self.segments], layer_idx)
+        keys, vals = _fragments(self.segments, layer_idx)
         return CacheStructure(keys=keys, values=vals, cos=self.cosines, sin=self.sines, loc=self.locations, frags=self.frags)
 
     def update(self, key_states: torch.Tensor, value_states: torch.Tensor, layer_idx: int,
