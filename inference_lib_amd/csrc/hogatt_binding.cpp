@@ -49,7 +49,8 @@ void check_status(int status, const char* where) {
 }
 
 // Geometry of a KV fragment [Hkv, L, D], read through the optional leading batch dimension of 1 ([1, Hkv, L, D]).  (Not
-// by a select() per tensor: that is a view to make and to drop for every fragment of every call.)
+// by a select() per tensor: that is a view to make and to drop for every fragment of every call, 361-392 against 344-360 us for
+// a step of 12 layers with three segments.)
 struct FragmentDims {
     int64_t heads, len, width, head_stride, row_stride, elem_stride;
 };
@@ -451,7 +452,7 @@ bool merge_segments(at::TensorList k_dst, at::TensorList v_dst, at::IntArrayRef 
 }
 
 // hw_rope_append on tensors: the append of HogwildCache, whose argument checks and pointer tables took most of a step's host
-// time in Python (12 layers, two workers, three segments: 694 -> 364 us a step with this, segment_views and fragment_dims).
+// time in Python (12 layers, two workers, three segments: 552 us a step through them, 359 with this).
 // Returns false, with nothing queued, for anything the checks below or the library do not take: the caller's general path then
 // handles it or names what is wrong.
 bool rope_append(at::TensorList k_dst, at::TensorList v_dst, at::IntArrayRef dst_len, at::IntArrayRef n_new, const at::Tensor& key_states,
@@ -510,7 +511,8 @@ bool rope_append(at::TensorList k_dst, at::TensorList v_dst, at::IntArrayRef dst
     return true;
 }
 
-// The filled parts of segment buffers [Hkv, cap, D] as fragments: [1, Hkv, len, D] views.
+// The filled parts of segment buffers [Hkv, cap, D] as fragments: [1, Hkv, len, D] views (the step of rope_append above: 463 us
+// with two slicing calls per view in Python, 358 with this).
 std::vector<at::Tensor> segment_views(at::TensorList buffers, at::IntArrayRef len) {
     TORCH_CHECK(buffers.size() == len.size(), "libhogatt: one length per buffer");
     std::vector<at::Tensor> out;

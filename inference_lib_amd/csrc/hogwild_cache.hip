@@ -185,7 +185,7 @@ __global__ __launch_bounds__(256) void rope_append_kernel(const AppendArgs a) {
 // head, layer).  Bound by memory: every byte is read and written once, with four 16-byte loads of a thread in
 // flight, and the one cos / sin row is worked out by every workgroup for itself (RotE / 2 angles, into LDS) instead of by
 // three launches in front.  One launch per layer left the chip idle between launches of 5.5 us that a host call of 23 us
-// each could not keep fed: 16 layers x 2 segments of 1000 and 777 tokens (8 kv heads, D = 128, bf16; 233 MB) 757 -> 51 us
+// each could not keep fed: 16 layers x 2 segments of 1000 and 777 tokens (8 kv heads, D = 128, bf16; 233 MB) 769 -> 52 us
 // (4.6 TB/s; a large copy reaches 4.9).
 constexpr int MERGE_ROWS = 64;     // rows of one kv head per workgroup: 4 value and 2 key chunk pairs per thread at D = 128
 template <class DT, bool EAGER, bool CS16, bool VEC>

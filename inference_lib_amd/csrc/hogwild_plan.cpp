@@ -218,7 +218,7 @@ int plan_call(const hw_problem* p, int num_cus, CallPlan* cp, int fused) {
 // 5) are 320 workgroups, so 256 CUs take two rounds of which the second is a quarter full.  Cut into equal runs across the
 // row groups every CU gets 1.25 row groups of work instead of 2.  A run that crosses into the next row group opens it anew
 // (queries, partial sums), so the runs are dealt by tiles plus openings at kJobCost and kOpenCost tiles.  (Runs dealt by
-// the kernel over the tiles that the locations leave visible were measured slower, 300 against 276 us for two layers of 1024
+// the kernel over the tiles that the locations leave visible were measured slower, 300 against 282 us for two layers of 1024
 // tokens behind 4096: a row group's unseen tiles cost next to nothing as it is, and the uneven row groups give some runs a
 // third one to open.)
 // Where to take them: a price of each launch in tiles, rounds against runs, with kJobPrice and kOpenPrice per opening.  The

@@ -181,10 +181,11 @@ struct WideRotation {
 };
 
 // STREAM: the workgroup's run of tiles may cross row groups (KH_STREAM): the whole body is then done once per row group.
-// Prompt chunk of 1024 tokens behind 4096 (40 / 8 heads, D = 128, bf16; 97 GFLOP): 131-133 us, 0.73 PFLOP/s (two layers with
-// their merges 276 us, against 342 us in two rounds of workgroups).  Bound by the arithmetic of two waves per SIMD: matrix units busy 92 k clocks of each SIMD's
-// 244 k, vector units 119 k (16 exponentials and about 90 others per 32 products), the rest waits at the barrier of a step
-// and for issue; LDS is in use a fifth of the time, without conflicts.
+// Prompt chunk of 1024 tokens behind 4096 (40 / 8 heads, D = 128, bf16; 97 GFLOP): two layers with their merges 263-275 us by
+// box, against 341 us in two rounds of workgroups; without a pause between passes, where the shader clock falls, 300-307
+// against 353.  In a kernel trace 131-133 us, 0.73 PFLOP/s, and 12 for the merge.  Bound by the arithmetic of two waves per
+// SIMD: matrix units busy 92 k clocks of each SIMD's 244 k, vector units 119 k (16 exponentials and about 90 others per 32
+// products), the rest waits at the barrier of a step and for issue; LDS is in use a fifth of the time, without conflicts.
 template <class DT, int E, int EV, int NS, bool PRE, int NW, int PAR, bool STREAM>
 __global__ __launch_bounds__(NW * 64, 1) void attention_wide_kernel(const KernelArgs args) {
     typedef Geo<DT, E, EV> G;
