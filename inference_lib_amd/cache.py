@@ -365,9 +365,9 @@ def merge_caches(target: SegmentCache, source: SegmentCache, model=None, *, inv_
         for layer in layers:          # grow like every other append (the reference's merge goes through target.update)
             if target.lengths[layer] + source.lengths[layer] > target.k[layer].size(1):
                 target.reserve(layer, source.lengths[layer])
-        k_dst, v_dst, k_src, v_src, at, added = ([of[layer] for layer in layers] for of in (target.k, target.v, source.k, source.v,
-                                                                                          target.lengths, source.lengths))
-        if torch.ops.libhogatt.merge_segments(k_dst, v_dst, at, k_src, v_src, added, inv_freq.to(dev), attention_scaling, position, tdt, mode):
+        n_layers, added = len(target.k), list(source.lengths)
+        if torch.ops.libhogatt.merge_segments(list(target.k), list(target.v), target.lengths, list(source.k)[:n_layers], list(source.v)[:n_layers],
+                                              added[:n_layers], inv_freq.to(dev), attention_scaling, position, tdt, mode):
             for layer in layers:
                 target.lengths[layer] += added[layer]
             return
