@@ -444,7 +444,7 @@ const char* hw_status_string(int status) {
         case HW_ERR_NULL: return "required pointer is NULL";
         case HW_ERR_DTYPE: return "unknown dtype";
         case HW_ERR_SHAPE: return "invalid or inconsistent shape";
-        case HW_ERR_UNSUPPORTED: return "no kernel instantiated for this shape (need E == Ev in {64, 128})";
+        case HW_ERR_UNSUPPORTED: return "no kernel instantiated for this shape (need E == Ev in {64, 128, 256})";
         case HW_ERR_FRAGMENTS: return "fragment count out of range";
         case HW_ERR_WORKSPACE: return "workspace missing, misaligned or too small";
         case HW_ERR_ALIGN: return "device pointer not 16-byte aligned";
