@@ -283,8 +283,8 @@ class HogwildCache:
             s.lengths[layer_idx] = end[id(s)]
 
     def _structure(self, key_states, layer_idx) -> CacheStructure:
-        W, S = key_states.size(0), key_states.size(2)
         if layer_idx == 0:
+            W, S = key_states.size(0), key_states.size(2)
             segments = list(self.cache_structure[0])                # the order of the first worker, attention.py:168-170,186-188
             index = {id(cs): f for f, cs in enumerate(segments)}
             pos_end = [[0] * W for _ in segments]
