@@ -49,6 +49,7 @@ constexpr int KH_DIRECT = 2;      // one workgroup per kv head and row group: it
 constexpr int KH_STREAM = 8;      // 128-row workgroups that run across row groups: wg_tile counts the tiles of all row groups one
                                   // behind the other, slot_stride = slots of PLAN_SLOT_ROWS rows per kv head, the piece of
                                   // workgroup g in row group rg goes to slot g + rg, a row table for the merge lies behind part_ml
+constexpr int KH_KEEP = 16;       // K/V tiles stay in the L2 for the other row groups (keep_in_l2; read by launch_attention_wide only)
 constexpr int KH_PREROTATED = 4;  // the queries arrive rotated, [F,W,Hq,S,E] (read by the launchers only)
 
 struct KernelArgs {

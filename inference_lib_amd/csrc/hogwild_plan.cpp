@@ -185,6 +185,14 @@ int make_plan(const hw_problem* p, int num_cus, hw_plan* plan, int fused) {
     return HW_OK;
 }
 
+// K/V tiles are streamed past the L2 (non-temporal) where whoever reads a tile reads it at about the same time: one row group, or
+// so few that all of them are under way together.  Once a CU works through row groups one after the other (more workgroups than
+// half the CUs even without a split) every tile is wanted again later, and is kept: 1024 tokens behind 4096 (40 row groups, 40/8
+// heads, D = 128) miss the L2 1.05 M times instead of 3.09 M (TCC_MISS), 136 -> 125 us a layer; 410 tokens behind 12 K and 16 K
+// 152 -> 125 and 203 -> 167; 1500 behind 12 K at 32/8 heads 426 -> 348; 2560 rows a head behind 1.2 K ... 8 K 1.00 to 1.12 times.
+// Below the line keeping costs: 256 ... 1024 rows a head of 8 heads 0.93 to 0.99, 1536 rows 0.98 to 1.06 by length.
+bool keep_in_l2(const hw_problem* p, const hw_plan& plan, int num_cus) { return 2ll * plan.row_groups * p->Hkv >= num_cus; }
+
 int plan_call(const hw_problem* p, int num_cus, CallPlan* cp, int fused) {
     if (cp == nullptr || p == nullptr) return HW_ERR_NULL;
     std::memset(cp, 0, sizeof(*cp));

@@ -21,6 +21,8 @@ int validate(const hw_problem* p, int fused);
 // fused != 0: size the workspace for hw_fused_attention (room for the rotated queries when the rotary width is not the head
 // dimension and the caller passes no rq buffer); 0: for hw_sdpa
 int make_plan(const hw_problem* p, int num_cus, hw_plan* plan, int fused = 1);
+// Whether the launch's K/V tiles are to stay in the L2 instead of being streamed past it (hogwild_plan.cpp).
+bool keep_in_l2(const hw_problem* p, const hw_plan& plan, int num_cus);
 // A call's fragments in groups of at most HW_MAX_LAUNCH_FRAGMENTS, one attention launch each.  Group i takes fragments
 // first[i] .. first[i] + count[i] - 1, is planned like a problem of its own (plan[i]; its workspace_bytes is not used) and
 // writes its split-K partials into slots slot_base[i] .. slot_base[i] + plan[i].wgs_per_head - 1 of every kv head's

@@ -68,25 +68,28 @@ __device__ __forceinline__ u32x4 raw_descriptor(unsigned long long base, unsigne
     d.w = 0x00020000u;
     return d;
 }
-// One 1 KB global->LDS transfer (lane l: 16 bytes from descriptor offset `voffset` to LDS byte `lds` + 16 l), non-temporal.
+// One 1 KB global->LDS transfer (lane l: 16 bytes from descriptor offset `voffset` to LDS byte `lds` + 16 l), non-temporal
+// unless KEEP (keep_in_l2: other row groups read the same tile, and the L2 is to hold it for them).
 // Issued from inline assembly on purpose: the compiler waits for every transfer it knows of before a read of LDS it
 // cannot prove disjoint, which would empty the look-ahead queue at every tile; these it does not know of, and the kernel
 // waits for them itself (s_waitcnt vmcnt before the barrier of each tile).  Loads complete in order, so a compiler-
 // generated wait for one of its own loads can only become longer through them, never too short.
 #pragma clang diagnostic push
 #pragma clang diagnostic ignored "-Winline-asm"   // m0 is a reserved register: it is set and used inside the one statement
+template <bool KEEP>
 __device__ __forceinline__ void lds_transfer(const u32x4& desc, unsigned lds, unsigned voffset) {
-    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, 0 offen nt lds" ::"s"(lds), "v"(voffset), "s"(desc) : "m0", "memory");
+    if constexpr (KEEP) asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, 0 offen lds" ::"s"(lds), "v"(voffset), "s"(desc) : "m0", "memory");
+    else asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, 0 offen nt lds" ::"s"(lds), "v"(voffset), "s"(desc) : "m0", "memory");
 }
 #pragma clang diagnostic pop
 
 // One wave's share of a tile's transfers: TPW 1 KB pieces of ONE image (the first half of the waves fill K, the second
 // half V), into LDS bytes `slot` + 1024 j.  `tile` = byte offset of the tile in the kv head's slice (OOB_OFFSET for a
 // tile that does not exist: the same number of transfers, no memory traffic, zeros in LDS).
-template <int TPW>
+template <int TPW, bool KEEP>
 __device__ __forceinline__ void wide_request(const u32x4& desc, unsigned slot, unsigned tile, const unsigned* off) {
 #pragma unroll
-    for (int j = 0; j < TPW; ++j) lds_transfer(desc, slot + j * 1024, tile + off[j]);
+    for (int j = 0; j < TPW; ++j) lds_transfer<KEEP>(desc, slot + j * 1024, tile + off[j]);
 }
 
 __device__ __forceinline__ unsigned lds_address(const void* p) {
@@ -186,7 +189,7 @@ struct WideRotation {
 // against 353.  In a kernel trace 131-133 us, 0.73 PFLOP/s, and 12 for the merge.  Bound by the arithmetic of two waves per
 // SIMD: matrix units busy 92 k clocks of each SIMD's 244 k, vector units 119 k (16 exponentials and about 90 others per 32
 // products), the rest waits at the barrier of a step and for issue; LDS is in use a fifth of the time, without conflicts.
-template <class DT, int E, int EV, int NS, bool PRE, int NW, int PAR, bool STREAM>
+template <class DT, int E, int EV, int NS, bool PRE, int NW, int PAR, bool STREAM, bool KEEP>
 __global__ __launch_bounds__(NW * 64, 1) void attention_wide_kernel(const KernelArgs args) {
     typedef Geo<DT, E, EV> G;
     constexpr int NT = NW * 64;                 // threads per workgroup
@@ -328,7 +331,7 @@ __global__ __launch_bounds__(NW * 64, 1) void attention_wide_kernel(const Kernel
 #pragma unroll
         for (int pp = 0; pp < PAR; ++pp) {
             const unsigned tile_bytes = (unsigned)((lt + pp) * TILE * image_row);
-            wide_request<TPW>(view, __builtin_amdgcn_readfirstlane(my_image + (ss * PAR + pp) * SLOT), lt + pp < lt1 ? tile_bytes : OOB_OFFSET, off);
+            wide_request<TPW, KEEP>(view, __builtin_amdgcn_readfirstlane(my_image + (ss * PAR + pp) * SLOT), lt + pp < lt1 ? tile_bytes : OOB_OFFSET, off);
         }
     };
 
@@ -1206,8 +1209,11 @@ static hipError_t launch_wide_dt(const KernelArgs& ka, int E, hipStream_t stream
     if (E != 64 && E != 128) return hipErrorInvalidValue;
     auto go = [&](auto head_dim, auto pre, auto stream_runs) {
         constexpr int HD = decltype(head_dim)::value;
-        hipLaunchKernelGGL((attention_wide_kernel<DT, HD, HD, NS, decltype(pre)::value, NW, PAR, decltype(stream_runs)::value>), dim3(ka.h.nwg),
-                           dim3(NW * 64), 0, stream, ka);
+        constexpr bool PRE = decltype(pre)::value, STREAM = decltype(stream_runs)::value;
+        if (ka.h.flags & KH_KEEP)
+            hipLaunchKernelGGL((attention_wide_kernel<DT, HD, HD, NS, PRE, NW, PAR, STREAM, true>), dim3(ka.h.nwg), dim3(NW * 64), 0, stream, ka);
+        else
+            hipLaunchKernelGGL((attention_wide_kernel<DT, HD, HD, NS, PRE, NW, PAR, STREAM, false>), dim3(ka.h.nwg), dim3(NW * 64), 0, stream, ka);
     };
     auto by_entry = [&](auto head_dim, auto stream_runs) {
         if (ka.h.flags & KH_PREROTATED) go(head_dim, std::true_type{}, stream_runs);
