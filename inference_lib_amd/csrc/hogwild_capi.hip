@@ -71,8 +71,16 @@ int run(const hw_problem* p, void* stream_, int fused, int stages = HW_STAGE_ATT
     // (a workspace sized for CallPlan only, as the static scratch may be, keeps to its launch; so do the stages on their own,
     // whose partials are for the caller to read: they are laid out by hw_plan)
     StreamPlan sp;
-    const bool stream_runs = stages == (HW_STAGE_ATTENTION | HW_STAGE_MERGE) && stream_size(p, cus, cp, &sp) && p->workspace_bytes >= sp.workspace_bytes;
-    if (stream_runs) stream_deal(p, cp, &sp);
+    const bool both = stages == (HW_STAGE_ATTENTION | HW_STAGE_MERGE);
+    WholePlan wp;
+    const bool whole = both && whole_size(p, cus, cp, &wp) && p->workspace_bytes >= wp.workspace_bytes;
+    const bool stream_runs = whole || (both && stream_size(p, cus, cp, &sp) && p->workspace_bytes >= sp.workspace_bytes);
+    if (whole) {
+        whole_deal(p, cp, &wp);
+        sp = wp.runs;
+    } else if (stream_runs) {
+        stream_deal(p, cp, &sp);
+    }
     // the VALU logits exist for what they are measured on: the fused entry with full rotary width, one row block, host lengths
     if (p->variant == HW_VARIANT_VALU_QK && (!fused || p->RotE != p->E || plan0.row_blocks != 1 || p->len_dev != nullptr)) return HW_ERR_UNSUPPORTED;
 
@@ -91,6 +99,7 @@ int run(const hw_problem* p, void* stream_, int fused, int stages = HW_STAGE_ATT
         prerotated = true;
     }
     const int rows = plan0.rows;
+    const int stream_wgs = whole ? wp.wgs : stream_runs ? sp.wgs : 0;
     float* const part_o = reinterpret_cast<float*>(p->workspace);
     const size_t part_rows = stream_runs ? (size_t)sp.slots * hw::PLAN_SLOT_ROWS : (size_t)cp.slots * rows;     // per kv head
     float* const part_ml = part_o + (size_t)p->Hkv * part_rows * p->Ev;
@@ -145,10 +154,14 @@ int run(const hw_problem* p, void* stream_, int fused, int stages = HW_STAGE_ATT
         if (stream_runs) {
             ka.h.nrg = 1;
             ka.h.magic_nrg = magic(1);
-            ka.h.wgs_per_head = sp.wgs;
-            ka.h.magic_wg = magic(sp.wgs);
-            ka.h.nwg = sp.wgs * p->Hkv;
+            ka.h.wgs_per_head = stream_wgs;
+            ka.h.magic_wg = magic(stream_wgs);
+            ka.h.nwg = stream_wgs * p->Hkv;
             ka.h.slot_stride = sp.slots;
+            ka.split = whole ? wp.split : plan.row_groups;
+            ka.whole = whole ? wp.whole : 0;
+            ka.out = p->out;
+            ka.lse = p->lse;
             ka.h.flags = ((ka.h.nwg % 8 == 0) ? hw::KH_XCD_REMAP : 0) | (prerotated ? hw::KH_PREROTATED : 0) | hw::KH_STREAM;
         }
         if (keep_in_l2(p, plan, cus)) ka.h.flags |= hw::KH_KEEP;
@@ -158,8 +171,9 @@ int run(const hw_problem* p, void* stream_, int fused, int stages = HW_STAGE_ATT
             e = hw::launch_attention(ka, p->dtype, p->E, plan.row_blocks, p->variant, stream);
         if (e != hipSuccess) return (int)e;
     }
-    if (!(stages & HW_STAGE_MERGE) || direct) return (int)e;
+    if (!(stages & HW_STAGE_MERGE) || direct || (whole && wp.split == 0)) return (int)e;
     hw::MergeArgs ma;
+    ma.rows = whole ? wp.split * hw::PLAN_SLOT_ROWS : rows;
     ma.part_o = part_o;
     ma.part_ml = part_ml;
     ma.out = p->out;
@@ -171,7 +185,7 @@ int run(const hw_problem* p, void* stream_, int fused, int stages = HW_STAGE_ATT
     ma.pslots = 0;
     if (stream_runs) {
         ma.wgs_per_head = sp.max_pieces;
-        ma.xcd_local = ((sp.wgs * p->Hkv) % 8 == 0 && p->Hkv % 8 == 0) ? 1 : 0;
+        ma.xcd_local = ((stream_wgs * p->Hkv) % 8 == 0 && p->Hkv % 8 == 0) ? 1 : 0;
         ma.row_tab = reinterpret_cast<const int*>(part_ml + (size_t)p->Hkv * part_rows * 2);
         ma.pslots = sp.slots;
     }
@@ -242,7 +256,7 @@ int paged_run(const hw_paged_problem* p, void* stream_, int stages) {
     ma.part_ml = ph.part_ml;
     ma.out = p->out;
     ma.lse = p->lse;
-    ma.W = ph.LW; ma.Hq = p->Hq; ma.Hkv = p->Hkv; ma.S = ph.LS; ma.R = plan.rows;
+    ma.W = ph.LW; ma.Hq = p->Hq; ma.Hkv = p->Hkv; ma.S = ph.LS; ma.R = ma.rows = plan.rows;
     ma.wgs_per_head = plan.splits;
     // a variable-length launch may leave row groups of the grid unused, and with them parts of an XCD's share
     // (a launch planned on the device keeps every slot of a kv head on the head's XCD whatever the slots do)
@@ -481,6 +495,8 @@ static int workspace_bytes_for(const hw_problem* p, int fused, size_t* bytes) {
     StreamPlan sp;
     *bytes = cp.workspace_bytes;
     if (stream_size(p, cus, cp, &sp) && sp.workspace_bytes > *bytes) *bytes = sp.workspace_bytes;
+    WholePlan wp;
+    if (whole_size(p, cus, cp, &wp) && wp.workspace_bytes > *bytes) *bytes = wp.workspace_bytes;
     return HW_OK;
 }
 

@@ -49,6 +49,7 @@ constexpr int KH_DIRECT = 2;      // one workgroup per kv head and row group: it
 constexpr int KH_STREAM = 8;      // 128-row workgroups that run across row groups: wg_tile counts the tiles of all row groups one
                                   // behind the other, slot_stride = slots of PLAN_SLOT_ROWS rows per kv head, the piece of
                                   // workgroup g in row group rg goes to slot g + rg, a row table for the merge lies behind part_ml
+                                  // (and see KernelArgs::split)
 constexpr int KH_KEEP = 16;       // K/V tiles stay in the L2 for the other row groups (keep_in_l2; read by launch_attention_wide only)
 constexpr int KH_PREROTATED = 4;  // the queries arrive rotated, [F,W,Hq,S,E] (read by the launchers only)
 
@@ -56,6 +57,11 @@ struct KernelArgs {
     KernelHeader h;
     FragTable frag;
     int wg_tile[MAX_SPLITS + 1];   // first tile of each workgroup of a head (same for all heads)
+    // KH_STREAM: row groups split .. split + whole - 1 of a head are dealt whole, every wgs_per_head-th to one workgroup, which writes
+    // their rows to out and lse itself; the runs of wg_tile go over row groups 0 .. split - 1
+    int split, whole;
+    void* out;
+    float* lse;
 };
 
 struct MergeArgs {
@@ -64,6 +70,7 @@ struct MergeArgs {
     void* out;
     float* lse;
     int W, Hq, Hkv, S, R, wgs_per_head;
+    int rows;           // rows 0 .. rows - 1 of every kv head are merged
     int xcd_local;      // kv head h was computed on XCD h / (Hkv/8): merge it there
     // Partials laid out by workgroup slot instead of by row (KH_STREAM, and the paged launch that is planned on the device,
     // see PagedHeader): row_tab[kv head][r] = {first slot | slots << 16, row within the slot}, a slot holds PLAN_SLOT_ROWS rows, pslots

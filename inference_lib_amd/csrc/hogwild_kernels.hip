@@ -324,7 +324,7 @@ __global__ __launch_bounds__(256) void merge_kernel(const MergeArgs a) {
 
     // Workgroups are dealt round-robin over the 8 XCDs.  When the attention kernel kept each kv head on one XCD, merge
     // that head's rows on the same XCD: its partials are then still in that XCD's L2.
-    const int nrb = (a.R + RPW - 1) / RPW;                // row blocks per kv head
+    const int nrb = (a.rows + RPW - 1) / RPW;             // row blocks per kv head
     int hkv, rblk;
     if (a.xcd_local) {
         const int hpx = a.Hkv >> 3;                       // heads per XCD
@@ -338,8 +338,8 @@ __global__ __launch_bounds__(256) void merge_kernel(const MergeArgs a) {
     const int tid = threadIdx.x;
     const int e4 = tid % V4, pg = tid / V4;
     const int rr = pg / GPR, pgl = pg % GPR;               // row within the workgroup, partial group within the row
-    const bool live = rblk * RPW + rr < a.R;
-    const int r = live ? rblk * RPW + rr : a.R - 1;        // (a row that does not exist re-reads the last one and stores nothing)
+    const bool live = rblk * RPW + rr < a.rows;
+    const int r = live ? rblk * RPW + rr : a.rows - 1;       // (a row that does not exist re-reads the last one and stores nothing)
     int ns = a.wgs_per_head;
     const float* ml = a.part_ml + ((size_t)hkv * ns * a.R + r) * 2;
     size_t mstride = (size_t)a.R * 2;
@@ -519,7 +519,7 @@ static hipError_t launch_merge_ev(const MergeArgs& ma, hipStream_t stream) {
     const int ns = ma.wgs_per_head;
     auto go = [&](auto rpw_tag) {
         constexpr int RPW = decltype(rpw_tag)::value;
-        const int blocks = ma.Hkv * ((ma.R + RPW - 1) / RPW);
+        const int blocks = ma.Hkv * ((ma.rows + RPW - 1) / RPW);
         hipLaunchKernelGGL((merge_kernel<DT, EV, RPW>), dim3(blocks), dim3(256), 0, stream, ma);
     };
     if constexpr (NPG >= 8) {       // (eight rows side by side need eight thread groups: not at head dimension 256)

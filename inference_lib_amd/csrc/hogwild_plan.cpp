@@ -332,6 +332,47 @@ void stream_deal(const hw_problem* p, const CallPlan& cp, StreamPlan* sp) {
     }
 }
 
+// Calls with at least a row group for every workgroup of a head (one workgroup per CU).  A run across row groups writes fp32
+// partial sums for both of its ends, 37 MB a layer for 1024 tokens at 40/8 heads, which the merge reads again in 11.6 us.  Here
+// floor(row groups / workgroups) row groups go whole to each workgroup, which holds complete rows at the end and writes the result,
+// and only the remainder is cut into runs (stream_deal), a fifth of the rows with 40 row groups on 32 workgroups.  With no
+// remainder there is no merge launch.  The remainder are the first row groups, which see least of a causal chunk.
+// Against runs, resp. rounds, a layer: 1024 tokens behind 4096 (40/8, D = 128) 124 -> 120 us (two layers, pauses between passes:
+// 248 -> 234), 2 x 574 behind 1333 88 -> 83.5; 1024 behind nothing at 32/8 (no remainder) 71.6 -> 61.5 in rounds, 1500 behind 128
+// 67 -> 60.  All 26 calls timed gained or stayed within the spread, so there is no price to weigh: wherever every workgroup has a
+// row group to itself, runs could only save what they pay for in partial sums.
+bool whole_size(const hw_problem* p, int num_cus, const CallPlan& cp, WholePlan* wp) {
+    const hw_plan& plan = cp.plan[0];
+    if (cp.groups != 1 || p->splits > 0 || plan.row_blocks != hw::WIDE_ROW_BLOCKS || plan.tiles_per_head < 1) return false;
+    const int nrg = plan.row_groups, T = plan.tiles_per_head;
+    int wgs = num_cus / p->Hkv;
+    if (wgs > hw::MAX_SPLITS) wgs = hw::MAX_SPLITS;
+    if (wgs < 1 || nrg < wgs || (long long)nrg * T >= (1ll << 30) || (long long)wgs + nrg >= (1 << 15)) return false;
+    // the kernel divides (head, workgroup) pairs by the workgroups per head (see magic_exact)
+    if ((unsigned long long)wgs * wgs * p->Hkv >= (1ull << 32)) return false;
+    wp->wgs = wgs;
+    wp->split = nrg % wgs;
+    wp->whole = nrg - wp->split;
+    StreamPlan& sp = wp->runs;
+    sp.wgs = wgs;
+    sp.slots = wp->split > 0 ? wgs + wp->split - 1 : 0;
+    const size_t rows = (size_t)sp.slots * hw::PLAN_SLOT_ROWS;
+    sp.partial_bytes = (size_t)p->Hkv * rows * ((size_t)p->Ev + 2) * sizeof(float);
+    sp.workspace_bytes = ((sp.partial_bytes + (size_t)p->Hkv * plan.rows * 2 * sizeof(int) + 255) & ~(size_t)255) + cp.rope_bytes;
+    wp->workspace_bytes = sp.workspace_bytes;
+    return true;
+}
+
+void whole_deal(const hw_problem* p, const CallPlan& cp, WholePlan* wp) {
+    StreamPlan& sp = wp->runs;
+    sp.max_pieces = 0;
+    for (int i = 0; i <= HW_MAX_SPLITS; ++i) sp.wg_tile_begin[i] = 0;
+    if (wp->split == 0) return;
+    CallPlan part = cp;
+    part.plan[0].row_groups = wp->split;
+    stream_deal(p, part, &sp);
+}
+
 int paged_validate(const hw_paged_problem* p) {
     if (p == nullptr) return HW_ERR_NULL;
     if (p->dtype != HW_F32 && p->dtype != HW_F16 && p->dtype != HW_BF16) return HW_ERR_DTYPE;

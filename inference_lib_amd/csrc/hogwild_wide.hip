@@ -183,12 +183,12 @@ struct WideRotation {
     }
 };
 
-// STREAM: the workgroup's run of tiles may cross row groups (KH_STREAM): the whole body is then done once per row group.
-// Prompt chunk of 1024 tokens behind 4096 (40 / 8 heads, D = 128, bf16; 97 GFLOP): two layers with their merges 263-275 us by
-// box, against 341 us in two rounds of workgroups; without a pause between passes, where the shader clock falls, 300-307
-// against 353.  In a kernel trace 131-133 us, 0.73 PFLOP/s, and 12 for the merge.  Bound by the arithmetic of two waves per
-// SIMD: matrix units busy 92 k clocks of each SIMD's 244 k, vector units 119 k (16 exponentials and about 90 others per 32
-// products), the rest waits at the barrier of a step and for issue; LDS is in use a fifth of the time, without conflicts.
+// STREAM: the workgroup's run of tiles may cross row groups, and it may have whole row groups of its own (KH_STREAM): the body is
+// then done once per row group.  Prompt chunk of 1024 tokens behind 4096 (40 / 8 heads, D = 128, bf16; 97 GFLOP): two layers
+// 288 -> 244 us (runs throughout and tiles streamed past the L2 -> whole row groups first and tiles kept, see keep_in_l2 and
+// whole_size), 341 in two rounds of workgroups.  What bounds it is power as much as the arithmetic of two waves per SIMD (matrix
+// units 39 %, vector units 50 % of the clocks): the shader clock follows the load, 2.37 GHz in this form and 2.08-2.12 GHz in one
+// with 32 x 32 x 16 products whose 13 % fewer clocks took the same time.
 template <class DT, int E, int EV, int NS, bool PRE, int NW, int PAR, bool STREAM, bool KEEP>
 __global__ __launch_bounds__(NW * 64, 1) void attention_wide_kernel(const KernelArgs args) {
     typedef Geo<DT, E, EV> G;
@@ -284,7 +284,10 @@ __global__ __launch_bounds__(NW * 64, 1) void attention_wide_kernel(const Kernel
     const int GQ = a.Hq / a.Hkv;
     [[maybe_unused]] const int tiles_head = STREAM ? __builtin_amdgcn_readlane(my_te, MAXF - 1) : 0;   // tiles of a row group
     [[maybe_unused]] const int run_begin = T0, run_end = T1;
-    int rgi = STREAM ? run_begin / tiles_head : rg;
+    // STREAM: first the row groups that are this workgroup's alone, then its run
+    [[maybe_unused]] const int split_groups = STREAM ? args.split : 0, groups = STREAM ? args.split + args.whole : 0;
+    [[maybe_unused]] bool whole = STREAM && split_groups + g < groups;
+    int rgi = STREAM ? (whole ? split_groups + g : run_begin / tiles_head) : rg;
     int r0, w0;                                 // first row of the workgroup, of this wave
     int ws_lo, nws;                             // (worker, token) pairs the rows of this workgroup belong to
     bool staged;                                // their tables go through LDS; uniform over the workgroup
@@ -295,8 +298,8 @@ __global__ __launch_bounds__(NW * 64, 1) void attention_wide_kernel(const Kernel
     // and first fragment are worked out, and are on their way while that happens.
     auto open_rows = [&]() {
         if constexpr (STREAM) {
-            T0 = max(run_begin - rgi * tiles_head, 0);
-            T1 = min(run_end - rgi * tiles_head, tiles_head);
+            T0 = whole ? 0 : max(run_begin - rgi * tiles_head, 0);
+            T1 = whole ? tiles_head : min(run_end - rgi * tiles_head, tiles_head);
         }
         r0 = rgi * WIDE_ROWS;
         w0 = r0 + rw * WROWS;
@@ -419,6 +422,29 @@ __global__ __launch_bounds__(NW * 64, 1) void attention_wide_kernel(const Kernel
             const float lsum = quarter_sum(st.l[rb]);
             const int row0 = w0 + rb * 16;                            // first row of the block
             const size_t prow0 = STREAM ? (size_t)(hkv * a.slot_stride + g + rgi) * PLAN_SLOT_ROWS + (row0 - r0) : (size_t)(hkv * a.slot_stride + g) * a.R + row0;
+            // STREAM, a row group of this workgroup's alone: the rows are complete, and leave normalised as the operator's result
+            // (with the arithmetic of the merge kernel on a single partial)
+            if constexpr (STREAM) {
+                if (whole) {
+                    const float inv = lsum > 0.f ? 1.0f / lsum : 0.f;
+#pragma unroll
+                    for (int c = 0; c < G::NOC; ++c)
+                        *reinterpret_cast<f32x4*>(stage + n * OSTR + 16 * c + 4 * q) = st.o[rb][c] * inv;
+                    if (args.lse != nullptr && q == 0 && row0 + n < a.R)
+                        reinterpret_cast<HW_GLOBAL float*>(reinterpret_cast<unsigned long long>(args.lse))[map_row(a, row0 + n, hkv, GQ).qrow] =
+                            lsum > 0.f ? (st.m[rb] + __builtin_amdgcn_logf(lsum)) * 0.69314718055994530942f : -__builtin_inff();
+                    HW_GLOBAL char* ob = reinterpret_cast<HW_GLOBAL char*>(reinterpret_cast<unsigned long long>(args.out));
+#pragma unroll
+                    for (int ps = 0; ps < 16 * EV / 512; ++ps) {      // 64 lanes x 8 elements per pass
+                        const int idx = ps * 512 + lane * 8;
+                        const int rr = idx / EV, e = idx % EV;
+                        const f32x4 lo = *reinterpret_cast<const f32x4*>(stage + rr * OSTR + e), hi = *reinterpret_cast<const f32x4*>(stage + rr * OSTR + e + 4);
+                        const float x[8] = {lo.x, lo.y, lo.z, lo.w, hi.x, hi.y, hi.z, hi.w};
+                        if (row0 + rr < a.R) *reinterpret_cast<HW_GLOBAL u32x4*>(ob + (map_row(a, row0 + rr, hkv, GQ).qrow * EV + e) * G::SZ) = Chunk<DT>::pack(x);
+                    }
+                    continue;
+                }
+            }
 #pragma unroll
             for (int c = 0; c < G::NOC; ++c)              // block c, accumulator rows 4q .. 4q+3 = elements 16c + 4q ..
                 *reinterpret_cast<f32x4*>(stage + n * OSTR + 16 * c + 4 * q) = st.o[rb][c];
@@ -562,9 +588,16 @@ __global__ __launch_bounds__(NW * 64, 1) void attention_wide_kernel(const Kernel
             open_segment(false);
         } else if constexpr (STREAM) {
             store_rows();
-            write_row_table();
-            ++rgi;
-            if (rgi * tiles_head < run_end) {          // the run goes on in the next row group
+            if (!whole) {
+                write_row_table();
+                ++rgi;
+            } else if (rgi + a.wgs_per_head < groups) {
+                rgi += a.wgs_per_head;
+            } else {
+                whole = false;
+                rgi = run_begin / tiles_head;
+            }
+            if (whole || max(run_begin, rgi * tiles_head) < run_end) {          // the next row group
                 __syncthreads();                       // every wave is done with the ring
                 open_rows();
                 open_segment(staged);
@@ -581,8 +614,15 @@ __global__ __launch_bounds__(NW * 64, 1) void attention_wide_kernel(const Kernel
     if (!PRE && a.rq != nullptr && (STREAM || g == 0)) {
         const unsigned long long all_empty = __ballot(lane < a.F && my_len == 0);
         unsigned long long empty = all_empty;
-        if constexpr (STREAM) rgi = (run_begin + tiles_head - 1) / tiles_head;
-        while (empty != 0 && (!STREAM || rgi * tiles_head < run_end)) {
+        if constexpr (STREAM) {
+            whole = false;
+            rgi = (run_begin + tiles_head - 1) / tiles_head;
+            if (rgi * tiles_head >= run_end) {
+                whole = true;
+                rgi = split_groups + g;
+            }
+        }
+        while (empty != 0 && (!STREAM || !whole || rgi < groups)) {
             f = __builtin_ctzll(empty);
             empty &= empty - 1;
             __syncthreads();
@@ -591,7 +631,12 @@ __global__ __launch_bounds__(NW * 64, 1) void attention_wide_kernel(const Kernel
             qempty.finish(a, q_lds, f, hkv, rgi * WIDE_ROWS, GQ, true, tid);
             if (STREAM && empty == 0) {
                 empty = all_empty;
-                ++rgi;
+                if (whole) {
+                    rgi += a.wgs_per_head;
+                } else if (++rgi * tiles_head >= run_end) {
+                    whole = true;
+                    rgi = split_groups + g;
+                }
             }
         }
     }
