@@ -78,6 +78,8 @@ int run(const hw_problem* p, void* stream_, int fused, int stages = HW_STAGE_ATT
     if (whole) {
         whole_deal(p, cp, &wp);
         sp = wp.runs;
+        cp.plan[0].row_blocks = hw::WIDE_ROW_BLOCKS;        // (at head dimension 256 the plan is the narrow kernel's)
+        cp.plan[0].row_groups = wp.split + wp.whole;
     } else if (stream_runs) {
         stream_deal(p, cp, &sp);
     }
@@ -173,7 +175,7 @@ int run(const hw_problem* p, void* stream_, int fused, int stages = HW_STAGE_ATT
     }
     if (!(stages & HW_STAGE_MERGE) || direct || (whole && wp.split == 0)) return (int)e;
     hw::MergeArgs ma;
-    ma.rows = whole ? wp.split * hw::PLAN_SLOT_ROWS : rows;
+    ma.rows = whole && wp.whole > 0 ? wp.split * hw::PLAN_SLOT_ROWS : rows;    // (the last row group may have fewer)
     ma.part_o = part_o;
     ma.part_ml = part_ml;
     ma.out = p->out;

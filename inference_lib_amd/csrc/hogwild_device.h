@@ -277,12 +277,12 @@ __device__ __forceinline__ void wait_k_landed() {
 // V image for transposed reads (the kernels whose waves share every tile, 16-bit types): rows of VROW bytes, the 32-byte
 // segments of a row (16 elements: what one MFMA block of outputs needs) stored at segment ^ key(row), the key chosen so
 // that the eight consecutive rows two neighbouring 16-lane groups read (2 x 4 rows x 32 bytes) cover all 64 banks:
-// rows of 256 bytes start at bank 0, so the key is row & 7; rows of 128 bytes alternate between the two halves of the
+// rows of 256 and 512 bytes start at bank 0, so the key is row & 7; rows of 128 bytes alternate between the two halves of the
 // banks by themselves and the key is (row >> 1) & 3.
 template <int VROW>
 __device__ __forceinline__ int vimg_segment_key(int row) {
-    static_assert(VROW == 256 || VROW == 128, "head dims 128 and 64 in 16-bit types");
-    return VROW == 256 ? (row & 7) : ((row >> 1) & 3);
+    static_assert(VROW == 512 || VROW == 256 || VROW == 128, "head dims 256, 128 and 64 in 16-bit types");
+    return VROW >= 256 ? (row & 7) : ((row >> 1) & 3);
 }
 
 typedef short v4i16 __attribute__((ext_vector_type(4)));
@@ -928,9 +928,9 @@ struct LaneRotation {
         const size_t fstride = (size_t)a.W * a.Hq * a.S * E;
 #pragma unroll
         for (int rb = 0; rb < RB; ++rb) {
-            // rows beyond R (MFMA padding) read the first row: harmless, and keeps the loads unconditional
+            // rows beyond R (MFMA padding) read the last row: harmless, and keeps the loads unconditional
             const int row = r0 + rb * 16 + n;
-            const RowMap rm = map_row(a, row < a.R ? row : r0, hkv, GQ);
+            const RowMap rm = map_row(a, min(row, a.R - 1), hkv, GQ);
             const HW_GLOBAL char* qp = a.q + (rm.qrow * E + (PRE ? f * fstride : 0)) * SZ;
 #pragma unroll
             for (int j = 0; j < KJ; ++j) x[rb][j] = *reinterpret_cast<const HW_GLOBAL u32x4*>(qp + (4 * j + q) * 16);

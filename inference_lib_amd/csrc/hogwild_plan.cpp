@@ -341,13 +341,22 @@ void stream_deal(const hw_problem* p, const CallPlan& cp, StreamPlan* sp) {
 // 248 -> 234), 2 x 574 behind 1333 88 -> 83.5; 1024 behind nothing at 32/8 (no remainder) 71.6 -> 61.5 in rounds, 1500 behind 128
 // 67 -> 60.  All 26 calls timed gained or stayed within the spread, so there is no price to weigh: wherever every workgroup has a
 // row group to itself, runs could only save what they pay for in partial sums.
+// Head dimension 256: the plan's kernel takes 16 rows a workgroup, so every 16 rows stream the K/V through a CU again.  Enough of
+// that, counted in tiles a CU takes in, and 128-row workgroups are faster, whose openings cost more (a launch of them takes about
+// 25 us whatever it holds).  16/8 heads, bf16, us a layer before / after: 1024 tokens behind 4096 (640 tiles a CU) 296 -> 111, 1500
+// behind 100 168 -> 70, 2 x 200 behind 5000 154 -> 79, 2 x 300 behind 500 (84) 75 -> 43, 100 behind 5000 (65) 50 -> 33, 150 behind 3000
+// (59) 49 -> 36; below the line 2 x 128 behind 1500 (55) 34 -> 36.5, 256 behind 1000 (40) 24 -> 35.5.
+constexpr int kWide256Visits = 56;
 bool whole_size(const hw_problem* p, int num_cus, const CallPlan& cp, WholePlan* wp) {
     const hw_plan& plan = cp.plan[0];
-    if (cp.groups != 1 || p->splits > 0 || plan.row_blocks != hw::WIDE_ROW_BLOCKS || plan.tiles_per_head < 1) return false;
-    const int nrg = plan.row_groups, T = plan.tiles_per_head;
+    if (cp.groups != 1 || p->splits > 0 || plan.tiles_per_head < 1) return false;
+    const bool wide_256 = p->E == 256 && p->dtype != HW_F32 && p->len_dev == nullptr && p->row_blocks == 0 &&
+                          (long long)plan.row_groups * plan.tiles_per_head * p->Hkv >= (long long)kWide256Visits * num_cus;
+    if (plan.row_blocks != hw::WIDE_ROW_BLOCKS && !wide_256) return false;
+    const int nrg = (plan.rows + hw::PLAN_SLOT_ROWS - 1) / hw::PLAN_SLOT_ROWS, T = plan.tiles_per_head;
     int wgs = num_cus / p->Hkv;
     if (wgs > hw::MAX_SPLITS) wgs = hw::MAX_SPLITS;
-    if (wgs < 1 || nrg < wgs || (long long)nrg * T >= (1ll << 30) || (long long)wgs + nrg >= (1 << 15)) return false;
+    if (wgs < 1 || (nrg < wgs && !wide_256) || (long long)nrg * T >= (1ll << 30) || (long long)wgs + nrg >= (1 << 15)) return false;
     // the kernel divides (head, workgroup) pairs by the workgroups per head (see magic_exact)
     if ((unsigned long long)wgs * wgs * p->Hkv >= (1ull << 32)) return false;
     wp->wgs = wgs;

@@ -208,10 +208,12 @@ __global__ __launch_bounds__(NW * 64, 1) void attention_wide_kernel(const Kernel
                       NW % PAR == 0 && (PAR == 1 || PAR == 2),
                   "16-bit types; a wave's transfers belong to one image");
 
-    __shared__ __attribute__((aligned(16))) char q_lds[WIDE_ROWS * G::QSTR];
-    __shared__ int lim_lds[WIDE_ROWS];
+    // Head dimension 256: every wave loads and rotates its own operands in registers (LaneRotation), the ring takes the LDS.
+    constexpr bool LANES = E > 128;
+    __shared__ __attribute__((aligned(16))) char q_lds[LANES ? 16 : WIDE_ROWS * G::QSTR];
+    __shared__ int lim_lds[LANES ? 1 : WIDE_ROWS];
     typedef WideRotation<DT, E, G::QSTR, NT> WRot;
-    __shared__ __attribute__((aligned(16))) float cs_lds[PRE ? 4 : WRot::CS_FLOATS];
+    __shared__ __attribute__((aligned(16))) float cs_lds[PRE || LANES ? 4 : WRot::CS_FLOATS];
     // ring slots: [K image | V image]; K is swizzled like in the narrow kernel, V is a plain row-major image
     __shared__ __attribute__((aligned(16))) char ring[NS * SLOT];
 
@@ -305,7 +307,7 @@ __global__ __launch_bounds__(NW * 64, 1) void attention_wide_kernel(const Kernel
         w0 = r0 + rw * WROWS;
         ws_lo = fast_div(r0, a.magic_gq);
         nws = fast_div(min(r0 + WIDE_ROWS, a.R) - 1, a.magic_gq) - ws_lo + 1;
-        staged = !PRE && nws <= WRot::CSMAX;
+        staged = !PRE && !LANES && nws <= WRot::CSMAX;
         int tids = tid;
         if constexpr (STREAM) asm volatile("" : "+v"(tids));      // (see open_segment)
         if (staged) wrot.load_queries(a, hkv, r0, GQ, tids);
@@ -326,6 +328,7 @@ __global__ __launch_bounds__(NW * 64, 1) void attention_wide_kernel(const Kernel
     bool opens_fragment = false;
     u32x4 view = {0, 0, 0, 0};                               // this wave's image of the current fragment (K or V slice)
     [[maybe_unused]] QueryRotation<DT, E, WIDE_ROWS, G::QSTR, true, NT> qrot;     // pre-rotated queries: a copy into LDS
+    [[maybe_unused]] LaneRotation<DT, E, RB, PRE> lrot;
     int lm = 0;
 
     // this wave's share of the PAR tiles of the step that starts at tile `lt` (fragment-local) into step slot `ss`; a tile
@@ -362,7 +365,10 @@ __global__ __launch_bounds__(NW * 64, 1) void attention_wide_kernel(const Kernel
         // would stay in registers across the tile loops, which have none to spare)
         int tids = tid;
         asm volatile("" : "+v"(tids));
-        if constexpr (PRE) {
+        if constexpr (LANES) {
+            lrot.load(a, f, hkv, w0, GQ, tids & 15, (tids >> 4) & 3);
+            return;
+        } else if constexpr (PRE) {
             qrot.load(a, f, hkv, r0, GQ, tids);
         } else if (staged) {
             if (!queries_requested) wrot.load_queries(a, hkv, r0, GQ, tids);
@@ -481,7 +487,7 @@ __global__ __launch_bounds__(NW * 64, 1) void attention_wide_kernel(const Kernel
     bool hw_first = true;
 
     while (more) {
-        __syncthreads();   // previous segment's readers are done with q_lds / lim_lds
+        if constexpr (!LANES) __syncthreads();   // previous segment's readers are done with q_lds / lim_lds
         if (hw_first) HW_MARK(7);
         int tids = tid;        // (see open_segment)
         asm volatile("" : "+v"(tids));
@@ -490,6 +496,13 @@ __global__ __launch_bounds__(NW * 64, 1) void attention_wide_kernel(const Kernel
         // below, the last load of open_segment -- would also wait for the look-ahead steps requested in between.
         // (Nothing is lost: the queries are needed now, and the first step was requested before them.)
         __builtin_amdgcn_s_waitcnt(0x0F70);   // vmcnt(0)
+        u32x4 qreg[RB * G::KJ];                      // this wave's query operands and mask bounds
+        int lim[RB];
+        if constexpr (LANES) {
+#pragma unroll
+            for (int i = 1; i < DP; ++i) request(i, lt0 + i * PAR);
+            lrot.finish(a, qreg, lim, f, hkv, w0, GQ, L, a.rq != nullptr && opens_fragment, tids & 15, (tids >> 4) & 3);
+        } else {
         int limv = (r0 + tids / TPR < a.R) ? min(L, max(0, lm + 1)) : 0x7fffffff;   // by every thread, see paged_wide_kernel
         asm volatile("" : "+v"(limv));
         if (!PRE && staged) {
@@ -523,25 +536,24 @@ __global__ __launch_bounds__(NW * 64, 1) void attention_wide_kernel(const Kernel
         asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
         if (hw_first) HW_MARK(1);
 
-        // this wave's query operands and mask bounds
-        u32x4 qreg[RB * G::KJ];
 #pragma unroll
-        for (int rb = 0; rb < RB; ++rb)
+        for (int rb = 0; rb < RB; ++rb) {
 #pragma unroll
             for (int j = 0; j < G::KJ; ++j)
                 qreg[rb * G::KJ + j] = *reinterpret_cast<const u32x4*>(q_lds + (rw * WROWS + rb * 16 + n) * G::QSTR + (4 * j + q) * 16);
-        int lim[RB];
+            lim[rb] = lim_lds[rw * WROWS + rb * 16 + n];
+        }
+        }
         int maxlim = 0, minlim = 0x7fffffff;
 #pragma unroll
         for (int rb = 0; rb < RB; ++rb) {
-            lim[rb] = lim_lds[rw * WROWS + rb * 16 + n];
             const bool pad = w0 + rb * 16 + n >= a.R;
             maxlim = max(maxlim, pad ? 0 : lim[rb]);
             minlim = min(minlim, lim[rb]);
         }
         maxlim = __builtin_amdgcn_readfirstlane(row_max16(maxlim));
         minlim = __builtin_amdgcn_readfirstlane(row_min16(minlim));
-        if (PRE || !staged) {
+        if (!LANES && (PRE || !staged)) {
 #pragma unroll
             for (int i = 1; i < DP; ++i) request(i, lt0 + i * PAR);
         }
@@ -628,7 +640,7 @@ __global__ __launch_bounds__(NW * 64, 1) void attention_wide_kernel(const Kernel
             __syncthreads();
             QueryRotation<DT, E, WIDE_ROWS, G::QSTR, PRE, NT> qempty;
             qempty.load(a, f, hkv, rgi * WIDE_ROWS, GQ, tid);
-            qempty.finish(a, q_lds, f, hkv, rgi * WIDE_ROWS, GQ, true, tid);
+            qempty.finish(a, LANES ? nullptr : q_lds, f, hkv, rgi * WIDE_ROWS, GQ, true, tid);
             if (STREAM && empty == 0) {
                 empty = all_empty;
                 if (whole) {
@@ -1246,11 +1258,33 @@ constexpr int WIDE_WAVES = 8;
 constexpr int WIDE_PAR = 2;
 constexpr int WIDE_SLOTS = 6;
 
+// Head dimension 256: a tile is 32 KB and a lane's accumulators of 32 rows are 128 registers, so four waves of 32 rows, one per SIMD
+// with 512 registers, that all take every tile, and a ring of four slots.
+constexpr int WIDE256_WAVES = 4;
+constexpr int WIDE256_SLOTS = 4;
+
+template <class DT>
+static hipError_t launch_wide_256(const KernelArgs& ka, hipStream_t stream) {
+    if (!(ka.h.flags & KH_STREAM)) return hipErrorInvalidValue;
+    auto go = [&](auto pre, auto keep) {
+        hipLaunchKernelGGL((attention_wide_kernel<DT, 256, 256, WIDE256_SLOTS, decltype(pre)::value, WIDE256_WAVES, 1, true, decltype(keep)::value>),
+                           dim3(ka.h.nwg), dim3(WIDE256_WAVES * 64), 0, stream, ka);
+    };
+    auto by_keep = [&](auto pre) {
+        if (ka.h.flags & KH_KEEP) go(pre, std::true_type{});
+        else go(pre, std::false_type{});
+    };
+    if (ka.h.flags & KH_PREROTATED) by_keep(std::true_type{});
+    else by_keep(std::false_type{});
+    return hipGetLastError();
+}
+
 template <class DT>
 static hipError_t launch_wide_dt(const KernelArgs& ka, int E, hipStream_t stream) {
     constexpr int NS = WIDE_SLOTS;
     constexpr int NW = WIDE_WAVES;
     constexpr int PAR = WIDE_PAR;
+    if (E == 256) return launch_wide_256<DT>(ka, stream);
     if (E != 64 && E != 128) return hipErrorInvalidValue;
     auto go = [&](auto head_dim, auto pre, auto stream_runs) {
         constexpr int HD = decltype(head_dim)::value;

@@ -12,7 +12,7 @@
 int main() {
     std::mt19937 rng(7);
     auto pick = [&](int lo, int hi) { return (int)(lo + rng() % (unsigned)(hi - lo + 1)); };
-    int taken = 0, left_over = 0;
+    int taken = 0, left_over = 0, taken_256 = 0;
     for (int it = 0; it < 20000; ++it) {
         hw_problem p{};
         p.dtype = pick(0, 2);
@@ -24,6 +24,7 @@ int main() {
         p.E = p.Ev = 64 << pick(0, 2);
         p.RotE = pick(0, 3) == 0 ? 32 : p.E;
         p.splits = pick(0, 9) == 0 ? 2 : 0;
+        p.row_blocks = p.E == 256 && pick(0, 9) == 0 ? 1 : 0;
         std::vector<int32_t> len(p.F);
         for (auto& n : len) n = pick(0, 4) == 0 ? pick(0, 3) : pick(0, 9000);
         p.len = len.data();
@@ -35,10 +36,13 @@ int main() {
         ++taken;
         hw::host::whole_deal(&p, cp, &wp);
         const hw::host::StreamPlan& sp = wp.runs;
-        const int T = cp.plan[0].tiles_per_head, nrg = cp.plan[0].row_groups;
-        CHECK(cp.groups == 1 && p.splits == 0 && T > 0 && cp.plan[0].row_blocks == hw::WIDE_ROW_BLOCKS);
+        const bool wide_256 = p.E == 256;           // its plan is the 16-row kernel's, and may have fewer row groups than workgroups
+        const int T = cp.plan[0].tiles_per_head, nrg = (cp.plan[0].rows + hw::PLAN_SLOT_ROWS - 1) / hw::PLAN_SLOT_ROWS;
+        CHECK(cp.groups == 1 && p.splits == 0 && T > 0 && p.dtype != HW_F32 && p.row_blocks == 0);
+        CHECK(wide_256 ? cp.plan[0].row_blocks == 1 : cp.plan[0].row_blocks == hw::WIDE_ROW_BLOCKS && cp.plan[0].row_groups == nrg && wp.whole > 0);
+        taken_256 += wide_256;
         CHECK(wp.wgs >= 1 && wp.wgs <= HW_MAX_SPLITS && (long long)wp.wgs * p.Hkv <= cus);
-        CHECK(wp.split >= 0 && wp.whole >= wp.wgs && wp.whole % wp.wgs == 0 && wp.split < wp.wgs && wp.split + wp.whole == nrg);
+        CHECK(wp.split >= 0 && wp.whole >= 0 && wp.whole % wp.wgs == 0 && wp.split < wp.wgs && wp.split + wp.whole == nrg);
         CHECK(sp.wg_tile_begin[0] == 0 && sp.wg_tile_begin[wp.wgs] == wp.split * T);
         std::vector<char> used(sp.slots > 0 ? sp.slots : 1, 0);
         std::vector<int> pieces(wp.split > 0 ? wp.split : 1, 0);
@@ -56,6 +60,6 @@ int main() {
         const size_t part = (size_t)p.Hkv * sp.slots * hw::PLAN_SLOT_ROWS * (p.Ev + 2) * 4;
         CHECK(sp.partial_bytes == part && wp.workspace_bytes >= part + (size_t)p.Hkv * cp.plan[0].rows * 8 + cp.rope_bytes && wp.workspace_bytes % 256 == 0);
     }
-    std::printf("%d calls, %d with row groups left over\n", taken, left_over);
-    return taken > 500 && left_over > 250 ? 0 : 1;
+    std::printf("%d calls, %d with row groups left over, %d of head dimension 256\n", taken, left_over, taken_256);
+    return taken > 500 && left_over > 250 && taken_256 > 100 ? 0 : 1;
 }
