@@ -28,6 +28,7 @@ from .attention import HAVE_TORCH_OPS
 if HAVE_TORCH_OPS:
     _rope_append = torch.ops.libhogatt.rope_append.default
     _segment_views = torch.ops.libhogatt.segment_views.default
+    _step_inputs = torch.ops.libhogatt.step_inputs.default
 
 
 class _LayerViews:
@@ -294,11 +295,17 @@ class HogwildCache:
                     pos += cs.get_seq_length(layer_idx)
                     pos_end[index[id(cs)]][w] = pos
             tdt = self.table_dtype if self.table_dtype is not None else key_states.dtype
-            self.locations, self.cosines, self.sines = _lib.build_inputs(
-                pos_end, S, self.inv_freq.to(key_states.device), attention_scaling=self.attention_scaling,
-                table_dtype=None if tdt == torch.float32 else tdt)
+            inv_freq, lens = self.inv_freq.to(key_states.device), [cs.get_seq_length(layer_idx) for cs in segments]
+            done = False
+            if HAVE_TORCH_OPS and inv_freq.is_cuda:         # (False for what it does not take, which _lib handles or refuses)
+                done, loc, cos, sin, frags = _step_inputs([x for row in pos_end for x in row], lens, S, inv_freq, self.attention_scaling, tdt)
+            if not done:
+                loc, cos, sin = _lib.build_inputs(pos_end, S, inv_freq, attention_scaling=self.attention_scaling,
+                                                  table_dtype=None if tdt == torch.float32 else tdt)
+                frags = torch.tensor(lens, dtype=torch.int32, device=key_states.device)
+            self.locations, self.cosines, self.sines = loc, cos, sin
             self.segments = segments
-            self.frags = torch.tensor([cs.get_seq_length(layer_idx) for cs in segments], dtype=torch.int32, device=key_states.device)
+            self.frags = frags
         # views; no .contiguous() copies (attention.py:160-162,199-203)
         keys, vals = _fragments(self.segments, layer_idx)
         return CacheStructure(keys=keys, values=vals, cos=self.cosines, sin=self.sines, loc=self.locations, frags=self.frags)

@@ -209,6 +209,14 @@ void hogwild_sdpa(at::Tensor& out, double scale, const at::Tensor& locations, co
     run(u, out, false);
 }
 
+void hogwild_sdpa_any(at::Tensor& out, double scale, const at::Tensor& locations, const at::Tensor& queries,
+                      const at::Tensor& fragment_lengths, const std::vector<at::Tensor>& key_fragments,
+                      const std::vector<at::Tensor>& value_fragments) {
+    Unpacked u;
+    unpack_common(u, out, scale, locations, queries, fragment_lengths, key_fragments, value_fragments, true, true);
+    run(u, out, false);
+}
+
 void hogwild_sdpa_lse(at::Tensor& out, at::Tensor& lse, double scale, const at::Tensor& locations, const at::Tensor& queries,
                       const at::Tensor& fragment_lengths, const std::vector<at::Tensor>& key_fragments,
                       const std::vector<at::Tensor>& value_fragments) {
@@ -526,6 +534,42 @@ std::vector<at::Tensor> segment_views(at::TensorList buffers, at::IntArrayRef le
     return out;
 }
 
+// What HogwildCache hands the attention in a step: locations [F, W, S], tables [F, W, S, RotE] and fragment lengths [F], from host
+// numbers in the kernel arguments (hw_build_inputs; the lengths are the locations of one worker with one token).  A host-to-device
+// copy of the lengths waits for the stream, i.e. for the step before, and with the rest through Python took 38 us a step.
+// Returns false, with nothing queued, for what the checks or the library refuse: the caller's general path then names it.
+std::tuple<bool, at::Tensor, at::Tensor, at::Tensor, at::Tensor> step_inputs(at::IntArrayRef pos_end, at::IntArrayRef len, int64_t S,
+                                                                             const at::Tensor& inv_freq, double scaling, at::ScalarType table_dtype) {
+    const int64_t F = (int64_t)len.size(), W = F > 0 ? (int64_t)pos_end.size() / F : 0;
+    const std::tuple<bool, at::Tensor, at::Tensor, at::Tensor, at::Tensor> refused;
+    if (F < 1 || W < 1 || F * W != (int64_t)pos_end.size() || F >= (1 << 20) || W >= (1 << 20) || S < 1 || S >= (1 << 20)) return refused;
+    if (inv_freq.dim() != 1 || inv_freq.scalar_type() != at::kFloat || !inv_freq.is_contiguous() || inv_freq.numel() >= (1 << 20)) return refused;
+    if (table_dtype != at::kFloat && table_dtype != at::kHalf && table_dtype != at::kBFloat16) return refused;
+    std::vector<int32_t> ends(pos_end.size()), lens(F);
+    for (size_t i = 0; i < pos_end.size(); ++i) {
+        if (pos_end[i] < 0 || pos_end[i] >= (1ll << 31)) return refused;
+        ends[i] = (int32_t)pos_end[i];
+    }
+    for (int64_t f = 0; f < F; ++f) {
+        if (len[f] < 0 || len[f] >= (1ll << 31) - 1) return refused;
+        lens[f] = (int32_t)len[f] + 1;
+    }
+    const int64_t rot = 2 * inv_freq.numel();
+    c10::hip::HIPGuardMasqueradingAsCUDA guard(inv_freq.device());
+    const auto ints = inv_freq.options().dtype(at::kInt);
+    at::Tensor loc = at::empty({F, W, S}, ints), cos = at::empty({F, W, S, rot}, inv_freq.options()), sin = at::empty({F, W, S, rot}, inv_freq.options());
+    at::Tensor frags = at::empty({F}, ints);
+    hipStream_t stream = c10::hip::getCurrentHIPStreamMasqueradingAsCUDA(inv_freq.device().index()).stream();
+    const int round = table_dtype == at::kFloat ? HW_F32 : table_dtype == at::kHalf ? HW_F16 : HW_BF16;
+    int status = hw_build_inputs(loc.data_ptr<int32_t>(), cos.data_ptr<float>(), sin.data_ptr<float>(), ends.data(), inv_freq.const_data_ptr<float>(),
+                                 (float)scaling, round, (int)F, (int)W, (int)S, (int)rot, stream);
+    if (status < 0) return refused;
+    check_status(status, "step_inputs");
+    status = hw_build_inputs(frags.data_ptr<int32_t>(), nullptr, nullptr, lens.data(), nullptr, 1.0f, HW_F32, (int)F, 1, 1, 0, stream);
+    check_status(status, "step_inputs");
+    return {true, loc, cos, sin, frags};
+}
+
 }  // namespace
 
 // `import hogatt` only has to load this shared object so that the registrations below run.
@@ -562,6 +606,11 @@ TORCH_LIBRARY(libhogatt, m) {
     m.def("rope_append(Tensor(a!)[] k_dst, Tensor(b!)[] v_dst, int[] dst_len, int[] n_new, Tensor key_states, Tensor value_states, "
           "Tensor? cosines, Tensor? sines, int mode) -> bool", tags);
     m.def("segment_views(Tensor(a)[] buffers, int[] len) -> Tensor(a)[]", tags);
+    m.def("step_inputs(int[] pos_end, int[] len, int S, Tensor inv_freq, float scaling, ScalarType table_dtype) -> "
+          "(bool, Tensor, Tensor, Tensor, Tensor)", tags);
+    // addition: hogwild_sdpa that copies fragments it cannot read in place, as the reference's wrapper does (:32-33)
+    m.def("hogwild_sdpa_any(Tensor(a!) output, float scale, Tensor locations, Tensor queries, "
+          "Tensor fragment_lengths, Tensor[] key_fragments, Tensor[] value_fragments) -> ()", tags);
 }
 
 TORCH_LIBRARY_IMPL(libhogatt, CUDA, m) {
@@ -577,4 +626,6 @@ TORCH_LIBRARY_IMPL(libhogatt, CUDA, m) {
     m.impl("merge_segments", merge_segments);
     m.impl("rope_append", rope_append);
     m.impl("segment_views", segment_views);
+    m.impl("step_inputs", step_inputs);
+    m.impl("hogwild_sdpa_any", hogwild_sdpa_any);
 }
