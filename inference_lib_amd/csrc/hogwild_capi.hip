@@ -237,7 +237,7 @@ int paged_run(const hw_paged_problem* p, void* stream_, int stages) {
     ph.nitems = plan.row_groups;
     ph.nrg = varlen ? 1 : plan.row_groups / p->W;
     ph.nwg = plan.workgroups;
-    ph.flags = ((plan.workgroups % 8 == 0) ? hw::PH_XCD_REMAP : 0) | (planned ? hw::PH_PLANNED : 0);
+    ph.flags = ((plan.workgroups % 8 == 0) ? hw::PH_XCD_REMAP : 0) | (planned ? hw::PH_PLANNED : 0) | (paged_keep_in_l2(p, plan) ? hw::PH_KEEP : 0);
     ph.sc = (float)((double)p->scale * 1.4426950408889634074);
     ph.magic_gq = magic(p->Hq / p->Hkv);
     ph.magic_ls = magic(ph.LS);

@@ -119,6 +119,7 @@ constexpr int PH_XCD_REMAP = 1;    // consecutive logical workgroup ids share an
 // kv head, and what slot j of a head does -- which row group of which sequence, which share of its tiles -- every
 // workgroup works out for itself from the query and KV lengths (plan_slot).  Behind part_ml the workgroups leave the
 // merge kernel a table per kv head of where each row's partial sums lie (MergeArgs::row_tab).
+constexpr int PH_KEEP = 4;         // K/V tiles stay in the L2 for the other row groups of a sequence (read by launch_paged_attention only)
 constexpr int PH_PLANNED = 2;
 
 struct CopyBlocksArgs {

@@ -33,8 +33,9 @@
 
 namespace hw {
 
-template <class DT, int E, int EV, int RB, int MINW>
+template <class DT, int E, int EV, int RB, int MINW, bool KEEP = false>
 __global__ __launch_bounds__(NTHREADS, MINW) void paged_attention_kernel(const PagedHeader args) {
+    constexpr int AUX = KEEP ? 0 : HW_KV_AUX;
     typedef Geo<DT, E, EV> G;
     constexpr int ROWS = RB * 16;
     typedef hw::Exchange<ROWS, EV> Ex;
@@ -172,7 +173,7 @@ __global__ __launch_bounds__(NTHREADS, MINW) void paged_attention_kernel(const P
             for (int i = 0; i < G::KL; ++i) {
                 const int r = __shfl(rid, i * RPL + lrow, 64);
                 const HW_GLOBAL char* src = ph.kcache + (unsigned long long)(unsigned)r * G::KROW + k_chunk(i);
-                __builtin_amdgcn_global_load_lds(src, HW_LDS_PTR(kslot + i * 1024), 16, 0, HW_KV_AUX);
+                __builtin_amdgcn_global_load_lds(src, HW_LDS_PTR(kslot + i * 1024), 16, 0, AUX);
             }
             asm volatile("" ::: "memory");
 #pragma unroll
@@ -182,14 +183,14 @@ __global__ __launch_bounds__(NTHREADS, MINW) void paged_attention_kernel(const P
 #pragma unroll
                 for (int hh = 0; hh < G::NVL; ++hh) {
                     if constexpr (G::VLD == 4) {
-                        const u32x4 x = HW_KV_AUX == 2 ? __builtin_nontemporal_load(reinterpret_cast<const HW_GLOBAL u32x4*>(src + hh * 256))
+                        const u32x4 x = AUX == 2 ? __builtin_nontemporal_load(reinterpret_cast<const HW_GLOBAL u32x4*>(src + hh * 256))
                                                         : *reinterpret_cast<const HW_GLOBAL u32x4*>(src + hh * 256);
                         tr.v[idx][hh * 4 + 0] = x.x;
                         tr.v[idx][hh * 4 + 1] = x.y;
                         tr.v[idx][hh * 4 + 2] = x.z;
                         tr.v[idx][hh * 4 + 3] = x.w;
                     } else {
-                        const u32x2 x = HW_KV_AUX == 2 ? __builtin_nontemporal_load(reinterpret_cast<const HW_GLOBAL u32x2*>(src))
+                        const u32x2 x = AUX == 2 ? __builtin_nontemporal_load(reinterpret_cast<const HW_GLOBAL u32x2*>(src))
                                                         : *reinterpret_cast<const HW_GLOBAL u32x2*>(src);
                         tr.v[idx][0] = x.x;
                         tr.v[idx][1] = x.y;
@@ -307,7 +308,8 @@ static hipError_t launch_paged_dt(const PagedHeader& ph, int E, int rb, hipStrea
     if (E == 256) {     // one 16-row block per workgroup, one wave per SIMD; 16-bit types (two fp32 K tiles per wave exceed the LDS)
         if constexpr (Elem<DT>::size == 2) {
             if (rb != 1) return hipErrorInvalidValue;
-            hipLaunchKernelGGL((paged_attention_kernel<DT, 256, 256, 1, 1>), dim3(ph.nwg), dim3(NTHREADS), 0, stream, ph);
+            if (ph.flags & PH_KEEP) hipLaunchKernelGGL((paged_attention_kernel<DT, 256, 256, 1, 1, true>), dim3(ph.nwg), dim3(NTHREADS), 0, stream, ph);
+            else hipLaunchKernelGGL((paged_attention_kernel<DT, 256, 256, 1, 1>), dim3(ph.nwg), dim3(NTHREADS), 0, stream, ph);
             return hipGetLastError();
         }
         return hipErrorInvalidValue;

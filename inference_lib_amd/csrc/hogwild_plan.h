@@ -68,6 +68,8 @@ bool whole_size(const hw_problem* p, int num_cus, const CallPlan& cp, WholePlan*
 void whole_deal(const hw_problem* p, const CallPlan& cp, WholePlan* wp);
 int paged_validate(const hw_paged_problem* p);
 int paged_plan(const hw_paged_problem* p, int num_cus, hw_paged_plan* plan);
+// Whether the tiles of a paged launch are to stay in the L2 (hogwild_plan.cpp).
+bool paged_keep_in_l2(const hw_paged_problem* p, const hw_paged_plan& plan);
 
 }  // namespace host
 }  // namespace hw

@@ -8,6 +8,8 @@ import torch
 
 from inference_lib_amd import _lib
 from inference_lib_amd import attention as ops
+from test_gpu_paged import build_paged
+from test_gpu_paged import check as check_paged
 from test_gpu_stream_runs import _inputs, _reference
 
 pytestmark = pytest.mark.gpu
@@ -65,3 +67,9 @@ def test_many_rows_of_256(W, S, Hq, Hkv, lens, dtype, rot, hide):
     _lib.Problem(q=q, locations=loc, keys=ks, values=vs, scale=scale, out=narrow, cosines=cos, sines=sin, row_blocks=1).run()
     assert bool(((narrow.double() - ref).abs() <= bound)[seen].all())
     assert not torch.equal(narrow, out), "not a call for 128-row workgroups"
+
+
+@pytest.mark.parametrize("Hq,S,block", [(10, 4, 16), (14, 3, 16), (8, 40, 7), (2, 129, 64)])
+def test_paged_rows_around_the_line_of_kept_tiles(Hq, S, block):
+    """20 and 21 rows a sequence (the K/V tiles are kept in the L2 from 21 on), and many row groups of 16."""
+    check_paged(build_paged("bf16", 1, 3, Hq, 2, 256, block, -(-900 // block), seq_lens=[900, S, 333], S=S, seed=S))
