@@ -337,10 +337,10 @@ void stream_deal(const hw_problem* p, const CallPlan& cp, StreamPlan* sp) {
 // floor(row groups / workgroups) row groups go whole to each workgroup, which holds complete rows at the end and writes the result,
 // and only the remainder is cut into runs (stream_deal), a fifth of the rows with 40 row groups on 32 workgroups.  With no
 // remainder there is no merge launch.  The remainder are the first row groups, which see least of a causal chunk.
-// Against runs, resp. rounds, a layer: 1024 tokens behind 4096 (40/8, D = 128) 124 -> 120 us (two layers, pauses between passes:
-// 248 -> 234), 2 x 574 behind 1333 88 -> 83.5; 1024 behind nothing at 32/8 (no remainder) 71.6 -> 61.5 in rounds, 1500 behind 128
-// 67 -> 60.  All 26 calls timed gained or stayed within the spread, so there is no price to weigh: wherever every workgroup has a
-// row group to itself, runs could only save what they pay for in partial sums.
+// Against runs, resp. rounds, a layer: 1024 tokens behind 4096 (40/8, D = 128) 124 -> 117 us, 2 x 574 behind 1333 88 -> 83.5, 1500
+// behind nothing at 32/8 69 -> 61.5, 1500 behind 128 66.5 -> 60 (and see whole_deal).  All 26 calls timed gained or stayed within
+// the spread, so there is no price to weigh: wherever every workgroup has a row group to itself, runs could only save what they
+// pay for in partial sums.
 // Head dimension 256: the plan's kernel takes 16 rows a workgroup, so every 16 rows stream the K/V through a CU again.  Enough of
 // that, counted in tiles a CU takes in, and 128-row workgroups are faster, whose openings cost more (a launch of them takes about
 // 25 us whatever it holds).  16/8 heads, bf16, us a layer before / after: 1024 tokens behind 4096 (640 tiles a CU) 296 -> 111, 1500

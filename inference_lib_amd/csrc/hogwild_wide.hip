@@ -1259,7 +1259,8 @@ constexpr int WIDE_PAR = 2;
 constexpr int WIDE_SLOTS = 6;
 
 // Head dimension 256: a tile is 32 KB and a lane's accumulators of 32 rows are 128 registers, so four waves of 32 rows, one per SIMD
-// with 512 registers, that all take every tile, and a ring of four slots.
+// with 512 registers, that all take every tile, and a ring of four slots.  1024 tokens behind 4096 at 16/8 heads, bf16: 111 us a layer
+// (0.70 PFLOP/s, matrix units busy 35 % of the clocks) against 296 of the 16-row workgroups, which stream the K/V once per 16 rows.
 constexpr int WIDE256_WAVES = 4;
 constexpr int WIDE256_SLOTS = 4;
 
