@@ -537,6 +537,7 @@ std::vector<at::Tensor> segment_views(at::TensorList buffers, at::IntArrayRef le
 // What HogwildCache hands the attention in a step: locations [F, W, S], tables [F, W, S, RotE] and fragment lengths [F], from host
 // numbers in the kernel arguments (hw_build_inputs; the lengths are the locations of one worker with one token).  A host-to-device
 // copy of the lengths waits for the stream, i.e. for the step before, and with the rest through Python took 38 us a step.
+// A stream that is being captured is refused, as it is by such a copy: the numbers would be the same in every replay.
 // Returns false, with nothing queued, for what the checks or the library refuse: the caller's general path then names it.
 std::tuple<bool, at::Tensor, at::Tensor, at::Tensor, at::Tensor> step_inputs(at::IntArrayRef pos_end, at::IntArrayRef len, int64_t S,
                                                                              const at::Tensor& inv_freq, double scaling, at::ScalarType table_dtype) {
@@ -556,10 +557,14 @@ std::tuple<bool, at::Tensor, at::Tensor, at::Tensor, at::Tensor> step_inputs(at:
     }
     const int64_t rot = 2 * inv_freq.numel();
     c10::hip::HIPGuardMasqueradingAsCUDA guard(inv_freq.device());
+    hipStream_t stream = c10::hip::getCurrentHIPStreamMasqueradingAsCUDA(inv_freq.device().index()).stream();
+    hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
+    if (hipStreamIsCapturing(stream, &capture) != hipSuccess) (void)hipGetLastError();     // (the launches below say what is wrong)
+    TORCH_CHECK(capture == hipStreamCaptureStatusNone, "libhogatt::step_inputs: a captured step with lengths from the host would repeat them "
+                "in every replay; call HogwildCache.use_device_lengths before the capture");
     const auto ints = inv_freq.options().dtype(at::kInt);
     at::Tensor loc = at::empty({F, W, S}, ints), cos = at::empty({F, W, S, rot}, inv_freq.options()), sin = at::empty({F, W, S, rot}, inv_freq.options());
     at::Tensor frags = at::empty({F}, ints);
-    hipStream_t stream = c10::hip::getCurrentHIPStreamMasqueradingAsCUDA(inv_freq.device().index()).stream();
     const int round = table_dtype == at::kFloat ? HW_F32 : table_dtype == at::kHalf ? HW_F16 : HW_BF16;
     int status = hw_build_inputs(loc.data_ptr<int32_t>(), cos.data_ptr<float>(), sin.data_ptr<float>(), ends.data(), inv_freq.const_data_ptr<float>(),
                                  (float)scaling, round, (int)F, (int)W, (int)S, (int)rot, stream);

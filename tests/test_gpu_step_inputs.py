@@ -5,6 +5,7 @@ import torch
 
 from inference_lib_amd import _lib
 from inference_lib_amd import attention as ops
+from inference_lib_amd import cache as hc
 
 pytestmark = pytest.mark.gpu
 
@@ -45,3 +46,43 @@ def test_sdpa_copies_what_it_cannot_read_in_place():
     assert not across[0].is_contiguous()
     assert torch.equal(ops.hogwild_sdpa(q, loc, across, across, 0.125, frag), want)
     assert torch.equal(ops.hogwild_sdpa(q, loc, tuple(across), tuple(across), 0.125), want)
+
+
+@pytest.mark.parametrize("fused", [True, False])
+def test_lengths_from_the_host_refuse_a_capture(fused):
+    """Every replay of such a graph would append to the same rows.  With lengths on the device the same step is captured, and its
+    replays append one behind the other."""
+    Hkv, D = 2, 64
+    segs = [hc.SegmentCache(1, Hkv, D, 64, dtype=torch.float16, device="cuda") for _ in range(2)]
+    for seg in segs:
+        seg.lengths = [5]
+        for buf in (seg.k[0], seg.v[0]):
+            buf.zero_()
+    cache = hc.HogwildCache([segs, segs[::-1]], inv_freq=torch.ones(D // 2, device="cuda"))
+    k, v = (torch.ones((2, Hkv, 1, D), dtype=torch.float16, device="cuda") for _ in range(2))
+    cos, sin = torch.ones((2, 1, D), dtype=torch.float16, device="cuda"), torch.zeros((2, 1, D), dtype=torch.float16, device="cuda")
+    step = (lambda: cache.update_fused(k, v, cos, sin, 0)) if fused else (lambda: cache.update(k, v, 0))
+    step()                                                       # outside a capture: a token each
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with pytest.raises(RuntimeError, match="use_device_lengths"):
+        with torch.cuda.graph(graph):
+            step()
+    for seg in segs:
+        seg.lengths = [6]
+    cache.use_device_lengths(headroom=8)
+    stream = torch.cuda.Stream()
+    stream.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(stream):
+        step()
+    torch.cuda.current_stream().wait_stream(stream)
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        step()
+    for _ in range(3):
+        graph.replay()
+    cache.sync_lengths()
+    for seg in segs:
+        assert seg.lengths == [10]
+        assert bool((seg.v[0][:, 5:10] == 1).all()) and bool((seg.v[0][:, :5] == 0).all()) and bool((seg.v[0][:, 10:] == 0).all())
