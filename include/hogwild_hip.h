@@ -130,7 +130,8 @@ typedef struct hw_problem {
  * the others an equal run of tiles across the row groups (often more workspace), if the workspace is as large as
  * hw_workspace_bytes / hw_sdpa_workspace_bytes say.  In a smaller one that still has hw_plan.workspace_bytes such a call runs as
  * described here, somewhat slower, wherever the other launch does not fit.  So do calls at head dimension 256 (16-bit types,
- * host lengths, row_blocks = 0, splits = 0) whose row groups of 16 would take in many tiles a CU: their plan says row_blocks = 1. */
+ * host lengths, row_blocks = 0, splits = 0) with several row groups of 16 that would take in many tiles a CU: their plan says
+ * row_blocks = 1. */
 typedef struct hw_plan {
     int32_t rows;             /* W*S*(Hq/Hkv): query rows that share one kv head */
     int32_t row_blocks;       /* 16-row MFMA blocks per workgroup (1, 2 or 8) */

@@ -342,21 +342,48 @@ void stream_deal(const hw_problem* p, const CallPlan& cp, StreamPlan* sp) {
 // the spread, so there is no price to weigh: wherever every workgroup has a row group to itself, runs could only save what they
 // pay for in partial sums.
 // Head dimension 256: the plan's kernel takes 16 rows a workgroup, so every 16 rows stream the K/V through a CU again.  Enough of
-// that, counted in tiles a CU takes in, and 128-row workgroups are faster, whose openings cost more (a launch of them takes about
-// 25 us whatever it holds).  16/8 heads, bf16, us a layer before / after: 1024 tokens behind 4096 (640 tiles a CU) 296 -> 111, 1500
-// behind 100 168 -> 70, 2 x 200 behind 5000 154 -> 79, 2 x 300 behind 500 (84) 75 -> 43, 100 behind 5000 (65) 50 -> 33, 150 behind 3000
-// (59) 49 -> 36; below the line 2 x 128 behind 1500 (55) 34 -> 36.5, 256 behind 1000 (40) 24 -> 35.5.
+// that, counted in tiles a CU takes in, and 128-row workgroups are faster, whose openings cost more.  16/8 heads, bf16, us a layer
+// before / after: 1024 tokens behind 4096 (640 tiles a CU) 296 -> 111, 1500 behind 100 168 -> 70, 2 x 200 behind 5000 154 -> 79, 2 x 300
+// behind 500 (84) 75 -> 43; below the line 2 x 128 behind 1500 (55) 34 -> 36.5, 256 behind 1000 (40) 24 -> 35.5.
+// With one row group nothing is streamed twice, whatever the context: 1 to 16 rows behind 4 K to 60 K at 16/8, 16/16, 32/32, 32/4 and
+// 64/8 heads take 0.60 to 1.01 times as long in the 16-row kernel (81.1 against 100.6 us: 4 workers x 4 tokens behind 30 K, 16/16).
+// Above that both launches are priced, in us, by fits to 1122 calls timed both ways (17 to 2000 rows of 1 to 8 workers, 2 to 17
+// fragments, 1 to 32 kv heads, 10 to 400 tiles a CU): the 16-row one by the tiles of its workgroups, less where their number lets
+// every kv head keep to an XCD, whose L2 its row groups then share; the 128-row one by its tiles and by the most fragments that one
+// workgroup opens, into whose run short ones crowd; both by the K/V itself (+-11 % each).  Of the 845 calls above the tile count
+// alone 54 lost, up to 1.49 times (a step of 17 fragments in 2 row groups).  The 736 that kWorth leaves gain 1.54 in the median, 5 of
+// them lose up to 1.12 times; the 44 that would have gained more than 1.03 gain 1.13 in the median.
 constexpr int kWide256Visits = 56;
+static bool wide_256(const hw_problem* p, int num_cus, const CallPlan& cp) {
+    const hw_plan& plan = cp.plan[0];
+    if (p->E != 256 || p->dtype == HW_F32 || p->len_dev != nullptr || p->row_blocks != 0 || plan.row_groups < 2) return false;
+    constexpr double kWorth = 1.12;
+    const double once = (double)plan.tiles_per_head * p->Hkv / num_cus;      // tiles a CU takes in where every tile is read once
+    if (plan.row_groups * once < kWide256Visits) return false;
+    const int rounds = (plan.workgroups + num_cus - 1) / num_cus, nrg = (plan.rows + hw::PLAN_SLOT_ROWS - 1) / hw::PLAN_SLOT_ROWS;
+    const double run16 = (double)rounds * plan.tiles_per_head / plan.wgs_per_head, run128 = (double)nrg * plan.tiles_per_head * p->Hkv / num_cus;
+    int nf = 0, crowd = 0, inside = 0;           // fragments; the most of them that a run of run128 tiles touches; those of the window
+    for (int f = 0, first = 0; f < p->F; ++f) {
+        if (p->len[f] == 0) continue;
+        ++nf;
+        ++inside;
+        for (; plan.tile_begin[f] - (plan.tile_begin[first + 1] - 1) >= run128 && first < f; ++first) inside -= p->len[first] > 0 ? 1 : 0;
+        crowd = std::max(crowd, inside);
+    }
+    const double narrow = 7.7 + (plan.workgroups % 8 == 0 ? 0.48 : 0.8) * run16 + 0.6 * nf + 0.8 * once;
+    const double wide = 17.4 + 1.58 * run128 + 3.6 * crowd - 0.56 * once;
+    return narrow > kWorth * wide;
+}
+
 bool whole_size(const hw_problem* p, int num_cus, const CallPlan& cp, WholePlan* wp) {
     const hw_plan& plan = cp.plan[0];
     if (cp.groups != 1 || p->splits > 0 || plan.tiles_per_head < 1) return false;
-    const bool wide_256 = p->E == 256 && p->dtype != HW_F32 && p->len_dev == nullptr && p->row_blocks == 0 &&
-                          (long long)plan.row_groups * plan.tiles_per_head * p->Hkv >= (long long)kWide256Visits * num_cus;
-    if (plan.row_blocks != hw::WIDE_ROW_BLOCKS && !wide_256) return false;
+    const bool few_groups = wide_256(p, num_cus, cp);        // may have fewer row groups than workgroups
+    if (plan.row_blocks != hw::WIDE_ROW_BLOCKS && !few_groups) return false;
     const int nrg = (plan.rows + hw::PLAN_SLOT_ROWS - 1) / hw::PLAN_SLOT_ROWS, T = plan.tiles_per_head;
     int wgs = num_cus / p->Hkv;
     if (wgs > hw::MAX_SPLITS) wgs = hw::MAX_SPLITS;
-    if (wgs < 1 || (nrg < wgs && !wide_256) || (long long)nrg * T >= (1ll << 30) || (long long)wgs + nrg >= (1 << 15)) return false;
+    if (wgs < 1 || (nrg < wgs && !few_groups) || (long long)nrg * T >= (1ll << 30) || (long long)wgs + nrg >= (1 << 15)) return false;
     // the kernel divides (head, workgroup) pairs by the workgroups per head (see magic_exact)
     if ((unsigned long long)wgs * wgs * p->Hkv >= (1ull << 32)) return false;
     wp->wgs = wgs;

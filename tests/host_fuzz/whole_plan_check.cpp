@@ -9,7 +9,33 @@
 
 #define CHECK(c) do { if (!(c)) { std::printf("failed: %s (Hkv %d rows %d F %d)\n", #c, p.Hkv, cp.plan[0].rows, p.F); return 1; } } while (0)
 
+// Does a call of head dimension 256 go to 128-row workgroups?  (256 CUs, bf16, one token a worker unless S says otherwise.)
+static bool wide_256(int W, int S, int Hq, int Hkv, std::vector<int32_t> len) {
+    hw_problem p{};
+    p.dtype = HW_BF16;
+    p.F = (int)len.size();
+    p.W = W; p.S = S; p.Hq = Hq; p.Hkv = Hkv;
+    p.E = p.Ev = p.RotE = 256;
+    p.len = len.data();
+    hw::host::CallPlan cp;
+    hw::host::WholePlan wp;
+    return hw::host::plan_call(&p, 256, &cp, 1) == HW_OK && hw::host::whole_size(&p, 256, cp, &wp);
+}
+
+// Decode steps keep the 16-row kernel however long the context: with one row group nothing is streamed twice.  With more, both
+// launches are priced: a prompt chunk and tokens of several workers behind a long prompt go to 128-row workgroups, a step of many
+// short fragments does not.
+static int head_dim_256() {
+    const bool ok = !wide_256(1, 1, 16, 16, {29000}) && !wide_256(1, 1, 16, 16, {120000}) && !wide_256(4, 1, 16, 16, {30000, 1, 1, 1, 1}) &&
+                    !wide_256(1, 1, 32, 32, {15000}) && !wide_256(4, 4, 16, 16, {60000, 4, 4, 4, 4}) && !wide_256(2, 1, 32, 4, {120000, 1, 1}) &&
+                    !wide_256(8, 1, 32, 8, {34000, 9, 9, 9, 9, 9, 9, 9, 9, 1, 1, 1, 1, 1, 1, 1, 1}) && !wide_256(4, 4, 8, 1, {60000, 4, 4, 4, 4}) &&
+                    wide_256(1, 1024, 16, 8, {4096, 1024}) && wide_256(4, 8, 16, 8, {60000, 8, 8, 8, 8}) && wide_256(1, 33, 32, 32, {12000, 33});
+    if (!ok) std::printf("failed: the choice of 128-row workgroups at head dimension 256\n");
+    return ok ? 0 : 1;
+}
+
 int main() {
+    if (head_dim_256() != 0) return 1;
     std::mt19937 rng(7);
     auto pick = [&](int lo, int hi) { return (int)(lo + rng() % (unsigned)(hi - lo + 1)); };
     int taken = 0, left_over = 0, taken_256 = 0;
