@@ -338,9 +338,12 @@ void stream_deal(const hw_problem* p, const CallPlan& cp, StreamPlan* sp) {
 // and only the remainder is cut into runs (stream_deal), a fifth of the rows with 40 row groups on 32 workgroups.  With no
 // remainder there is no merge launch.  The remainder are the first row groups, which see least of a causal chunk.
 // Against runs, resp. rounds, a layer: 1024 tokens behind 4096 (40/8, D = 128) 124 -> 117 us, 2 x 574 behind 1333 88 -> 83.5, 1500
-// behind nothing at 32/8 69 -> 61.5, 1500 behind 128 66.5 -> 60 (and see whole_deal).  All 26 calls timed gained or stayed within
-// the spread, so there is no price to weigh: wherever every workgroup has a row group to itself, runs could only save what they
-// pay for in partial sums.
+// behind nothing at 32/8 69 -> 61.5, 1500 behind 128 66.5 -> 60 (and see whole_deal).  Where the heads divide the CUs this is never
+// more work a CU than rounds.  Where they do not, CUs stay idle that rounds would use, and the workgroups take nrg / wgs row groups
+// one after the other against the rounds: 9 row groups of 56 heads (1119 tokens behind 1200, D = 128) 2.25 against 2, 105.6 against
+// 100.6 us; 5 of 96 2.5 against 2 (D = 64: 65 against 60 behind 1200, 131 against 116 behind 4000), 3 of 140 3 against 2 (144 against
+// 115).  What is saved in partial sums is worth about 16 tiles of that: 621 tokens behind 150 at 96 heads (25 tiles) 39 against 43 us.  (Of 400 calls
+// of 1 to 160 heads 9 lost 3 % or more, up to 31 %, with whole row groups throughout, 1 with the line, 5 %.)
 // Head dimension 256: the plan's kernel takes 16 rows a workgroup, so every 16 rows stream the K/V through a CU again.  Enough of
 // that, counted in tiles a CU takes in, and 128-row workgroups are faster, whose openings cost more.  16/8 heads, bf16, us a layer
 // before / after: 1024 tokens behind 4096 (640 tiles a CU) 296 -> 111, 1500 behind 100 168 -> 70, 2 x 200 behind 5000 154 -> 79, 2 x 300
@@ -386,6 +389,8 @@ bool whole_size(const hw_problem* p, int num_cus, const CallPlan& cp, WholePlan*
     if (wgs < 1 || (nrg < wgs && !few_groups) || (long long)nrg * T >= (1ll << 30) || (long long)wgs + nrg >= (1 << 15)) return false;
     // the kernel divides (head, workgroup) pairs by the workgroups per head (see magic_exact)
     if ((unsigned long long)wgs * wgs * p->Hkv >= (1ull << 32)) return false;
+    const int rounds = (plan.workgroups + num_cus - 1) / num_cus;
+    if (!few_groups && (long long)(nrg - rounds * wgs) * T > 16ll * wgs) return false;
     wp->wgs = wgs;
     wp->split = nrg % wgs;
     wp->whole = nrg - wp->split;

@@ -9,18 +9,20 @@
 
 #define CHECK(c) do { if (!(c)) { std::printf("failed: %s (Hkv %d rows %d F %d)\n", #c, p.Hkv, cp.plan[0].rows, p.F); return 1; } } while (0)
 
-// Does a call of head dimension 256 go to 128-row workgroups?  (256 CUs, bf16, one token a worker unless S says otherwise.)
-static bool wide_256(int W, int S, int Hq, int Hkv, std::vector<int32_t> len) {
+// Is a call dealt in whole row groups of 128 rows?  (256 CUs, bf16.)
+static bool whole(int D, int W, int S, int Hq, int Hkv, std::vector<int32_t> len) {
     hw_problem p{};
     p.dtype = HW_BF16;
     p.F = (int)len.size();
     p.W = W; p.S = S; p.Hq = Hq; p.Hkv = Hkv;
-    p.E = p.Ev = p.RotE = 256;
+    p.E = p.Ev = p.RotE = D;
     p.len = len.data();
     hw::host::CallPlan cp;
     hw::host::WholePlan wp;
     return hw::host::plan_call(&p, 256, &cp, 1) == HW_OK && hw::host::whole_size(&p, 256, cp, &wp);
 }
+
+static bool wide_256(int W, int S, int Hq, int Hkv, std::vector<int32_t> len) { return whole(256, W, S, Hq, Hkv, len); }
 
 // Decode steps keep the 16-row kernel however long the context: with one row group nothing is streamed twice.  With more, both
 // launches are priced: a prompt chunk and tokens of several workers behind a long prompt go to 128-row workgroups, a step of many
@@ -34,7 +36,18 @@ static int head_dim_256() {
     return ok ? 0 : 1;
 }
 
+// Head counts that leave CUs idle with one workgroup a CU: not where rounds would take fewer row groups one after the other.
+static int rounds_instead() {
+    const bool ok = !whole(128, 1, 1152, 56, 56, {1200, 1152}) && !whole(64, 1, 640, 96, 96, {4000, 640}) && !whole(64, 1, 384, 140, 140, {1200, 384}) &&
+                    !whole(128, 1, 640, 96, 96, {4000, 640}) && whole(128, 1, 512, 56, 56, {1200, 512}) && whole(128, 1, 1024, 56, 56, {1200, 1024}) &&
+                    whole(128, 1, 640, 56, 56, {4000, 640}) && whole(64, 1, 621, 96, 96, {150, 621}) && whole(128, 1, 1024, 40, 8, {4096, 1024}) &&
+                    whole(128, 1, 1500, 32, 8, {12000, 1500}) && whole(128, 1, 1354, 36, 12, {1200, 1354});
+    if (!ok) std::printf("failed: whole row groups or rounds\n");
+    return ok ? 0 : 1;
+}
+
 int main() {
+    if (rounds_instead() != 0) return 1;
     if (head_dim_256() != 0) return 1;
     std::mt19937 rng(7);
     auto pick = [&](int lo, int hi) { return (int)(lo + rng() % (unsigned)(hi - lo + 1)); };
