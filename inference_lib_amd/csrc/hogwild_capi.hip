@@ -494,11 +494,7 @@ static int workspace_bytes_for(const hw_problem* p, int fused, size_t* bytes) {
     CallPlan cp;
     st = plan_call(p, cus, &cp, fused);
     if (st != HW_OK) return st;
-    StreamPlan sp;
-    *bytes = cp.workspace_bytes;
-    if (stream_size(p, cus, cp, &sp) && sp.workspace_bytes > *bytes) *bytes = sp.workspace_bytes;
-    WholePlan wp;
-    if (whole_size(p, cus, cp, &wp) && wp.workspace_bytes > *bytes) *bytes = wp.workspace_bytes;
+    *bytes = call_workspace_bytes(p, cus, cp);
     return HW_OK;
 }
 

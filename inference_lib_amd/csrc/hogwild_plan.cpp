@@ -463,6 +463,13 @@ void whole_deal(const hw_problem* p, const CallPlan& cp, WholePlan* wp) {
     }
 }
 
+size_t call_workspace_bytes(const hw_problem* p, int num_cus, const CallPlan& cp) {
+    WholePlan wp;
+    StreamPlan sp;
+    if (whole_size(p, num_cus, cp, &wp)) return std::max(cp.workspace_bytes, wp.workspace_bytes);
+    return stream_size(p, num_cus, cp, &sp) ? std::max(cp.workspace_bytes, sp.workspace_bytes) : cp.workspace_bytes;
+}
+
 int paged_validate(const hw_paged_problem* p) {
     if (p == nullptr) return HW_ERR_NULL;
     if (p->dtype != HW_F32 && p->dtype != HW_F16 && p->dtype != HW_BF16) return HW_ERR_DTYPE;

@@ -66,6 +66,9 @@ struct WholePlan {
 };
 bool whole_size(const hw_problem* p, int num_cus, const CallPlan& cp, WholePlan* wp);
 void whole_deal(const hw_problem* p, const CallPlan& cp, WholePlan* wp);
+// What a call asks for: room for CallPlan, the caller's fallback, and for the launch that is preferred to it (whole row groups
+// before runs; 1024 tokens behind 4096 at 40/8 heads, D = 128: 21.3 MB, where the runs that are not taken there would need 38.1).
+size_t call_workspace_bytes(const hw_problem* p, int num_cus, const CallPlan& cp);
 int paged_validate(const hw_paged_problem* p);
 int paged_plan(const hw_paged_problem* p, int num_cus, hw_paged_plan* plan);
 // Whether the tiles of a paged launch are to stay in the L2 (hogwild_plan.cpp).

@@ -1,5 +1,6 @@
 // whole_size and whole_deal over random calls of 128-row workgroups: the row groups dealt whole and the runs cover every row group
 // once, every piece of a run has a slot inside the workspace, max_pieces bounds the pieces of a row group.
+#include <algorithm>
 #include <cstdio>
 #include <random>
 #include <vector>
@@ -73,6 +74,8 @@ int main() {
         hw::host::WholePlan wp;
         if (!hw::host::whole_size(&p, cus, cp, &wp)) continue;
         ++taken;
+        // what is asked for is what the launch uses, or hw_plan's own where that is more; not what the runs it replaces would need
+        CHECK(hw::host::call_workspace_bytes(&p, cus, cp) == std::max(cp.workspace_bytes, wp.workspace_bytes));
         hw::host::whole_deal(&p, cp, &wp);
         const hw::host::StreamPlan& sp = wp.runs;
         const bool wide_256 = p.E == 256;           // its plan is the 16-row kernel's, and may have fewer row groups than workgroups
