@@ -404,14 +404,28 @@ bool whole_size(const hw_problem* p, int num_cus, const CallPlan& cp, WholePlan*
     return true;
 }
 
+// One worker that brings the newest S tokens of the last fragment (a causal chunk) sees of that fragment what lies before its own
+// tokens.  Dealing the remainder by the tiles seen pays where they are few enough and the remainder is large enough: plain / this, us
+// a layer, 1400 tokens at 40/8 heads (23 row groups left for 32 workgroups) with the chunk 0.8, 0.5 and a third of the tiles 1.15,
+// 1.05 and 1.03 times, 830 (one left) 0.94, 0.96 and 0.97, 1024 (eight left) 1.08, 0.96 to 1.06 and 1.00.  The lines are drawn through
+// 623 calls of 13 head layouts.  With more than a quarter of the workgroups' number left, the chunk above a third: means of 1.00 to
+// 1.14 by share, 0.97 at worst; with less left but more than one, above a half: 1.00 to 1.11, 0.98 at worst.  With one left 0.97
+// whatever the share, and below a third 1.00.  Head dimension 256 with all row groups in runs: 0.75 to 1.09 with less than half the
+// workgroups' number, 0.97 to 1.16 above the lines here.
+bool deal_by_seen(const hw_problem* p, const CallPlan& cp, const WholePlan& wp) {
+    const int T = cp.plan[0].tiles_per_head, chunk = (p->S + hw::TILE - 1) / hw::TILE;
+    int last = p->F - 1;
+    while (last > 0 && p->len[last] == 0) --last;
+    if (p->W != 1 || p->len[last] < p->S) return false;
+    if (wp.whole == 0) return 2 * wp.split > wp.wgs && (2 * chunk > T || (3 * chunk > T && 8 * wp.split > 5 * wp.wgs));
+    return (2 * chunk > T && wp.split > 1) || (3 * chunk > T && 4 * wp.split > wp.wgs);
+}
+
 // The remainder in runs: the smallest share (tiles, with openings) at which the workgroups, taking one after the other what fits,
-// use up the row groups, found by bisection.  One worker that brings the newest S tokens of the last fragment (a causal chunk) sees
-// of that fragment what lies before its own tokens: the tiles behind them go with the piece in front, so that no workgroup opens
-// a row group for tiles that none of its rows sees.  (Should the locations say otherwise, the launch is merely less even.)
-// Against stream_deal on the same remainder: 1500 tokens behind 128 at 32/8 heads 59.6 -> 53 us, 900 behind nothing at 64/8
-// 57 -> 51, 1300 at 32/8 behind 512, 1024, 2048, 3000 and 4096 1.10, 1.05, 1.06, 1.02 and 1.00 times, 1024 at 40/8 1.06, 0.98, 1.00,
-// 0.99 and 0.98 times, which is why the chunk has to be a quarter of the tiles.  Unseen tiles cost as much here as the others:
-// priced at 0.15, 0.3, 0.5 and 0.8, with the workgroups' shares unequal to match, the launches took as long or longer.
+// use up the row groups, found by bisection.  Dealt by the tiles seen, those behind them go with the piece in front, so that no
+// workgroup opens a row group for tiles that none of its rows sees.  (Should the locations say otherwise, the launch is merely less
+// even.)  Unseen tiles cost as much here as the others: priced at 0.15, 0.3, 0.5 and 0.8, with the workgroups' shares unequal to
+// match, the launches took as long or longer.
 void whole_deal(const hw_problem* p, const CallPlan& cp, WholePlan* wp) {
     constexpr double kPieceCost = 8.0, kOpenCost = 2.0;      // in tiles: a piece's prologue and epilogue; a row group's fragments
     const hw_plan& plan = cp.plan[0];
@@ -424,10 +438,10 @@ void whole_deal(const hw_problem* p, const CallPlan& cp, WholePlan* wp) {
         ++nf;
     }
     const double tile = 1.0 + kOpenCost * nf / T;            // a row group's openings spread over its tiles
-    const bool causal = p->W == 1 && p->len[last] >= p->S && 4 * (T - plan.tile_begin[last]) > T;
+    const bool by_seen = deal_by_seen(p, cp, *wp);
     const int gq = p->Hq / p->Hkv;
     auto seen_tiles = [&](int rg) {                          // up to the token of the row group's last row
-        if (!causal) return T;
+        if (!by_seen) return T;
         const int token = (std::min((rg + 1) * hw::PLAN_SLOT_ROWS, plan.rows) - 1) / gq;
         return plan.tile_begin[last] + (p->len[last] - p->S + token + hw::TILE) / hw::TILE;
     };

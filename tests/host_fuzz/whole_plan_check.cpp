@@ -47,7 +47,31 @@ static int rounds_instead() {
     return ok ? 0 : 1;
 }
 
+// Are the runs of a prompt chunk of one worker dealt by the tiles that it sees?
+static bool by_seen(int D, int S, int Hq, int Hkv, std::vector<int32_t> len) {
+    hw_problem p{};
+    p.dtype = HW_F16;
+    p.F = (int)len.size();
+    p.W = 1; p.S = S; p.Hq = Hq; p.Hkv = Hkv;
+    p.E = p.Ev = p.RotE = D;
+    p.len = len.data();
+    hw::host::CallPlan cp;
+    hw::host::WholePlan wp;
+    return hw::host::plan_call(&p, 256, &cp, 1) == HW_OK && hw::host::whole_size(&p, 256, cp, &wp) && hw::host::deal_by_seen(&p, cp, wp);
+}
+
+// Where that was measured to pay: the share of the chunk in the tiles, the row groups left over, in one fragment as in two.
+static int seen_tiles() {
+    const bool ok = by_seen(128, 1400, 40, 8, {350, 1400}) && by_seen(128, 1400, 40, 8, {2700, 1400}) && by_seen(128, 1400, 40, 8, {4100}) &&
+                    by_seen(128, 1024, 40, 8, {900, 1024, 0}) && by_seen(256, 1400, 16, 8, {1000, 1400}) && !by_seen(128, 1400, 40, 8, {2900, 1400}) && !by_seen(128, 1024, 40, 8, {1024, 1024}) &&
+                    !by_seen(128, 1024, 40, 8, {4096, 1024}) && !by_seen(128, 1024, 40, 8, {5120}) && !by_seen(128, 830, 40, 8, {200, 830}) &&
+                    !by_seen(64, 1400, 24, 8, {350, 1400}) && !by_seen(256, 950, 16, 8, {511, 950}) && !by_seen(256, 600, 16, 8, {676, 600});
+    if (!ok) std::printf("failed: dealing by the tiles seen\n");
+    return ok ? 0 : 1;
+}
+
 int main() {
+    if (seen_tiles() != 0) return 1;
     if (rounds_instead() != 0) return 1;
     if (head_dim_256() != 0) return 1;
     std::mt19937 rng(7);
