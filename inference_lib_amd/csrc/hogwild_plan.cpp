@@ -445,35 +445,45 @@ void whole_deal(const hw_problem* p, const CallPlan& cp, WholePlan* wp) {
         const int token = (std::min((rg + 1) * hw::PLAN_SLOT_ROWS, plan.rows) - 1) / gq;
         return plan.tile_begin[last] + (p->len[last] - p->S + token + hw::TILE) / hw::TILE;
     };
+    const double per_tile = 1.0 / tile;
     auto deal = [&](double share) {                          // false if something is left
-        int rg = 0, t = 0;
+        int rg = 0, t = 0, seen = seen_tiles(0);
         for (int g = 0; g < wgs; ++g) {
             sp.wg_tile_begin[g] = rg * T + t;
             for (double room = share; rg < split;) {
-                const int seen = seen_tiles(rg), take = std::min((int)((room - kPieceCost) / tile), seen - t);
+                const int take = std::min((int)((room - kPieceCost) * per_tile), seen - t);
                 if (take < std::min(kMinPiece, seen - t)) break;
                 room -= kPieceCost + take * tile;
                 t += take;
                 if (t < seen) break;
                 room -= T - seen;
                 t = 0;
-                ++rg;
+                seen = seen_tiles(++rg);
             }
         }
         return rg == split;
     };
-    double low = 0.0, high = split * (kPieceCost + (T + 1) * tile);      // all of it for the first workgroup
-    for (int i = 0; i < 12; ++i) {
+    // Between an equal part of the tiles seen and that of all tiles with what a workgroup opens and leaves at most besides.
+    double low = 0.0, unseen = 0.0;
+    for (int rg = 0; rg < split; ++rg) {
+        low += kPieceCost + seen_tiles(rg) * tile;
+        unseen += T - seen_tiles(rg);
+    }
+    low /= wgs;
+    double high = low + unseen / wgs + 2.0 * kPieceCost + (kMinPiece + 1) * tile;
+    while (!deal(high)) high *= 2.0;
+    while (high - low > 0.25) {
         const double mid = 0.5 * (low + high);
         (deal(mid) ? high : low) = mid;
     }
     deal(high);
     for (int i = wgs; i <= HW_MAX_SPLITS; ++i) sp.wg_tile_begin[i] = split * T;
     sp.max_pieces = 0;
-    for (int rg = 0; rg < split; ++rg) {
-        int pieces = 0;
-        for (int g = 0; g < wgs; ++g) pieces += std::max(sp.wg_tile_begin[g], rg * T) < std::min(sp.wg_tile_begin[g + 1], (rg + 1) * T) ? 1 : 0;
-        sp.max_pieces = std::max(sp.max_pieces, pieces);
+    for (int rg = 0, g = 0; rg < split; ++rg) {
+        while (sp.wg_tile_begin[g + 1] <= rg * T) ++g;
+        int last = g;
+        while (sp.wg_tile_begin[last + 1] < (rg + 1) * T) ++last;
+        sp.max_pieces = std::max(sp.max_pieces, last - g + 1);
     }
 }
 

@@ -65,6 +65,9 @@ struct WholePlan {
     size_t workspace_bytes;
 };
 bool whole_size(const hw_problem* p, int num_cus, const CallPlan& cp, WholePlan* wp);
+// Every call of the kind deals about nine times over row groups and workgroups until the share is found: 0.9 us on the host with 8 row
+// groups left for 32 workgroups, 4.0 with 47 for 128, 12 with 94 for one kv head's 256 (1.9, 12 and 27 when the bisection began at all
+// of the work for one workgroup and the pieces were counted for every pair).  Sizing takes 0.02.
 void whole_deal(const hw_problem* p, const CallPlan& cp, WholePlan* wp);
 // Whether whole_deal counts the tiles that a causal chunk sees (hogwild_plan.cpp).
 bool deal_by_seen(const hw_problem* p, const CallPlan& cp, const WholePlan& wp);
