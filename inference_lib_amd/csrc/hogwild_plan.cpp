@@ -520,11 +520,20 @@ int paged_validate(const hw_paged_problem* p) {
 }
 
 // At head dimension 256 the paged kernel takes 16 rows a workgroup, and the row groups of a sequence read its K/V one after the
-// other: from 20 rows a sequence on the tiles are kept in the L2 instead of being streamed past it.  16/8 heads, bf16, us a
-// layer: 128 query tokens on 12 528 166 -> 114, 4 x 100 on 2 ... 5 K 163 -> 123, 29/4/98/23/17 on 640 ... 4.8 K 71 -> 56.5, 4 x 12 on 12 K
-// 96 -> 92; 4 x 9 (18 rows) on 3 K 27.8 -> 28.0.  (The 128-row form for D <= 128 reads a sequence a few times at most and lost
-// 1 to 11 % with kept tiles, except with three row groups a sequence and more, 1 to 6 %, which only the device knows.)
-bool paged_keep_in_l2(const hw_paged_problem* p, const hw_paged_plan& plan) { return p->E == 256 && plan.rows > 20ll * p->W; }
+// other: with more than two of them the tiles are kept in the L2 instead of being streamed past it.  16/8 heads, bf16, us a layer: 128
+// query tokens on 12 528 166 -> 114, 4 x 64 on 12 000 291 -> 203, 4 x 24 131 -> 121, 4 x 24 on 3000 39.3 -> 39.4.  Two row groups
+// of a sequence are under way together: 21 to 32 rows at 8 and 16 kv heads 0.93 to 1.13 times, 0.996 in the mean of 44 calls (4 x 16 on
+// 3000 27.4 -> 28.8, on 12 000 84.7 -> 81.4), and 16 rows lose 0.87 to 0.91; 33 to 48 rows 0.94 to 1.20, 1.05 in the mean.
+// Packed sequences share a launch whatever they bring, and only the device knows it, so the line is their mean, and it lies lower, as
+// their rows are in few long chunks: 21 to 32 rows in the mean 0.97 to 1.29, 1.08 over 14 batches (31 decoding sequences and a chunk of
+// 64 on 3000 at 32/4 128 -> 99); up to 20 rows 0.91 to 1.00; from 64 on 1.01 to 1.82 (7 decoding and a chunk of 128 on 12 000 at 64/8
+// 639 -> 468).  What the decoding sequences beside a chunk lose is 3 % at most of the launch (63 and a chunk of 1024 on 1500 at 16/8
+// 230 -> 237).  Ten head layouts, bf16 and fp16, 1 to 64 sequences; bit-identical both ways.
+// (The 128-row form for D <= 128 reads a sequence a few times at most and lost 1 to 11 % with kept tiles, except with three row groups
+// a sequence and more, 1 to 6 %, which only the device knows.)
+bool paged_keep_in_l2(const hw_paged_problem* p, const hw_paged_plan& plan) {
+    return p->E == 256 && plan.rows > (p->cu_seqlens_q != nullptr ? 20ll : 32ll) * p->W;
+}
 
 int paged_plan(const hw_paged_problem* p, int num_cus, hw_paged_plan* plan) {
     if (plan == nullptr) return HW_ERR_NULL;

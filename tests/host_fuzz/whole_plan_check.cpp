@@ -70,7 +70,29 @@ static int seen_tiles() {
     return ok ? 0 : 1;
 }
 
+// Paged queries of head dimension 256: K/V tiles are kept with more than two row groups of 16 a sequence, packed ones with more than
+// 20 rows in the mean.
+static int kept_tiles() {
+    auto keep = [](int D, int W, int Hq, int Hkv, int S, int total_q) {
+        static const int32_t cu = 0;
+        hw_paged_problem p{};
+        p.dtype = HW_BF16;
+        p.F = 1; p.W = W; p.Hq = Hq; p.Hkv = Hkv; p.E = p.Ev = D; p.S = S; p.total_q = total_q;
+        p.cu_seqlens_q = total_q > 0 ? &cu : nullptr;
+        p.block_size = 16;
+        p.max_blocks = 800;
+        hw_paged_plan plan;
+        return hw::host::paged_plan(&p, 256, &plan) == HW_OK && hw::host::paged_keep_in_l2(&p, plan);
+    };
+    const bool ok = !keep(256, 4, 16, 8, 8, 0) && !keep(256, 4, 16, 8, 12, 0) && !keep(256, 4, 16, 8, 16, 0) && keep(256, 4, 16, 8, 17, 0) &&
+                    keep(256, 1, 16, 8, 128, 0) && !keep(256, 4, 16, 8, 0, 40) && keep(256, 4, 16, 8, 0, 41) && !keep(256, 32, 16, 8, 0, 31 + 128) &&
+                    keep(256, 8, 64, 8, 0, 7 + 128) && !keep(128, 4, 40, 8, 64, 0) && !keep(128, 4, 40, 8, 0, 400);
+    if (!ok) std::printf("failed: paged tiles kept in the L2\n");
+    return ok ? 0 : 1;
+}
+
 int main() {
+    if (kept_tiles() != 0) return 1;
     if (seen_tiles() != 0) return 1;
     if (rounds_instead() != 0) return 1;
     if (head_dim_256() != 0) return 1;

@@ -69,7 +69,13 @@ def test_many_rows_of_256(W, S, Hq, Hkv, lens, dtype, rot, hide):
     assert not torch.equal(narrow, out), "not a call for 128-row workgroups"
 
 
-@pytest.mark.parametrize("Hq,S,block", [(10, 4, 16), (14, 3, 16), (8, 40, 7), (2, 129, 64)])
+@pytest.mark.parametrize("Hq,S,block", [(10, 4, 16), (14, 3, 16), (8, 8, 16), (22, 3, 16), (8, 40, 7), (2, 129, 64)])
 def test_paged_rows_around_the_line_of_kept_tiles(Hq, S, block):
-    """20 and 21 rows a sequence (the K/V tiles are kept in the L2 from 21 on), and many row groups of 16."""
+    """20, 21, 32 and 33 rows a sequence (the K/V tiles are kept in the L2 from 33 on), and many row groups of 16."""
     check_paged(build_paged("bf16", 1, 3, Hq, 2, 256, block, -(-900 // block), seq_lens=[900, S, 333], S=S, seed=S))
+
+
+@pytest.mark.parametrize("q_lens", [(10, 1, 49), (10, 2, 49), (1, 64, 30)])
+def test_packed_rows_around_the_line_of_kept_tiles(q_lens):
+    """60 and 61 query rows of three packed sequences (kept from 61 on), and more."""
+    check_paged(build_paged("bf16", 1, 3, 2, 2, 256, 16, 57, seq_lens=[900, 70, 333], q_lens=list(q_lens), seed=sum(q_lens)))
