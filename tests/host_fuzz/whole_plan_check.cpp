@@ -132,18 +132,35 @@ int main() {
         CHECK(wp.wgs >= 1 && wp.wgs <= HW_MAX_SPLITS && (long long)wp.wgs * p.Hkv <= cus);
         CHECK(wp.split >= 0 && wp.whole >= 0 && wp.whole % wp.wgs == 0 && wp.split < wp.wgs && wp.split + wp.whole == nrg);
         CHECK(sp.wg_tile_begin[0] == 0 && sp.wg_tile_begin[wp.wgs] == wp.split * T);
-        std::vector<char> used(sp.slots > 0 ? sp.slots : 1, 0);
+        std::vector<int> used(sp.slots > 0 ? sp.slots : 1, -1);           // row group of the piece in a slot
         std::vector<int> pieces(wp.split > 0 ? wp.split : 1, 0);
         for (int g = 0; g < wp.wgs; ++g) {
             const int b = sp.wg_tile_begin[g], e = sp.wg_tile_begin[g + 1];
             CHECK(b <= e);
             for (int rg = b / T; rg * T < e && b < e; ++rg) {
-                CHECK(g + rg < sp.slots && !used[g + rg]);
-                used[g + rg] = 1;
+                CHECK(g + rg < sp.slots && used[g + rg] < 0);
+                used[g + rg] = rg;
                 ++pieces[rg];
             }
         }
-        for (int rg = 0; rg < wp.split; ++rg) CHECK(pieces[rg] >= 1 && pieces[rg] <= sp.max_pieces);
+        // what the merge is told (write_row_table): the workgroup with a row group's first tile counts the workgroups that begin before
+        // the row group ends, and lists the slots from its own on; an empty run among them would be a slot that nobody wrote
+        int most = 0;
+        for (int rg = 0; rg < wp.split; ++rg) {
+            int first = -1, begun = 0;
+            for (int g = 0; g < wp.wgs; ++g) {
+                const int b = sp.wg_tile_begin[g], e = sp.wg_tile_begin[g + 1];
+                begun += b < (rg + 1) * T;
+                if (std::max(b, rg * T) < std::min(e, (rg + 1) * T) && b <= rg * T) {
+                    CHECK(first < 0);
+                    first = g;
+                }
+            }
+            CHECK(first >= 0 && pieces[rg] >= 1 && begun - first == pieces[rg]);
+            for (int i = first; i < begun; ++i) CHECK(used[i + rg] == rg);
+            most = std::max(most, pieces[rg]);
+        }
+        CHECK(most == sp.max_pieces);
         left_over += wp.split > 0;
         const size_t part = (size_t)p.Hkv * sp.slots * hw::PLAN_SLOT_ROWS * (p.Ev + 2) * 4;
         CHECK(sp.partial_bytes == part && wp.workspace_bytes >= part + (size_t)p.Hkv * cp.plan[0].rows * 8 + cp.rope_bytes && wp.workspace_bytes % 256 == 0);
