@@ -222,18 +222,19 @@ int plan_call(const hw_problem* p, int num_cus, CallPlan* cp, int fused) {
     return HW_OK;
 }
 
-// Row groups of 128 rows that do not fill the CUs evenly: 40 row groups of 8 kv heads (1024 prompt tokens at a GQA ratio of
-// 5) are 320 workgroups, so 256 CUs take two rounds of which the second is a quarter full.  Cut into equal runs across the
-// row groups every CU gets 1.25 row groups of work instead of 2.  A run that crosses into the next row group opens it anew
+// Row groups of 128 rows that do not fill the CUs evenly, fewer than one for every workgroup of a head (the others are whole_size's):
+// 24 row groups of 8 kv heads (600 prompt tokens at a GQA ratio of 5) are 192 workgroups, which leave 64 of 256 CUs idle.  Cut into
+// equal runs across the row groups every CU gets three quarters of a row group of work instead of one.  A run that crosses into the next row group opens it anew
 // (queries, partial sums), so the runs are dealt by tiles plus openings at kJobCost and kOpenCost tiles.  (Runs dealt by
 // the kernel over the tiles that the locations leave visible were measured slower, 300 against 282 us for two layers of 1024
 // tokens behind 4096: a row group's unseen tiles cost next to nothing as it is, and the uneven row groups give some runs a
 // third one to open.)
 // Where to take them: a price of each launch in tiles, rounds against runs, with kJobPrice and kOpenPrice per opening.  The
 // prices and the line at kWorth were fitted to 1626 calls timed both ways, merge launches included (24 to 1500 new tokens of
-// 1 to 8 workers behind 0 to 16 K, eight head layouts, D = 64 and 128): the 1305 that the rule takes gain 0.994 to 1.66,
-// 1.21 in the median (1024 tokens behind 4096 at 40/8 heads, D = 128: 180 -> 138 us a layer); the 321 that it leaves in rounds
-// would give 0.88 to 1.17, 1.03 in the median (133 tokens of two workers behind 761: 28 -> 32 us).
+// 1 to 8 workers behind 0 to 16 K, eight head layouts, D = 64 and 128; before there were whole row groups, whose calls are among
+// them): the 1305 that the rule takes gain 0.994 to 1.66, 1.21 in the median (600 tokens behind 8192 at 40/8 heads, D = 128: 144 -> 124
+// us a layer); the 321 that it leaves in rounds would give 0.88 to 1.17, 1.03 in the median (133 tokens of two workers behind 761:
+// 28 -> 32 us).
 constexpr int kMinPiece = 4;      // tiles worth opening a row group for
 bool stream_size(const hw_problem* p, int num_cus, const CallPlan& cp, StreamPlan* sp) {
     const hw_plan& plan = cp.plan[0];
@@ -332,18 +333,19 @@ void stream_deal(const hw_problem* p, const CallPlan& cp, StreamPlan* sp) {
     }
 }
 
-// Calls with at least a row group for every workgroup of a head (one workgroup per CU).  A run across row groups writes fp32
-// partial sums for both of its ends, 37 MB a layer for 1024 tokens at 40/8 heads, which the merge reads again in 11.6 us.  Here
-// floor(row groups / workgroups) row groups go whole to each workgroup, which holds complete rows at the end and writes the result,
-// and only the remainder is cut into runs (stream_deal), a fifth of the rows with 40 row groups on 32 workgroups.  With no
-// remainder there is no merge launch.  The remainder are the first row groups, which see least of a causal chunk.
+// Calls with at least a row group for every workgroup of a head (one workgroup per CU; at head dimension 256 also with fewer, which
+// are then all in runs).  A run across row groups writes fp32 partial sums for both of its ends, 37 MB a layer for 1024 tokens at 40/8
+// heads, which the merge reads again in 11.6 us.  Here floor(row groups / workgroups) row groups go whole to each workgroup, which holds
+// complete rows at the end and writes the result, and only the remainder is cut into runs (whole_deal), a fifth of the rows with 40 row
+// groups on 32 workgroups.  With no remainder there is no merge launch.  The remainder are the first row groups, which see least of a
+// causal chunk.
 // Against runs, resp. rounds, a layer: 1024 tokens behind 4096 (40/8, D = 128) 124 -> 117 us, 2 x 574 behind 1333 88 -> 83.5, 1500
 // behind nothing at 32/8 69 -> 61.5, 1500 behind 128 66.5 -> 60 (and see whole_deal).  Where the heads divide the CUs this is never
 // more work a CU than rounds.  Where they do not, CUs stay idle that rounds would use, and the workgroups take nrg / wgs row groups
-// one after the other against the rounds: 9 row groups of 56 heads (1119 tokens behind 1200, D = 128) 2.25 against 2, 105.6 against
-// 100.6 us; 5 of 96 2.5 against 2 (D = 64: 65 against 60 behind 1200, 131 against 116 behind 4000), 3 of 140 3 against 2 (144 against
-// 115).  What is saved in partial sums is worth about 16 tiles of that: 621 tokens behind 150 at 96 heads (25 tiles) 39 against 43 us.  (Of 400 calls
-// of 1 to 160 heads 9 lost 3 % or more, up to 31 %, with whole row groups throughout, 1 with the line, 5 %.)
+// one after the other against the rounds: 9 row groups of 56 heads (1119 tokens behind 1200, D = 128) 2.25 against 2, 106 against
+// 101 us; 5 of 96 2.5 against 2 (D = 64: 65 against 60 behind 1200, 131 against 116 behind 4000), 3 of 140 3 against 2 (144 against
+// 115).  What is saved in partial sums is worth about 16 tiles of that: 621 tokens behind 150 at 96 heads (25 tiles) 39 against 43 us.
+// (Of 400 calls of 1 to 160 heads 9 took longer by 3 % or more, up to 31 %, with whole row groups throughout; 1 does with the line, 5 %.)
 // Head dimension 256: the plan's kernel takes 16 rows a workgroup, so every 16 rows stream the K/V through a CU again.  Enough of
 // that, counted in tiles a CU takes in, and 128-row workgroups are faster, whose openings cost more.  16/8 heads, bf16, us a layer
 // before / after: 1024 tokens behind 4096 (640 tiles a CU) 296 -> 111, 1500 behind 100 168 -> 70, 2 x 200 behind 5000 154 -> 79, 2 x 300

@@ -56,8 +56,8 @@ bool stream_size(const hw_problem* p, int num_cus, const CallPlan& cp, StreamPla
 // take a loop over row groups and workgroups (40 row groups, 32 workgroups: 1.7 us with 2 fragments, 2.6 with 60, 46 when it
 // visited every fragment of every row group; sizing 0.02).
 void stream_deal(const hw_problem* p, const CallPlan& cp, StreamPlan* sp);
-// The same for calls with at least a row group for every workgroup (see whole_size in the source): as many row groups as go
-// round are dealt whole -- their workgroups write the result, no partial sums -- and the others in runs.
+// The same for calls with at least a row group for every workgroup, and at head dimension 256 (see whole_size in the source): as many
+// row groups as go round are dealt whole -- their workgroups write the result, no partial sums -- and the others in runs.
 struct WholePlan {
     int split, whole;                    // row groups 0 .. split - 1 in runs, the `whole` behind them one to a workgroup
     int wgs;                             // workgroups per kv head

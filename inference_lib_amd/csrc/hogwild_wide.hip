@@ -185,7 +185,7 @@ struct WideRotation {
 
 // STREAM: the workgroup's run of tiles may cross row groups, and it may have whole row groups of its own (KH_STREAM): the body is
 // then done once per row group.  Prompt chunk of 1024 tokens behind 4096 (40 / 8 heads, D = 128, bf16; 97 GFLOP): two layers
-// 288 -> 244 us (runs throughout and tiles streamed past the L2 -> whole row groups first and tiles kept, see keep_in_l2 and
+// 271 -> 235 us (runs throughout and tiles streamed past the L2 -> whole row groups first and tiles kept, see keep_in_l2 and
 // whole_size), 341 in two rounds of workgroups.  What bounds it is power as much as the arithmetic of two waves per SIMD (matrix
 // units 39 %, vector units 50 % of the clocks): the shader clock follows the load, 2.37 GHz in this form and 2.08-2.12 GHz in one
 // with 32 x 32 x 16 products whose 13 % fewer clocks took the same time.

@@ -1,5 +1,6 @@
 // whole_size and whole_deal over random calls of 128-row workgroups: the row groups dealt whole and the runs cover every row group
-// once, every piece of a run has a slot inside the workspace, max_pieces bounds the pieces of a row group.
+// once, every piece of a run has a slot inside the workspace, the merge is told of the slots that were written and of no others.  And
+// the lines of the rules: which calls are dealt so, at head dimension 256 too, which by the tiles seen, which paged ones keep their tiles.
 #include <algorithm>
 #include <cstdio>
 #include <random>

@@ -1,5 +1,5 @@
 """step_inputs, the one native call behind layer 0 of a HogwildCache step, against build_inputs and the lengths themselves; what it
-refuses comes back as False.  hogwild_sdpa on fragments that have to be copied."""
+refuses comes back as False, a stream that is being captured as an error.  hogwild_sdpa on fragments that have to be copied."""
 import pytest
 import torch
 

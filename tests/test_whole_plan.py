@@ -1,4 +1,4 @@
-"""The plan that deals row groups of 128 rows whole, checked over random calls on the CPU."""
+"""The plan that deals row groups of 128 rows whole, checked over random calls on the CPU, and the rules that choose it."""
 import os
 import shutil
 import subprocess
