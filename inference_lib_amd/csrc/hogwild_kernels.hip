@@ -419,7 +419,8 @@ __global__ __launch_bounds__(256) void merge_kernel(const MergeArgs a) {
     }
 }
 
-// Standalone rotation: out[f,w,h,s,:] = rope(q[w,h,s,:], cos/sin[f,w,s,:])   (src/rope.cuh:2-52)
+// Standalone rotation: out[f,w,h,s,:] = rope(q[w,h,s,:], cos/sin[f,w,s,:])   (src/rope.cuh:2-52).  One element per thread, for widths and
+// addresses that rope_chunks_kernel cannot take.
 template <class DT>
 __global__ __launch_bounds__(256) void rope_kernel(void* out_, const void* q_, const float* cosv, const float* sinv, int F, int W,
                                                    int Hq, int S, int E, int RotE) {
@@ -446,6 +447,52 @@ __global__ __launch_bounds__(256) void rope_kernel(void* out_, const void* q_, c
             else val = x * cosv[cs + e - h] + Elem<DT>::to_float(qp[e - h]) * sinv[cs + e - h];
         }
         out[idx] = Elem<DT>::from_float(val);
+    }
+}
+
+// The same rotation, 16 bytes of either half of a row per thread: one unit = the chunk pair (u, u + half) of a row, or a chunk behind the
+// rotary width, which is copied.  A workgroup stays within one (fragment, worker) pair, so what is left of the index arithmetic are two
+// 32-bit divisions a thread.  (With one element per thread and five 64-bit divisions around it, instructions were what the launch waited
+// for: 9 fragments x 8 workers x 5 tokens x 64 heads, D = 128, 14.7 -> 5.3 us; 4 x 3 x 2 x 8, D = 64, a launch's minimum, 3.0 -> 2.6.)
+template <class DT>
+__global__ __launch_bounds__(256) void rope_chunks_kernel(void* out_, const void* q_, const float* cosv, const float* sinv, unsigned FW, unsigned W,
+                                                          unsigned Hq, unsigned S, unsigned E, unsigned RotE, unsigned blocks_per_pair) {
+    constexpr int CH = Chunk<DT>::CH;
+    const unsigned half = RotE / (2 * CH), units = E / CH - half;      // chunks of half the rotary width; units of a row
+    const unsigned per = Hq * S * units;                               // units of a (fragment, worker) pair
+    const u32x4* qb = reinterpret_cast<const u32x4*>(q_);
+    u32x4* out = reinterpret_cast<u32x4*>(out_);
+    for (unsigned b = blockIdx.x; b < FW * blocks_per_pair; b += gridDim.x) {
+        const unsigned fw = b / blocks_per_pair, w = fw % W;           // (uniform)
+        const unsigned idx = (b - fw * blocks_per_pair) * blockDim.x + threadIdx.x;
+        if (idx >= per) continue;
+        const unsigned row = idx / units, u = idx - row * units;       // row = head * S + token
+        const unsigned s = row % S;
+        const u32x4* src = qb + ((size_t)w * Hq * S + row) * (E / CH);
+        u32x4* dst = out + ((size_t)fw * Hq * S + row) * (E / CH);
+        if (u >= half) {
+            dst[u + half] = src[u + half];
+            continue;
+        }
+        const u32x4 xa = src[u], xb = src[u + half];
+        const size_t co = ((size_t)fw * S + s) * RotE + u * CH;
+        f32x4 cs[CH / 4], sn[CH / 4];
+#pragma unroll
+        for (int i = 0; i < CH / 4; ++i) {
+            cs[i] = *reinterpret_cast<const f32x4*>(cosv + co + 4 * i);
+            sn[i] = *reinterpret_cast<const f32x4*>(sinv + co + 4 * i);
+        }
+        float x1[CH], x2[CH], y1[CH], y2[CH];
+        Chunk<DT>::unpack(xa, x1);
+        Chunk<DT>::unpack(xb, x2);
+#pragma unroll
+        for (int i = 0; i < CH; ++i) {
+            const float c = cs[i >> 2][i & 3], sv = sn[i >> 2][i & 3];
+            y1[i] = x1[i] * c - x2[i] * sv;
+            y2[i] = x2[i] * c + x1[i] * sv;
+        }
+        dst[u] = Chunk<DT>::pack(y1);
+        dst[u + half] = Chunk<DT>::pack(y2);
     }
 }
 
@@ -549,18 +596,37 @@ hipError_t launch_merge(const MergeArgs& ma, int dtype, int EV, hipStream_t stre
     }
 }
 
+template <class DT>
+static hipError_t launch_rope_dt(void* out, const void* q, const float* cosv, const float* sinv, int F, int W, int Hq, int S, int E, int RotE,
+                                 hipStream_t stream) {
+    constexpr int CH = Chunk<DT>::CH;
+    const size_t total = (size_t)F * W * Hq * S * E;
+    const uintptr_t tables = RotE > 0 ? reinterpret_cast<uintptr_t>(cosv) | reinterpret_cast<uintptr_t>(sinv) : 0;
+    // rope_chunks_kernel moves 16-byte pieces: rows and halves of the rotary width have to be whole numbers of them, and aligned (tables
+    // with such a width then are, row by row)
+    const bool chunks = E % CH == 0 && RotE % (2 * CH) == 0 && ((reinterpret_cast<uintptr_t>(out) | reinterpret_cast<uintptr_t>(q) | tables) & 15u) == 0;
+    const size_t per = (size_t)Hq * S * (size_t)(E / CH - RotE / (2 * CH));      // units of a (fragment, worker) pair
+    const size_t pair_blocks = (per + 255) / 256, nblocks = (size_t)F * W * pair_blocks;
+    if (chunks && per < (1u << 31) && nblocks < (1u << 31)) {
+        const unsigned threads = per < 256 ? (unsigned)((per + 63) & ~(size_t)63) : 256;
+        const unsigned grid = nblocks < (1u << 20) ? (unsigned)nblocks : 1u << 20;
+        hipLaunchKernelGGL((rope_chunks_kernel<DT>), dim3(grid), dim3(threads), 0, stream, out, q, cosv, sinv, (unsigned)F * (unsigned)W, (unsigned)W,
+                           (unsigned)Hq, (unsigned)S, (unsigned)E, (unsigned)RotE, (unsigned)pair_blocks);
+        return hipGetLastError();
+    }
+    int blocks = total < (size_t)4096 * 256 ? (int)((total + 255) / 256) : 4096;
+    if (blocks < 1) blocks = 1;
+    hipLaunchKernelGGL((rope_kernel<DT>), dim3(blocks), dim3(256), 0, stream, out, q, cosv, sinv, F, W, Hq, S, E, RotE);
+    return hipGetLastError();
+}
+
 hipError_t launch_rope(void* out, const void* q, const float* cosv, const float* sinv, int dtype, int F, int W, int Hq, int S,
                        int E, int RotE, hipStream_t stream) {
-    const size_t total = (size_t)F * W * Hq * S * E;
-    int blocks = (int)((total + 255) / 256);
-    if (blocks > 4096) blocks = 4096;
-    if (blocks < 1) blocks = 1;
     switch (dtype) {
-        case 0: hipLaunchKernelGGL((rope_kernel<F32>), dim3(blocks), dim3(256), 0, stream, out, q, cosv, sinv, F, W, Hq, S, E, RotE); break;
-        case 1: hipLaunchKernelGGL((rope_kernel<F16>), dim3(blocks), dim3(256), 0, stream, out, q, cosv, sinv, F, W, Hq, S, E, RotE); break;
-        default: hipLaunchKernelGGL((rope_kernel<BF16>), dim3(blocks), dim3(256), 0, stream, out, q, cosv, sinv, F, W, Hq, S, E, RotE); break;
+        case 0: return launch_rope_dt<F32>(out, q, cosv, sinv, F, W, Hq, S, E, RotE, stream);
+        case 1: return launch_rope_dt<F16>(out, q, cosv, sinv, F, W, Hq, S, E, RotE, stream);
+        default: return launch_rope_dt<BF16>(out, q, cosv, sinv, F, W, Hq, S, E, RotE, stream);
     }
-    return hipGetLastError();
 }
 
 }  // namespace hw
