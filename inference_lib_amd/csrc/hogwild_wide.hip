@@ -60,12 +60,13 @@ constexpr int WIDE_ROWS = 128;      // query rows per workgroup: 32 per wave
 
 // A slice of device memory as a raw buffer descriptor (base, stride 0, size in bytes, flags): reads beyond the size
 // return zero.  Held as plain words: the transfers below are issued from inline assembly.
+constexpr u32 RAW_FLAGS = 0x00020000u;
 __device__ __forceinline__ u32x4 raw_descriptor(unsigned long long base, unsigned bytes) {
     u32x4 d;
     d.x = __builtin_amdgcn_readfirstlane((u32)base);
     d.y = __builtin_amdgcn_readfirstlane((u32)(base >> 32) & 0xffffu);
     d.z = __builtin_amdgcn_readfirstlane(bytes);
-    d.w = 0x00020000u;
+    d.w = RAW_FLAGS;
     return d;
 }
 // One 1 KB global->LDS transfer (lane l: 16 bytes from descriptor offset `voffset` to LDS byte `lds` + 16 l), non-temporal
@@ -83,6 +84,18 @@ __device__ __forceinline__ void lds_transfer(const u32x4& desc, unsigned lds, un
 }
 #pragma clang diagnostic pop
 
+// The same with a 64-bit address per lane (rows that no descriptor could bound: the paged cache, queries): lane l brings 16 bytes
+// from `src` to LDS byte `lds` + 16 l, or, with DWORD, 4 bytes to `lds` + 4 l.
+#pragma clang diagnostic push
+#pragma clang diagnostic ignored "-Winline-asm"
+template <bool KEEP, bool DWORD = false>
+__device__ __forceinline__ void lds_transfer_flat(unsigned lds, unsigned long long src) {
+    if constexpr (DWORD) asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dword %1, off" ::"s"(lds), "v"(src) : "m0", "memory");
+    else if constexpr (KEEP) asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off" ::"s"(lds), "v"(src) : "m0", "memory");
+    else asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off nt" ::"s"(lds), "v"(src) : "m0", "memory");
+}
+#pragma clang diagnostic pop
+
 // One wave's share of a tile's transfers: TPW 1 KB pieces of ONE image (the first half of the waves fill K, the second
 // half V), into LDS bytes `slot` + 1024 j.  `tile` = byte offset of the tile in the kv head's slice (OOB_OFFSET for a
 // tile that does not exist: the same number of transfers, no memory traffic, zeros in LDS).
@@ -95,6 +108,103 @@ __device__ __forceinline__ void wide_request(const u32x4& desc, unsigned slot, u
 __device__ __forceinline__ unsigned lds_address(const void* p) {
     return __builtin_amdgcn_readfirstlane((unsigned)(size_t)HW_LDS_PTR(p));
 }
+
+// What the opening of a fragment needs besides its tiles, for the 128 rows of a workgroup: the queries, the cos/sin table rows of
+// their (worker, token) pairs and the rows' locations.  All of it is brought into LDS by transfers that nobody waits for until the
+// fragment is opened -- for every fragment but the workgroup's first they run beside the tiles of the one before -- and the queries are
+// rotated where they lie.  The rows of one (worker, token) pair share their table row, so the distinct rows are staged (first halves
+// only: both halves of the rotation read cos/sin at the first-half index, src/rope.cuh:30-46), CSMAX of them; a workgroup whose
+// rows span more pairs than that (GQA ratio below 4) reads them from memory where it rotates.
+template <class DT, int E, bool PRE, int NW>
+struct WideQueries {
+    typedef Geo<DT, E, E> G;
+    static constexpr int SZ = Elem<DT>::size;
+    static constexpr int CH = Chunk<DT>::CH;
+    static constexpr int NT = NW * 64;
+    static constexpr int IPR = E / (2 * CH);                        // chunk pairs per row
+    static constexpr int NIT = WIDE_ROWS * IPR / NT;                // chunk pairs per thread
+    static constexpr int CSMAX = 36;                                // table rows staged per workgroup
+    static constexpr int CPW = E / 2 / 4;                           // float4 per half table row
+    static constexpr int CS_FLOATS = CSMAX * E;                     // [row][cos half | sin half]
+    static constexpr int NQ = WIDE_ROWS * G::KROW / 1024 / NW;      // query transfers per wave
+    static constexpr int RPQ = 1024 / G::KROW;                      // rows of each
+    static constexpr int RPC = 1024 / (E * 4);                      // table rows of a transfer
+    static_assert(WIDE_ROWS * IPR % NT == 0 && WIDE_ROWS * G::KROW % (1024 * NW) == 0 && CSMAX % RPC == 0, "whole transfers");
+
+    // The image of the queries in LDS is that of a K tile: rows of KROW bytes, 16-byte chunks XOR-swizzled by the row.
+    // Rows beyond R (MFMA padding) read the first row of the group; they are zeroed where the operands are read.
+    static __device__ __forceinline__ void request_queries(const DevHeader& a, unsigned q_base, int f, int hkv, int r0, int GQ, int wv, int lane) {
+#pragma unroll
+        for (int j = 0; j < NQ; ++j) {
+            const int piece = wv * NQ + j;
+            const int rr = piece * RPQ + lane / G::CPR, slot = lane % G::CPR;
+            const int key = G::CPR >= 16 ? (rr & 15) : ((rr >> 1) & (G::CPR - 1));
+            const RowMap rm = map_row(a, r0 + rr < a.R ? r0 + rr : r0, hkv, GQ);
+            const size_t row = rm.qrow + (PRE ? (size_t)f * a.W * a.Hq * a.S : 0);
+            lds_transfer_flat<true>(__builtin_amdgcn_readfirstlane(q_base + piece * 1024), reinterpret_cast<unsigned long long>(a.q) + (row * E * SZ + ((slot ^ key) << 4)));
+        }
+    }
+    // fragment f's table rows ws_lo .. ws_lo + nws - 1 (nws <= CSMAX), and the locations of the rows
+    static __device__ __forceinline__ void request_tables(const DevHeader& a, unsigned cs_base, unsigned loc_base, int f, int r0, int ws_lo, int nws, bool staged,
+                                                          int wv, int lane) {
+        if (staged) {
+            for (int piece = wv; piece * RPC < nws; piece += NW) {
+                const int wi = min(piece * RPC + lane / (2 * CPW), nws - 1), part = lane % (2 * CPW);      // beyond the last row: re-read it
+                const unsigned long long cosv = reinterpret_cast<unsigned long long>(a.cos), to_sin = reinterpret_cast<unsigned long long>(a.sin) - cosv;
+                const unsigned long long tab = cosv + (part < CPW ? 0ull : to_sin);
+                lds_transfer_flat<true>(__builtin_amdgcn_readfirstlane(cs_base + piece * 1024), tab + (((size_t)f * a.W * a.S + ws_lo + wi) * E + (part % CPW) * 4) * 4);
+            }
+        }
+        if (wv < WIDE_ROWS / 64) {
+            const int ws = fast_div(min(r0 + wv * 64 + lane, a.R - 1), a.magic_gq);
+            lds_transfer_flat<true, true>(__builtin_amdgcn_readfirstlane(loc_base + wv * 256), reinterpret_cast<unsigned long long>(a.loc) + ((size_t)f * a.W * a.S + ws) * 4);
+        }
+    }
+    template <bool STAGED>
+    static __device__ __forceinline__ void rotate(const DevHeader& a, char* q_lds, const float* cs_lds, int f, int hkv, int r0, int GQ, bool write_rq, int tid, int ws_lo) {
+        const size_t fstride = (size_t)a.W * a.Hq * a.S * E;
+#pragma unroll
+        for (int it = 0; it < NIT; ++it) {
+            const int item = tid + it * NT;
+            // (rows with bits 2 and 3 exchanged: the chunks that a wave takes at once then lie in both halves of the rows)
+            const int ri = item / IPR, slot = item % IPR, rr = (ri & ~12) | ((ri & 4) << 1) | ((ri & 8) >> 1);
+            const bool pad = r0 + rr >= a.R;
+            const RowMap rm = map_row(a, pad ? r0 : r0 + rr, hkv, GQ);
+            char* lo = q_lds + kstage_offset<G>(rr, slot);
+            char* hi = q_lds + kstage_offset<G>(rr, slot + IPR);
+            f32x4 cs[CH / 4], sn[CH / 4];
+#pragma unroll
+            for (int i = 0; i < CH / 4; ++i) {
+                if constexpr (STAGED) {
+                    const float* tab = cs_lds + (rm.ws - ws_lo) * E + slot * CH + 4 * i;
+                    cs[i] = *reinterpret_cast<const f32x4*>(tab);
+                    sn[i] = *reinterpret_cast<const f32x4*>(tab + E / 2);
+                } else {
+                    const size_t co = ((size_t)f * a.W * a.S + rm.ws) * E + slot * CH + 4 * i;
+                    cs[i] = *reinterpret_cast<const HW_GLOBAL f32x4*>(a.cos + co);
+                    sn[i] = *reinterpret_cast<const HW_GLOBAL f32x4*>(a.sin + co);
+                }
+            }
+            float x1[CH], x2[CH], y1[CH], y2[CH];
+            Chunk<DT>::unpack(*reinterpret_cast<const u32x4*>(lo), x1);
+            Chunk<DT>::unpack(*reinterpret_cast<const u32x4*>(hi), x2);
+#pragma unroll
+            for (int i = 0; i < CH; ++i) {
+                const float c = cs[i >> 2][i & 3], sv = sn[i >> 2][i & 3];
+                y1[i] = x1[i] * c - x2[i] * sv;
+                y2[i] = x2[i] * c + x1[i] * sv;
+            }
+            const u32x4 ya = Chunk<DT>::pack(y1), yb = Chunk<DT>::pack(y2);
+            *reinterpret_cast<u32x4*>(lo) = ya;
+            *reinterpret_cast<u32x4*>(hi) = yb;
+            if (write_rq && !pad) {
+                HW_GLOBAL char* rqp = a.rq + (f * fstride + rm.qrow * E) * SZ;
+                *reinterpret_cast<HW_GLOBAL u32x4*>(rqp + slot * 16) = ya;
+                *reinterpret_cast<HW_GLOBAL u32x4*>(rqp + (slot + IPR) * 16) = yb;
+            }
+        }
+    }
+};
 
 // Query rotation of one fragment for the 128 rows of a workgroup (the role of QueryRotation in the narrow kernel).  The
 // rows of one (worker, token) pair share their cos/sin table row, and with 128 rows per workgroup loading it per query
@@ -210,10 +320,19 @@ __global__ __launch_bounds__(NW * 64, 1) void attention_wide_kernel(const Kernel
 
     // Head dimension 256: every wave loads and rotates its own operands in registers (LaneRotation), the ring takes the LDS.
     constexpr bool LANES = E > 128;
-    __shared__ __attribute__((aligned(16))) char q_lds[LANES ? 16 : WIDE_ROWS * G::QSTR];
-    __shared__ int lim_lds[LANES ? 1 : WIDE_ROWS];
+    // AHEAD: what opening a fragment needs is brought into LDS beside the tiles of the one before (WideQueries), the fragment's first
+    // tiles follow the last of the one before without a pause, and tiles that no row of the workgroup sees are not taken in.  Prompt
+    // chunks of several workers, which open a row group and two or three fragments per workgroup and row group (D = 128, bf16 and fp16, us
+    // a layer): 2 x 574 tokens behind 1333 at 40/8 heads 86 -> 83, 2 x 799 behind 791 109 -> 104, 2 x 657 behind 75 at 32/8 58 -> 55; 50 calls
+    // of 2 to 4 workers 0.99 to 1.05 times as fast, 1.017 in the mean.  Pre-rotated, 7 x 6 tokens: 26.2 -> 24.9 (40/8), 29.2 -> 28.1
+    // (28/4).  Not where it costs more than it hides: with one or two openings a launch (the other fused calls, 0.95 to 0.99 times),
+    // at D = 64 (0.94 to 0.98: half the arithmetic a tile beside the same scalar work) and 256 (0.97 to 0.99: a barrier per tile).
+    constexpr bool AHEAD = E <= 128 && (PRE || (STREAM && E == 128));
+    typedef WideQueries<DT, LANES ? 128 : E, PRE, NW> WQ;         // (not used at head dimension 256)
     typedef WideRotation<DT, E, G::QSTR, NT> WRot;
-    __shared__ __attribute__((aligned(16))) float cs_lds[PRE || LANES ? 4 : WRot::CS_FLOATS];
+    __shared__ __attribute__((aligned(16))) char q_lds[LANES ? 16 : WIDE_ROWS * (AHEAD ? G::KROW : G::QSTR)];
+    __shared__ int lim_lds[LANES ? 1 : WIDE_ROWS];        // the rows' bounds, with AHEAD their locations
+    __shared__ __attribute__((aligned(16))) float cs_lds[PRE || LANES ? 4 : WQ::CS_FLOATS];
     // ring slots: [K image | V image]; K is swizzled like in the narrow kernel, V is a plain row-major image
     __shared__ __attribute__((aligned(16))) char ring[NS * SLOT];
 
@@ -291,92 +410,9 @@ __global__ __launch_bounds__(NW * 64, 1) void attention_wide_kernel(const Kernel
     [[maybe_unused]] bool whole = STREAM && split_groups + g < groups;
     int rgi = STREAM ? (whole ? split_groups + g : run_begin / tiles_head) : rg;
     int r0, w0;                                 // first row of the workgroup, of this wave
-    int ws_lo, nws;                             // (worker, token) pairs the rows of this workgroup belong to
-    bool staged;                                // their tables go through LDS; uniform over the workgroup
     unsigned long long todo;                    // fragments with tiles of this workgroup
-    WRot wrot;
     WaveState<RB, G::NOC> st;
-    // The queries to rotate are the same for every fragment: they are requested here, before the workgroup's tile range
-    // and first fragment are worked out, and are on their way while that happens.
-    auto open_rows = [&]() {
-        if constexpr (STREAM) {
-            T0 = whole ? 0 : max(run_begin - rgi * tiles_head, 0);
-            T1 = whole ? tiles_head : min(run_end - rgi * tiles_head, tiles_head);
-        }
-        r0 = rgi * WIDE_ROWS;
-        w0 = r0 + rw * WROWS;
-        ws_lo = fast_div(r0, a.magic_gq);
-        nws = fast_div(min(r0 + WIDE_ROWS, a.R) - 1, a.magic_gq) - ws_lo + 1;
-        staged = !PRE && !LANES && nws <= WRot::CSMAX;
-        int tids = tid;
-        if constexpr (STREAM) asm volatile("" : "+v"(tids));      // (see open_segment)
-        if (staged) wrot.load_queries(a, hkv, r0, GQ, tids);
-#pragma unroll
-        for (int rb = 0; rb < RB; ++rb) {
-            st.m[rb] = NEG_BIG;
-            st.l[rb] = 0.f;
-#pragma unroll
-            for (int c = 0; c < G::NOC; ++c) st.o[rb][c] = f32x4{0.f, 0.f, 0.f, 0.f};
-        }
-        st.fresh = true;
-        todo = __ballot(lane < a.F && max(T0, my_tb) < min(T1, my_te));
-    };
-    open_rows();
 
-    HW_MARK(10);
-    int f = 0, L = 0, lt0 = 0, lt1 = 0;
-    bool opens_fragment = false;
-    u32x4 view = {0, 0, 0, 0};                               // this wave's image of the current fragment (K or V slice)
-    [[maybe_unused]] QueryRotation<DT, E, WIDE_ROWS, G::QSTR, true, NT> qrot;     // pre-rotated queries: a copy into LDS
-    [[maybe_unused]] LaneRotation<DT, E, RB, PRE> lrot;
-    int lm = 0;
-
-    // this wave's share of the PAR tiles of the step that starts at tile `lt` (fragment-local) into step slot `ss`; a tile
-    // that does not exist is requested out of range: the same number of transfers, no memory traffic, zeros in LDS
-    auto request = [&](int ss, int lt) {
-#pragma unroll
-        for (int pp = 0; pp < PAR; ++pp) {
-            const unsigned tile_bytes = (unsigned)((lt + pp) * TILE * image_row);
-            wide_request<TPW, KEEP>(view, __builtin_amdgcn_readfirstlane(my_image + (ss * PAR + pp) * SLOT), lt + pp < lt1 ? tile_bytes : OOB_OFFSET, off);
-        }
-    };
-
-    auto open_segment = [&](bool queries_requested) {
-        f = __builtin_ctzll(todo);
-        todo &= todo - 1;
-        const int fb = __builtin_amdgcn_readlane(my_tb, f);
-        const int fe = __builtin_amdgcn_readlane(my_te, f);
-        const int s0 = max(T0, fb), s1 = min(T1, fe);
-        L = __builtin_amdgcn_readlane(my_len, f);
-        const unsigned long long base = ((unsigned long long)(unsigned)__builtin_amdgcn_readlane((int)(my_image_ptr >> 32), f) << 32) |
-                                        (unsigned)__builtin_amdgcn_readlane((int)my_image_ptr, f);
-        const int cap = __builtin_amdgcn_readlane(my_cap, f);
-        view = raw_descriptor(base + (unsigned long long)hkv * cap * image_row, (unsigned)(L * image_row));
-        lt0 = s0 - fb;
-        lt1 = s1 - fb;
-        opens_fragment = s0 == fb;
-        // The first step is requested before the queries: the compiler's wait for the query loads then also waits for it
-        // (loads complete in order), which costs nothing, its tiles being needed first anyway.  The other look-ahead
-        // steps follow when the queries have arrived, so that the rotation does not wait for them as well.
-        request(0, lt0);
-        HW_MARK(11);
-        // (the thread index as the compiler cannot see through it: what is derived from it -- rows, addresses of the
-        // queries -- is then formed per segment instead of once in front of the loop over the segments, from where it
-        // would stay in registers across the tile loops, which have none to spare)
-        int tids = tid;
-        asm volatile("" : "+v"(tids));
-        if constexpr (LANES) {
-            lrot.load(a, f, hkv, w0, GQ, tids & 15, (tids >> 4) & 3);
-            return;
-        } else if constexpr (PRE) {
-            qrot.load(a, f, hkv, r0, GQ, tids);
-        } else if (staged) {
-            if (!queries_requested) wrot.load_queries(a, hkv, r0, GQ, tids);
-            wrot.load_tables(a, f, tids, ws_lo, nws);
-        }
-        // the bound of row tid / TPR (TPR threads per row, all load: keeps the load unconditional)
-        lm = a.loc[(size_t)f * a.W * a.S + fast_div(min(r0 + tids / TPR, a.R - 1), a.magic_gq)];
-    };
     // ---- The PAR waves that share their rows hold a partial sum each: block rb of the rows goes to wave rb % PAR of them
     // through LDS, lane for lane in the accumulator layout, and is added up there.  Then every wave stores the blocks it
     // owns.  The accumulator layout scatters a row over the lanes in 16-byte pieces; written like that, a partial (17 MB
@@ -481,141 +517,491 @@ __global__ __launch_bounds__(NW * 64, 1) void attention_wide_kernel(const Kernel
         }
     };
 
-    bool more = todo != 0;
-    if (more) open_segment(staged);
-    HW_MARK(6);
-    bool hw_first = true;
-
-    while (more) {
-        if constexpr (!LANES) __syncthreads();   // previous segment's readers are done with q_lds / lim_lds
-        if (hw_first) HW_MARK(7);
-        int tids = tid;        // (see open_segment)
-        asm volatile("" : "+v"(tids));
-        // Every load of open_segment is waited for here, in a form the compiler sees: it waits for a load where its result
-        // is first used and counts only the loads it knows of, so a wait that it places further down -- for the bound
-        // below, the last load of open_segment -- would also wait for the look-ahead steps requested in between.
-        // (Nothing is lost: the queries are needed now, and the first step was requested before them.)
-        __builtin_amdgcn_s_waitcnt(0x0F70);   // vmcnt(0)
-        u32x4 qreg[RB * G::KJ];                      // this wave's query operands and mask bounds
-        int lim[RB];
-        if constexpr (LANES) {
+    if constexpr (AHEAD) {
+        // The rows of a row group: (worker, token) pairs they belong to, and whether their tables go through LDS; uniform over the workgroup.
+        struct Rows {
+            int r0, ws_lo, nws;
+            int staged;
+        };
+        auto rows_of = [&](int group) {
+            Rows r;
+            r.r0 = group * WIDE_ROWS;
+            r.ws_lo = fast_div(r.r0, a.magic_gq);
+            r.nws = fast_div(min(r.r0 + WIDE_ROWS, a.R) - 1, a.magic_gq) - r.ws_lo + 1;
+            r.staged = !PRE && r.nws <= WQ::CSMAX;
+            return r;
+        };
+        // One segment = the part of a fragment that lies in the workgroup's tile range.
+        struct Segment {
+            int f, L, lt0, lt1;                     // fragment, its length, tiles (fragment-local)
+            int opens;                              // this workgroup owns the fragment's first tile (and writes its rotated queries)
+            u32 lo, hi, bytes;                      // this wave's image of the fragment (K or V slice, see raw_descriptor)
+        };   // (no padding: the compiler copies it through memory)
+        auto segment_of = [&](int f) {
+            Segment s;
+            const int fb = __builtin_amdgcn_readlane(my_tb, f);
+            const int fe = __builtin_amdgcn_readlane(my_te, f);
+            const int s0 = max(T0, fb), s1 = min(T1, fe);
+            s.f = f;
+            s.L = __builtin_amdgcn_readlane(my_len, f);
+            const unsigned long long base = ((unsigned long long)(unsigned)__builtin_amdgcn_readlane((int)(my_image_ptr >> 32), f) << 32) |
+                                            (unsigned)__builtin_amdgcn_readlane((int)my_image_ptr, f);
+            const int cap = __builtin_amdgcn_readlane(my_cap, f);
+            const u32x4 d = raw_descriptor(base + (unsigned long long)hkv * cap * image_row, (unsigned)(s.L * image_row));
+            s.lo = d.x;
+            s.hi = d.y;
+            s.bytes = d.z;
+            s.lt0 = s0 - fb;
+            s.lt1 = s1 - fb;
+            s.opens = s0 == fb;
+            return s;
+        };
+        auto open_rows = [&]() {
+            if constexpr (STREAM) {
+                T0 = whole ? 0 : max(run_begin - rgi * tiles_head, 0);
+                T1 = whole ? tiles_head : min(run_end - rgi * tiles_head, tiles_head);
+            }
+            r0 = rgi * WIDE_ROWS;
+            w0 = r0 + rw * WROWS;
 #pragma unroll
-            for (int i = 1; i < DP; ++i) request(i, lt0 + i * PAR);
-            lrot.finish(a, qreg, lim, f, hkv, w0, GQ, L, a.rq != nullptr && opens_fragment, tids & 15, (tids >> 4) & 3);
+            for (int rb = 0; rb < RB; ++rb) {
+                st.m[rb] = NEG_BIG;
+                st.l[rb] = 0.f;
+#pragma unroll
+                for (int c = 0; c < G::NOC; ++c) st.o[rb][c] = f32x4{0.f, 0.f, 0.f, 0.f};
+            }
+            st.fresh = true;
+            todo = __ballot(lane < a.F && max(T0, my_tb) < min(T1, my_te));
+        };
+        // The row group that comes behind the present one (STREAM): its number, or -1; below split_groups it is part of the run.
+        [[maybe_unused]] auto next_group = [&]() {
+            int group = whole ? rgi + a.wgs_per_head : rgi + 1;
+            if (whole && group < groups) return group;
+            if (whole) group = run_begin / tiles_head;
+            return max(run_begin, group * tiles_head) < run_end ? group : -1;
+        };
+        // the largest value over the wave (uniform)
+        auto wave_max = [&](int v) {
+            v = row_max16(v);
+            return max(max(__builtin_amdgcn_readlane(v, 0), __builtin_amdgcn_readlane(v, 16)),
+                       max(__builtin_amdgcn_readlane(v, 32), __builtin_amdgcn_readlane(v, 48)));
+        };
+        [[maybe_unused]] const unsigned q_base = lds_address(q_lds), cs_base = lds_address(cs_lds), loc_base = lds_address(lim_lds);
+        // (the lane as the compiler cannot see through it: what is derived from it -- rows, addresses of the queries -- is then
+        // formed where it is used instead of once in front of the loop over the segments, from where it would stay in registers across
+        // the tile loops, which have none to spare)
+        auto request_queries = [&](int f, const Rows& r) {
+            int ln = lane;
+            asm volatile("" : "+v"(ln));
+            WQ::request_queries(a, q_base, f, hkv, r.r0, GQ, wv, ln);
+        };
+        auto request_tables = [&](int f, const Rows& r) {
+            int ln = lane;
+            asm volatile("" : "+v"(ln));
+            WQ::request_tables(a, cs_base, loc_base, f, r.r0, r.ws_lo, r.nws, r.staged, wv, ln);
+        };
+        // The queries to rotate are the same for every fragment: they are requested here, before the workgroup's tile range
+        // and first fragment are worked out, and are on their way while that happens.  (A run without tiles has no rows: run_begin then
+        // lies behind the last row group.)
+        Rows rows = rows_of(rgi);
+        __builtin_amdgcn_s_waitcnt(0x0F70);   // vmcnt(0): the tables in the arguments, ahead of transfers that the compiler does not count
+        if (!PRE && (!STREAM || whole || run_begin < run_end)) request_queries(0, rows);
+        open_rows();
+        HW_MARK(10);
+        Segment seg, nxt;                                        // the open segment; the one behind it in the same rows (lt1 == 0: none)
+        int ss = 0, l = 0, lend = 0;                             // step slot and first tile of the current step; end of the segment's steps
+
+        // This wave's share of the PAR tiles of the next step into step slot `slot`.  A tile that does not exist is requested out of
+        // range: the same number of transfers, no memory traffic, zeros in LDS.
+        u32x4 view = {0, 0, 0, RAW_FLAGS};                       // of the segment that is requested, the open one or the one behind it
+        int rt = 0, rend = 0;                                    // the next step's first tile there, and the segment's end
+        auto request = [&](int slot) {
+#pragma unroll
+            for (int pp = 0; pp < PAR; ++pp) {
+                const unsigned tile_bytes = (unsigned)((rt + pp) * TILE * image_row);
+                wide_request<TPW, KEEP>(view, __builtin_amdgcn_readfirstlane(my_image + (slot * PAR + pp) * SLOT), rt + pp < rend ? tile_bytes : OOB_OFFSET, off);
+            }
+            rt += PAR;
+        };
+        auto turn_to = [&](const Segment& s) {
+            view.x = s.lo;
+            view.y = s.hi;
+            view.z = s.bytes;
+            rt = s.lt0;
+            rend = s.lt1;
+        };
+        // The first segment of the rows.  Its first step is requested here, the other look-ahead steps when its queries have arrived: a CU
+        // takes in about 16 B/clk, and the queries of a wave would wait behind the tiles that others have requested.
+        constexpr int ALL_ITS_OWN = 0x7fffffff;                  // lend until the segment's steps are counted
+        auto open_first = [&]() {
+            seg = segment_of(__builtin_ctzll(todo));
+            todo &= todo - 1;
+            ss = 0;
+            l = seg.lt0;
+            lend = ALL_ITS_OWN;
+            nxt = seg;
+            turn_to(seg);
+            request(0);
+        };
+        auto request_look_ahead = [&]() {
+            if (lend == ALL_ITS_OWN) {
+#pragma unroll
+                for (int i = 1; i < DP; ++i) request(i);
+            }
+        };
+        bool more = todo != 0;
+        if (more) {
+            const int f = __builtin_ctzll(todo);
+            if constexpr (PRE) request_queries(f, rows);
+            open_first();
+            request_tables(f, rows);
+            // the first step, queries, tables and locations have landed, for every wave
+            asm volatile("s_waitcnt vmcnt(0)\n\ts_barrier" ::: "memory");
         } else {
-        int limv = (r0 + tids / TPR < a.R) ? min(L, max(0, lm + 1)) : 0x7fffffff;   // by every thread, see paged_wide_kernel
-        asm volatile("" : "+v"(limv));
-        if (!PRE && staged) {
-            wrot.stage(cs_lds, tids, nws);
-            if (hw_first) HW_MARK(13);
-            // The barrier above has waited for every load of open_segment: the other look-ahead steps can be requested
-            // here, ahead of the rotation arithmetic, which waits for nothing from memory any more.  (An LDS-only barrier
-            // again: __syncthreads() would wait for the requests just issued.)
-#pragma unroll
-            for (int i = 1; i < DP; ++i) request(i, lt0 + i * PAR);
-            asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
-            if (hw_first) HW_MARK(14);
-            wrot.rotate(a, q_lds, cs_lds, f, hkv, r0, GQ, a.rq != nullptr && opens_fragment, tids, ws_lo);
-        } else if constexpr (PRE) {
-            qrot.finish(a, q_lds, f, hkv, r0, GQ, false, tids);
-        } else {
-            // too many (worker, token) pairs for the staged tables (GQA ratio below 4): every row loads its own table row,
-            // here and not ahead of time in open_segment, so that the registers of this path are not held across the tile
-            // loops of the common one
-            QueryRotation<DT, E, WIDE_ROWS, G::QSTR, false, NT> qslow;
-            qslow.load(a, f, hkv, r0, GQ, tids);
-            qslow.finish(a, q_lds, f, hkv, r0, GQ, a.rq != nullptr && opens_fragment, tids);
-            // (said once more where the compiler sees it: without it, it takes this path's loads for outstanding on the
-            // other path of the next segment and waits there, in the middle of the rotation, for "everything")
-            __builtin_amdgcn_s_waitcnt(0x0F70);   // vmcnt(0)
+            asm volatile("s_waitcnt vmcnt(0)" ::: "memory");      // (no transfer outlives the workgroup)
         }
-        if (tids % TPR == 0) lim_lds[tids / TPR] = limv;
-        if (hw_first) HW_MARK(12);
-        // q_lds and lim_lds become visible: a barrier for LDS only.  __syncthreads() would also wait for the stores of
-        // the rotated queries to be acknowledged by memory, which nobody here depends on.
-        asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
-        if (hw_first) HW_MARK(1);
+        HW_MARK(6);
+        bool hw_first = true;
 
+        // An opened segment: its queries, tables and locations lie in LDS, visible to all waves, its first steps are under way.
+        while (more) {
+            int tids = tid;        // (see request_queries)
+            asm volatile("" : "+v"(tids));
+            const bool write_rq = a.rq != nullptr && seg.opens;
+            u32x4 qreg[RB * G::KJ];                      // this wave's query operands and mask bounds
+            int lim[RB];
+            int most = 0;                                // the largest bound of the workgroup's rows (uniform)
+            request_look_ahead();
+            if constexpr (!PRE) {
+                if (rows.staged) WQ::template rotate<true>(a, q_lds, cs_lds, seg.f, hkv, r0, GQ, write_rq, tids, rows.ws_lo);
+                else WQ::template rotate<false>(a, q_lds, cs_lds, seg.f, hkv, r0, GQ, write_rq, tids, rows.ws_lo);
+                if (hw_first) HW_MARK(12);
+                lds_barrier();
+                if (hw_first) HW_MARK(1);
+            }
+            const u32x4 z = {0, 0, 0, 0};
 #pragma unroll
-        for (int rb = 0; rb < RB; ++rb) {
+            for (int rb = 0; rb < RB; ++rb) {
+                const int row = rw * WROWS + rb * 16 + (tids & 15);
+                const bool pad = r0 + row >= a.R;         // padding rows of the 16-row MFMA block hold zeros and "see everything"
 #pragma unroll
-            for (int j = 0; j < G::KJ; ++j)
-                qreg[rb * G::KJ + j] = *reinterpret_cast<const u32x4*>(q_lds + (rw * WROWS + rb * 16 + n) * G::QSTR + (4 * j + q) * 16);
-            lim[rb] = lim_lds[rw * WROWS + rb * 16 + n];
-        }
-        }
-        int maxlim = 0, minlim = 0x7fffffff;
+                for (int j = 0; j < G::KJ; ++j) {
+                    const u32x4 x = *reinterpret_cast<const u32x4*>(q_lds + kstage_offset<G>(row, 4 * j + ((tids >> 4) & 3)));
+                    qreg[rb * G::KJ + j] = pad ? z : x;
+                }
+                lim[rb] = pad ? 0x7fffffff : min(seg.L, max(0, lim_lds[row] + 1));
+            }
 #pragma unroll
-        for (int rb = 0; rb < RB; ++rb) {
-            const bool pad = w0 + rb * 16 + n >= a.R;
-            maxlim = max(maxlim, pad ? 0 : lim[rb]);
-            minlim = min(minlim, lim[rb]);
-        }
-        maxlim = __builtin_amdgcn_readfirstlane(row_max16(maxlim));
-        minlim = __builtin_amdgcn_readfirstlane(row_min16(minlim));
-        if (!LANES && (PRE || !staged)) {
+            for (int h = 0; h < WIDE_ROWS / 64; ++h) most = max(most, r0 + h * 64 + (tids & 63) < a.R ? lim_lds[h * 64 + (tids & 63)] + 1 : 0);
+            int maxlim = 0, minlim = 0x7fffffff;
 #pragma unroll
-            for (int i = 1; i < DP; ++i) request(i, lt0 + i * PAR);
-        }
+            for (int rb = 0; rb < RB; ++rb) {
+                const bool pad = w0 + rb * 16 + (tids & 15) >= a.R;
+                maxlim = max(maxlim, pad ? 0 : lim[rb]);
+                minlim = min(minlim, lim[rb]);
+            }
+            maxlim = __builtin_amdgcn_readfirstlane(row_max16(maxlim));
+            minlim = __builtin_amdgcn_readfirstlane(row_min16(minlim));
+            // tiles that no row of the workgroup sees are not taken in
+            seg.lt1 = min(seg.lt1, (min(seg.L, wave_max(most)) + TILE - 1) / TILE);
+            rend = seg.lt1;
+            l = seg.lt0;
 
-        {
-            // A step = PAR tiles behind one barrier, one for each of the waves that share their rows.  Two loops, one
-            // instantiation of the tile arithmetic in each: first the steps in which every row of this wave sees its tile
-            // completely, then the rest.  With both instantiations in one loop body the compiler merges their accumulators
-            // through copies (48 v_mov_b64 per tile).  The waves of a workgroup may change loops at different steps; each
-            // still passes one barrier per step.
-            int ss = 0;                                   // step slot of the current step
-            int l = lt0;                                  // its first tile
-            auto arrive = [&]() {
-                // this wave's transfers of the step have landed (the DP - 1 steps requested since may stay in flight: loads
-                // complete in order), then every wave's.  Behind the barrier the slots of the step before are free:
-                // request step + DP into them.
-                asm volatile("s_waitcnt vmcnt(%0)\n\ts_barrier" ::"n"((DP - 1) * TPS) : "memory");
-                request(ss == 0 ? NSTEP - 1 : ss - 1, l + DP * PAR);
-                if (hw_first) { HW_MARK(2); hw_first = false; }
+            // The first step is complete, and every wave holds its operands and bounds: what the next opening needs can follow into the
+            // memory they came from -- requested ahead of the next step's tiles, so that the wait of the segment's second step covers
+            // it.
+            asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"((DP - 1) * TPS) : "memory");
+            if (hw_first) { HW_MARK(2); hw_first = false; }
+            bool behind = todo != 0;
+            if (behind) {                                // the segment behind this one in the same rows
+                nxt = segment_of(__builtin_ctzll(todo));
+                request_queries(nxt.f, rows);
+                request_tables(nxt.f, rows);
+            } else {
+                nxt.lt1 = 0;
+                if constexpr (STREAM) {
+                    const int group = next_group();
+                    behind = group >= 0;
+                    if (behind) {
+                        const bool wh = group >= split_groups;
+                        rows = rows_of(group);
+                        const int t0 = wh ? 0 : max(run_begin - group * tiles_head, 0), t1 = wh ? tiles_head : min(run_end - group * tiles_head, tiles_head);
+                        const int f = __builtin_ctzll(__ballot(lane < a.F && max(t0, my_tb) < min(t1, my_te)));
+                        request_queries(f, rows);
+                        request_tables(f, rows);
+                    }
+                }
+            }
+            // With something behind it a segment has at least the DP steps that were requested: the first steps of the next one are
+            // requested behind its own.
+            lend = l + max(behind ? DP : 1, (max(seg.lt1 - l, 0) + PAR - 1) / PAR) * PAR;
+            // The two loops over steps of the other form (see there), but that a step is waited for behind the one before.  Behind the
+            // segment's own steps the next one's are requested, and the last wait is for the first of them.
+            auto request_next = [&]() {
+                if (l + DP * PAR == lend) turn_to(nxt);
+                request(ss == 0 ? NSTEP - 1 : ss - 1);
             };
-            const int lfast = maxlim > 0 ? min(lt1, minlim / TILE) : lt0;
+            auto arrive = [&]() {
+                ss = ss + 1 == NSTEP ? 0 : ss + 1;
+                asm volatile("s_waitcnt vmcnt(%0)\n\ts_barrier" ::"n"((DP - 1) * TPS) : "memory");
+            };
+            const int lfast = maxlim > 0 ? min(seg.lt1, minlim / TILE) : seg.lt0;
 #pragma unroll 1
             for (; l + par < lfast; l += PAR) {
-                arrive();
+                request_next();
                 const char* slot = ring + (ss * PAR + par) * SLOT;
                 compute_tile<DT, E, EV, RB, false, true, false, true>(TileRegs<DT, E, EV>(), q_lds, qreg, lim, st, (l + par) * TILE, n, q, a.sc, slot, slot + KBYTES, voff);
-                ss = ss + 1 == NSTEP ? 0 : ss + 1;
+                arrive();
             }
 #pragma unroll 1
-            for (; l < lt1; l += PAR) {
-                arrive();
-                if (l + par < lt1 && (l + par) * TILE < maxlim) {
+            for (; l < lend; l += PAR) {
+                request_next();
+                if (l + par < seg.lt1 && (l + par) * TILE < maxlim) {
                     const char* slot = ring + (ss * PAR + par) * SLOT;
                     compute_tile<DT, E, EV, RB, true, true, false, true>(TileRegs<DT, E, EV>(), q_lds, qreg, lim, st, (l + par) * TILE, n, q, a.sc, slot, slot + KBYTES, voff);
                 }
-                ss = ss + 1 == NSTEP ? 0 : ss + 1;
+                arrive();
             }
-        }
-        // the requests behind the last tile (they fetched nothing) must have landed before the ring is used again
-        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-        more = todo != 0;
-        if (more) {
-            __syncthreads();   // every wave is done with the ring
-            open_segment(false);
-        } else if constexpr (STREAM) {
-            store_rows();
-            if (!whole) {
-                write_row_table();
-                ++rgi;
-            } else if (rgi + a.wgs_per_head < groups) {
-                rgi += a.wgs_per_head;
+            more = todo != 0;
+            if (more) {
+                seg = nxt;
+                todo &= todo - 1;
             } else {
-                whole = false;
-                rgi = run_begin / tiles_head;
-            }
-            if (whole || max(run_begin, rgi * tiles_head) < run_end) {          // the next row group
-                __syncthreads();                       // every wave is done with the ring
-                open_rows();
-                open_segment(staged);
-                more = true;
+                // the requests behind the last tile (they fetched nothing) and what the next rows need have landed, before the ring
+                // is used for the results
+                asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+                if constexpr (STREAM) {
+                    store_rows();
+                    if (!whole) write_row_table();
+                    const int group = next_group();
+                    if (group >= 0) {
+                        rgi = group;
+                        whole = group >= split_groups;
+                        __syncthreads();                       // every wave is done with the ring
+                        open_rows();
+                        open_first();
+                        more = true;
+                    }
+                }
             }
         }
+    } else {
+        WRot wrot;
+        int ws_lo, nws;                             // (worker, token) pairs the rows of this workgroup belong to
+        bool staged;                                // their tables go through LDS; uniform over the workgroup
+        // The queries to rotate are the same for every fragment: they are requested here, before the workgroup's tile range
+        // and first fragment are worked out, and are on their way while that happens.
+        auto open_rows = [&]() {
+            if constexpr (STREAM) {
+                T0 = whole ? 0 : max(run_begin - rgi * tiles_head, 0);
+                T1 = whole ? tiles_head : min(run_end - rgi * tiles_head, tiles_head);
+            }
+            r0 = rgi * WIDE_ROWS;
+            w0 = r0 + rw * WROWS;
+            ws_lo = fast_div(r0, a.magic_gq);
+            nws = fast_div(min(r0 + WIDE_ROWS, a.R) - 1, a.magic_gq) - ws_lo + 1;
+            staged = !LANES && nws <= WRot::CSMAX;
+            int tids = tid;
+            if constexpr (STREAM) asm volatile("" : "+v"(tids));      // (see open_segment)
+            if (staged) wrot.load_queries(a, hkv, r0, GQ, tids);
+#pragma unroll
+            for (int rb = 0; rb < RB; ++rb) {
+                st.m[rb] = NEG_BIG;
+                st.l[rb] = 0.f;
+#pragma unroll
+                for (int c = 0; c < G::NOC; ++c) st.o[rb][c] = f32x4{0.f, 0.f, 0.f, 0.f};
+            }
+            st.fresh = true;
+            todo = __ballot(lane < a.F && max(T0, my_tb) < min(T1, my_te));
+        };
+        open_rows();
+
+        HW_MARK(10);
+        int f = 0, L = 0, lt0 = 0, lt1 = 0;
+        bool opens_fragment = false;
+        u32x4 view = {0, 0, 0, 0};                               // this wave's image of the current fragment (K or V slice)
+        [[maybe_unused]] LaneRotation<DT, E, RB, PRE> lrot;
+        int lm = 0;
+
+        // this wave's share of the PAR tiles of the step that starts at tile `lt` (fragment-local) into step slot `ss`; a tile
+        // that does not exist is requested out of range: the same number of transfers, no memory traffic, zeros in LDS
+        auto request = [&](int ss, int lt) {
+#pragma unroll
+            for (int pp = 0; pp < PAR; ++pp) {
+                const unsigned tile_bytes = (unsigned)((lt + pp) * TILE * image_row);
+                wide_request<TPW, KEEP>(view, __builtin_amdgcn_readfirstlane(my_image + (ss * PAR + pp) * SLOT), lt + pp < lt1 ? tile_bytes : OOB_OFFSET, off);
+            }
+        };
+
+        auto open_segment = [&](bool queries_requested) {
+            f = __builtin_ctzll(todo);
+            todo &= todo - 1;
+            const int fb = __builtin_amdgcn_readlane(my_tb, f);
+            const int fe = __builtin_amdgcn_readlane(my_te, f);
+            const int s0 = max(T0, fb), s1 = min(T1, fe);
+            L = __builtin_amdgcn_readlane(my_len, f);
+            const unsigned long long base = ((unsigned long long)(unsigned)__builtin_amdgcn_readlane((int)(my_image_ptr >> 32), f) << 32) |
+                                            (unsigned)__builtin_amdgcn_readlane((int)my_image_ptr, f);
+            const int cap = __builtin_amdgcn_readlane(my_cap, f);
+            view = raw_descriptor(base + (unsigned long long)hkv * cap * image_row, (unsigned)(L * image_row));
+            lt0 = s0 - fb;
+            lt1 = s1 - fb;
+            opens_fragment = s0 == fb;
+            // The first step is requested before the queries: the compiler's wait for the query loads then also waits for it
+            // (loads complete in order), which costs nothing, its tiles being needed first anyway.  The other look-ahead
+            // steps follow when the queries have arrived, so that the rotation does not wait for them as well.
+            request(0, lt0);
+            HW_MARK(11);
+            // (the thread index as the compiler cannot see through it: what is derived from it -- rows, addresses of the
+            // queries -- is then formed per segment instead of once in front of the loop over the segments, from where it
+            // would stay in registers across the tile loops, which have none to spare)
+            int tids = tid;
+            asm volatile("" : "+v"(tids));
+            if constexpr (LANES) {
+                lrot.load(a, f, hkv, w0, GQ, tids & 15, (tids >> 4) & 3);
+                return;
+            } else if (staged) {
+                if (!queries_requested) wrot.load_queries(a, hkv, r0, GQ, tids);
+                wrot.load_tables(a, f, tids, ws_lo, nws);
+            }
+            // the bound of row tid / TPR (TPR threads per row, all load: keeps the load unconditional)
+            lm = a.loc[(size_t)f * a.W * a.S + fast_div(min(r0 + tids / TPR, a.R - 1), a.magic_gq)];
+        };
+        bool more = todo != 0;
+        if (more) open_segment(staged);
+        HW_MARK(6);
+        bool hw_first = true;
+
+        while (more) {
+            if constexpr (!LANES) __syncthreads();   // previous segment's readers are done with q_lds / lim_lds
+            if (hw_first) HW_MARK(7);
+            int tids = tid;        // (see open_segment)
+            asm volatile("" : "+v"(tids));
+            // Every load of open_segment is waited for here, in a form the compiler sees: it waits for a load where its result
+            // is first used and counts only the loads it knows of, so a wait that it places further down -- for the bound
+            // below, the last load of open_segment -- would also wait for the look-ahead steps requested in between.
+            // (Nothing is lost: the queries are needed now, and the first step was requested before them.)
+            __builtin_amdgcn_s_waitcnt(0x0F70);   // vmcnt(0)
+            u32x4 qreg[RB * G::KJ];                      // this wave's query operands and mask bounds
+            int lim[RB];
+            if constexpr (LANES) {
+#pragma unroll
+                for (int i = 1; i < DP; ++i) request(i, lt0 + i * PAR);
+                lrot.finish(a, qreg, lim, f, hkv, w0, GQ, L, a.rq != nullptr && opens_fragment, tids & 15, (tids >> 4) & 3);
+            } else {
+            int limv = (r0 + tids / TPR < a.R) ? min(L, max(0, lm + 1)) : 0x7fffffff;   // by every thread, see paged_wide_kernel
+            asm volatile("" : "+v"(limv));
+            if (staged) {
+                wrot.stage(cs_lds, tids, nws);
+                if (hw_first) HW_MARK(13);
+                // The barrier above has waited for every load of open_segment: the other look-ahead steps can be requested
+                // here, ahead of the rotation arithmetic, which waits for nothing from memory any more.  (An LDS-only barrier
+                // again: __syncthreads() would wait for the requests just issued.)
+#pragma unroll
+                for (int i = 1; i < DP; ++i) request(i, lt0 + i * PAR);
+                asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+                if (hw_first) HW_MARK(14);
+                wrot.rotate(a, q_lds, cs_lds, f, hkv, r0, GQ, a.rq != nullptr && opens_fragment, tids, ws_lo);
+            } else {
+                // too many (worker, token) pairs for the staged tables (GQA ratio below 4): every row loads its own table row,
+                // here and not ahead of time in open_segment, so that the registers of this path are not held across the tile
+                // loops of the common one
+                QueryRotation<DT, E, WIDE_ROWS, G::QSTR, false, NT> qslow;
+                qslow.load(a, f, hkv, r0, GQ, tids);
+                qslow.finish(a, q_lds, f, hkv, r0, GQ, a.rq != nullptr && opens_fragment, tids);
+                // (said once more where the compiler sees it: without it, it takes this path's loads for outstanding on the
+                // other path of the next segment and waits there, in the middle of the rotation, for "everything")
+                __builtin_amdgcn_s_waitcnt(0x0F70);   // vmcnt(0)
+            }
+            if (tids % TPR == 0) lim_lds[tids / TPR] = limv;
+            if (hw_first) HW_MARK(12);
+            // q_lds and lim_lds become visible: a barrier for LDS only.  __syncthreads() would also wait for the stores of
+            // the rotated queries to be acknowledged by memory, which nobody here depends on.
+            asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+            if (hw_first) HW_MARK(1);
+
+#pragma unroll
+            for (int rb = 0; rb < RB; ++rb) {
+#pragma unroll
+                for (int j = 0; j < G::KJ; ++j)
+                    qreg[rb * G::KJ + j] = *reinterpret_cast<const u32x4*>(q_lds + (rw * WROWS + rb * 16 + n) * G::QSTR + (4 * j + q) * 16);
+                lim[rb] = lim_lds[rw * WROWS + rb * 16 + n];
+            }
+            }
+            int maxlim = 0, minlim = 0x7fffffff;
+#pragma unroll
+            for (int rb = 0; rb < RB; ++rb) {
+                const bool pad = w0 + rb * 16 + n >= a.R;
+                maxlim = max(maxlim, pad ? 0 : lim[rb]);
+                minlim = min(minlim, lim[rb]);
+            }
+            maxlim = __builtin_amdgcn_readfirstlane(row_max16(maxlim));
+            minlim = __builtin_amdgcn_readfirstlane(row_min16(minlim));
+            if (!LANES && !staged) {
+#pragma unroll
+                for (int i = 1; i < DP; ++i) request(i, lt0 + i * PAR);
+            }
+
+            {
+                // A step = PAR tiles behind one barrier, one for each of the waves that share their rows.  Two loops, one
+                // instantiation of the tile arithmetic in each: first the steps in which every row of this wave sees its tile
+                // completely, then the rest.  With both instantiations in one loop body the compiler merges their accumulators
+                // through copies (48 v_mov_b64 per tile).  The waves of a workgroup may change loops at different steps; each
+                // still passes one barrier per step.
+                int ss = 0;                                   // step slot of the current step
+                int l = lt0;                                  // its first tile
+                auto arrive = [&]() {
+                    // this wave's transfers of the step have landed (the DP - 1 steps requested since may stay in flight: loads
+                    // complete in order), then every wave's.  Behind the barrier the slots of the step before are free:
+                    // request step + DP into them.
+                    asm volatile("s_waitcnt vmcnt(%0)\n\ts_barrier" ::"n"((DP - 1) * TPS) : "memory");
+                    request(ss == 0 ? NSTEP - 1 : ss - 1, l + DP * PAR);
+                    if (hw_first) { HW_MARK(2); hw_first = false; }
+                };
+                const int lfast = maxlim > 0 ? min(lt1, minlim / TILE) : lt0;
+#pragma unroll 1
+                for (; l + par < lfast; l += PAR) {
+                    arrive();
+                    const char* slot = ring + (ss * PAR + par) * SLOT;
+                    compute_tile<DT, E, EV, RB, false, true, false, true>(TileRegs<DT, E, EV>(), q_lds, qreg, lim, st, (l + par) * TILE, n, q, a.sc, slot, slot + KBYTES, voff);
+                    ss = ss + 1 == NSTEP ? 0 : ss + 1;
+                }
+#pragma unroll 1
+                for (; l < lt1; l += PAR) {
+                    arrive();
+                    if (l + par < lt1 && (l + par) * TILE < maxlim) {
+                        const char* slot = ring + (ss * PAR + par) * SLOT;
+                        compute_tile<DT, E, EV, RB, true, true, false, true>(TileRegs<DT, E, EV>(), q_lds, qreg, lim, st, (l + par) * TILE, n, q, a.sc, slot, slot + KBYTES, voff);
+                    }
+                    ss = ss + 1 == NSTEP ? 0 : ss + 1;
+                }
+            }
+            // the requests behind the last tile (they fetched nothing) must have landed before the ring is used again
+            asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+            more = todo != 0;
+            if (more) {
+                __syncthreads();   // every wave is done with the ring
+                open_segment(false);
+            } else if constexpr (STREAM) {
+                store_rows();
+                if (!whole) {
+                    write_row_table();
+                    ++rgi;
+                } else if (rgi + a.wgs_per_head < groups) {
+                    rgi += a.wgs_per_head;
+                } else {
+                    whole = false;
+                    rgi = run_begin / tiles_head;
+                }
+                if (whole || max(run_begin, rgi * tiles_head) < run_end) {          // the next row group
+                    __syncthreads();                       // every wave is done with the ring
+                    open_rows();
+                    open_segment(staged);
+                    more = true;
+                }
+            }
+        }
+
     }
 
     if constexpr (!STREAM) store_rows();
@@ -635,12 +1021,12 @@ __global__ __launch_bounds__(NW * 64, 1) void attention_wide_kernel(const Kernel
             }
         }
         while (empty != 0 && (!STREAM || !whole || rgi < groups)) {
-            f = __builtin_ctzll(empty);
+            const int f = __builtin_ctzll(empty);
             empty &= empty - 1;
             __syncthreads();
             QueryRotation<DT, E, WIDE_ROWS, G::QSTR, PRE, NT> qempty;
             qempty.load(a, f, hkv, rgi * WIDE_ROWS, GQ, tid);
-            qempty.finish(a, LANES ? nullptr : q_lds, f, hkv, rgi * WIDE_ROWS, GQ, true, tid);
+            qempty.finish(a, LANES || AHEAD ? nullptr : q_lds, f, hkv, rgi * WIDE_ROWS, GQ, true, tid);
             if (STREAM && empty == 0) {
                 empty = all_empty;
                 if (whole) {
@@ -653,16 +1039,6 @@ __global__ __launch_bounds__(NW * 64, 1) void attention_wide_kernel(const Kernel
         }
     }
 }
-
-// One 1 KB global->LDS transfer with a 64-bit address per lane (the paged cache has no contiguous slice a buffer
-// descriptor could bound): lane l brings 16 bytes from `src` to LDS byte `lds` + 16 l, non-temporal.  Issued from inline
-// assembly and waited for by hand, like lds_transfer.
-#pragma clang diagnostic push
-#pragma clang diagnostic ignored "-Winline-asm"
-__device__ __forceinline__ void lds_transfer_flat(unsigned lds, unsigned long long src) {
-    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off nt" ::"s"(lds), "v"(src) : "m0", "memory");
-}
-#pragma clang diagnostic pop
 
 // The split of a packed-query launch, decided on the device (query lengths and KV lengths are device tensors,
 // src/binding.cu:144-181) -- by every workgroup for itself, in its prologue: the inputs are a few hundred bytes that
@@ -1128,7 +1504,7 @@ __global__ __launch_bounds__(NW * 64, 1) void paged_wide_kernel(const PagedHeade
                         for (int j = 0; j < NP; ++j)
 #pragma unroll
                             for (int im = 0; im < NI; ++im)
-                                lds_transfer_flat(__builtin_amdgcn_readfirstlane(my_image[im] + (step_slot * PAR + pp) * SLOT + j * 1024),
+                                lds_transfer_flat<false>(__builtin_amdgcn_readfirstlane(my_image[im] + (step_slot * PAR + pp) * SLOT + j * 1024),
                                                   src[(pp * NP + j) * NI + im]);
                 };
 
