@@ -423,13 +423,25 @@ bool deal_by_seen(const hw_problem* p, const CallPlan& cp, const WholePlan& wp) 
     return (2 * chunk > T && wp.split > 1) || (3 * chunk > T && 4 * wp.split > wp.wgs);
 }
 
+// One worker that brings the newest S tokens of the last fragment.
+static bool causal_chunk(const hw_problem* p) {
+    int last = p->F - 1;
+    while (last > 0 && p->len[last] == 0) --last;
+    return p->W == 1 && p->len[last] >= p->S;
+}
+
 // The remainder in runs: the smallest share (tiles, with openings) at which the workgroups, taking one after the other what fits,
 // use up the row groups, found by bisection.  Dealt by the tiles seen, those behind them go with the piece in front, so that no
 // workgroup opens a row group for tiles that none of its rows sees.  (Should the locations say otherwise, the launch is merely less
-// even.)  Unseen tiles cost as much here as the others: priced at 0.15, 0.3, 0.5 and 0.8, with the workgroups' shares unequal to
-// match, the launches took as long or longer.
+// even.)
+// At head dimension 128 the kernel does not take unseen tiles in.  Then a causal chunk is dealt by the tiles seen whatever its share,
+// and the workgroups with the later row groups, which see most, get less of the remainder or none of it.  (Taking in fewer tiles alone
+// gave nothing, the last row group's workgroup having as many as before; nor did unequal shares while unseen tiles cost as much as
+// others.)  us a layer: 938 tokens behind 577 at 40/8 heads 51 -> 44, 1088 behind 527 at 32/8 48 -> 40, 1112 behind 62 46 -> 41.5, 1024
+// behind 4096 117 -> 115; 70 calls of four head layouts 0.96 to 1.20 times as fast, 1.068 in the mean, two of them below 0.98.  The
+// costs of a piece and a fragment are from the same calls: at 8 and 2 tiles 1.046 in the mean, at 5 and 1 1.027, 12 and 2 1.063, 16 and 4
+// 1.065, 24 and 4 1.069; of several workers, dealt by all tiles, 1.015 at 8 and 2, 1.017 at 12 and 2, 1.016 at 24 and 4.
 void whole_deal(const hw_problem* p, const CallPlan& cp, WholePlan* wp) {
-    constexpr double kPieceCost = 8.0, kOpenCost = 2.0;      // in tiles: a piece's prologue and epilogue; a row group's fragments
     const hw_plan& plan = cp.plan[0];
     const int T = plan.tiles_per_head, wgs = wp->wgs, split = wp->split;
     StreamPlan& sp = wp->runs;
@@ -439,8 +451,11 @@ void whole_deal(const hw_problem* p, const CallPlan& cp, WholePlan* wp) {
         last = f;
         ++nf;
     }
-    const double tile = 1.0 + kOpenCost * nf / T;            // a row group's openings spread over its tiles
-    const bool by_seen = deal_by_seen(p, cp, *wp);
+    const bool trimmed = p->E == 128;                        // the kernel does not take unseen tiles in
+    const bool by_seen = trimmed ? causal_chunk(p) : deal_by_seen(p, cp, *wp);
+    // in tiles: a piece's prologue and epilogue; a row group's fragments, spread over its tiles
+    const double kPieceCost = !trimmed ? 8.0 : by_seen ? 20.0 : 12.0, kOpenCost = trimmed && by_seen ? 4.0 : 2.0;
+    const double tile = 1.0 + kOpenCost * nf / T;
     const int gq = p->Hq / p->Hkv;
     auto seen_tiles = [&](int rg) {                          // up to the token of the row group's last row
         if (!by_seen) return T;
@@ -448,31 +463,38 @@ void whole_deal(const hw_problem* p, const CallPlan& cp, WholePlan* wp) {
         return plan.tile_begin[last] + (p->len[last] - p->S + token + hw::TILE) / hw::TILE;
     };
     const double per_tile = 1.0 / tile;
+    // what workgroup g has in hand with the row groups that are its alone, above workgroup 0 (later row groups see more)
+    const int own = wp->whole / wgs;
+    auto ahead = [&](int g) {
+        int more = 0;
+        for (int i = 0; i < (trimmed ? own : 0); ++i) more += seen_tiles(split + i * wgs + g) - seen_tiles(split + i * wgs);
+        return more * tile;
+    };
     auto deal = [&](double share) {                          // false if something is left
         int rg = 0, t = 0, seen = seen_tiles(0);
         for (int g = 0; g < wgs; ++g) {
             sp.wg_tile_begin[g] = rg * T + t;
-            for (double room = share; rg < split;) {
+            for (double room = share - ahead(g); rg < split;) {
                 const int take = std::min((int)((room - kPieceCost) * per_tile), seen - t);
                 if (take < std::min(kMinPiece, seen - t)) break;
                 room -= kPieceCost + take * tile;
                 t += take;
                 if (t < seen) break;
-                room -= T - seen;
+                if (!trimmed) room -= T - seen;
                 t = 0;
-                seen = seen_tiles(++rg);
+                if (++rg < split) seen = seen_tiles(rg);
             }
         }
         return rg == split;
     };
-    // Between an equal part of the tiles seen and that of all tiles with what a workgroup opens and leaves at most besides.
+    // Between an equal part of the tiles seen and that of all with what a workgroup opens and leaves at most besides.
     double low = 0.0, unseen = 0.0;
     for (int rg = 0; rg < split; ++rg) {
         low += kPieceCost + seen_tiles(rg) * tile;
-        unseen += T - seen_tiles(rg);
+        unseen += trimmed ? 0 : T - seen_tiles(rg);
     }
     low /= wgs;
-    double high = low + unseen / wgs + 2.0 * kPieceCost + (kMinPiece + 1) * tile;
+    double high = low + unseen / wgs + ahead(wgs - 1) + 2.0 * kPieceCost + (kMinPiece + 1) * tile;
     while (!deal(high)) high *= 2.0;
     while (high - low > 0.25) {
         const double mid = 0.5 * (low + high);
