@@ -184,8 +184,10 @@ int run(const hw_problem* p, void* stream_, int fused, int stages = HW_STAGE_ATT
     ma.wgs_per_head = cp.slots;
     ma.xcd_local = (cp.groups == 1 && plan0.workgroups % 8 == 0 && p->Hkv % 8 == 0) ? 1 : 0;
     ma.row_tab = nullptr;
-    ma.pslots = 0;
+    ma.pslots = ma.slot_rows = ma.guess = 0;
+    ma.magic_rows = 0;
     if (stream_runs) {
+        ma.slot_rows = hw::PLAN_SLOT_ROWS;
         ma.wgs_per_head = sp.max_pieces;
         ma.xcd_local = ((stream_wgs * p->Hkv) % 8 == 0 && p->Hkv % 8 == 0) ? 1 : 0;
         ma.row_tab = reinterpret_cast<const int*>(part_ml + (size_t)p->Hkv * part_rows * 2);
@@ -237,7 +239,9 @@ int paged_run(const hw_paged_problem* p, void* stream_, int stages) {
     ph.nitems = plan.row_groups;
     ph.nrg = varlen ? 1 : plan.row_groups / p->W;
     ph.nwg = plan.workgroups;
-    ph.flags = ((plan.workgroups % 8 == 0) ? hw::PH_XCD_REMAP : 0) | (planned ? hw::PH_PLANNED : 0) | (paged_keep_in_l2(p, plan) ? hw::PH_KEEP : 0);
+    // (with the stages on their own, and in a workspace sized for hw_paged_plan only, the partials are laid out by it)
+    const bool shared = stages == (HW_STAGE_ATTENTION | HW_STAGE_MERGE) && paged_shared(p, plan) && p->workspace_bytes >= paged_call_bytes(p, plan);
+    ph.flags = ((plan.workgroups % 8 == 0) ? hw::PH_XCD_REMAP : 0) | (shared ? hw::PH_SHARED : 0) | (planned ? hw::PH_PLANNED : 0) | (paged_keep_in_l2(p, plan) ? hw::PH_KEEP : 0);
     ph.sc = (float)((double)p->scale * 1.4426950408889634074);
     ph.magic_gq = magic(p->Hq / p->Hkv);
     ph.magic_ls = magic(ph.LS);
@@ -263,8 +267,11 @@ int paged_run(const hw_paged_problem* p, void* stream_, int stages) {
     // a variable-length launch may leave row groups of the grid unused, and with them parts of an XCD's share
     // (a launch planned on the device keeps every slot of a kv head on the head's XCD whatever the slots do)
     ma.xcd_local = ((!varlen || planned) && plan.workgroups % 8 == 0 && p->Hkv % 8 == 0) ? 1 : 0;
-    ma.row_tab = planned ? row_tab : nullptr;
-    ma.pslots = planned ? plan.row_groups : 0;
+    ma.row_tab = planned || shared ? row_tab : nullptr;
+    ma.pslots = planned ? plan.row_groups : shared ? plan.row_groups * plan.splits : 0;
+    ma.slot_rows = planned ? hw::PLAN_SLOT_ROWS : shared ? plan.rows / p->W : 0;
+    ma.guess = shared ? plan.splits : 0;
+    ma.magic_rows = magic(shared ? ma.slot_rows : 1);
     if (planned) ma.wgs_per_head = 8;       // a row's slots are device data: the merge shape that suits a handful of them
     e = hw::launch_merge(ma, p->dtype, p->Ev, stream);
     return (int)e;
@@ -564,7 +571,7 @@ int hw_paged_workspace_bytes(const hw_paged_problem* p, size_t* bytes) {
     hw_paged_plan plan;
     st = hw_paged_plan_debug(p, cus, &plan);
     if (st != HW_OK) return st;
-    *bytes = plan.workspace_bytes;
+    *bytes = paged_call_bytes(p, plan);
     return HW_OK;
 }
 

@@ -143,6 +143,17 @@ __device__ __forceinline__ int row_min16(int v) {
     return min(v, row_dpp<0x140>(v));
 }
 
+// inclusive sum over the wave's lanes
+__device__ __forceinline__ int wave_scan_inclusive(int v) {
+    v += __builtin_amdgcn_update_dpp(0, v, 0x111, 0xf, 0xf, false);    // row_shr:1
+    v += __builtin_amdgcn_update_dpp(0, v, 0x112, 0xf, 0xf, false);    // row_shr:2
+    v += __builtin_amdgcn_update_dpp(0, v, 0x114, 0xf, 0xf, false);    // row_shr:4
+    v += __builtin_amdgcn_update_dpp(0, v, 0x118, 0xf, 0xf, false);    // row_shr:8: inclusive within rows of 16 lanes
+    v += __builtin_amdgcn_update_dpp(0, v, 0x142, 0xa, 0xf, false);    // row_bcast:15 into rows 1 and 3
+    v += __builtin_amdgcn_update_dpp(0, v, 0x143, 0xc, 0xf, false);    // row_bcast:31 into rows 2 and 3
+    return v;
+}
+
 // token (relative to the tile start) held in reduction slot `idx` (0..7) of quarter-wave `q`:
 // slots 0..3 come from the first 16-token S^T block, 4..7 from the second (accumulator rows 4q..4q+3).
 __device__ __forceinline__ int slot_token(int q, int idx) { return ((idx >> 2) << 4) + (q << 2) + (idx & 3); }

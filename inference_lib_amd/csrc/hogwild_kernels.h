@@ -72,11 +72,13 @@ struct MergeArgs {
     int W, Hq, Hkv, S, R, wgs_per_head;
     int rows;           // rows 0 .. rows - 1 of every kv head are merged
     int xcd_local;      // kv head h was computed on XCD h / (Hkv/8): merge it there
-    // Partials laid out by workgroup slot instead of by row (KH_STREAM, and the paged launch that is planned on the device,
-    // see PagedHeader): row_tab[kv head][r] = {first slot | slots << 16, row within the slot}, a slot holds PLAN_SLOT_ROWS rows, pslots
+    // Partials laid out by workgroup slot instead of by row (KH_STREAM, and the paged launches that are dealt on the device,
+    // see PagedHeader): row_tab[kv head][r] = {first slot | slots << 16, row within the slot}, a slot holds slot_rows rows, pslots
     // slots per kv head; wgs_per_head then only bounds the slots of a row (for the choice of the merge kernel's shape).
     const int* row_tab;
-    int pslots;
+    int pslots, slot_rows;
+    int guess;          // > 0: slots of a row where every slot_rows rows have the same number, one behind the other; requested ahead of the table
+    unsigned magic_rows;   // ceil(2^32 / slot_rows), for guess
 };
 
 hipError_t launch_attention(const KernelArgs& ka, int dtype, int E, int rb, int variant, hipStream_t stream);
@@ -121,6 +123,10 @@ constexpr int PH_XCD_REMAP = 1;    // consecutive logical workgroup ids share an
 // merge kernel a table per kv head of where each row's partial sums lie (MergeArgs::row_tab).
 constexpr int PH_KEEP = 4;         // K/V tiles stay in the L2 for the other row groups of a sequence (read by launch_paged_attention only)
 constexpr int PH_PLANNED = 2;
+// One row group per sequence (the fixed-length operator): the nitems * nsplit workgroups of a kv head are shared out by the
+// sequences' visible tiles instead of nsplit to each (paged_share).  Partial sums by workgroup slot, LS * (Hq / Hkv) rows each, the
+// merge's row table right behind part_ml.
+constexpr int PH_SHARED = 8;
 
 struct CopyBlocksArgs {
     const void* key_states;    // [B, Hkv, S_new, E]   (element strides below, innermost contiguous)

@@ -345,33 +345,55 @@ __global__ __launch_bounds__(256) void merge_kernel(const MergeArgs a) {
     size_t mstride = (size_t)a.R * 2;
     const float* po = a.part_o + ((size_t)hkv * ns * a.R + r) * EV + e4 * 4;
     size_t ostride = (size_t)a.R * EV;
-    if (a.row_tab != nullptr) {     // partials by workgroup slot: this row's are in slots first .. first + ns - 1, at row `rl` of each
-        // (clamped: the table is device data, and a malformed prefix array of query lengths leaves rows that no entry
-        // was written for)
-        const int* tab = a.row_tab + ((size_t)hkv * a.R + r) * 2;
-        const int x = tab[0];
-        const int rl = min(max(tab[1], 0), PLAN_SLOT_ROWS - 1);
-        ns = min(max(x >> 16, 0), a.pslots);
-        const int first = min(x & 0xffff, a.pslots - ns);
-        const size_t base = ((size_t)hkv * a.pslots + first) * PLAN_SLOT_ROWS + rl;
-        ml = a.part_ml + base * 2;
-        mstride = (size_t)PLAN_SLOT_ROWS * 2;
-        po = a.part_o + base * EV + e4 * 4;
-        ostride = (size_t)PLAN_SLOT_ROWS * EV;
-    }
-
-    float m_run = NEG_BIG, l_run = 0.f;
-    f32x4 acc = {0.f, 0.f, 0.f, 0.f};
-    for (int s0 = pgl; s0 < ns; s0 += UN * GPR) {
-        f32x4 o[UN];
-        f32x2 mlv[UN];
+    f32x4 o[UN];
+    f32x2 mlv[UN];
+    auto fetch = [&](int s0) {
 #pragma unroll
         for (int u = 0; u < UN; ++u) {
             const int s = s0 + u * GPR;
             const int sc = s < ns ? s : pgl;                // clamp: the loads stay unconditional
             o[u] = *reinterpret_cast<const f32x4*>(po + (size_t)sc * ostride);
             mlv[u] = *reinterpret_cast<const f32x2*>(ml + (size_t)sc * mstride);
-            if (s >= ns) mlv[u] = f32x2{NEG_BIG, 0.f};
+        }
+    };
+    bool fetched = false;
+    if (a.row_tab != nullptr) {     // partials by workgroup slot: this row's are in slots first .. first + ns - 1, at row `rl` of each
+        // (clamped: the table is device data, and a malformed prefix array of query lengths leaves rows that no entry
+        // was written for)
+        const int* tab = a.row_tab + ((size_t)hkv * a.R + r) * 2;
+        const int x = tab[0];
+        const int rl = min(max(tab[1], 0), a.slot_rows - 1);
+        mstride = (size_t)a.slot_rows * 2;
+        ostride = (size_t)a.slot_rows * EV;
+        auto place = [&](int slot, int row) {
+            const size_t base = ((size_t)hkv * a.pslots + slot) * a.slot_rows + row;
+            ml = a.part_ml + base * 2;
+            po = a.part_o + base * EV + e4 * 4;
+        };
+        int guessed = 0;
+        if (a.guess > 0) {
+            const int group = fast_div(r, a.magic_rows);
+            guessed = (group * a.guess) | (a.guess << 16);
+            ns = a.guess;
+            place(group * a.guess, r - group * a.slot_rows);
+            fetch(pgl);
+            fetched = true;
+        }
+        if (a.guess <= 0 || x != guessed) {
+            ns = min(max(x >> 16, 0), a.pslots);
+            place(min(x & 0xffff, a.pslots - ns), rl);
+            fetched = false;
+        }
+    }
+
+    float m_run = NEG_BIG, l_run = 0.f;
+    f32x4 acc = {0.f, 0.f, 0.f, 0.f};
+    for (int s0 = pgl; s0 < ns; s0 += UN * GPR) {
+        if (!fetched) fetch(s0);
+        fetched = false;
+#pragma unroll
+        for (int u = 0; u < UN; ++u) {
+            if (s0 + u * GPR >= ns) mlv[u] = f32x2{NEG_BIG, 0.f};
         }
         float mb = m_run;
 #pragma unroll

@@ -10,9 +10,9 @@
 // min(fragment_lengths, location + 1) (kernel_v21.cuh:385-388).
 //
 // Work decomposition: a workgroup owns one kv head, one row group of one worker (up to 16 or 32 query rows, a row
-// being one (token, q-head-in-group) pair of that worker) and every nsplit-th stripe of the sequence's 32-token
-// tiles: tile t goes to wave t mod (4 * nsplit) of the (kv head, row group).  Nothing about the sequence lengths
-// is known on the host (they are device tensors), so the stripes balance themselves.  The per-tile arithmetic,
+// being one (token, q-head-in-group) pair of that worker) and every ns-th stripe of the sequence's 32-token
+// tiles: tile t goes to wave t mod (4 * ns) of the (kv head, row group).  Nothing about the sequence lengths
+// is known on the host (they are device tensors): ns is the host's nsplit, or what paged_share makes of it.  The per-tile arithmetic,
 // the LDS staging and the partial/merge scheme are those of the fragment kernel; what differs is the address
 // generation: each lane computes the cache row of "its" token of the tile from the block table (one table entry
 // per lane and tile, prefetched two tiles ahead), the rows a lane has to fetch are picked from those with
@@ -22,6 +22,8 @@
 
 #include <hip/hip_runtime.h>
 #include <stdint.h>
+
+#include <type_traits>
 
 #include "hogwild_kernels.h"
 #include "hogwild_device.h"
@@ -33,6 +35,58 @@
 
 namespace hw {
 
+// The workgroups of a kv head shared out by the lengths of the sequences (fixed-length operator, one row group per sequence; the lengths
+// are device data, so every wave works the shares out for itself).  nsplit workgroups for each sequence whatever its length left the
+// launch waiting for those of the longest: append and attention of five sequences of 296 to 10 543 tokens (40/8 heads, D = 128, bf16)
+// 31.7 -> 22.3 us, eight of 210 to 9000 at 32/8 37 -> 24, four of 300 to 11 000 at 16/8 and D = 256 41 -> 28.6, five of 844 to 5868 23.8 -> 22.2.
+// The shares are the smallest bound on the tiles of a workgroup (in steps of the four waves) at which the sequences' workgroups
+// are no more than there are, found by trying one bound in every lane.  Sequences within a fifth of the first one's length keep nsplit
+// each, at no more than before (four of 12 528 tokens 41.4 -> 41.2, eight of 1200 17.0 both): the lengths are read ahead of the queries,
+// which are requested for equal shares, as are the partial sums in the merge.
+struct PagedShare {
+    int w, split, ns, slot0;      // sequence, which of its ns workgroups, the first one's slot
+    bool found;                   // false: a slot that is left over
+};
+// (loc0, len0: the first location of sequence min(lane, W - 1) and the first fragment's length, requested ahead of what the workgroup
+// needs besides, so that this is worked out while the rest is on its way)
+__device__ __forceinline__ PagedShare paged_share(const PagedDevHeader& ph, int item, int split, int lane, int loc0, int len0) {
+    const int cap = ph.block_size * ph.max_blocks, T = ph.LW * ph.LS, w = min(lane, ph.W - 1);
+    // lane = sequence: the tiles that its workgroups go through
+    auto tiles_to = [&](int most, int len) { return (max(min(min(len, cap), most < cap ? most + 1 : cap), 0) + TILE - 1) / TILE; };
+    int most = loc0;
+    for (int s = 1; s < ph.LS; ++s) most = max(most, ph.loc[w * ph.LS + s]);
+    int tiles = tiles_to(most, len0);
+    for (int f = 1; f < ph.F; ++f) {
+        most = -1;
+        for (int s = 0; s < ph.LS; ++s) most = max(most, ph.loc[f * T + w * ph.LS + s]);
+        tiles += tiles_to(most, ph.frag_len[f]);
+    }
+    // sequences of about the same length keep nsplit each
+    const int first = __builtin_amdgcn_readlane(tiles, 0);
+    if (__ballot(lane < ph.W && (5 * tiles > 6 * first || 6 * tiles < 5 * first)) == 0) return PagedShare{item, split, ph.nsplit, item * ph.nsplit, true};
+    const float mine = lane < ph.W ? (float)tiles : 0.f;
+    const int slots = ph.W * ph.nsplit, slot = item * ph.nsplit + split;
+    const int all = __builtin_amdgcn_readlane(wave_scan_inclusive(lane < ph.W ? tiles : 0), 63);
+    // lane = a bound on the tiles of a workgroup, multiples of the four waves: does every sequence get its workgroups?
+    const int least = max(1, (int)((float)all * __builtin_amdgcn_rcpf(4.0f * (float)slots)));
+    const float per = __builtin_amdgcn_rcpf(4.0f * (float)(least + lane * (1 + (least >> 5))));
+    auto groups = [&](float t, float per_group) { return max(1, (int)__builtin_ceilf(t * per_group - 0.01f)); };
+    int need = 0;
+    for (int sq = 0; sq < ph.W; ++sq) need += groups(__int_as_float(__builtin_amdgcn_readlane(__float_as_int(mine), sq)), per);
+    const unsigned long long fits = __ballot(need <= slots);
+    const float best = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(per), fits != 0 ? __builtin_ctzll(fits) : 63));
+    int n = lane < ph.W ? (fits != 0 ? groups(mine, best) : ph.nsplit) : 0;
+    const int slot0 = wave_scan_inclusive(n) - n;
+    const unsigned long long owner = __ballot(slot >= slot0 && slot < slot0 + n);
+    PagedShare r;
+    r.found = owner != 0;
+    r.w = r.found ? __builtin_ctzll(owner) : 0;
+    r.slot0 = __builtin_amdgcn_readlane(slot0, r.w);
+    r.split = slot - r.slot0;
+    r.ns = __builtin_amdgcn_readlane(n, r.w);
+    return r;
+}
+
 template <class DT, int E, int EV, int RB, int MINW, bool KEEP = false>
 __global__ __launch_bounds__(NTHREADS, MINW) void paged_attention_kernel(const PagedHeader args) {
     constexpr int AUX = KEEP ? 0 : HW_KV_AUX;
@@ -41,7 +95,6 @@ __global__ __launch_bounds__(NTHREADS, MINW) void paged_attention_kernel(const P
     typedef hw::Exchange<ROWS, EV> Ex;
     constexpr int SBYTES = NWAVES * G::KSTAGE;
     __shared__ __attribute__((aligned(16))) char q_lds[ROWS * G::QSTR];
-    __shared__ int lim_lds[ROWS];
     union Slot0 {
         char k[SBYTES];
         Ex ex;
@@ -83,22 +136,14 @@ __global__ __launch_bounds__(NTHREADS, MINW) void paged_attention_kernel(const P
     int bid = blockIdx.x;
     if (ph.flags & PH_XCD_REMAP) bid = (bid & 7) * (ph.nwg >> 3) + (bid >> 3);
     const int hi = fast_div(bid, ph.magic_nsplit);
-    const int split = bid - hi * ph.nsplit;
     const int hkv = fast_div(hi, ph.magic_nitems);
-    const int item = hi - hkv * ph.nitems;
     const int GQ = ph.Hq / ph.Hkv;
-
-    const PagedItem it = paged_item<ROWS>(ph, item, lane, GQ);
-    if (!it.found) return;                  // the grid is sized for the worst case; uniform over the workgroup
-    const int w = it.w, rg = it.rg, qs = it.qs, qe = it.qe;
     const int T = ph.LW * ph.LS;
-    const int r0 = qs * GQ + rg * ROWS;     // first row (global numbering: token * GQ + head in group)
-    const int rend = qe * GQ;               // end of the worker's rows
-    if (r0 >= rend) return;                 // uniform over the workgroup
     const int cap = ph.block_size * ph.max_blocks;
-    const int NW = ph.nsplit * NWAVES;      // waves that share the tiles of this (kv head, row group)
-    const int gw = split * NWAVES + wv;
-    const HW_GLOBAL int* btw = ph.block_table + (size_t)w * ph.max_blocks;
+    const bool shared = (ph.flags & PH_SHARED) != 0;
+    int item = hi - hkv * ph.nitems, split = bid - hi * ph.nsplit;
+    int ns = ph.nsplit;                     // workgroups that share the sequence's tiles
+    const int slot = item * ns + split;
 
     // what QueryRotation / map_row need, in the [LW, Hq, LS] layout, with the worker's row end as the row limit
     DevHeader a;
@@ -110,45 +155,74 @@ __global__ __launch_bounds__(NTHREADS, MINW) void paged_attention_kernel(const P
     a.part_o = ph.part_o;
     a.part_ml = ph.part_ml;
     a.len_dev = nullptr;
-    a.F = ph.F; a.W = ph.LW; a.Hq = ph.Hq; a.Hkv = ph.Hkv; a.S = ph.LS; a.R = rend;
+    a.F = ph.F; a.W = ph.LW; a.Hq = ph.Hq; a.Hkv = ph.Hkv; a.S = ph.LS;
     a.nrg = 1; a.wgs_per_head = ph.nsplit; a.nwg = ph.nwg;
     a.slot_stride = ph.nsplit; a.flags = KH_PREROTATED; a.sc = ph.sc;
     a.magic_gq = ph.magic_gq; a.magic_s = ph.magic_ls; a.magic_nrg = 0; a.magic_wg = 0;
 
+    int w = 0, r0 = 0, rend = 0;            // sequence; first row (global numbering: token * GQ + head in group), end of its rows
+    int NW = 0, gw = 0;                     // waves that share the tiles of this (kv head, row group); this one
+    const HW_GLOBAL int* btw = nullptr;
+    auto place = [&](int seq, int row_group, int qs, int qe) {
+        w = seq;
+        r0 = qs * GQ + row_group * ROWS;
+        rend = qe * GQ;
+        a.R = rend;
+        NW = ns * NWAVES;
+        gw = split * NWAVES + wv;
+        btw = ph.block_table + (size_t)w * ph.max_blocks;
+    };
     // block-table entry of the token this lane stands for in tile t
     auto bt_load = [&](int t) -> int {
         const int tok = min(t * TILE + (lane & 31), cap - 1);
         return btw[fast_div(tok, ph.magic_bs)];
     };
+    // one batch of independent loads: queries, locations, fragment length, the table entries of two tiles
+    QueryRotation<DT, E, ROWS, G::QSTR, true> qrot;
+    int lm = 0, flen = 0, bt_a = 0, bt_b = 0;
+    auto request = [&](int f) {
+        qrot.load(a, f, hkv, r0, GQ, tid);
+        lm = ph.loc[(size_t)f * T + fast_div(min(r0 + (tid & (ROWS - 1)), rend - 1), ph.magic_gq)];
+        flen = ph.frag_len[ph.cu_q != nullptr ? f * ph.W + w : f];
+        bt_a = bt_load(gw);
+        bt_b = bt_load(gw + NW);
+    };
+    {
+        const PagedItem it = paged_item<ROWS>(ph, item, lane, GQ);
+        if (!it.found) return;              // the grid is sized for the worst case; uniform over the workgroup
+        place(it.w, it.rg, it.qs, it.qe);
+    }
+    if (r0 >= rend) return;                 // uniform over the workgroup
+    int loc0 = 0, len0 = 0, first_slot = 0;
+    if (shared) {
+        loc0 = ph.loc[min(lane, ph.W - 1) * ph.LS];
+        len0 = ph.frag_len[0];
+    }
+    request(0);
+    if (shared) {
+        // (what is requested holds for equal sequences: only where the share turns out another is it requested again)
+        const PagedShare sh = paged_share(ph, item, split, lane, loc0, len0);
+        if (!sh.found) return;              // uniform over the workgroup
+        first_slot = sh.slot0;
+        if (sh.w != item || sh.split != split || sh.ns != ns) {
+            item = sh.w;
+            split = sh.split;
+            ns = sh.ns;
+            place(item, 0, item * ph.LS, item * ph.LS + ph.LS);
+            request(0);
+        }
+    }
 
     for (int f = 0; f < ph.F; ++f) {
-        // one batch of independent loads: queries, locations, fragment length, the table entries of two tiles
-        QueryRotation<DT, E, ROWS, G::QSTR, true> qrot;
-        qrot.load(a, f, hkv, r0, GQ, tid);
-        const int lm = ph.loc[(size_t)f * T + fast_div(min(r0 + (tid & (ROWS - 1)), rend - 1), ph.magic_gq)];
-        const int flen = ph.frag_len[ph.cu_q != nullptr ? f * ph.W + w : f];
-        int bt_a = bt_load(gw);
-        int bt_b = bt_load(gw + NW);
+        if (f > 0) request(f);
 
-        __syncthreads();   // the previous fragment's readers are done with q_lds / lim_lds
-        qrot.finish(a, q_lds, f, hkv, r0, GQ, false, tid);
-        if (tid < ROWS) lim_lds[tid] = (r0 + tid < rend) ? max(0, min(min(flen, cap), lm < cap ? lm + 1 : cap)) : 0x7fffffff;
-        __syncthreads();
-
-        constexpr bool QREG = MINW == 1;
-        u32x4 qreg[QREG ? RB * G::KJ : 1];
-        if constexpr (QREG) {
-#pragma unroll
-            for (int rb = 0; rb < RB; ++rb)
-#pragma unroll
-                for (int j = 0; j < G::KJ; ++j)
-                    qreg[rb * G::KJ + j] = *reinterpret_cast<const u32x4*>(q_lds + (rb * 16 + n) * G::QSTR + (4 * j + q) * 16);
-        }
+        // The bounds of the rows: lane l holds that of row l % ROWS.
+        const int limv = (r0 + (lane & (ROWS - 1)) < rend) ? max(0, min(min(flen, cap), lm < cap ? lm + 1 : cap)) : 0x7fffffff;
         int lim[RB];
         int maxlim = 0, minlim = 0x7fffffff;
 #pragma unroll
         for (int rb = 0; rb < RB; ++rb) {
-            lim[rb] = lim_lds[rb * 16 + n];
+            lim[rb] = RB == 1 ? limv : __shfl(limv, rb * 16 + n, 64);
             const bool pad = r0 + rb * 16 + n >= rend;
             maxlim = max(maxlim, pad ? 0 : lim[rb]);
             minlim = min(minlim, lim[rb]);
@@ -199,12 +273,27 @@ __global__ __launch_bounds__(NTHREADS, MINW) void paged_attention_kernel(const P
             }
         };
 
+        // The first tile is requested as soon as the bounds are known, and the queries go through LDS while it is on its way (barriers
+        // for LDS only: __syncthreads() would wait for it): eight sequences of 1200 tokens 17.3 -> 17.0 us with the append.
+        TileRegs<DT, E, EV> tr[2];
+        issue_tile(tr[0], kslots[0], bt_a, gw);
+        lds_barrier();   // the previous fragment's readers are done with q_lds
+        qrot.finish(a, q_lds, f, hkv, r0, GQ, false, tid);
+        lds_barrier();
+        constexpr bool QREG = MINW == 1;
+        u32x4 qreg[QREG ? RB * G::KJ : 1];
+        if constexpr (QREG) {
+#pragma unroll
+            for (int rb = 0; rb < RB; ++rb)
+#pragma unroll
+                for (int j = 0; j < G::KJ; ++j)
+                    qreg[rb * G::KJ + j] = *reinterpret_cast<const u32x4*>(q_lds + (rb * 16 + n) * G::QSTR + (4 * j + q) * 16);
+        }
+
         if (maxlim > 0) {   // uniform
             // Two tiles in flight per wave.  Per step: request the table entries two tiles ahead, then the K/V of
             // the next tile (its entries were requested one step earlier, ahead of the previous K/V request, so
             // they have arrived by the time the current tile's data has), then compute the current tile.
-            TileRegs<DT, E, EV> tr[2];
-            issue_tile(tr[0], kslots[0], bt_a, gw);
             // Two loops with one instantiation of the tile arithmetic each (see attention_kernel): pairs of tiles every
             // row of the wave sees completely, then the rest.
             int t = gw;
@@ -248,31 +337,41 @@ __global__ __launch_bounds__(NTHREADS, MINW) void paged_attention_kernel(const P
         }
     }
 
-    store_partials<DT, EV, RB, true>(st, slot0.ex, wv, n, q, tid, ph.part_o, ph.part_ml, (size_t)(hkv * ph.nsplit + split) * ph.R + r0,
+    store_partials<DT, EV, RB, true>(st, slot0.ex, wv, n, q, tid, ph.part_o, ph.part_ml,
+                               shared ? (size_t)(hkv * ph.nitems * ph.nsplit + slot) * (ph.LS * GQ) : (size_t)(hkv * ph.nsplit + split) * ph.R + r0,
                                min(ROWS, rend - r0));
+    // where the merge finds the rows' partial sums
+    if (shared && split == 0 && tid < rend - r0) {
+        HW_GLOBAL int* row_tab = reinterpret_cast<HW_GLOBAL int*>(ph.part_ml + (size_t)ph.Hkv * ph.nsplit * ph.R * 2) + ((size_t)hkv * ph.R + r0) * 2;
+        row_tab[2 * tid] = first_slot | (ns << 16);
+        row_tab[2 * tid + 1] = tid;
+    }
 }
 
 // Scatter of new K/V rows into the paged caches, one 16-byte chunk (or, for odd sizes, one element) per thread.
 // A position whose block index lies outside the table, or whose table entry lies outside the cache, is skipped.
-template <int VEC>   // bytes per thread
+// IDX: 32 bits, unless there are more pieces than that (a division in 64 bits is a hundred instructions, and five of them stood in front
+// of three dependent accesses: one token of eight sequences, 8 heads, D = 128, append and attention 18.0 -> 17.8 us, see paged_share).
+template <int VEC, class IDX>   // bytes per thread
 __global__ __launch_bounds__(256) void copy_to_blocks_kernel(const CopyBlocksArgs a, int sz) {
     const int ck = a.E * sz / VEC, cv = a.Ev * sz / VEC;
-    const size_t rows = (size_t)a.B * a.Hkv * a.S_new;
-    const size_t total = rows * (size_t)(ck + cv);
-    for (size_t idx = (size_t)blockIdx.x * blockDim.x + threadIdx.x; idx < total; idx += (size_t)gridDim.x * blockDim.x) {
-        const size_t row = idx / (size_t)(ck + cv);
-        const int c = (int)(idx - row * (size_t)(ck + cv));
-        const int t = (int)(row % a.S_new);
-        const size_t bh = row / a.S_new;
-        const int h = (int)(bh % a.Hkv);
-        const int b = (int)(bh / a.Hkv);
-        const long long pos = (long long)a.seq_lengths[b] + t;
-        if (pos < 0) continue;
-        const long long bi = pos / a.block_size;
-        if (bi >= a.max_blocks) continue;
+    const IDX rows = (IDX)a.B * a.Hkv * a.S_new;
+    const IDX total = rows * (unsigned)(ck + cv);
+    for (IDX idx = (IDX)blockIdx.x * blockDim.x + threadIdx.x; idx < total; idx += (IDX)gridDim.x * blockDim.x) {
+        const IDX row = idx / (unsigned)(ck + cv);
+        const int c = (int)(idx - row * (unsigned)(ck + cv));
+        const IDX bh = row / (unsigned)a.S_new;
+        const int t = (int)(row - bh * (unsigned)a.S_new);
+        const int b = (int)(bh / (unsigned)a.Hkv);
+        const int h = (int)(bh - (IDX)b * (unsigned)a.Hkv);
+        const int length = a.seq_lengths[b];
+        if (length < 0 && length + t < 0) continue;
+        const unsigned pos = (unsigned)length + (unsigned)t;               // (two numbers below 2^31)
+        const unsigned bi = pos / (unsigned)a.block_size;
+        if (bi >= (unsigned)a.max_blocks) continue;
         const int blk = a.block_table[(size_t)b * a.max_blocks + bi];
         if (blk < 0 || blk >= a.num_blocks) continue;
-        const int off = (int)(pos - bi * a.block_size);
+        const int off = (int)(pos - bi * (unsigned)a.block_size);
         const size_t dst_row = ((size_t)blk * a.Hkv + h) * a.block_size + off;
         const bool is_k = c < ck;
         const char* src = is_k ? reinterpret_cast<const char*>(a.key_states) + ((long long)b * a.ks_b + (long long)h * a.ks_h + (long long)t * a.ks_s) * sz + (size_t)c * VEC
@@ -338,9 +437,14 @@ hipError_t launch_copy_to_blocks(const CopyBlocksArgs& ca, int dtype, hipStream_
     if (total == 0) return hipSuccess;
     size_t blocks = (total + 255) / 256;
     if (blocks > 8192) blocks = 8192;
-    if (vec == 16) hipLaunchKernelGGL((copy_to_blocks_kernel<16>), dim3((unsigned)blocks), dim3(256), 0, stream, ca, sz);
-    else if (vec == 4) hipLaunchKernelGGL((copy_to_blocks_kernel<4>), dim3((unsigned)blocks), dim3(256), 0, stream, ca, sz);
-    else hipLaunchKernelGGL((copy_to_blocks_kernel<2>), dim3((unsigned)blocks), dim3(256), 0, stream, ca, sz);
+    auto go = [&](auto vec_tag) {
+        constexpr int VEC = decltype(vec_tag)::value;
+        if (total < (1ull << 31)) hipLaunchKernelGGL((copy_to_blocks_kernel<VEC, unsigned>), dim3((unsigned)blocks), dim3(256), 0, stream, ca, sz);
+        else hipLaunchKernelGGL((copy_to_blocks_kernel<VEC, unsigned long long>), dim3((unsigned)blocks), dim3(256), 0, stream, ca, sz);
+    };
+    if (vec == 16) go(std::integral_constant<int, 16>{});
+    else if (vec == 4) go(std::integral_constant<int, 4>{});
+    else go(std::integral_constant<int, 2>{});
     return hipGetLastError();
 }
 

@@ -559,6 +559,19 @@ bool paged_keep_in_l2(const hw_paged_problem* p, const hw_paged_plan& plan) {
     return p->E == 256 && plan.rows > (p->cu_seqlens_q != nullptr ? 20ll : 32ll) * p->W;
 }
 
+// One row group per sequence, and what the waves go through to find a length (F * S locations) is little: a decode step, a draft of a few
+// tokens.  The measurements are at paged_share in hogwild_paged.hip.  (A caller that fixes the split keeps it.)
+bool paged_shared(const hw_paged_problem* p, const hw_paged_plan& plan) {
+    return p->cu_seqlens_q == nullptr && p->splits <= 0 && plan.row_blocks != hw::WIDE_ROW_BLOCKS && p->W >= 2 && p->W <= 64 &&
+           plan.row_groups == p->W && plan.splits >= 2 && (long long)p->F * p->S <= 8;
+}
+
+size_t paged_call_bytes(const hw_paged_problem* p, const hw_paged_plan& plan) {
+    if (!paged_shared(p, plan)) return plan.workspace_bytes;
+    const size_t bytes = (size_t)p->Hkv * plan.splits * plan.rows * ((size_t)p->Ev + 2) * sizeof(float) + (size_t)p->Hkv * plan.rows * 2 * sizeof(int);
+    return std::max(plan.workspace_bytes, (bytes + 255) & ~(size_t)255);
+}
+
 int paged_plan(const hw_paged_problem* p, int num_cus, hw_paged_plan* plan) {
     if (plan == nullptr) return HW_ERR_NULL;
     if (num_cus < 1) return HW_ERR_SHAPE;

@@ -76,6 +76,10 @@ bool deal_by_seen(const hw_problem* p, const CallPlan& cp, const WholePlan& wp);
 size_t call_workspace_bytes(const hw_problem* p, int num_cus, const CallPlan& cp);
 int paged_validate(const hw_paged_problem* p);
 int paged_plan(const hw_paged_problem* p, int num_cus, hw_paged_plan* plan);
+// Whether the workgroups of a paged launch may be shared out by the lengths of the sequences (hogwild_plan.cpp), and what a call asks
+// for: hw_paged_plan's workspace, the caller's fallback, and the merge's row table.
+bool paged_shared(const hw_paged_problem* p, const hw_paged_plan& plan);
+size_t paged_call_bytes(const hw_paged_problem* p, const hw_paged_plan& plan);
 // Whether the tiles of a paged launch are to stay in the L2 (hogwild_plan.cpp).
 bool paged_keep_in_l2(const hw_paged_problem* p, const hw_paged_plan& plan);
 

@@ -1080,15 +1080,6 @@ __device__ __forceinline__ void plan_row_table(const PagedDevHeader& ph, const P
 // The same plan for launches of at most 64 sequences and 64 slots per kv head, worked out by every wave for itself with
 // cross-lane operations (lane = sequence, then lane = row group): no LDS, no barriers.  (The general form below meets
 // sixteen workgroup barriers; on four sequences it took 2.6 us of every workgroup's prologue.)
-__device__ __forceinline__ int wave_scan_inclusive(int v) {
-    v += __builtin_amdgcn_update_dpp(0, v, 0x111, 0xf, 0xf, false);    // row_shr:1
-    v += __builtin_amdgcn_update_dpp(0, v, 0x112, 0xf, 0xf, false);    // row_shr:2
-    v += __builtin_amdgcn_update_dpp(0, v, 0x114, 0xf, 0xf, false);    // row_shr:4
-    v += __builtin_amdgcn_update_dpp(0, v, 0x118, 0xf, 0xf, false);    // row_shr:8: inclusive within rows of 16 lanes
-    v += __builtin_amdgcn_update_dpp(0, v, 0x142, 0xa, 0xf, false);    // row_bcast:15 into rows 1 and 3
-    v += __builtin_amdgcn_update_dpp(0, v, 0x143, 0xc, 0xf, false);    // row_bcast:31 into rows 2 and 3
-    return v;
-}
 template <int NTW>
 __device__ __forceinline__ PlanSlot plan_slot_wave(const PagedDevHeader& ph, int item, int hkv, int GQ, int T, int tid) {
     const int lane = tid & 63;

@@ -1,0 +1,68 @@
+"""Paged decode steps of sequences of different length: the workgroups of a kv head are shared out by the visible tiles (paged_share) --
+against the same call with the split fixed by the caller, which keeps equal shares, and in a workspace sized for those."""
+import pytest
+import torch
+
+from inference_lib_amd import _lib
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("dtype,lens,S,F,Hq,Hkv,D,bs", [
+    (torch.bfloat16, (1, 5000), 1, 1, 8, 8, 128, 16),                            # one tile beside many
+    (torch.float16, (300, 0, 7000, 33, 64, 1), 1, 1, 28, 4, 64, 32),             # a sequence that sees nothing
+    (torch.bfloat16, (9000, 40, 40, 40, 40, 40, 40), 2, 1, 40, 8, 128, 16),      # several tokens; nearly all to the first
+    (torch.float32, (700, 2900, 31), 1, 1, 8, 2, 64, 16),
+    (torch.bfloat16, (100, 11000, 900, 2500), 1, 1, 16, 8, 256, 64),
+    (torch.float16, (4000, 200, 1500), 1, 3, 16, 4, 128, 16),                    # three fragments of the same sequences
+    (torch.bfloat16, tuple(64 + 97 * i for i in range(31)), 1, 1, 8, 2, 128, 16),
+    (torch.bfloat16, (1000, 1190, 850), 1, 1, 40, 8, 128, 16),                   # within a fifth: equal shares
+])
+def test_shares_by_length(dtype, lens, S, F, Hq, Hkv, D, bs):
+    g = torch.Generator(device="cuda").manual_seed(len(lens) + D)
+    W, mb = len(lens), -(-max(lens) // bs) + 3
+    rnd = lambda *shape: torch.randn(shape, generator=g, device="cuda").to(dtype)
+    kc, vc = rnd(W * mb, Hkv, bs, D), rnd(W * mb, Hkv, bs, D)
+    table = torch.randperm(W * mb, generator=g, device="cuda").to(torch.int32).reshape(W, mb)
+    q = rnd(F, W, Hq, S, D)
+    pos = torch.tensor([[n - S + s for s in range(S)] for n in lens], dtype=torch.int32, device="cuda").clamp(min=-1)
+    loc = torch.stack([pos - 50 * f for f in range(F)]).clamp(min=-1).contiguous()
+    frag = torch.full((F,), bs * mb, dtype=torch.int32, device="cuda")
+    results = []
+    for splits, sized_for_equal in ((0, False), (0, True), (3, False)):
+        out, lse = torch.full((W, Hq, S, D), 7.0, dtype=dtype, device="cuda"), torch.full((W, Hq, S), 7.0, device="cuda")
+        pr = _lib.PagedProblem(q=q, locations=loc, fragment_lengths=frag, key_cache=kc, value_cache=vc, block_table=table, scale=D ** -0.5, out=out, lse=lse,
+                               splits=splits)
+        need = pr.workspace_bytes()
+        if sized_for_equal:                        # the row table does not fit: equal shares
+            equal = _lib.paged_plan(W=W, Hq=Hq, Hkv=Hkv, Ev=D, block_size=bs, max_blocks=mb, num_cus=_lib.lib.hw_device_cus(), S=S, dtype=_lib._DTYPE_CODE[dtype])
+            assert equal.splits > 1 and equal.workspace_bytes < need
+            need = equal.workspace_bytes
+        space = torch.full((need + 4096,), 165, dtype=torch.uint8, device="cuda")
+        pr.set_workspace(space[:need])
+        pr.run()
+        assert bool((space[need:] == 165).all())
+        results.append((out.double(), lse.double()))
+    # float64, of the values as stored
+    ref, ref_lse = torch.zeros((W, Hq, S, D), dtype=torch.float64, device="cuda"), torch.full((W, Hq, S), float("-inf"), dtype=torch.float64, device="cuda")
+    bound = torch.zeros_like(ref)
+    u = {torch.bfloat16: 2.0 ** -8, torch.float16: 2.0 ** -11, torch.float32: 2.0 ** -24}[dtype]
+    for w in range(W):
+        n = max(lens[w], 1)
+        rows = table[w, : -(-n // bs)].long()
+        k, v = (c[rows].transpose(1, 2).reshape(-1, Hkv, D)[:n].double() for c in (kc, vc))          # [n, Hkv, D]
+        for h in range(Hq):
+            kh, vh = k[:, h // (Hq // Hkv)], v[:, h // (Hq // Hkv)]
+            x = torch.cat([(q[f, w, h].double() @ kh.t().contiguous() * D ** -0.5).masked_fill(torch.arange(n, device="cuda")[None] > loc[f, w][:, None], float("-inf"))
+                           for f in range(F)], dim=1)
+            ref_lse[w, h] = torch.logsumexp(x, dim=1)
+            p = torch.nan_to_num(torch.softmax(x, dim=1))
+            vv = vh.repeat(F, 1)
+            ref[w, h] = p @ vv
+            # probabilities and the result are rounded once (fp16: to 2^-25 where subnormal), the fp32 sums are worth another 2^-16
+            bound[w, h] = (u + 2.0 ** -16) * (p @ vv.abs()) + u * ref[w, h].abs() + (2.0 ** -25 * vv.abs().sum(0) if dtype == torch.float16 else 0.0)
+    seen = ~torch.isneginf(ref_lse)
+    for out, lse in results:
+        assert bool(((out - ref).abs() <= bound)[seen].all())
+        assert bool((out[~seen] == 0).all()) and bool(torch.isneginf(lse[~seen]).all())
+        assert float((lse - ref_lse)[seen].abs().max()) <= 1e-4
