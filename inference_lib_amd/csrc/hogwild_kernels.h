@@ -127,6 +127,7 @@ constexpr int PH_PLANNED = 2;
 // sequences' visible tiles instead of nsplit to each (paged_share).  Partial sums by workgroup slot, LS * (Hq / Hkv) rows each, the
 // merge's row table right behind part_ml.
 constexpr int PH_SHARED = 8;
+constexpr int PH_SMALL = 16;       // the K cache is less than 4 GB: one buffer descriptor reaches all of it (read by launch_paged_attention only)
 
 struct CopyBlocksArgs {
     const void* key_states;    // [B, Hkv, S_new, E]   (element strides below, innermost contiguous)

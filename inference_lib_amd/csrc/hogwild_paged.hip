@@ -87,10 +87,31 @@ __device__ __forceinline__ PagedShare paged_share(const PagedDevHeader& ph, int 
     return r;
 }
 
-template <class DT, int E, int EV, int RB, int MINW, bool KEEP = false>
+// SMALL: below 4 GB the K cache is reached through one buffer descriptor, and its transfers are buffer loads.  A transfer by 64-bit address
+// is a flat-encoded instruction with an LDS operand, for which the compiler waits until nothing is outstanding: it emptied the
+// look-ahead at every tile (vmcnt(0) in front of each request, where 16 and 17 operations may be in flight).  Four sequences of 12 528
+// tokens, append and attention 41.2 -> 39.3 us (6.3 TB/s in the attention), 2500 to 3600 tokens 18.2 -> 17.1, five of 296 to 10 543 22.3 -> 20.4;
+// bit-identical.
+struct CacheView {
+    __amdgpu_buffer_rsrc_t k;
+};
+__device__ __forceinline__ CacheView make_cache_view(const PagedDevHeader& ph, int krow) {
+    CacheView v;
+    v.k = __builtin_amdgcn_make_buffer_rsrc(reinterpret_cast<void*>(reinterpret_cast<unsigned long long>(ph.kcache)), 0,
+                                            (int)((unsigned)ph.num_blocks * (unsigned)ph.Hkv * (unsigned)ph.block_size * (unsigned)krow), 0x00020000);
+    return v;
+}
+
+template <int AUX>
+__device__ __forceinline__ void cache_transfer(const CacheView& v, char* lds, unsigned offset) {
+    __builtin_amdgcn_raw_ptr_buffer_load_lds(v.k, HW_LDS_PTR(lds), 16, offset, 0, 0, AUX);
+}
+
+template <class DT, int E, int EV, int RB, int MINW, bool SMALL, bool KEEP = false>
 __global__ __launch_bounds__(NTHREADS, MINW) void paged_attention_kernel(const PagedHeader args) {
     constexpr int AUX = KEEP ? 0 : HW_KV_AUX;
     typedef Geo<DT, E, EV> G;
+    constexpr bool STATED = G::KL + 8 * G::NVL >= 32;      // the waits for K are stated by hand (wait_k_landed)
     constexpr int ROWS = RB * 16;
     typedef hw::Exchange<ROWS, EV> Ex;
     constexpr int SBYTES = NWAVES * G::KSTAGE;
@@ -144,6 +165,9 @@ __global__ __launch_bounds__(NTHREADS, MINW) void paged_attention_kernel(const P
     int item = hi - hkv * ph.nitems, split = bid - hi * ph.nsplit;
     int ns = ph.nsplit;                     // workgroups that share the sequence's tiles
     const int slot = item * ns + split;
+
+    [[maybe_unused]] CacheView all;                        // the whole K cache (SMALL)
+    if constexpr (SMALL) all = make_cache_view(ph, G::KROW);
 
     // what QueryRotation / map_row need, in the [LW, Hq, LS] layout, with the worker's row end as the row limit
     DevHeader a;
@@ -246,8 +270,12 @@ __global__ __launch_bounds__(NTHREADS, MINW) void paged_attention_kernel(const P
 #pragma unroll
             for (int i = 0; i < G::KL; ++i) {
                 const int r = __shfl(rid, i * RPL + lrow, 64);
-                const HW_GLOBAL char* src = ph.kcache + (unsigned long long)(unsigned)r * G::KROW + k_chunk(i);
-                __builtin_amdgcn_global_load_lds(src, HW_LDS_PTR(kslot + i * 1024), 16, 0, AUX);
+                if constexpr (SMALL) {
+                    cache_transfer<AUX>(all, kslot + i * 1024, (unsigned)r * G::KROW + k_chunk(i));
+                } else {
+                    const HW_GLOBAL char* src = ph.kcache + (unsigned long long)(unsigned)r * G::KROW + k_chunk(i);
+                    __builtin_amdgcn_global_load_lds(src, HW_LDS_PTR(kslot + i * 1024), 16, 0, AUX);
+                }
             }
             asm volatile("" ::: "memory");
 #pragma unroll
@@ -302,14 +330,14 @@ __global__ __launch_bounds__(NTHREADS, MINW) void paged_attention_kernel(const P
                 {
                     const int bt_n = bt_load(t + 2 * NW);
                     issue_tile(tr[1], kslots[1], bt_b, t + NW);
-                    if constexpr (E > 128) wait_k_landed<G, 1>();   // (see wait_k_landed: the table load in between only adds to what is behind)
+                    if constexpr (STATED) wait_k_landed<G, 1>();   // (see wait_k_landed: the table load in between only adds to what is behind)
                     compute_tile<DT, E, EV, RB, false, QREG>(tr[0], q_lds, qreg, lim, st, t * TILE, n, q, ph.sc, kslots[0]);
                     bt_a = bt_n;
                 }
                 {
                     const int bt_n = bt_load(t + 3 * NW);
                     issue_tile(tr[0], kslots[0], bt_a, t + 2 * NW);
-                    if constexpr (E > 128) wait_k_landed<G, 1>();
+                    if constexpr (STATED) wait_k_landed<G, 1>();
                     compute_tile<DT, E, EV, RB, false, QREG>(tr[1], q_lds, qreg, lim, st, (t + NW) * TILE, n, q, ph.sc, kslots[1]);
                     bt_b = bt_n;
                 }
@@ -318,7 +346,7 @@ __global__ __launch_bounds__(NTHREADS, MINW) void paged_attention_kernel(const P
                 {
                     const int bt_n = bt_load(t + 2 * NW);
                     issue_tile(tr[1], kslots[1], bt_b, t + NW);
-                    if constexpr (E > 128) wait_k_landed<G, 1>();
+                    if constexpr (STATED) wait_k_landed<G, 1>();
                     const int t0 = t * TILE;
                     if (G::SZ == 4 && t0 + TILE <= minlim) compute_tile<DT, E, EV, RB, false, QREG>(tr[0], q_lds, qreg, lim, st, t0, n, q, ph.sc, kslots[0]);
                     else compute_tile<DT, E, EV, RB, true, QREG>(tr[0], q_lds, qreg, lim, st, t0, n, q, ph.sc, kslots[0]);
@@ -327,7 +355,7 @@ __global__ __launch_bounds__(NTHREADS, MINW) void paged_attention_kernel(const P
                 {
                     const int bt_n = bt_load(t + 3 * NW);
                     issue_tile(tr[0], kslots[0], bt_a, t + 2 * NW);
-                    if constexpr (E > 128) wait_k_landed<G, 1>();
+                    if constexpr (STATED) wait_k_landed<G, 1>();
                     const int t0 = (t + NW) * TILE;
                     if (G::SZ == 4 && t0 + TILE <= minlim) compute_tile<DT, E, EV, RB, false, QREG>(tr[1], q_lds, qreg, lim, st, t0, n, q, ph.sc, kslots[1]);
                     else if (t0 < maxlim) compute_tile<DT, E, EV, RB, true, QREG>(tr[1], q_lds, qreg, lim, st, t0, n, q, ph.sc, kslots[1]);
@@ -387,43 +415,48 @@ __global__ __launch_bounds__(256) void copy_to_blocks_kernel(const CopyBlocksArg
 // ------------------------------------------------------------------------------------------------
 // launchers
 // ------------------------------------------------------------------------------------------------
-template <class DT, int E, int EV>
+template <class DT, int E, int EV, bool SMALL>
 static hipError_t launch_paged_rb(const PagedHeader& ph, int rb, hipStream_t stream) {
     constexpr bool half = Elem<DT>::size == 2;
     // fp32 operands with two row blocks do not fit the register file; the planner never asks for them
     if constexpr (half) {
         if (rb == 2) {
-            hipLaunchKernelGGL((paged_attention_kernel<DT, E, EV, 2, 1>), dim3(ph.nwg), dim3(NTHREADS), 0, stream, ph);
+            hipLaunchKernelGGL((paged_attention_kernel<DT, E, EV, 2, 1, SMALL>), dim3(ph.nwg), dim3(NTHREADS), 0, stream, ph);
             return hipGetLastError();
         }
     }
     if (rb != 1) return hipErrorInvalidValue;
-    hipLaunchKernelGGL((paged_attention_kernel<DT, E, EV, 1, half ? HW_PAGED_MINW : 1>), dim3(ph.nwg), dim3(NTHREADS), 0, stream, ph);
+    hipLaunchKernelGGL((paged_attention_kernel<DT, E, EV, 1, half ? HW_PAGED_MINW : 1, SMALL>), dim3(ph.nwg), dim3(NTHREADS), 0, stream, ph);
     return hipGetLastError();
 }
 
-template <class DT>
+template <class DT, bool SMALL>
 static hipError_t launch_paged_dt(const PagedHeader& ph, int E, int rb, hipStream_t stream) {
     if (E == 256) {     // one 16-row block per workgroup, one wave per SIMD; 16-bit types (two fp32 K tiles per wave exceed the LDS)
         if constexpr (Elem<DT>::size == 2) {
             if (rb != 1) return hipErrorInvalidValue;
-            if (ph.flags & PH_KEEP) hipLaunchKernelGGL((paged_attention_kernel<DT, 256, 256, 1, 1, true>), dim3(ph.nwg), dim3(NTHREADS), 0, stream, ph);
-            else hipLaunchKernelGGL((paged_attention_kernel<DT, 256, 256, 1, 1>), dim3(ph.nwg), dim3(NTHREADS), 0, stream, ph);
+            if (ph.flags & PH_KEEP) hipLaunchKernelGGL((paged_attention_kernel<DT, 256, 256, 1, 1, SMALL, true>), dim3(ph.nwg), dim3(NTHREADS), 0, stream, ph);
+            else hipLaunchKernelGGL((paged_attention_kernel<DT, 256, 256, 1, 1, SMALL>), dim3(ph.nwg), dim3(NTHREADS), 0, stream, ph);
             return hipGetLastError();
         }
         return hipErrorInvalidValue;
     }
-    if (E == 128) return launch_paged_rb<DT, 128, 128>(ph, rb, stream);
+    if (E == 128) return launch_paged_rb<DT, 128, 128, SMALL>(ph, rb, stream);
     if (E != 64) return hipErrorInvalidValue;
-    return launch_paged_rb<DT, 64, 64>(ph, rb, stream);
+    return launch_paged_rb<DT, 64, 64, SMALL>(ph, rb, stream);
+}
+
+template <bool SMALL>
+static hipError_t launch_paged_small(const PagedHeader& ph, int dtype, int E, int rb, hipStream_t stream) {
+    switch (dtype) {
+        case 0: return launch_paged_dt<F32, SMALL>(ph, E, rb, stream);
+        case 1: return launch_paged_dt<F16, SMALL>(ph, E, rb, stream);
+        default: return launch_paged_dt<BF16, SMALL>(ph, E, rb, stream);
+    }
 }
 
 hipError_t launch_paged_attention(const PagedHeader& ph, int dtype, int E, int rb, hipStream_t stream) {
-    switch (dtype) {
-        case 0: return launch_paged_dt<F32>(ph, E, rb, stream);
-        case 1: return launch_paged_dt<F16>(ph, E, rb, stream);
-        default: return launch_paged_dt<BF16>(ph, E, rb, stream);
-    }
+    return ph.flags & PH_SMALL ? launch_paged_small<true>(ph, dtype, E, rb, stream) : launch_paged_small<false>(ph, dtype, E, rb, stream);
 }
 
 hipError_t launch_copy_to_blocks(const CopyBlocksArgs& ca, int dtype, hipStream_t stream) {

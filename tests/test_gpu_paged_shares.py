@@ -66,3 +66,26 @@ def test_shares_by_length(dtype, lens, S, F, Hq, Hkv, D, bs):
         assert bool(((out - ref).abs() <= bound)[seen].all())
         assert bool((out[~seen] == 0).all()) and bool(torch.isneginf(lse[~seen]).all())
         assert float((lse - ref_lse)[seen].abs().max()) <= 1e-4
+
+
+@pytest.mark.parametrize("dtype,Hq,Hkv,D,S", [(torch.bfloat16, 40, 8, 128, 1), (torch.float16, 16, 8, 256, 3), (torch.float32, 8, 8, 128, 1), (torch.float16, 64, 8, 64, 4)])
+def test_caches_of_4_gb_and_more(dtype, Hq, Hkv, D, S):
+    """K rows are reached through one buffer descriptor below 4 GB and through 64-bit addresses from there on: the same blocks at the end of
+    a cache of 4.3 GB and in a small one give the same bits."""
+    bs, lens = 32, (700, 90, 2500)
+    W, mb = len(lens), -(-max(lens) // bs)
+    g = torch.Generator(device="cuda").manual_seed(D)
+    rnd = lambda *shape: torch.randn(shape, generator=g, device="cuda").to(dtype)
+    k, v, q = rnd(W * mb, Hkv, bs, D), rnd(W * mb, Hkv, bs, D), rnd(1, W, Hq, S, D)
+    table = torch.randperm(W * mb, generator=g, device="cuda").to(torch.int32).reshape(W, mb)
+    loc = torch.tensor([[[n - S + s for s in range(S)] for n in lens]], dtype=torch.int32, device="cuda")
+    frag = torch.tensor([max(lens)], dtype=torch.int32, device="cuda")
+    many = -(-(2 ** 32 + 2 ** 20) // (Hkv * bs * D * k.element_size()))
+    results = []
+    for blocks in (W * mb, many):
+        kc, vc = (torch.empty((blocks, Hkv, bs, D), dtype=dtype, device="cuda") for _ in range(2))
+        kc[blocks - W * mb:], vc[blocks - W * mb:] = k, v
+        out = torch.empty((W, Hq, S, D), dtype=dtype, device="cuda")
+        _lib.PagedProblem(q=q, locations=loc, fragment_lengths=frag, key_cache=kc, value_cache=vc, block_table=table + (blocks - W * mb), scale=D ** -0.5, out=out).run()
+        results.append(out)
+    assert torch.equal(*results) and bool(torch.isfinite(results[0].float()).all())
