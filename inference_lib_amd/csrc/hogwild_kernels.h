@@ -73,7 +73,7 @@ struct MergeArgs {
     int rows;           // rows 0 .. rows - 1 of every kv head are merged
     int xcd_local;      // kv head h was computed on XCD h / (Hkv/8): merge it there
     // Partials laid out by workgroup slot instead of by row (KH_STREAM, and the paged launches that are dealt on the device,
-    // see PagedHeader): row_tab[kv head][r] = {first slot | slots << 16, row within the slot}, a slot holds slot_rows rows, pslots
+    // see PagedHeader): row_tab[kv head][r] = {first slot | slots << 16, row within the slot}, a slot holds slot_rows rows (PLAN_SLOT_ROWS without guess), pslots
     // slots per kv head; wgs_per_head then only bounds the slots of a row (for the choice of the merge kernel's shape).
     const int* row_tab;
     int pslots, slot_rows;
@@ -108,7 +108,7 @@ struct alignas(64) PagedHeader {
     int block_size, max_blocks, num_blocks;
     int nsplit;                // workgroups that share one (kv head, row group)
     int nitems;                // row groups over all workers (an upper bound when cu_q is given)
-    int nrg;                   // row groups per worker (fixed-length operator)
+    int nrg;                   // row groups per worker (fixed-length operator); planned: workgroups of a kv head that are under way at once
     int nwg;
     int flags;                 // PH_*
     float sc;                  // scale * log2(e)
@@ -123,6 +123,7 @@ constexpr int PH_XCD_REMAP = 1;    // consecutive logical workgroup ids share an
 // merge kernel a table per kv head of where each row's partial sums lie (MergeArgs::row_tab).
 constexpr int PH_KEEP = 4;         // K/V tiles stay in the L2 for the other row groups of a sequence (read by launch_paged_attention only)
 constexpr int PH_PLANNED = 2;
+constexpr int PH_GROUPS_SHIFT = 8;   // from this bit on, planned: the most row groups that the query tokens may come to
 // One row group per sequence (the fixed-length operator): the nitems * nsplit workgroups of a kv head are shared out by the
 // sequences' visible tiles instead of nsplit to each (paged_share).  Partial sums by workgroup slot, LS * (Hq / Hkv) rows each, the
 // merge's row table right behind part_ml.

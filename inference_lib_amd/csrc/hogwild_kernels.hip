@@ -311,7 +311,7 @@ __global__ __launch_bounds__(NTHREADS, MINW) void attention_kernel(const KernelA
 // its own, and the NPG partial groups are combined through LDS.
 // RPW = rows per workgroup: with few partials per row (at most 4 * NPG / RPW) a workgroup merges RPW rows side by side,
 // each with its share of the partial groups, instead of leaving most of its threads without a partial to load.
-template <class DT, int EV, int RPW>
+template <class DT, int EV, int RPW, bool GUESS>
 __global__ __launch_bounds__(256) void merge_kernel(const MergeArgs a) {
     typedef typename Elem<DT>::store_t store_t;
     constexpr int V4 = EV / 4;          // threads along the head dim (4 floats each)
@@ -356,30 +356,31 @@ __global__ __launch_bounds__(256) void merge_kernel(const MergeArgs a) {
             mlv[u] = *reinterpret_cast<const f32x2*>(ml + (size_t)sc * mstride);
         }
     };
-    bool fetched = false;
+    [[maybe_unused]] bool fetched = false;
     if (a.row_tab != nullptr) {     // partials by workgroup slot: this row's are in slots first .. first + ns - 1, at row `rl` of each
         // (clamped: the table is device data, and a malformed prefix array of query lengths leaves rows that no entry
         // was written for)
         const int* tab = a.row_tab + ((size_t)hkv * a.R + r) * 2;
         const int x = tab[0];
-        const int rl = min(max(tab[1], 0), a.slot_rows - 1);
-        mstride = (size_t)a.slot_rows * 2;
-        ostride = (size_t)a.slot_rows * EV;
+        const int slot_rows = GUESS ? a.slot_rows : PLAN_SLOT_ROWS;
+        const int rl = min(max(tab[1], 0), slot_rows - 1);
+        mstride = (size_t)slot_rows * 2;
+        ostride = (size_t)slot_rows * EV;
         auto place = [&](int slot, int row) {
-            const size_t base = ((size_t)hkv * a.pslots + slot) * a.slot_rows + row;
+            const size_t base = ((size_t)hkv * a.pslots + slot) * slot_rows + row;
             ml = a.part_ml + base * 2;
             po = a.part_o + base * EV + e4 * 4;
         };
-        int guessed = 0;
-        if (a.guess > 0) {
+        int guessed = -1;
+        if constexpr (GUESS) {
             const int group = fast_div(r, a.magic_rows);
             guessed = (group * a.guess) | (a.guess << 16);
             ns = a.guess;
-            place(group * a.guess, r - group * a.slot_rows);
+            place(group * a.guess, r - group * slot_rows);
             fetch(pgl);
             fetched = true;
         }
-        if (a.guess <= 0 || x != guessed) {
+        if (!GUESS || x != guessed) {
             ns = min(max(x >> 16, 0), a.pslots);
             place(min(x & 0xffff, a.pslots - ns), rl);
             fetched = false;
@@ -389,7 +390,7 @@ __global__ __launch_bounds__(256) void merge_kernel(const MergeArgs a) {
     float m_run = NEG_BIG, l_run = 0.f;
     f32x4 acc = {0.f, 0.f, 0.f, 0.f};
     for (int s0 = pgl; s0 < ns; s0 += UN * GPR) {
-        if (!fetched) fetch(s0);
+        if (!GUESS || !fetched) fetch(s0);
         fetched = false;
 #pragma unroll
         for (int u = 0; u < UN; ++u) {
@@ -589,7 +590,8 @@ static hipError_t launch_merge_ev(const MergeArgs& ma, hipStream_t stream) {
     auto go = [&](auto rpw_tag) {
         constexpr int RPW = decltype(rpw_tag)::value;
         const int blocks = ma.Hkv * ((ma.rows + RPW - 1) / RPW);
-        hipLaunchKernelGGL((merge_kernel<DT, EV, RPW>), dim3(blocks), dim3(256), 0, stream, ma);
+        if (ma.guess > 0) hipLaunchKernelGGL((merge_kernel<DT, EV, RPW, true>), dim3(blocks), dim3(256), 0, stream, ma);
+        else hipLaunchKernelGGL((merge_kernel<DT, EV, RPW, false>), dim3(blocks), dim3(256), 0, stream, ma);
     };
     if constexpr (NPG >= 8) {       // (eight rows side by side need eight thread groups: not at head dimension 256)
         if (ns <= 4) {

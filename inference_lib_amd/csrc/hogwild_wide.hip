@@ -575,10 +575,14 @@ __global__ __launch_bounds__(NW * 64, 1) void attention_wide_kernel(const Kernel
         };
         // The row group that comes behind the present one (STREAM): its number, or -1; below split_groups it is part of the run.
         [[maybe_unused]] auto next_group = [&]() {
-            int group = whole ? rgi + a.wgs_per_head : rgi + 1;
-            if (whole && group < groups) return group;
-            if (whole) group = run_begin / tiles_head;
-            return max(run_begin, group * tiles_head) < run_end ? group : -1;
+            int group = -1;
+            if constexpr (STREAM) {
+                group = whole ? rgi + a.wgs_per_head : rgi + 1;
+                if (whole && group < groups) return group;
+                if (whole) group = run_begin / tiles_head;
+                if (max(run_begin, group * tiles_head) >= run_end) group = -1;
+            }
+            return group;
         };
         // the largest value over the wave (uniform)
         auto wave_max = [&](int v) {
@@ -1077,9 +1081,14 @@ __device__ __forceinline__ void plan_row_table(const PagedDevHeader& ph, const P
     }
 }
 
-// The same plan for launches of at most 64 sequences and 64 slots per kv head, worked out by every wave for itself with
+// The plan for launches of at most 64 sequences and 64 row groups, worked out by every wave for itself with
 // cross-lane operations (lane = sequence, then lane = row group): no LDS, no barriers.  (The general form below meets
 // sixteen workgroup barriers; on four sequences it took 2.6 us of every workgroup's prologue.)
+// The host provides slots for the row groups that there might be; the ones beyond the CUs begin another round, and the plan now takes
+// them only where that is the shorter way.  Append-less packed launches, us a layer (bf16 but the third): 120, 100, 60, 40, 20 tokens on
+// 800 to 9000 at 40/8 heads, D = 128 55 -> 44; 4 x 128 on 4000 at 32/8 67 -> 53; seven sequences of 2 to 128 tokens at 64/8 (24 groups
+// for 32 CUs, fp16), where two rounds stay, 78 both; 7 x 128 at 64/8 (56 groups) 152 -> 138.  Shares in proportion to the work, one
+// after the other, gave the third 95 in one round.
 template <int NTW>
 __device__ __forceinline__ PlanSlot plan_slot_wave(const PagedDevHeader& ph, int item, int hkv, int GQ, int T, int tid) {
     const int lane = tid & 63;
@@ -1109,21 +1118,32 @@ __device__ __forceinline__ PlanSlot plan_slot_wave(const PagedDevHeader& ph, int
     const int rows = min((w_qe - w_qs) * GQ - rg * WIDE_ROWS, WIDE_ROWS);
     const int work = valid ? w_tiles * (rows > WIDE_ROWS / 2 ? 4 : 3) : 0;
     const int most = max(1, w_tiles / 4);
-    auto wave_total = [&](int v) { return __builtin_amdgcn_readlane(wave_scan_inclusive(v), 63); };
-    // one slot each, and the other pslots - G in proportion to the work (see plan_slot)
-    const int all_work = wave_total(work);
-    const float share = (float)(pslots - G) * (1.0f - 1.0f / (1 << 20)) * __builtin_amdgcn_rcpf((float)max(all_work, 1));
-    int n = valid ? min(1 + (int)((float)work * share), most) : 0;
-    const int left = pslots - wave_total(n);
-    const int load = (valid && n < most) ? __float_as_int((float)work * __builtin_amdgcn_rcpf((float)n)) : -1;
-    int ahead = 0;
-    for (int g = 0; g < G; ++g) {
-        const int lg = __builtin_amdgcn_readlane(load, g);
-        ahead += (lg > load || (lg == load && g < lane)) ? 1 : 0;
-    }
-    if (load >= 0 && ahead < left) ++n;
+    // The smallest bound on the work of a slot at which the groups need no more slots than there are, found by trying one in every
+    // lane: from an equal share in steps of 2^(1/16), the last lane the largest group whole.  The slots: as many as are under way at once
+    // (a whole number of times that with more groups), or that many more again, whichever comes to less with the openings (12 tiles of
+    // the dearer kind each).
+    const int fill = ph.nrg;
+    const int rounds = G <= fill ? 1 : (G + fill - 1) / fill;
+    const int few = min(pslots, rounds * fill), many = min(pslots, few + fill);
+    const int all_work = max(__builtin_amdgcn_readlane(wave_scan_inclusive(work), 63), 1);
+    const int row_most = row_max16(work);
+    const int largest = max(max(max(__builtin_amdgcn_readlane(row_most, 0), __builtin_amdgcn_readlane(row_most, 16)),
+                                max(__builtin_amdgcn_readlane(row_most, 32), __builtin_amdgcn_readlane(row_most, 48))), 1);
+    const float bound = lane == 63 ? (float)largest : (float)all_work * __builtin_amdgcn_rcpf((float)many) * fast_exp2(0.0625f * (float)lane);
+    const float per = __builtin_amdgcn_rcpf(bound);
+    auto share = [&](int work_, float per_slot) { return max(1, (int)__builtin_ceilf((float)work_ * per_slot - 0.01f)); };
+    int need = 0;
+    for (int g = 0; g < G; ++g) need += share(__builtin_amdgcn_readlane(work, g), per);
+    const unsigned long long fit_few = __ballot(need <= few) | (1ull << 63), fit_many = __ballot(need <= many) | (1ull << 63);
+    const int lane_few = __builtin_ctzll(fit_few), lane_many = __builtin_ctzll(fit_many);
+    auto at = [&](float v, int l) { return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), l)); };
+    constexpr float OPENING = 48.0f;
+    const bool more = ((float)rounds + 1.0f) * (at(bound, lane_many) + OPENING) < (float)rounds * (at(bound, lane_few) + OPENING);
+    const int slots = more ? many : few;
+    const float best = at(per, more ? lane_many : lane_few);
+    int n = valid ? min(share(work, best), most) : 0;
     const int slot0 = wave_scan_inclusive(n) - n;
-    n = max(min(n, pslots - slot0), 0);                 // (cannot bite)
+    n = max(min(n, slots - slot0), 0);                 // (cannot bite)
     const unsigned long long owner = __ballot(valid && item >= slot0 && item < slot0 + n);
     PlanSlot r;
     r.found = owner != 0;
@@ -1347,7 +1367,7 @@ __global__ __launch_bounds__(NW * 64, 1) void paged_wide_kernel(const PagedHeade
     int w, rg, qs, qe, ns;
     size_t pbase;                           // row of the partial arrays that holds the workgroup's first row
     if (ph.flags & PH_PLANNED) {
-        const PlanSlot ps = (ph.W <= 64 && ph.nitems <= 64)      // uniform over the launch
+        const PlanSlot ps = (ph.W <= 64 && (ph.flags >> PH_GROUPS_SHIFT) <= 64)      // uniform over the launch
                                 ? plan_slot_wave<NT>(ph, item, hkv, GQ, T, tid)
                                 : plan_slot<NT>(ph, reinterpret_cast<int*>(ring), item, hkv, GQ, T, tid);   // (the ring is not in use yet)
         if (!ps.found) return;              // a slot the plan left empty; uniform over the workgroup

@@ -89,3 +89,44 @@ def test_caches_of_4_gb_and_more(dtype, Hq, Hkv, D, S):
         _lib.PagedProblem(q=q, locations=loc, fragment_lengths=frag, key_cache=kc, value_cache=vc, block_table=table + (blocks - W * mb), scale=D ** -0.5, out=out).run()
         results.append(out)
     assert torch.equal(*results) and bool(torch.isfinite(results[0].float()).all())
+
+
+@pytest.mark.parametrize("dtype,tokens,lens,Hq,Hkv,D", [
+    (torch.bfloat16, (120, 100, 60, 40, 20), (1200, 5200, 800, 3000, 9000), 40, 8, 128),     # 16 row groups of 32 slots, 51 provided
+    (torch.float16, (30, 90, 5, 128, 60, 2, 17), (1300, 3200, 700, 5100, 400, 2000, 6000), 64, 8, 128),      # 24: two rounds
+    (torch.bfloat16, (128,) * 5, (1300, 3200, 700, 5100, 400), 64, 8, 128),                  # 40: more than the CUs of a head
+    (torch.float16, (30, 0, 60), (3000, 700, 64), 8, 2, 64),                                 # 128 slots a head, a sequence without tokens
+    (torch.bfloat16, (40,) + (1,) * 40, (4000,) + tuple(60 + 31 * i for i in range(40)), 40, 8, 128),
+])
+def test_packed_rounds(dtype, tokens, lens, Hq, Hkv, D):
+    g = torch.Generator(device="cuda").manual_seed(sum(tokens))
+    bs, W, T = 32, len(lens), sum(tokens)
+    mb = -(-max(lens) // bs)
+    rnd = lambda *shape: torch.randn(shape, generator=g, device="cuda").to(dtype)
+    kc, vc, q = rnd(W * mb, Hkv, bs, D), rnd(W * mb, Hkv, bs, D), rnd(1, T, Hq, D)
+    table = torch.randperm(W * mb, generator=g, device="cuda").to(torch.int32).reshape(W, mb)
+    cu = torch.tensor([sum(tokens[:w]) for w in range(W + 1)], dtype=torch.int32, device="cuda")
+    pos = torch.cat([torch.arange(n - t, n, dtype=torch.int32) for t, n in zip(tokens, lens)]).cuda()
+    frag = torch.tensor([lens], dtype=torch.int32, device="cuda")
+    out, lse = torch.full((T, Hq, D), 7.0, dtype=dtype, device="cuda"), torch.full((T, Hq), 7.0, device="cuda")
+    pr = _lib.PagedProblem(q=q, locations=pos[None].contiguous(), fragment_lengths=frag, key_cache=kc, value_cache=vc, block_table=table, scale=D ** -0.5,
+                           out=out, lse=lse, cu_seqlens_q=cu)
+    need = pr.workspace_bytes()
+    space = torch.full((need + 4096,), 165, dtype=torch.uint8, device="cuda")
+    pr.set_workspace(space[:need])
+    pr.run()
+    assert bool((space[need:] == 165).all())
+    u = {torch.bfloat16: 2.0 ** -8, torch.float16: 2.0 ** -11}[dtype]
+    for w in range(W):
+        n, rows = lens[w], slice(int(cu[w]), int(cu[w + 1]))
+        blocks = table[w, : -(-n // bs)].long()
+        k, v = (c[blocks].transpose(1, 2).reshape(-1, Hkv, D)[:n].double() for c in (kc, vc))
+        hidden = torch.arange(n, device="cuda")[None] > pos[rows][:, None]
+        for h in range(Hq):
+            kh, vh = k[:, h // (Hq // Hkv)], v[:, h // (Hq // Hkv)]
+            x = (q[0, rows, h].double() @ kh.t().contiguous() * D ** -0.5).masked_fill(hidden, float("-inf"))
+            p = torch.softmax(x, dim=1)
+            ref = p @ vh
+            bound = (u + 2.0 ** -16) * (p @ vh.abs()) + u * ref.abs() + (2.0 ** -25 * vh.abs().sum(0) if dtype == torch.float16 else 0.0)
+            assert bool(((out[rows, h].double() - ref).abs() <= bound).all())
+            assert bool(((lse[rows, h].double() - torch.logsumexp(x, dim=1)).abs() <= 1e-4).all())
