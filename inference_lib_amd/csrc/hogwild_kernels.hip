@@ -345,17 +345,8 @@ __global__ __launch_bounds__(256) void merge_kernel(const MergeArgs a) {
     size_t mstride = (size_t)a.R * 2;
     const float* po = a.part_o + ((size_t)hkv * ns * a.R + r) * EV + e4 * 4;
     size_t ostride = (size_t)a.R * EV;
-    f32x4 o[UN];
-    f32x2 mlv[UN];
-    auto fetch = [&](int s0) {
-#pragma unroll
-        for (int u = 0; u < UN; ++u) {
-            const int s = s0 + u * GPR;
-            const int sc = s < ns ? s : pgl;                // clamp: the loads stay unconditional
-            o[u] = *reinterpret_cast<const f32x4*>(po + (size_t)sc * ostride);
-            mlv[u] = *reinterpret_cast<const f32x2*>(ml + (size_t)sc * mstride);
-        }
-    };
+    [[maybe_unused]] f32x4 o_first[GUESS ? UN : 1];        // the first batch, where the guess holds
+    [[maybe_unused]] f32x2 ml_first[GUESS ? UN : 1];
     [[maybe_unused]] bool fetched = false;
     if (a.row_tab != nullptr) {     // partials by workgroup slot: this row's are in slots first .. first + ns - 1, at row `rl` of each
         // (clamped: the table is device data, and a malformed prefix array of query lengths leaves rows that no entry
@@ -377,7 +368,12 @@ __global__ __launch_bounds__(256) void merge_kernel(const MergeArgs a) {
             guessed = (group * a.guess) | (a.guess << 16);
             ns = a.guess;
             place(group * a.guess, r - group * slot_rows);
-            fetch(pgl);
+#pragma unroll
+            for (int u = 0; u < UN; ++u) {
+                const int sc = pgl + u * GPR < ns ? pgl + u * GPR : min(pgl, ns - 1);
+                o_first[u] = *reinterpret_cast<const f32x4*>(po + (size_t)sc * ostride);
+                ml_first[u] = *reinterpret_cast<const f32x2*>(ml + (size_t)sc * mstride);
+            }
             fetched = true;
         }
         if (!GUESS || x != guessed) {
@@ -390,11 +386,24 @@ __global__ __launch_bounds__(256) void merge_kernel(const MergeArgs a) {
     float m_run = NEG_BIG, l_run = 0.f;
     f32x4 acc = {0.f, 0.f, 0.f, 0.f};
     for (int s0 = pgl; s0 < ns; s0 += UN * GPR) {
-        if (!GUESS || !fetched) fetch(s0);
-        fetched = false;
+        f32x4 o[UN];
+        f32x2 mlv[UN];
+        if (GUESS && fetched) {
 #pragma unroll
-        for (int u = 0; u < UN; ++u) {
-            if (s0 + u * GPR >= ns) mlv[u] = f32x2{NEG_BIG, 0.f};
+            for (int u = 0; u < UN; ++u) {
+                o[u] = o_first[GUESS ? u : 0];
+                mlv[u] = s0 + u * GPR < ns ? ml_first[GUESS ? u : 0] : f32x2{NEG_BIG, 0.f};
+            }
+            fetched = false;
+        } else {
+#pragma unroll
+            for (int u = 0; u < UN; ++u) {
+                const int s = s0 + u * GPR;
+                const int sc = s < ns ? s : pgl;                // clamp: the loads stay unconditional
+                o[u] = *reinterpret_cast<const f32x4*>(po + (size_t)sc * ostride);
+                mlv[u] = *reinterpret_cast<const f32x2*>(ml + (size_t)sc * mstride);
+                if (s >= ns) mlv[u] = f32x2{NEG_BIG, 0.f};
+            }
         }
         float mb = m_run;
 #pragma unroll
