@@ -167,6 +167,7 @@ int run(const hw_problem* p, void* stream_, int fused, int stages = HW_STAGE_ATT
             ka.h.flags = ((ka.h.nwg % 8 == 0) ? hw::KH_XCD_REMAP : 0) | (prerotated ? hw::KH_PREROTATED : 0) | hw::KH_STREAM;
         }
         if (keep_in_l2(p, plan, cus)) ka.h.flags |= hw::KH_KEEP;
+        if (openings_ahead(p, plan, prerotated, stream_runs, whole ? &wp : nullptr)) ka.h.flags |= hw::KH_AHEAD;
         if (plan.row_blocks == hw::WIDE_ROW_BLOCKS)
             e = hw::launch_attention_wide(ka, p->dtype, p->E, stream);
         else

@@ -51,6 +51,7 @@ constexpr int KH_STREAM = 8;      // 128-row workgroups that run across row grou
                                   // workgroup g in row group rg goes to slot g + rg, a row table for the merge lies behind part_ml
                                   // (and see KernelArgs::split)
 constexpr int KH_KEEP = 16;       // K/V tiles stay in the L2 for the other row groups (keep_in_l2; read by launch_attention_wide only)
+constexpr int KH_AHEAD = 32;      // openings are prepared ahead (openings_ahead; read by launch_attention_wide only)
 constexpr int KH_PREROTATED = 4;  // the queries arrive rotated, [F,W,Hq,S,E] (read by the launchers only)
 
 struct KernelArgs {

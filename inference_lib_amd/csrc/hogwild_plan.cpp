@@ -430,6 +430,14 @@ static bool causal_chunk(const hw_problem* p) {
     return p->W == 1 && p->len[last] >= p->S;
 }
 
+// Whether the openings of a launch are prepared beside the tiles before them (attention_wide_kernel, AHEAD).  At head dimension 128, where
+// that was measured to pay.  At 64 a tile is half the arithmetic beside the same scalar work: pre-rotated queries of 1 to 8 workers and
+// 2 to 200 tokens at four head layouts took 1.00 to 1.035 times as long, 1.018 in the mean of 26 calls (4 workers x 32 tokens behind 4781
+// at 32/8 heads, fp16, 22.2 -> 21.5 us a layer without), prompt chunks 1.02 to 1.06.
+bool openings_ahead(const hw_problem* p, const hw_plan&, bool prerotated, bool stream_runs, const WholePlan*) {
+    return p->E == 128 && (prerotated || stream_runs);
+}
+
 // The remainder in runs: the smallest share (tiles, with openings) at which the workgroups, taking one after the other what fits,
 // use up the row groups, found by bisection.  Dealt by the tiles seen, those behind them go with the piece in front, so that no
 // workgroup opens a row group for tiles that none of its rows sees.  (Should the locations say otherwise, the launch is merely less

@@ -71,6 +71,8 @@ bool whole_size(const hw_problem* p, int num_cus, const CallPlan& cp, WholePlan*
 void whole_deal(const hw_problem* p, const CallPlan& cp, WholePlan* wp);
 // Whether whole_deal counts the tiles that a causal chunk sees (hogwild_plan.cpp).
 bool deal_by_seen(const hw_problem* p, const CallPlan& cp, const WholePlan& wp);
+// Whether a launch of 128-row workgroups prepares its openings ahead (hogwild_plan.cpp).  `whole`: of a launch in whole row groups, else null.
+bool openings_ahead(const hw_problem* p, const hw_plan& plan, bool prerotated, bool stream_runs, const WholePlan* whole);
 // What a call asks for: room for CallPlan, the caller's fallback, and for the launch that is preferred to it (whole row groups
 // before runs; 1024 tokens behind 4096 at 40/8 heads, D = 128: 21.3 MB, where the runs that are not taken there would need 38.1).
 size_t call_workspace_bytes(const hw_problem* p, int num_cus, const CallPlan& cp);

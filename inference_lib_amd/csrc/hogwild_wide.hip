@@ -299,7 +299,7 @@ struct WideRotation {
 // whole_size), 341 in two rounds of workgroups.  What bounds it is power as much as the arithmetic of two waves per SIMD (matrix
 // units 39 %, vector units 50 % of the clocks): the shader clock follows the load, 2.37 GHz in this form and 2.08-2.12 GHz in one
 // with 32 x 32 x 16 products whose 13 % fewer clocks took the same time.
-template <class DT, int E, int EV, int NS, bool PRE, int NW, int PAR, bool STREAM, bool KEEP>
+template <class DT, int E, int EV, int NS, bool PRE, int NW, int PAR, bool STREAM, bool KEEP, bool AHEAD>
 __global__ __launch_bounds__(NW * 64, 1) void attention_wide_kernel(const KernelArgs args) {
     typedef Geo<DT, E, EV> G;
     constexpr int NT = NW * 64;                 // threads per workgroup
@@ -325,14 +325,14 @@ __global__ __launch_bounds__(NW * 64, 1) void attention_wide_kernel(const Kernel
     // chunks of several workers, which open a row group and two or three fragments per workgroup and row group (D = 128, bf16 and fp16, us
     // a layer): 2 x 574 tokens behind 1333 at 40/8 heads 86 -> 83, 2 x 799 behind 791 109 -> 104, 2 x 657 behind 75 at 32/8 58 -> 55; 50 calls
     // of 2 to 4 workers 0.99 to 1.05 times as fast, 1.017 in the mean.  Pre-rotated, 7 x 6 tokens: 26.2 -> 24.9 (40/8), 29.2 -> 28.1
-    // (28/4).  Not where it costs more than it hides: with one or two openings a launch (the other fused calls, 0.95 to 0.99 times),
-    // at D = 64 (0.94 to 0.98: half the arithmetic a tile beside the same scalar work) and 256 (0.97 to 0.99: a barrier per tile).
-    constexpr bool AHEAD = E <= 128 && (PRE || (STREAM && E == 128));
-    typedef WideQueries<DT, LANES ? 128 : E, PRE, NW> WQ;         // (not used at head dimension 256)
+    // (28/4).  Not at head dimension 256 (0.97 to 0.99 times as fast: a barrier per tile); openings_ahead says which of the other calls
+    // take it.
+    static_assert(!AHEAD || E == 128, "head dimension 128 only (openings_ahead)");
+    typedef WideQueries<DT, LANES ? 128 : E, PRE, NW> WQ;         // (used where AHEAD is)
     typedef WideRotation<DT, E, G::QSTR, NT> WRot;
     __shared__ __attribute__((aligned(16))) char q_lds[LANES ? 16 : WIDE_ROWS * (AHEAD ? G::KROW : G::QSTR)];
     __shared__ int lim_lds[LANES ? 1 : WIDE_ROWS];        // the rows' bounds, with AHEAD their locations
-    __shared__ __attribute__((aligned(16))) float cs_lds[PRE || LANES ? 4 : WQ::CS_FLOATS];
+    __shared__ __attribute__((aligned(16))) float cs_lds[PRE || LANES ? 4 : AHEAD ? WQ::CS_FLOATS : WRot::CS_FLOATS];
     // ring slots: [K image | V image]; K is swizzled like in the narrow kernel, V is a plain row-major image
     __shared__ __attribute__((aligned(16))) char ring[NS * SLOT];
 
@@ -804,7 +804,7 @@ __global__ __launch_bounds__(NW * 64, 1) void attention_wide_kernel(const Kernel
             w0 = r0 + rw * WROWS;
             ws_lo = fast_div(r0, a.magic_gq);
             nws = fast_div(min(r0 + WIDE_ROWS, a.R) - 1, a.magic_gq) - ws_lo + 1;
-            staged = !LANES && nws <= WRot::CSMAX;
+            staged = !PRE && !LANES && nws <= WRot::CSMAX;
             int tids = tid;
             if constexpr (STREAM) asm volatile("" : "+v"(tids));      // (see open_segment)
             if (staged) wrot.load_queries(a, hkv, r0, GQ, tids);
@@ -824,6 +824,7 @@ __global__ __launch_bounds__(NW * 64, 1) void attention_wide_kernel(const Kernel
         int f = 0, L = 0, lt0 = 0, lt1 = 0;
         bool opens_fragment = false;
         u32x4 view = {0, 0, 0, 0};                               // this wave's image of the current fragment (K or V slice)
+        [[maybe_unused]] QueryRotation<DT, E, WIDE_ROWS, G::QSTR, true, NT> qrot;     // pre-rotated queries: a copy into LDS
         [[maybe_unused]] LaneRotation<DT, E, RB, PRE> lrot;
         int lm = 0;
 
@@ -864,6 +865,8 @@ __global__ __launch_bounds__(NW * 64, 1) void attention_wide_kernel(const Kernel
             if constexpr (LANES) {
                 lrot.load(a, f, hkv, w0, GQ, tids & 15, (tids >> 4) & 3);
                 return;
+            } else if constexpr (PRE) {
+                qrot.load(a, f, hkv, r0, GQ, tids);
             } else if (staged) {
                 if (!queries_requested) wrot.load_queries(a, hkv, r0, GQ, tids);
                 wrot.load_tables(a, f, tids, ws_lo, nws);
@@ -895,7 +898,7 @@ __global__ __launch_bounds__(NW * 64, 1) void attention_wide_kernel(const Kernel
             } else {
             int limv = (r0 + tids / TPR < a.R) ? min(L, max(0, lm + 1)) : 0x7fffffff;   // by every thread, see paged_wide_kernel
             asm volatile("" : "+v"(limv));
-            if (staged) {
+            if (!PRE && staged) {
                 wrot.stage(cs_lds, tids, nws);
                 if (hw_first) HW_MARK(13);
                 // The barrier above has waited for every load of open_segment: the other look-ahead steps can be requested
@@ -906,6 +909,8 @@ __global__ __launch_bounds__(NW * 64, 1) void attention_wide_kernel(const Kernel
                 asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
                 if (hw_first) HW_MARK(14);
                 wrot.rotate(a, q_lds, cs_lds, f, hkv, r0, GQ, a.rq != nullptr && opens_fragment, tids, ws_lo);
+            } else if constexpr (PRE) {
+                qrot.finish(a, q_lds, f, hkv, r0, GQ, false, tids);
             } else {
                 // too many (worker, token) pairs for the staged tables (GQA ratio below 4): every row loads its own table row,
                 // here and not ahead of time in open_segment, so that the registers of this path are not held across the tile
@@ -941,7 +946,7 @@ __global__ __launch_bounds__(NW * 64, 1) void attention_wide_kernel(const Kernel
             }
             maxlim = __builtin_amdgcn_readfirstlane(row_max16(maxlim));
             minlim = __builtin_amdgcn_readfirstlane(row_min16(minlim));
-            if (!LANES && !staged) {
+            if (!LANES && (PRE || !staged)) {
 #pragma unroll
                 for (int i = 1; i < DP; ++i) request(i, lt0 + i * PAR);
             }
@@ -1655,7 +1660,7 @@ template <class DT>
 static hipError_t launch_wide_256(const KernelArgs& ka, hipStream_t stream) {
     if (!(ka.h.flags & KH_STREAM)) return hipErrorInvalidValue;
     auto go = [&](auto pre, auto keep) {
-        hipLaunchKernelGGL((attention_wide_kernel<DT, 256, 256, WIDE256_SLOTS, decltype(pre)::value, WIDE256_WAVES, 1, true, decltype(keep)::value>),
+        hipLaunchKernelGGL((attention_wide_kernel<DT, 256, 256, WIDE256_SLOTS, decltype(pre)::value, WIDE256_WAVES, 1, true, decltype(keep)::value, false>),
                            dim3(ka.h.nwg), dim3(WIDE256_WAVES * 64), 0, stream, ka);
     };
     auto by_keep = [&](auto pre) {
@@ -1674,13 +1679,19 @@ static hipError_t launch_wide_dt(const KernelArgs& ka, int E, hipStream_t stream
     constexpr int PAR = WIDE_PAR;
     if (E == 256) return launch_wide_256<DT>(ka, stream);
     if (E != 64 && E != 128) return hipErrorInvalidValue;
-    auto go = [&](auto head_dim, auto pre, auto stream_runs) {
+    auto launch = [&](auto head_dim, auto pre, auto stream_runs, auto ahead) {
         constexpr int HD = decltype(head_dim)::value;
-        constexpr bool PRE = decltype(pre)::value, STREAM = decltype(stream_runs)::value;
+        constexpr bool PRE = decltype(pre)::value, STREAM = decltype(stream_runs)::value, AHEAD = decltype(ahead)::value;
         if (ka.h.flags & KH_KEEP)
-            hipLaunchKernelGGL((attention_wide_kernel<DT, HD, HD, NS, PRE, NW, PAR, STREAM, true>), dim3(ka.h.nwg), dim3(NW * 64), 0, stream, ka);
+            hipLaunchKernelGGL((attention_wide_kernel<DT, HD, HD, NS, PRE, NW, PAR, STREAM, true, AHEAD>), dim3(ka.h.nwg), dim3(NW * 64), 0, stream, ka);
         else
-            hipLaunchKernelGGL((attention_wide_kernel<DT, HD, HD, NS, PRE, NW, PAR, STREAM, false>), dim3(ka.h.nwg), dim3(NW * 64), 0, stream, ka);
+            hipLaunchKernelGGL((attention_wide_kernel<DT, HD, HD, NS, PRE, NW, PAR, STREAM, false, AHEAD>), dim3(ka.h.nwg), dim3(NW * 64), 0, stream, ka);
+    };
+    auto go = [&](auto head_dim, auto pre, auto stream_runs) {
+        if constexpr (decltype(head_dim)::value == 128 && (decltype(pre)::value || decltype(stream_runs)::value)) {      // (the forms that openings_ahead may choose)
+            if (ka.h.flags & KH_AHEAD) return launch(head_dim, pre, stream_runs, std::true_type{});
+        }
+        launch(head_dim, pre, stream_runs, std::false_type{});
     };
     auto by_entry = [&](auto head_dim, auto stream_runs) {
         if (ka.h.flags & KH_PREROTATED) go(head_dim, std::true_type{}, stream_runs);

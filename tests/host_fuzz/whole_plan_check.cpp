@@ -71,6 +71,32 @@ static int seen_tiles() {
     return ok ? 0 : 1;
 }
 
+// Does a call prepare its openings ahead?
+static bool ahead(int D, int W, int S, int Hq, int Hkv, std::vector<int32_t> len, bool prerotated) {
+    hw_problem p{};
+    p.dtype = HW_BF16;
+    p.F = (int)len.size();
+    p.W = W; p.S = S; p.Hq = Hq; p.Hkv = Hkv;
+    p.E = p.Ev = p.RotE = D;
+    p.len = len.data();
+    hw::host::CallPlan cp;
+    hw::host::WholePlan wp;
+    hw::host::StreamPlan sp;
+    if (hw::host::plan_call(&p, 256, &cp, 1) != HW_OK) return false;
+    const bool whole = hw::host::whole_size(&p, 256, cp, &wp);
+    return hw::host::openings_ahead(&p, cp.plan[0], prerotated, whole || hw::host::stream_size(&p, 256, cp, &sp), whole ? &wp : nullptr);
+}
+
+// Where that pays: at head dimension 128.
+static int openings() {
+    const bool ok = !ahead(64, 4, 32, 32, 8, {4781, 131, 350, 32, 1577}, true) && !ahead(64, 6, 64, 8, 2, {840, 166, 692, 1162, 64, 64, 64}, true) &&
+                    !ahead(64, 1, 1400, 40, 8, {350, 1400}, false) && !ahead(256, 1, 1024, 16, 8, {4096, 1024}, false) &&
+                    ahead(128, 4, 20, 64, 8, {3000, 205, 205, 205, 205}, true) && ahead(128, 1, 1024, 40, 8, {4096, 1024}, false) &&
+                    ahead(128, 2, 657, 32, 8, {75, 657, 657}, false) && !ahead(128, 4, 4, 64, 8, {8192, 2048, 2048, 2048, 2048}, false);
+    if (!ok) std::printf("failed: openings ahead\n");
+    return ok ? 0 : 1;
+}
+
 // Paged queries of head dimension 256: K/V tiles are kept with more than two row groups of 16 a sequence, packed ones with more than
 // 20 rows in the mean.
 static int kept_tiles() {
@@ -95,6 +121,7 @@ static int kept_tiles() {
 int main() {
     if (kept_tiles() != 0) return 1;
     if (seen_tiles() != 0) return 1;
+    if (openings() != 0) return 1;
     if (rounds_instead() != 0) return 1;
     if (head_dim_256() != 0) return 1;
     std::mt19937 rng(7);
