@@ -434,8 +434,22 @@ static bool causal_chunk(const hw_problem* p) {
 // that was measured to pay.  At 64 a tile is half the arithmetic beside the same scalar work: pre-rotated queries of 1 to 8 workers and
 // 2 to 200 tokens at four head layouts took 1.00 to 1.035 times as long, 1.018 in the mean of 26 calls (4 workers x 32 tokens behind 4781
 // at 32/8 heads, fp16, 22.2 -> 21.5 us a layer without), prompt chunks 1.02 to 1.06.
-bool openings_ahead(const hw_problem* p, const hw_plan&, bool prerotated, bool stream_runs, const WholePlan*) {
-    return p->E == 128 && (prerotated || stream_runs);
+// With one or two openings a workgroup there is little to hide, and the opening itself is longer.  bf16, how many times as fast:
+//   whole row groups, one for each workgroup and none left over: 0.954 to 0.991 below 64 tiles (512 tokens from nothing at 64/8 heads
+//     17.4 against 18.1 us a layer, 802 behind 479 at 40/8 31.8 against 32.4; three of 16 calls gained, up to 1.015), 0.99 to 1.034 from
+//     there on, 1.009 in the mean of 17; with a second one each 1.015 to 1.08, with a remainder to deal 0.985 to 1.55 (it is dealt for
+//     this form);
+//   runs alone: 0.970 to 1.038 with up to three fragments, 0.992 in the mean of 49 calls, 0.997 in the mean of 21 with four and five,
+//     0.982 to 1.054 with six and more, 1.007 in the mean of 40.
+// Pre-rotated queries have no rotation to wait for: 1.007 to 1.22 in whole row groups and in runs; in rounds 1.00 to 1.11 with three
+// fragments or a workgroup to a row group, but for two calls of 0.98; with one opening a workgroup 0.974 to 1.03, 0.997 in the mean of ten.
+bool openings_ahead(const hw_problem* p, const hw_plan& plan, bool prerotated, bool stream_runs, const WholePlan* whole) {
+    if (p->E != 128) return false;
+    int nf = 0;
+    for (int f = 0; f < p->F; ++f) nf += p->len[f] > 0 ? 1 : 0;
+    if (prerotated) return stream_runs || nf > 2 || plan.wgs_per_head == 1;
+    if (whole != nullptr) return whole->split > 0 || whole->whole > whole->wgs || plan.tiles_per_head >= 64;
+    return stream_runs && nf >= 6;
 }
 
 // The remainder in runs: the smallest share (tiles, with openings) at which the workgroups, taking one after the other what fits,

@@ -87,12 +87,17 @@ static bool ahead(int D, int W, int S, int Hq, int Hkv, std::vector<int32_t> len
     return hw::host::openings_ahead(&p, cp.plan[0], prerotated, whole || hw::host::stream_size(&p, 256, cp, &sp), whole ? &wp : nullptr);
 }
 
-// Where that pays: at head dimension 128.
+// Where that pays: at head dimension 128, with more than one or two openings a workgroup.
 static int openings() {
     const bool ok = !ahead(64, 4, 32, 32, 8, {4781, 131, 350, 32, 1577}, true) && !ahead(64, 6, 64, 8, 2, {840, 166, 692, 1162, 64, 64, 64}, true) &&
                     !ahead(64, 1, 1400, 40, 8, {350, 1400}, false) && !ahead(256, 1, 1024, 16, 8, {4096, 1024}, false) &&
                     ahead(128, 4, 20, 64, 8, {3000, 205, 205, 205, 205}, true) && ahead(128, 1, 1024, 40, 8, {4096, 1024}, false) &&
-                    ahead(128, 2, 657, 32, 8, {75, 657, 657}, false) && !ahead(128, 4, 4, 64, 8, {8192, 2048, 2048, 2048, 2048}, false);
+                    ahead(128, 2, 657, 32, 8, {75, 657, 657}, false) && !ahead(128, 4, 4, 64, 8, {8192, 2048, 2048, 2048, 2048}, false) &&
+                    !ahead(128, 1, 512, 64, 8, {512}, false) && !ahead(128, 1, 802, 40, 8, {479, 802}, false) && ahead(128, 1, 819, 40, 8, {5000, 819}, false) &&
+                    ahead(128, 1, 528, 64, 8, {528}, false) && ahead(128, 1, 1020, 64, 8, {70, 1020}, false) && ahead(128, 1, 512, 64, 8, {512}, true) &&
+                    !ahead(128, 1, 655, 28, 4, {817, 655}, false) && !ahead(128, 2, 317, 28, 4, {1202, 620, 317}, false) && ahead(128, 1, 663, 28, 4, {3204, 795}, true) &&
+                    ahead(128, 8, 76, 32, 4, {1249, 76, 76, 76, 76, 76, 76, 76, 76}, false) && !ahead(128, 1, 110, 40, 8, {114, 110}, true) &&
+                    ahead(128, 1, 555, 32, 8, {37, 555}, true);
     if (!ok) std::printf("failed: openings ahead\n");
     return ok ? 0 : 1;
 }
