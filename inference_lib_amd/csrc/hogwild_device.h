@@ -143,6 +143,12 @@ __device__ __forceinline__ int row_min16(int v) {
     return min(v, row_dpp<0x140>(v));
 }
 
+// the largest value over the wave (uniform)
+__device__ __forceinline__ int wave_max(int v) {
+    v = row_max16(v);
+    return max(max(__builtin_amdgcn_readlane(v, 0), __builtin_amdgcn_readlane(v, 16)), max(__builtin_amdgcn_readlane(v, 32), __builtin_amdgcn_readlane(v, 48)));
+}
+
 // inclusive sum over the wave's lanes
 __device__ __forceinline__ int wave_scan_inclusive(int v) {
     v += __builtin_amdgcn_update_dpp(0, v, 0x111, 0xf, 0xf, false);    // row_shr:1

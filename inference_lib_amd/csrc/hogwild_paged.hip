@@ -40,9 +40,10 @@ namespace hw {
 // launch waiting for those of the longest: append and attention of five sequences of 296 to 10 543 tokens (40/8 heads, D = 128, bf16)
 // 31.7 -> 22.3 us, eight of 210 to 9000 at 32/8 37 -> 24, four of 300 to 11 000 at 16/8 and D = 256 41 -> 28.6, five of 844 to 5868 23.8 -> 22.2.
 // The shares are the smallest bound on the tiles of a workgroup (in steps of the four waves) at which the sequences' workgroups
-// are no more than there are, found by trying one bound in every lane.  Sequences within a fifth of the first one's length keep nsplit
-// each, at no more than before (four of 12 528 tokens 41.4 -> 41.2, eight of 1200 17.0 both): the lengths are read ahead of the queries,
-// which are requested for equal shares, as are the partial sums in the merge.
+// are no more than there are, found by trying one bound in every lane.  Working that out and requesting the queries again takes 0.9 us,
+// a step of the four waves 1.1 to 1.2 (fit over 63 decode steps of 2 to 12 sequences, all head layouts): nsplit each wherever the longest sequence needs two
+// steps at most, or no more than it would need with even shares.  The lengths are read ahead of the queries, which are requested for
+// equal shares, as are the partial sums in the merge.
 struct PagedShare {
     int w, split, ns, slot0;      // sequence, which of its ns workgroups, the first one's slot
     bool found;                   // false: a slot that is left over
@@ -61,21 +62,27 @@ __device__ __forceinline__ PagedShare paged_share(const PagedDevHeader& ph, int 
         for (int s = 0; s < ph.LS; ++s) most = max(most, ph.loc[f * T + w * ph.LS + s]);
         tiles += tiles_to(most, ph.frag_len[f]);
     }
-    // sequences of about the same length keep nsplit each
-    const int first = __builtin_amdgcn_readlane(tiles, 0);
-    if (__ballot(lane < ph.W && (5 * tiles > 6 * first || 6 * tiles < 5 * first)) == 0) return PagedShare{item, split, ph.nsplit, item * ph.nsplit, true};
-    const float mine = lane < ph.W ? (float)tiles : 0.f;
+    if (lane >= ph.W) tiles = 0;
+    // (nothing here depends on the order of the sequences: a sequence's share, and so its result, is the same wherever it is listed)
+    const PagedShare equal = {item, split, ph.nsplit, item * ph.nsplit, true};
     const int slots = ph.W * ph.nsplit, slot = item * ph.nsplit + split;
-    const int all = __builtin_amdgcn_readlane(wave_scan_inclusive(lane < ph.W ? tiles : 0), 63);
+    const int longest = wave_max(tiles);
+    if (longest <= 2 * NWAVES * ph.nsplit) return equal;       // (on its own: short steps leave here, 0.1 us sooner than behind the sum)
+    const int all = __builtin_amdgcn_readlane(wave_scan_inclusive(tiles), 63);
+    const int least = max(1, (int)((float)all * __builtin_amdgcn_rcpf((float)(NWAVES * slots))));          // steps with even shares, less what is left over
+    if (longest <= NWAVES * ph.nsplit * (least + (least * NWAVES * slots < all ? 1 : 0))) return equal;
     // lane = a bound on the tiles of a workgroup, multiples of the four waves: does every sequence get its workgroups?
-    const int least = max(1, (int)((float)all * __builtin_amdgcn_rcpf(4.0f * (float)slots)));
-    const float per = __builtin_amdgcn_rcpf(4.0f * (float)(least + lane * (1 + (least >> 5))));
+    const float mine = (float)tiles;
+    const int bound = NWAVES * (least + lane * (1 + (least >> 5)));
+    const float per = __builtin_amdgcn_rcpf((float)bound);
     auto groups = [&](float t, float per_group) { return max(1, (int)__builtin_ceilf(t * per_group - 0.01f)); };
     int need = 0;
     for (int sq = 0; sq < ph.W; ++sq) need += groups(__int_as_float(__builtin_amdgcn_readlane(__float_as_int(mine), sq)), per);
     const unsigned long long fits = __ballot(need <= slots);
-    const float best = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(per), fits != 0 ? __builtin_ctzll(fits) : 63));
-    int n = lane < ph.W ? (fits != 0 ? groups(mine, best) : ph.nsplit) : 0;
+    const int fit = fits != 0 ? __builtin_ctzll(fits) : 0;
+    if (fits == 0 || longest <= ph.nsplit * __builtin_amdgcn_readlane(bound, fit)) return equal;
+    const float best = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(per), fit));
+    const int n = lane < ph.W ? groups(mine, best) : 0;
     const int slot0 = wave_scan_inclusive(n) - n;
     const unsigned long long owner = __ballot(slot >= slot0 && slot < slot0 + n);
     PagedShare r;

@@ -584,12 +584,6 @@ __global__ __launch_bounds__(NW * 64, 1) void attention_wide_kernel(const Kernel
             }
             return group;
         };
-        // the largest value over the wave (uniform)
-        auto wave_max = [&](int v) {
-            v = row_max16(v);
-            return max(max(__builtin_amdgcn_readlane(v, 0), __builtin_amdgcn_readlane(v, 16)),
-                       max(__builtin_amdgcn_readlane(v, 32), __builtin_amdgcn_readlane(v, 48)));
-        };
         [[maybe_unused]] const unsigned q_base = lds_address(q_lds), cs_base = lds_address(cs_lds), loc_base = lds_address(lim_lds);
         // (the lane as the compiler cannot see through it: what is derived from it -- rows, addresses of the queries -- is then
         // formed where it is used instead of once in front of the loop over the segments, from where it would stay in registers across
@@ -1131,9 +1125,7 @@ __device__ __forceinline__ PlanSlot plan_slot_wave(const PagedDevHeader& ph, int
     const int rounds = G <= fill ? 1 : (G + fill - 1) / fill;
     const int few = min(pslots, rounds * fill), many = min(pslots, few + fill);
     const int all_work = max(__builtin_amdgcn_readlane(wave_scan_inclusive(work), 63), 1);
-    const int row_most = row_max16(work);
-    const int largest = max(max(max(__builtin_amdgcn_readlane(row_most, 0), __builtin_amdgcn_readlane(row_most, 16)),
-                                max(__builtin_amdgcn_readlane(row_most, 32), __builtin_amdgcn_readlane(row_most, 48))), 1);
+    const int largest = max(wave_max(work), 1);
     const float bound = lane == 63 ? (float)largest : (float)all_work * __builtin_amdgcn_rcpf((float)many) * fast_exp2(0.0625f * (float)lane);
     const float per = __builtin_amdgcn_rcpf(bound);
     auto share = [&](int work_, float per_slot) { return max(1, (int)__builtin_ceilf((float)work_ * per_slot - 0.01f)); };

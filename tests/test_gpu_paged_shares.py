@@ -68,6 +68,56 @@ def test_shares_by_length(dtype, lens, S, F, Hq, Hkv, D, bs):
         assert float((lse - ref_lse)[seen].abs().max()) <= 1e-4
 
 
+def _step(lens, dtype, Hq, Hkv, D, bs, mb, seed, splits=0):
+    """One decode step; sequence i has the data of its number in `lens`, a list of (number, length), wherever it is listed."""
+    W, n = len(lens), len(lens) * mb
+    g = torch.Generator(device="cuda").manual_seed(seed)
+    rnd = lambda *shape: torch.randn(shape, generator=g, device="cuda").to(dtype)
+    kc, vc, q = rnd(n, Hkv, bs, D), rnd(n, Hkv, bs, D), rnd(1, W, Hq, 1, D)
+    table = torch.randperm(n, generator=g, device="cuda").to(torch.int32).reshape(W, mb)
+    order = [i for i, _ in lens]
+    loc = torch.tensor([[[m - 1] for _, m in lens]], dtype=torch.int32, device="cuda")
+    out, lse = torch.empty((W, Hq, 1, D), dtype=dtype, device="cuda"), torch.empty((W, Hq, 1), device="cuda")
+    frag = torch.tensor([bs * mb], dtype=torch.int32, device="cuda")
+    _lib.PagedProblem(q=q[:, order].contiguous(), locations=loc, fragment_lengths=frag, key_cache=kc, value_cache=vc, block_table=table[order].contiguous(),
+                      scale=D ** -0.5, out=out, lse=lse, splits=splits).run()
+    back = torch.tensor(order).argsort().cuda()
+    return out[back], lse[back]
+
+
+@pytest.mark.parametrize("dtype,lens,Hq,Hkv,D", [
+    (torch.bfloat16, (9600, 10880, 8160, 8160), 40, 8, 128),      # the first within a fifth of all others, the longest a fifth above the mean
+    (torch.float16, (3000, 3550, 2550, 2550, 2550), 16, 8, 256),
+    (torch.bfloat16, (400, 9000, 2000, 64, 5000, 33), 32, 8, 128),
+    (torch.float32, (300, 4100, 900), 8, 8, 64),
+])
+def test_order_of_the_sequences_does_not_matter(dtype, lens, Hq, Hkv, D):
+    """The same sequences listed in other orders: the same bits for each."""
+    bs, mb = 32, -(-max(lens) // 32) + 1
+    listed = list(enumerate(lens))
+    first = _step(listed, dtype, Hq, Hkv, D, bs, mb, D)
+    for order in (listed[::-1], listed[1:] + listed[:1], sorted(listed, key=lambda x: -x[1])):
+        for a, b in zip(first, _step(order, dtype, Hq, Hkv, D, bs, mb, D)):
+            assert torch.equal(a, b)
+
+
+@pytest.mark.parametrize("dtype,lens,Hq,Hkv,D", [
+    (torch.bfloat16, (1318, 2139, 1454, 101, 419, 62, 2291, 197, 900), 8, 2, 64),      # two steps of a wave: nothing to gain by other shares
+    (torch.bfloat16, (465, 191, 997, 358, 388, 1028, 84, 1466, 456, 213), 28, 4, 128),
+    (torch.float16, (184, 101, 104, 74), 16, 8, 256),
+    (torch.bfloat16, (886, 3433), 40, 8, 128),
+    (torch.bfloat16, (4096, 4000, 4064, 3969), 40, 8, 128),                              # as many steps with even shares
+])
+def test_short_and_even_steps_keep_equal_shares(dtype, lens, Hq, Hkv, D):
+    """The bits of the call whose split is fixed at that of equal shares, which is launched so whatever the lengths."""
+    bs, mb = 32, -(-max(lens) // 32)
+    equal = _lib.paged_plan(W=len(lens), Hq=Hq, Hkv=Hkv, Ev=D, block_size=bs, max_blocks=mb, num_cus=_lib.lib.hw_device_cus(), S=1, dtype=_lib._DTYPE_CODE[dtype])
+    assert equal.splits > 1
+    listed = list(enumerate(lens))
+    for a, b in zip(_step(listed, dtype, Hq, Hkv, D, bs, mb, D), _step(listed, dtype, Hq, Hkv, D, bs, mb, D, splits=equal.splits)):
+        assert torch.equal(a, b)
+
+
 @pytest.mark.parametrize("dtype,Hq,Hkv,D,S", [(torch.bfloat16, 40, 8, 128, 1), (torch.float16, 16, 8, 256, 3), (torch.float32, 8, 8, 128, 1), (torch.float16, 64, 8, 64, 4)])
 def test_caches_of_4_gb_and_more(dtype, Hq, Hkv, D, S):
     """K rows are reached through one buffer descriptor below 4 GB and through 64-bit addresses from there on: the same blocks at the end of
