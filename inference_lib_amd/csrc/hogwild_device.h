@@ -326,6 +326,7 @@ struct WaveState {
     f32x4 o[RB][NOC];
     float m[RB];   // reference of the exponentials (base-2 units): within 2^8 below/above the running max
     float l[RB];   // lane-partial sum: this lane's quarter of the tokens
+    float top[RB]; // running max (kept with compute_tile's FOLLOW only)
     bool fresh;    // no tile accumulated yet (uniform over the wave)
 };
 
@@ -336,10 +337,13 @@ struct WaveState {
 // kernels whose waves share every tile, 16-bit types): the K operands are read first (LDS answers in order, and the
 // logits wait for K only), the V^T operands come straight out of the image (lds_read_tr16, per-lane offsets `voff` from
 // vtr_lane_offsets), and output block c then holds elements 16c .. 16c+15.  `t_in` is not used.
-template <class DT, int E, int EV, int RB, bool MASKED, bool QREG, bool VS = false, bool VLDS = false>
+// FOLLOW = the reference may follow the tiles (`follow`, uniform): it is moved to every tile's maximum, down as well as up, but not
+// further than 2^LAZY_LOG2 below the running one.  The largest weights of a row are then 1 in their tiles, which the storage type holds
+// exactly; otherwise those of a wave's first tile are.
+template <class DT, int E, int EV, int RB, bool MASKED, bool QREG, bool VS = false, bool VLDS = false, bool FOLLOW = false>
 __device__ __forceinline__ void compute_tile(const TileRegs<DT, E, EV>& t_in, const char* q_lds, const u32x4* qreg, const int (&lim)[RB],
                                              WaveState<RB, Geo<DT, E, EV>::NOC>& st, int t0, int n, int q, float sc, const char* kstage,
-                                             const char* vimg = nullptr, const unsigned* voff = nullptr) {
+                                             const char* vimg = nullptr, const unsigned* voff = nullptr, bool follow = false) {
     typedef Geo<DT, E, EV> G;
     const TileRegs<DT, E, EV>& t = t_in;
 #ifdef HW_NO_COMPUTE   // tuning aid: consume the tile without doing the arithmetic
@@ -458,12 +462,16 @@ __device__ __forceinline__ void compute_tile(const TileRegs<DT, E, EV>& t_in, co
         const float mine = MASKED ? (mx < -1.0e29f ? NEG_BIG : mx * sc) : mx * sc;
         need = need || (mine > st.m[rb] + LAZY_LOG2);
     }
-    if (__builtin_amdgcn_ballot_w64(need) != 0) {        // uniform over the wave
+    if ((FOLLOW && follow) || __builtin_amdgcn_ballot_w64(need) != 0) {        // uniform over the wave
 #pragma unroll
         for (int rb = 0; rb < RB; ++rb) {
             const float mx = quarter_max(mxl[rb]);
             const float mxs = MASKED ? (mx < -1.0e29f ? NEG_BIG : mx * sc) : mx * sc;
-            const float mnew = mxs > st.m[rb] + LAZY_LOG2 ? mxs : st.m[rb];
+            float mnew = mxs > st.m[rb] + LAZY_LOG2 ? mxs : st.m[rb];
+            if constexpr (FOLLOW) {
+                st.top[rb] = fmaxf(st.top[rb], mxs);
+                if (follow) mnew = fmaxf(mxs, st.top[rb] - LAZY_LOG2);
+            }
             const float alpha = fast_exp2(st.m[rb] - mnew);   // 1 for rows that keep their reference
             st.m[rb] = mnew;
             st.l[rb] *= alpha;

@@ -44,9 +44,13 @@ namespace hw {
 // a step of the four waves 1.1 to 1.2 (fit over 63 decode steps of 2 to 12 sequences, all head layouts): nsplit each wherever the longest sequence needs two
 // steps at most, or no more than it would need with even shares.  The lengths are read ahead of the queries, which are requested for
 // equal shares, as are the partial sums in the merge.
+// A sequence with fewer workgroups has fewer tiles that are a wave's first, whose largest weight the storage type holds exactly: 1.04 to
+// 1.09 times the error against float64 (nine ragged steps x 6 seeds, bf16 and fp16).  With other than equal shares the reference of the
+// exponentials therefore follows the tiles (compute_tile's FOLLOW), 0.94 to 0.99 times the error of equal shares for 0.1 us.
 struct PagedShare {
     int w, split, ns, slot0;      // sequence, which of its ns workgroups, the first one's slot
     bool found;                   // false: a slot that is left over
+    bool other;                   // not equal shares (the same for every workgroup of the launch)
 };
 // (loc0, len0: the first location of sequence min(lane, W - 1) and the first fragment's length, requested ahead of what the workgroup
 // needs besides, so that this is worked out while the rest is on its way)
@@ -64,7 +68,7 @@ __device__ __forceinline__ PagedShare paged_share(const PagedDevHeader& ph, int 
     }
     if (lane >= ph.W) tiles = 0;
     // (nothing here depends on the order of the sequences: a sequence's share, and so its result, is the same wherever it is listed)
-    const PagedShare equal = {item, split, ph.nsplit, item * ph.nsplit, true};
+    const PagedShare equal = {item, split, ph.nsplit, item * ph.nsplit, true, false};
     const int slots = ph.W * ph.nsplit, slot = item * ph.nsplit + split;
     const int longest = wave_max(tiles);
     if (longest <= 2 * NWAVES * ph.nsplit) return equal;       // (on its own: short steps leave here, 0.1 us sooner than behind the sum)
@@ -86,6 +90,7 @@ __device__ __forceinline__ PagedShare paged_share(const PagedDevHeader& ph, int 
     const int slot0 = wave_scan_inclusive(n) - n;
     const unsigned long long owner = __ballot(slot >= slot0 && slot < slot0 + n);
     PagedShare r;
+    r.other = true;
     r.found = owner != 0;
     r.w = r.found ? __builtin_ctzll(owner) : 0;
     r.slot0 = __builtin_amdgcn_readlane(slot0, r.w);
@@ -152,7 +157,7 @@ __global__ __launch_bounds__(NTHREADS, MINW) void paged_attention_kernel(const P
     WaveState<RB, G::NOC> st;
 #pragma unroll
     for (int rb = 0; rb < RB; ++rb) {
-        st.m[rb] = NEG_BIG;
+        st.m[rb] = st.top[rb] = NEG_BIG;
         st.l[rb] = 0.f;
 #pragma unroll
         for (int c = 0; c < G::NOC; ++c) st.o[rb][c] = f32x4{0.f, 0.f, 0.f, 0.f};
@@ -225,6 +230,7 @@ __global__ __launch_bounds__(NTHREADS, MINW) void paged_attention_kernel(const P
     }
     if (r0 >= rend) return;                 // uniform over the workgroup
     int loc0 = 0, len0 = 0, first_slot = 0;
+    bool other_shares = false;              // than equal ones
     if (shared) {
         loc0 = ph.loc[min(lane, ph.W - 1) * ph.LS];
         len0 = ph.frag_len[0];
@@ -235,6 +241,7 @@ __global__ __launch_bounds__(NTHREADS, MINW) void paged_attention_kernel(const P
         const PagedShare sh = paged_share(ph, item, split, lane, loc0, len0);
         if (!sh.found) return;              // uniform over the workgroup
         first_slot = sh.slot0;
+        other_shares = sh.other;
         if (sh.w != item || sh.split != split || sh.ns != ns) {
             item = sh.w;
             split = sh.split;
@@ -338,14 +345,14 @@ __global__ __launch_bounds__(NTHREADS, MINW) void paged_attention_kernel(const P
                     const int bt_n = bt_load(t + 2 * NW);
                     issue_tile(tr[1], kslots[1], bt_b, t + NW);
                     if constexpr (STATED) wait_k_landed<G, 1>();   // (see wait_k_landed: the table load in between only adds to what is behind)
-                    compute_tile<DT, E, EV, RB, false, QREG>(tr[0], q_lds, qreg, lim, st, t * TILE, n, q, ph.sc, kslots[0]);
+                    compute_tile<DT, E, EV, RB, false, QREG, false, false, G::SZ == 2>(tr[0], q_lds, qreg, lim, st, t * TILE, n, q, ph.sc, kslots[0], nullptr, nullptr, other_shares);
                     bt_a = bt_n;
                 }
                 {
                     const int bt_n = bt_load(t + 3 * NW);
                     issue_tile(tr[0], kslots[0], bt_a, t + 2 * NW);
                     if constexpr (STATED) wait_k_landed<G, 1>();
-                    compute_tile<DT, E, EV, RB, false, QREG>(tr[1], q_lds, qreg, lim, st, (t + NW) * TILE, n, q, ph.sc, kslots[1]);
+                    compute_tile<DT, E, EV, RB, false, QREG, false, false, G::SZ == 2>(tr[1], q_lds, qreg, lim, st, (t + NW) * TILE, n, q, ph.sc, kslots[1], nullptr, nullptr, other_shares);
                     bt_b = bt_n;
                 }
             }
@@ -355,8 +362,8 @@ __global__ __launch_bounds__(NTHREADS, MINW) void paged_attention_kernel(const P
                     issue_tile(tr[1], kslots[1], bt_b, t + NW);
                     if constexpr (STATED) wait_k_landed<G, 1>();
                     const int t0 = t * TILE;
-                    if (G::SZ == 4 && t0 + TILE <= minlim) compute_tile<DT, E, EV, RB, false, QREG>(tr[0], q_lds, qreg, lim, st, t0, n, q, ph.sc, kslots[0]);
-                    else compute_tile<DT, E, EV, RB, true, QREG>(tr[0], q_lds, qreg, lim, st, t0, n, q, ph.sc, kslots[0]);
+                    if (G::SZ == 4 && t0 + TILE <= minlim) compute_tile<DT, E, EV, RB, false, QREG, false, false, G::SZ == 2>(tr[0], q_lds, qreg, lim, st, t0, n, q, ph.sc, kslots[0], nullptr, nullptr, other_shares);
+                    else compute_tile<DT, E, EV, RB, true, QREG, false, false, G::SZ == 2>(tr[0], q_lds, qreg, lim, st, t0, n, q, ph.sc, kslots[0], nullptr, nullptr, other_shares);
                     bt_a = bt_n;
                 }
                 {
@@ -364,8 +371,8 @@ __global__ __launch_bounds__(NTHREADS, MINW) void paged_attention_kernel(const P
                     issue_tile(tr[0], kslots[0], bt_a, t + 2 * NW);
                     if constexpr (STATED) wait_k_landed<G, 1>();
                     const int t0 = (t + NW) * TILE;
-                    if (G::SZ == 4 && t0 + TILE <= minlim) compute_tile<DT, E, EV, RB, false, QREG>(tr[1], q_lds, qreg, lim, st, t0, n, q, ph.sc, kslots[1]);
-                    else if (t0 < maxlim) compute_tile<DT, E, EV, RB, true, QREG>(tr[1], q_lds, qreg, lim, st, t0, n, q, ph.sc, kslots[1]);
+                    if (G::SZ == 4 && t0 + TILE <= minlim) compute_tile<DT, E, EV, RB, false, QREG, false, false, G::SZ == 2>(tr[1], q_lds, qreg, lim, st, t0, n, q, ph.sc, kslots[1], nullptr, nullptr, other_shares);
+                    else if (t0 < maxlim) compute_tile<DT, E, EV, RB, true, QREG, false, false, G::SZ == 2>(tr[1], q_lds, qreg, lim, st, t0, n, q, ph.sc, kslots[1], nullptr, nullptr, other_shares);
                     bt_b = bt_n;
                 }
             }

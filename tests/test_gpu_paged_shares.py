@@ -68,14 +68,17 @@ def test_shares_by_length(dtype, lens, S, F, Hq, Hkv, D, bs):
         assert float((lse - ref_lse)[seen].abs().max()) <= 1e-4
 
 
-def _step(lens, dtype, Hq, Hkv, D, bs, mb, seed, splits=0):
-    """One decode step; sequence i has the data of its number in `lens`, a list of (number, length), wherever it is listed."""
+def _step(lens, dtype, Hq, Hkv, D, bs, mb, seed, splits=0, change=None):
+    """One decode step; sequence i has the data of its number in `lens`, a list of (number, length), wherever it is listed.
+    change(q, keys, values, table) alters the data."""
     W, n = len(lens), len(lens) * mb
     g = torch.Generator(device="cuda").manual_seed(seed)
     rnd = lambda *shape: torch.randn(shape, generator=g, device="cuda").to(dtype)
     kc, vc, q = rnd(n, Hkv, bs, D), rnd(n, Hkv, bs, D), rnd(1, W, Hq, 1, D)
     table = torch.randperm(n, generator=g, device="cuda").to(torch.int32).reshape(W, mb)
     order = [i for i, _ in lens]
+    if change is not None:
+        change(q, kc, vc, table)
     loc = torch.tensor([[[m - 1] for _, m in lens]], dtype=torch.int32, device="cuda")
     out, lse = torch.empty((W, Hq, 1, D), dtype=dtype, device="cuda"), torch.empty((W, Hq, 1), device="cuda")
     frag = torch.tensor([bs * mb], dtype=torch.int32, device="cuda")
@@ -116,6 +119,53 @@ def test_short_and_even_steps_keep_equal_shares(dtype, lens, Hq, Hkv, D):
     listed = list(enumerate(lens))
     for a, b in zip(_step(listed, dtype, Hq, Hkv, D, bs, mb, D), _step(listed, dtype, Hq, Hkv, D, bs, mb, D, splits=equal.splits)):
         assert torch.equal(a, b)
+
+
+@pytest.mark.parametrize("dtype,lens,Hq,Hkv,D", [
+    (torch.bfloat16, (8989, 493, 7242, 1180, 231, 1815, 3425, 8850), 32, 8, 128),
+    (torch.float16, (2194, 3461, 4600, 1232, 2019, 6230, 2042, 395), 16, 8, 256),
+    (torch.bfloat16, (895, 7978, 64), 64, 8, 128),
+    (torch.float16, (2852, 3640, 4675, 11537, 220, 2552, 4251, 578), 8, 2, 64),
+])
+def test_shares_cost_no_precision(dtype, lens, Hq, Hkv, D):
+    """Short sequences get fewer workgroups than with equal shares, so fewer of their weights are the largest of a wave's first tile, which
+    the storage type holds exactly; the reference follows the tiles instead, and every tile's largest is exact: no further from float64
+    than equal shares, which hold a part of those."""
+    bs, mb, kept = 32, -(-max(lens) // 32), []
+    listed = list(enumerate(lens))
+    equal = _lib.paged_plan(W=len(lens), Hq=Hq, Hkv=Hkv, Ev=D, block_size=bs, max_blocks=mb, num_cus=_lib.lib.hw_device_cus(), S=1, dtype=_lib._DTYPE_CODE[dtype])
+    shared, _ = _step(listed, dtype, Hq, Hkv, D, bs, mb, D, change=lambda *data: kept.extend(data))
+    fixed, _ = _step(listed, dtype, Hq, Hkv, D, bs, mb, D, splits=equal.splits)
+    assert not torch.equal(shared, fixed)
+    q, kc, vc, table = kept
+    ref = torch.empty(shared.shape, dtype=torch.float64, device="cuda")
+    for w, n in listed:
+        rows = table[w, : -(-n // bs)].long()
+        k, v = (c[rows].transpose(1, 2).reshape(-1, Hkv, D)[:n].double() for c in (kc, vc))
+        for h in range(Hq):
+            ref[w, h] = torch.softmax(q[0, w, h].double() @ k[:, h // (Hq // Hkv)].t().contiguous() * D ** -0.5, dim=1) @ v[:, h // (Hq // Hkv)]
+    assert float((shared.double() - ref).norm()) <= float((fixed.double() - ref).norm())
+
+
+@pytest.mark.parametrize("dtype,Hq,Hkv,D", [(torch.bfloat16, 40, 8, 128), (torch.float16, 16, 8, 256)])
+def test_infinite_logits_under_shares(dtype, Hq, Hkv, D):
+    """Logits of minus infinity (one, a whole tile, a sequence's first tiles) weigh nothing, as with equal shares."""
+    lens, bs = (700, 6000, 90, 2500), 32
+    mb, listed = -(-max(lens) // bs), list(enumerate(lens))
+
+    def change(q, kc, vc, table):
+        q.abs_()
+        for w, block, row in ((0, 3, 5), (3, 1, slice(None)), (1, 0, slice(None)), (1, 1, slice(None)), (2, 1, 3)):
+            kc[int(table[w, block]), :, row] = float("-inf")
+
+    equal = _lib.paged_plan(W=len(lens), Hq=Hq, Hkv=Hkv, Ev=D, block_size=bs, max_blocks=mb, num_cus=_lib.lib.hw_device_cus(), S=1, dtype=_lib._DTYPE_CODE[dtype])
+    out, lse = _step(listed, dtype, Hq, Hkv, D, bs, mb, 3, change=change)
+    want, want_lse = _step(listed, dtype, Hq, Hkv, D, bs, mb, 3, splits=equal.splits, change=change)
+    assert not torch.equal(out, want) and bool(torch.isfinite(out).all())
+    # the probabilities and the results of two launches, each rounded once; |values| < 6
+    u = {torch.bfloat16: 2.0 ** -8, torch.float16: 2.0 ** -11}[dtype]
+    assert float((out.double() - want.double()).abs().max()) <= 4 * u * 6.0
+    assert float((lse - want_lse).abs().max()) <= 1e-4
 
 
 @pytest.mark.parametrize("dtype,Hq,Hkv,D,S", [(torch.bfloat16, 40, 8, 128, 1), (torch.float16, 16, 8, 256, 3), (torch.float32, 8, 8, 128, 1), (torch.float16, 64, 8, 64, 4)])
