@@ -467,6 +467,11 @@ void whole_deal(const hw_problem* p, const CallPlan& cp, WholePlan* wp) {
     const hw_plan& plan = cp.plan[0];
     const int T = plan.tiles_per_head, wgs = wp->wgs, split = wp->split;
     StreamPlan& sp = wp->runs;
+    if (split == 0) {
+        std::fill(sp.wg_tile_begin, sp.wg_tile_begin + HW_MAX_SPLITS + 1, 0);
+        sp.max_pieces = 0;
+        return;
+    }
     int nf = 0, last = 0;
     for (int f = 0; f < p->F; ++f) {
         if (p->len[f] == 0) continue;
@@ -485,38 +490,42 @@ void whole_deal(const hw_problem* p, const CallPlan& cp, WholePlan* wp) {
         return plan.tile_begin[last] + (p->len[last] - p->S + token + hw::TILE) / hw::TILE;
     };
     const double per_tile = 1.0 / tile;
+    // (Both once and not in every step of the bisection: their divisions were most of its time.)
+    int seen_of[HW_MAX_SPLITS];                              // of the row groups to deal, fewer than there are workgroups
+    double low = 0.0, unseen = 0.0;
+    for (int rg = 0; rg < split; ++rg) {
+        seen_of[rg] = seen_tiles(rg);
+        low += kPieceCost + seen_of[rg] * tile;
+        unseen += trimmed ? 0 : T - seen_of[rg];
+    }
     // what workgroup g has in hand with the row groups that are its alone, above workgroup 0 (later row groups see more)
-    const int own = wp->whole / wgs;
-    auto ahead = [&](int g) {
-        int more = 0;
-        for (int i = 0; i < (trimmed ? own : 0); ++i) more += seen_tiles(split + i * wgs + g) - seen_tiles(split + i * wgs);
-        return more * tile;
-    };
+    double ahead[HW_MAX_SPLITS];
+    const int own = trimmed && by_seen ? wp->whole / wgs : 0;
+    std::fill(ahead, ahead + wgs, 0.0);
+    for (int i = 0; i < own; ++i) {
+        const int first = seen_tiles(split + i * wgs);
+        for (int g = 1; g < wgs; ++g) ahead[g] += (seen_tiles(split + i * wgs + g) - first) * tile;
+    }
     auto deal = [&](double share) {                          // false if something is left
-        int rg = 0, t = 0, seen = seen_tiles(0);
+        int rg = 0, t = 0;
         for (int g = 0; g < wgs; ++g) {
             sp.wg_tile_begin[g] = rg * T + t;
-            for (double room = share - ahead(g); rg < split;) {
-                const int take = std::min((int)((room - kPieceCost) * per_tile), seen - t);
-                if (take < std::min(kMinPiece, seen - t)) break;
+            for (double room = share - ahead[g]; rg < split;) {
+                const int rest = seen_of[rg] - t, take = std::min((int)((room - kPieceCost) * per_tile), rest);
+                if (take < std::min(kMinPiece, rest)) break;
                 room -= kPieceCost + take * tile;
                 t += take;
-                if (t < seen) break;
-                if (!trimmed) room -= T - seen;
+                if (take < rest) break;
+                if (!trimmed) room -= T - seen_of[rg];
                 t = 0;
-                if (++rg < split) seen = seen_tiles(rg);
+                ++rg;
             }
         }
         return rg == split;
     };
     // Between an equal part of the tiles seen and that of all with what a workgroup opens and leaves at most besides.
-    double low = 0.0, unseen = 0.0;
-    for (int rg = 0; rg < split; ++rg) {
-        low += kPieceCost + seen_tiles(rg) * tile;
-        unseen += trimmed ? 0 : T - seen_tiles(rg);
-    }
     low /= wgs;
-    double high = low + unseen / wgs + ahead(wgs - 1) + 2.0 * kPieceCost + (kMinPiece + 1) * tile;
+    double high = low + unseen / wgs + ahead[wgs - 1] + 2.0 * kPieceCost + (kMinPiece + 1) * tile;
     while (!deal(high)) high *= 2.0;
     while (high - low > 0.25) {
         const double mid = 0.5 * (low + high);

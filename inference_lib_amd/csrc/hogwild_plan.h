@@ -65,9 +65,9 @@ struct WholePlan {
     size_t workspace_bytes;
 };
 bool whole_size(const hw_problem* p, int num_cus, const CallPlan& cp, WholePlan* wp);
-// Every call of the kind deals about nine times over row groups and workgroups until the share is found: 0.9 us on the host with 8 row
-// groups left for 32 workgroups, 4.0 with 47 for 128, 12 with 94 for one kv head's 256 (1.9, 12 and 27 when the bisection began at all
-// of the work for one workgroup and the pieces were counted for every pair).  Sizing takes 0.02.
+// Every call of the kind deals about ten times over row groups and workgroups until the share is found: 2.0 us on the host with 8 row
+// groups left for 32 workgroups, 2.4 with 17 for 64, 29 with 213 for one kv head's 256 (5.2, 6.2 and 39 when what a workgroup has in
+// hand and sees was worked out again in every one of them).  Sizing takes 0.02.
 void whole_deal(const hw_problem* p, const CallPlan& cp, WholePlan* wp);
 // Whether whole_deal counts the tiles that a causal chunk sees (hogwild_plan.cpp).
 bool deal_by_seen(const hw_problem* p, const CallPlan& cp, const WholePlan& wp);

@@ -18,3 +18,15 @@ def test_workgroups_open_only_row_groups_that_exist(tmp_path):
                    check=True)
     r = subprocess.run([str(exe)], capture_output=True, text=True, timeout=300)
     assert r.returncode == 0, r.stdout + r.stderr
+
+
+def test_the_deal_is_the_rule_in_less_time(tmp_path):
+    if shutil.which("g++") is None:
+        pytest.skip("no g++")
+    exe = tmp_path / "whole_deal_check"
+    csrc = os.path.join(ROOT, "inference_lib_amd", "csrc")
+    subprocess.run(["g++", "-std=c++17", "-O2", "-I", os.path.join(ROOT, "include"), "-I", csrc,
+                    os.path.join(ROOT, "tests", "host_fuzz", "whole_deal_check.cpp"), os.path.join(csrc, "hogwild_plan.cpp"), "-o", str(exe)],
+                   check=True)
+    r = subprocess.run([str(exe)], capture_output=True, text=True, timeout=300)
+    assert r.returncode == 0, r.stdout + r.stderr
