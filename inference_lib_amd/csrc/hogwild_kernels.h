@@ -75,7 +75,7 @@ struct MergeArgs {
     int xcd_local;      // kv head h was computed on XCD h / (Hkv/8): merge it there
     // Partials laid out by workgroup slot instead of by row (KH_STREAM, and the paged launches that are dealt on the device,
     // see PagedHeader): row_tab[kv head][r] = {first slot | slots << 16, row within the slot}, a slot holds slot_rows rows (PLAN_SLOT_ROWS without guess), pslots
-    // slots per kv head; wgs_per_head then only bounds the slots of a row (for the choice of the merge kernel's shape).
+    // slots per kv head; wgs_per_head then is what most rows have (for the choice of the merge kernel's shape).
     const int* row_tab;
     int pslots, slot_rows;
     int guess;          // > 0: slots of a row where every slot_rows rows have the same number, one behind the other; requested ahead of the table

@@ -324,12 +324,12 @@ void stream_deal(const hw_problem* p, const CallPlan& cp, StreamPlan* sp) {
     }
     sp->wgs = wg + 1;
     for (int i = sp->wgs; i <= HW_MAX_SPLITS; ++i) sp->wg_tile_begin[i] = nrg * T;
-    sp->max_pieces = 1;
+    sp->max_pieces = sp->usual_pieces = 1;
     for (int rg = 0, g = 0; rg < nrg; ++rg) {
         while (sp->wg_tile_begin[g + 1] <= rg * T) ++g;
         int last = g;
         while (sp->wg_tile_begin[last + 1] < (rg + 1) * T) ++last;
-        if (last - g + 1 > sp->max_pieces) sp->max_pieces = last - g + 1;
+        if (last - g + 1 > sp->max_pieces) sp->max_pieces = sp->usual_pieces = last - g + 1;
     }
 }
 
@@ -469,7 +469,7 @@ void whole_deal(const hw_problem* p, const CallPlan& cp, WholePlan* wp) {
     StreamPlan& sp = wp->runs;
     if (split == 0) {
         std::fill(sp.wg_tile_begin, sp.wg_tile_begin + HW_MAX_SPLITS + 1, 0);
-        sp.max_pieces = 0;
+        sp.max_pieces = sp.usual_pieces = 0;
         return;
     }
     int nf = 0, last = 0;
@@ -534,12 +534,15 @@ void whole_deal(const hw_problem* p, const CallPlan& cp, WholePlan* wp) {
     deal(high);
     for (int i = wgs; i <= HW_MAX_SPLITS; ++i) sp.wg_tile_begin[i] = split * T;
     sp.max_pieces = 0;
+    int pieces = 0;
     for (int rg = 0, g = 0; rg < split; ++rg) {
         while (sp.wg_tile_begin[g + 1] <= rg * T) ++g;
         int last = g;
         while (sp.wg_tile_begin[last + 1] < (rg + 1) * T) ++last;
         sp.max_pieces = std::max(sp.max_pieces, last - g + 1);
+        pieces += last - g + 1;
     }
+    sp.usual_pieces = (pieces + split / 2) / split;
 }
 
 size_t call_workspace_bytes(const hw_problem* p, int num_cus, const CallPlan& cp) {

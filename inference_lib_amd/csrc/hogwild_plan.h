@@ -44,7 +44,7 @@ int plan_call(const hw_problem* p, int num_cus, CallPlan* cp, int fused);
 struct StreamPlan {
     int wgs;                             // workgroups per kv head
     int slots;                           // partial slots of PLAN_SLOT_ROWS rows per kv head, not all of them used
-    int max_pieces;                      // pieces of one row group, at most
+    int max_pieces, usual_pieces;        // pieces of one row group, at most and for most of them
     int wg_tile_begin[HW_MAX_SPLITS + 1];   // first tile of each workgroup, counted through all row groups
     size_t partial_bytes;                // part_o + part_ml of all slots
     size_t workspace_bytes;              // partials, the merge's row table, and CallPlan::rope_bytes

@@ -102,6 +102,22 @@ static int openings() {
     return ok ? 0 : 1;
 }
 
+// One row group in more pieces than the others does not decide how all rows are merged.
+static int usual_pieces() {
+    hw_problem p{};
+    const int32_t len[2] = {4096, 1024};
+    p.dtype = HW_BF16;
+    p.F = 2; p.W = 1; p.S = 1024; p.Hq = 40; p.Hkv = 8; p.E = p.Ev = p.RotE = 128;
+    p.len = len;
+    hw::host::CallPlan cp;
+    hw::host::WholePlan wp;
+    if (hw::host::plan_call(&p, 256, &cp, 1) != HW_OK || !hw::host::whole_size(&p, 256, cp, &wp)) return 1;
+    hw::host::whole_deal(&p, cp, &wp);
+    const bool ok = wp.runs.max_pieces > 4 && wp.runs.usual_pieces <= 4;
+    if (!ok) std::printf("failed: pieces of the row groups, %d at most, usually %d\n", wp.runs.max_pieces, wp.runs.usual_pieces);
+    return ok ? 0 : 1;
+}
+
 // Paged queries of head dimension 256: K/V tiles are kept with more than two row groups of 16 a sequence, packed ones with more than
 // 20 rows in the mean.
 static int kept_tiles() {
@@ -127,6 +143,7 @@ int main() {
     if (kept_tiles() != 0) return 1;
     if (seen_tiles() != 0) return 1;
     if (openings() != 0) return 1;
+    if (usual_pieces() != 0) return 1;
     if (rounds_instead() != 0) return 1;
     if (head_dim_256() != 0) return 1;
     std::mt19937 rng(7);
@@ -193,7 +210,7 @@ int main() {
             for (int i = first; i < begun; ++i) CHECK(used[i + rg] == rg);
             most = std::max(most, pieces[rg]);
         }
-        CHECK(most == sp.max_pieces);
+        CHECK(most == sp.max_pieces && sp.usual_pieces <= most && sp.usual_pieces >= (wp.split > 0));
         left_over += wp.split > 0;
         const size_t part = (size_t)p.Hkv * sp.slots * hw::PLAN_SLOT_ROWS * (p.Ev + 2) * 4;
         CHECK(sp.partial_bytes == part && wp.workspace_bytes >= part + (size_t)p.Hkv * cp.plan[0].rows * 8 + cp.rope_bytes && wp.workspace_bytes % 256 == 0);

@@ -13,6 +13,7 @@ pytestmark = pytest.mark.gpu
 @pytest.mark.parametrize("W,S,Hq,Hkv,D,lens,dtype", [
     (1, 1100, 28, 4, 128, (1, 40, 33, 0, 1100), torch.bfloat16),                  # one and two tiles, an empty one: whole row groups
     (1, 840, 40, 8, 128, (3, 31, 32, 65, 1, 1, 840, 17), torch.float16),          # eight fragments, the chunk not the last
+    (1, 1879, 28, 4, 128, (208, 1879), torch.bfloat16),                           # a row group in five pieces, most in two: merged eight rows to a workgroup
     (1, 700, 20, 20, 128, (300, 20, 700), torch.bfloat16),                        # GQA 1: tables out of memory
     (2, 640, 16, 8, 128, (64, 640, 1, 640), torch.float16),                       # GQA 2, two workers
     (5, 7, 28, 4, 128, (1, 33, 7, 20, 64, 7, 200), torch.bfloat16),               # few rows: pre-rotated only
