@@ -403,6 +403,8 @@ __global__ __launch_bounds__(256) void merge_kernel(const MergeArgs a) {
                 o[u] = *reinterpret_cast<const f32x4*>(po + (size_t)sc * ostride);
                 mlv[u] = *reinterpret_cast<const f32x2*>(ml + (size_t)sc * mstride);
                 if (s >= ns) mlv[u] = f32x2{NEG_BIG, 0.f};
+                // (a sequence with another number of slots than the guess: its infinite values stay infinite)
+                if (GUESS && s >= ns) o[u] = f32x4{0.f, 0.f, 0.f, 0.f};
             }
         }
         float mb = m_run;
