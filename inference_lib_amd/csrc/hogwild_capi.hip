@@ -244,10 +244,11 @@ int paged_run(const hw_paged_problem* p, void* stream_, int stages) {
     ph.nrg = planned ? (cus / p->Hkv > 0 ? cus / p->Hkv : 1) : varlen ? 1 : plan.row_groups / p->W;
     ph.nwg = plan.workgroups;
     // (with the stages on their own, and in a workspace sized for hw_paged_plan only, the partials are laid out by it)
-    const bool shared = stages == (HW_STAGE_ATTENTION | HW_STAGE_MERGE) && paged_shared(p, plan) && p->workspace_bytes >= paged_call_bytes(p, plan);
+    const bool shared = stages == (HW_STAGE_ATTENTION | HW_STAGE_MERGE) && paged_shared(p, plan) && paged_shares_save(p, plan, cus) >= 0 && p->workspace_bytes >= paged_call_bytes(p, plan);
     ph.flags = ((plan.workgroups % 8 == 0) ? hw::PH_XCD_REMAP : 0) | (shared ? hw::PH_SHARED : 0) | (planned ? hw::PH_PLANNED : 0) | (paged_keep_in_l2(p, plan) ? hw::PH_KEEP : 0);
     if ((unsigned long long)p->num_blocks * p->Hkv * p->block_size * p->E * elem_size(p->dtype) < 0xffff0000ull) ph.flags |= hw::PH_SMALL;
     if (planned) ph.flags |= (p->W + plan.rows / hw::PLAN_SLOT_ROWS) << hw::PH_GROUPS_SHIFT;
+    if (shared) ph.flags |= paged_shares_save(p, plan, cus) << hw::PH_SAVED_SHIFT;
     ph.sc = (float)((double)p->scale * 1.4426950408889634074);
     ph.magic_gq = magic(p->Hq / p->Hkv);
     ph.magic_ls = magic(ph.LS);

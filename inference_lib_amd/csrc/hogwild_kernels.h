@@ -129,6 +129,7 @@ constexpr int PH_GROUPS_SHIFT = 8;   // from this bit on, planned: the most row 
 // sequences' visible tiles instead of nsplit to each (paged_share).  Partial sums by workgroup slot, LS * (Hq / Hkv) rows each, the
 // merge's row table right behind part_ml.
 constexpr int PH_SHARED = 8;
+constexpr int PH_SAVED_SHIFT = 8;    // from this bit on, shared: steps that other than equal shares have to save (paged_shares_save); > 0: more workgroups than CUs
 constexpr int PH_SMALL = 16;       // the K cache is less than 4 GB: one buffer descriptor reaches all of it (read by launch_paged_attention only)
 
 struct CopyBlocksArgs {

@@ -42,7 +42,7 @@ namespace hw {
 // The shares are the smallest bound on the tiles of a workgroup (in steps of the four waves) at which the sequences' workgroups
 // are no more than there are, found by trying one bound in every lane.  Working that out and requesting the queries again takes 0.9 us,
 // a step of the four waves 1.1 to 1.2 (fit over 63 decode steps of 2 to 12 sequences, all head layouts): nsplit each wherever the longest sequence needs two
-// steps at most, or no more than it would need with even shares.  The lengths are read ahead of the queries, which are requested for
+// steps at most, or no more than it would need with even shares (more workgroups than CUs: paged_shares_save).  The lengths are read ahead of the queries, which are requested for
 // equal shares, as are the partial sums in the merge.
 // A sequence with fewer workgroups has fewer tiles that are a wave's first, whose largest weight the storage type holds exactly: 1.04 to
 // 1.09 times the error against float64 (nine ragged steps x 6 seeds, bf16 and fp16).  With other than equal shares the reference of the
@@ -71,10 +71,14 @@ __device__ __forceinline__ PagedShare paged_share(const PagedDevHeader& ph, int 
     const PagedShare equal = {item, split, ph.nsplit, item * ph.nsplit, true, false};
     const int slots = ph.W * ph.nsplit, slot = item * ph.nsplit + split;
     const int longest = wave_max(tiles);
+    const int saved = NWAVES * (ph.flags >> PH_SAVED_SHIFT);   // (in tiles, like the bounds)
     if (longest <= 2 * NWAVES * ph.nsplit) return equal;       // (on its own: short steps leave here, 0.1 us sooner than behind the sum)
     const int all = __builtin_amdgcn_readlane(wave_scan_inclusive(tiles), 63);
     const int least = max(1, (int)((float)all * __builtin_amdgcn_rcpf((float)(NWAVES * slots))));          // steps with even shares, less what is left over
-    if (longest <= NWAVES * ph.nsplit * (least + (least * NWAVES * slots < all ? 1 : 0))) return equal;
+    int even = NWAVES * (least + (least * NWAVES * slots < all ? 1 : 0));
+    // (with many sequences the search is long; what half a workgroup of each leaves over is estimated instead)
+    if (saved > 0) even = (int)((float)all * __builtin_amdgcn_rcpf((float)(slots - (ph.W >> 1)))) + saved;
+    if (longest <= ph.nsplit * even) return equal;
     // lane = a bound on the tiles of a workgroup, multiples of the four waves: does every sequence get its workgroups?
     const float mine = (float)tiles;
     const int bound = NWAVES * (least + lane * (1 + (least >> 5)));

@@ -82,6 +82,8 @@ int paged_plan(const hw_paged_problem* p, int num_cus, hw_paged_plan* plan);
 // for: hw_paged_plan's workspace, the caller's fallback, and the merge's row table.
 bool paged_shared(const hw_paged_problem* p, const hw_paged_plan& plan);
 size_t paged_call_bytes(const hw_paged_problem* p, const hw_paged_plan& plan);
+// How many steps of its waves the longest sequence has to need less with other than equal shares, or -1: equal ones always.
+int paged_shares_save(const hw_paged_problem* p, const hw_paged_plan& plan, int num_cus);
 // Whether the tiles of a paged launch are to stay in the L2 (hogwild_plan.cpp).
 bool paged_keep_in_l2(const hw_paged_problem* p, const hw_paged_plan& plan);
 

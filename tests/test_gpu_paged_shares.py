@@ -93,6 +93,7 @@ def _step(lens, dtype, Hq, Hkv, D, bs, mb, seed, splits=0, change=None):
     (torch.float16, (3000, 3550, 2550, 2550, 2550), 16, 8, 256),
     (torch.bfloat16, (400, 9000, 2000, 64, 5000, 33), 32, 8, 128),
     (torch.float32, (300, 4100, 900), 8, 8, 64),
+    (torch.bfloat16, (7000,) + tuple(100 + 61 * i for i in range(23)), 40, 8, 128),      # more workgroups than CUs, and shares save many steps
 ])
 def test_order_of_the_sequences_does_not_matter(dtype, lens, Hq, Hkv, D):
     """The same sequences listed in other orders: the same bits for each."""
@@ -110,6 +111,8 @@ def test_order_of_the_sequences_does_not_matter(dtype, lens, Hq, Hkv, D):
     (torch.float16, (184, 101, 104, 74), 16, 8, 256),
     (torch.bfloat16, (886, 3433), 40, 8, 128),
     (torch.bfloat16, (4096, 4000, 4064, 3969), 40, 8, 128),                              # as many steps with even shares
+    (torch.bfloat16, (2016,) + tuple(200 + 40 * i for i in range(47)), 28, 4, 128),      # more workgroups than CUs, and shares save few steps
+    (torch.float16, tuple(60 + 50 * i for i in range(64)), 40, 8, 128),
 ])
 def test_short_and_even_steps_keep_equal_shares(dtype, lens, Hq, Hkv, D):
     """The bits of the call whose split is fixed at that of equal shares, which is launched so whatever the lengths."""
