@@ -32,6 +32,13 @@ def test_openings(W, S, Hq, Hkv, D, lens, dtype):
     eps = 2.0 ** -8 if dtype == torch.bfloat16 else 2.0 ** -11
     want_rq = ops.hogwild_rope(q, cos, sin)
     assert float((rq.float() - want_rq.float()).abs().max()) <= 4 * eps * float(want_rq.float().abs().max())
+    # and every element against float64: two fp32 roundings on the way, one to the storage type (2^-25: half the spacing of fp16's subnormals)
+    h = D // 2
+    x1, x2 = q.double()[None, ..., :h], q.double()[None, ..., h:]
+    c, s = cos[:, :, None, :, :h].double(), sin[:, :, None, :, :h].double()
+    rotated = torch.cat([x1 * c - x2 * s, x2 * c + x1 * s], dim=-1)
+    size = torch.cat([(x1 * c).abs() + (x2 * s).abs(), (x2 * c).abs() + (x1 * s).abs()], dim=-1)
+    assert bool(((rq.double() - rotated).abs() <= eps * rotated.abs() + 2.0 ** -22 * size + (2.0 ** -25 if dtype == torch.float16 else 0.0)).all())
     ref, ref_lse, bound = _reference(rq, loc, keys, values, scale, Hkv)
     seen = ~torch.isneginf(ref_lse)
     assert bool(((out.double() - ref).abs() <= bound)[seen].all())

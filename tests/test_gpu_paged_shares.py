@@ -68,6 +68,35 @@ def test_shares_by_length(dtype, lens, S, F, Hq, Hkv, D, bs):
         assert float((lse - ref_lse)[seen].abs().max()) <= 1e-4
 
 
+@pytest.mark.parametrize("dtype,lens,S,F,Hq,Hkv,D,bs,within", [
+    # 64 sequences (a lane of a wave each) and F * S = 8; beyond them equal shares
+    (torch.bfloat16, (6000,) + tuple(40 + 29 * i for i in range(62)) + (4500,), 1, 1, 8, 2, 64, 32, True),
+    (torch.float16, (6000,) + tuple(40 + 29 * i for i in range(63)) + (4500,), 1, 1, 8, 2, 64, 32, False),
+    (torch.bfloat16, (300, 7000, 1200, 8), 8, 1, 16, 8, 128, 32, True),
+    (torch.float16, (300, 5000, 64), 4, 2, 28, 7, 128, 16, True),
+    (torch.bfloat16, (300, 7000, 1200), 3, 3, 40, 8, 128, 16, False),
+])
+def test_limits_of_the_rule(dtype, lens, S, F, Hq, Hkv, D, bs, within):
+    W, mb = len(lens), -(-max(lens) // bs) + 3
+    g = torch.Generator(device="cuda").manual_seed(W)
+    rnd = lambda *shape: torch.randn(shape, generator=g, device="cuda").to(dtype)
+    table = torch.randperm(W * mb, generator=g, device="cuda").to(torch.int32).reshape(W, mb)
+    pos = torch.tensor([[n - S + s for s in range(S)] for n in lens], dtype=torch.int32, device="cuda")
+    args = dict(q=rnd(F, W, Hq, S, D), locations=torch.stack([pos - 7 * f for f in range(F)]).clamp(min=-1).contiguous(), key_cache=rnd(W * mb, Hkv, bs, D),
+                value_cache=rnd(W * mb, Hkv, bs, D), block_table=table, scale=D ** -0.5, fragment_lengths=torch.full((F,), bs * mb, dtype=torch.int32, device="cuda"))
+    equal = _lib.paged_plan(W=W, Hq=Hq, Hkv=Hkv, Ev=D, block_size=bs, max_blocks=mb, num_cus=_lib.lib.hw_device_cus(), S=S, dtype=_lib._DTYPE_CODE[dtype])
+    assert equal.splits > 1
+    outs = []
+    for splits in (0, equal.splits):
+        outs.append(torch.full((W, Hq, S, D), 7.0, dtype=dtype, device="cuda"))
+        pr = _lib.PagedProblem(out=outs[-1], splits=splits, **args)
+        assert (pr.workspace_bytes() > equal.workspace_bytes) == (within and splits == 0)      # room for the row table of other shares
+        pr.run()
+    assert torch.equal(*outs) == (not within)
+    if within:
+        test_shares_by_length(dtype, lens, S, F, Hq, Hkv, D, bs)
+
+
 def _step(lens, dtype, Hq, Hkv, D, bs, mb, seed, splits=0, change=None):
     """One decode step; sequence i has the data of its number in `lens`, a list of (number, length), wherever it is listed.
     change(q, keys, values, table) alters the data."""
