@@ -52,6 +52,7 @@ __device__ unsigned long long hw_wide_clock_buf[1024 * 4 * 16];
 }  // namespace hw
 
 #include "hogwild_device.h"
+#include "hogwild_walk.h"
 
 namespace hw {
 
@@ -407,8 +408,9 @@ __global__ __launch_bounds__(NW * 64, 1) void attention_wide_kernel(const Kernel
     [[maybe_unused]] const int run_begin = T0, run_end = T1;
     // STREAM: first the row groups that are this workgroup's alone, then its run
     [[maybe_unused]] const int split_groups = STREAM ? args.split : 0, groups = STREAM ? args.split + args.whole : 0;
-    [[maybe_unused]] bool whole = STREAM && split_groups + g < groups;
-    int rgi = STREAM ? (whole ? split_groups + g : run_begin / tiles_head) : rg;
+    [[maybe_unused]] const Walk walk = {run_begin, run_end, tiles_head, split_groups, groups, a.wgs_per_head};
+    [[maybe_unused]] bool whole = STREAM && walk_whole(walk, g);
+    int rgi = STREAM ? walk_first(walk, g) : rg;
     int r0, w0;                                 // first row of the workgroup, of this wave
     unsigned long long todo;                    // fragments with tiles of this workgroup
     WaveState<RB, G::NOC> st;
@@ -558,8 +560,8 @@ __global__ __launch_bounds__(NW * 64, 1) void attention_wide_kernel(const Kernel
         };
         auto open_rows = [&]() {
             if constexpr (STREAM) {
-                T0 = whole ? 0 : max(run_begin - rgi * tiles_head, 0);
-                T1 = whole ? tiles_head : min(run_end - rgi * tiles_head, tiles_head);
+                T0 = walk_from(walk, whole, rgi);
+                T1 = walk_to(walk, whole, rgi);
             }
             r0 = rgi * WIDE_ROWS;
             w0 = r0 + rw * WROWS;
@@ -572,17 +574,6 @@ __global__ __launch_bounds__(NW * 64, 1) void attention_wide_kernel(const Kernel
             }
             st.fresh = true;
             todo = __ballot(lane < a.F && max(T0, my_tb) < min(T1, my_te));
-        };
-        // The row group that comes behind the present one (STREAM): its number, or -1; below split_groups it is part of the run.
-        [[maybe_unused]] auto next_group = [&]() {
-            int group = -1;
-            if constexpr (STREAM) {
-                group = whole ? rgi + a.wgs_per_head : rgi + 1;
-                if (whole && group < groups) return group;
-                if (whole) group = run_begin / tiles_head;
-                if (max(run_begin, group * tiles_head) >= run_end) group = -1;
-            }
-            return group;
         };
         [[maybe_unused]] const unsigned q_base = lds_address(q_lds), cs_base = lds_address(cs_lds), loc_base = lds_address(lim_lds);
         // (the lane as the compiler cannot see through it: what is derived from it -- rows, addresses of the queries -- is then
@@ -599,11 +590,11 @@ __global__ __launch_bounds__(NW * 64, 1) void attention_wide_kernel(const Kernel
             WQ::request_tables(a, cs_base, loc_base, f, r.r0, r.ws_lo, r.nws, r.staged, wv, ln);
         };
         // The queries to rotate are the same for every fragment: they are requested here, before the workgroup's tile range
-        // and first fragment are worked out, and are on their way while that happens.  (A run without tiles has no rows: run_begin then
-        // lies behind the last row group.)
+        // and first fragment are worked out, and are on their way while that happens.  (No launch of head dimension 128 has a workgroup
+        // without tiles, but should one have, its run_begin lies behind the last row group.)
         Rows rows = rows_of(rgi);
         __builtin_amdgcn_s_waitcnt(0x0F70);   // vmcnt(0): the tables in the arguments, ahead of transfers that the compiler does not count
-        if (!PRE && (!STREAM || whole || run_begin < run_end)) request_queries(0, rows);
+        if (!PRE && (!STREAM || walk_opens(walk, whole))) request_queries(0, rows);
         open_rows();
         HW_MARK(10);
         Segment seg, nxt;                                        // the open segment; the one behind it in the same rows (lt1 == 0: none)
@@ -718,12 +709,12 @@ __global__ __launch_bounds__(NW * 64, 1) void attention_wide_kernel(const Kernel
             } else {
                 nxt.lt1 = 0;
                 if constexpr (STREAM) {
-                    const int group = next_group();
+                    const int group = walk_next(walk, whole, rgi);
                     behind = group >= 0;
                     if (behind) {
                         const bool wh = group >= split_groups;
                         rows = rows_of(group);
-                        const int t0 = wh ? 0 : max(run_begin - group * tiles_head, 0), t1 = wh ? tiles_head : min(run_end - group * tiles_head, tiles_head);
+                        const int t0 = walk_from(walk, wh, group), t1 = walk_to(walk, wh, group);
                         const int f = __builtin_ctzll(__ballot(lane < a.F && max(t0, my_tb) < min(t1, my_te)));
                         request_queries(f, rows);
                         request_tables(f, rows);
@@ -771,7 +762,7 @@ __global__ __launch_bounds__(NW * 64, 1) void attention_wide_kernel(const Kernel
                 if constexpr (STREAM) {
                     store_rows();
                     if (!whole) write_row_table();
-                    const int group = next_group();
+                    const int group = walk_next(walk, whole, rgi);
                     if (group >= 0) {
                         rgi = group;
                         whole = group >= split_groups;
@@ -791,8 +782,8 @@ __global__ __launch_bounds__(NW * 64, 1) void attention_wide_kernel(const Kernel
         // and first fragment are worked out, and are on their way while that happens.
         auto open_rows = [&]() {
             if constexpr (STREAM) {
-                T0 = whole ? 0 : max(run_begin - rgi * tiles_head, 0);
-                T1 = whole ? tiles_head : min(run_end - rgi * tiles_head, tiles_head);
+                T0 = walk_from(walk, whole, rgi);
+                T1 = walk_to(walk, whole, rgi);
             }
             r0 = rgi * WIDE_ROWS;
             w0 = r0 + rw * WROWS;
@@ -987,16 +978,11 @@ __global__ __launch_bounds__(NW * 64, 1) void attention_wide_kernel(const Kernel
                 open_segment(false);
             } else if constexpr (STREAM) {
                 store_rows();
-                if (!whole) {
-                    write_row_table();
-                    ++rgi;
-                } else if (rgi + a.wgs_per_head < groups) {
-                    rgi += a.wgs_per_head;
-                } else {
-                    whole = false;
-                    rgi = run_begin / tiles_head;
-                }
-                if (whole || max(run_begin, rgi * tiles_head) < run_end) {          // the next row group
+                if (!whole) write_row_table();
+                const int group = walk_next(walk, whole, rgi);
+                if (group >= 0) {
+                    rgi = group;
+                    whole = group >= split_groups;
                     __syncthreads();                       // every wave is done with the ring
                     open_rows();
                     open_segment(staged);

@@ -210,7 +210,8 @@ int main() {
             for (int i = first; i < begun; ++i) CHECK(used[i + rg] == rg);
             most = std::max(most, pieces[rg]);
         }
-        CHECK(most == sp.max_pieces && sp.usual_pieces <= most && sp.usual_pieces >= (wp.split > 0));
+        CHECK(most == sp.max_pieces);
+        CHECK(sp.usual_pieces <= most && sp.usual_pieces >= (wp.split > 0));
         left_over += wp.split > 0;
         const size_t part = (size_t)p.Hkv * sp.slots * hw::PLAN_SLOT_ROWS * (p.Ev + 2) * 4;
         CHECK(sp.partial_bytes == part && wp.workspace_bytes >= part + (size_t)p.Hkv * cp.plan[0].rows * 8 + cp.rope_bytes && wp.workspace_bytes % 256 == 0);
