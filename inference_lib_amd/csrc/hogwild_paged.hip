@@ -46,7 +46,7 @@ namespace hw {
 // equal shares, as are the partial sums in the merge.
 // A sequence with fewer workgroups has fewer tiles that are a wave's first, whose largest weight the storage type holds exactly: 1.04 to
 // 1.09 times the error against float64 (nine ragged steps x 6 seeds, bf16 and fp16).  With other than equal shares the reference of the
-// exponentials therefore follows the tiles (compute_tile's FOLLOW), 0.94 to 0.99 times the error of equal shares for 0.1 us.
+// exponentials therefore follows the tiles of such a sequence (compute_tile's FOLLOW), 0.94 to 0.99 times the error of equal shares.
 struct PagedShare {
     int w, split, ns, slot0;      // sequence, which of its ns workgroups, the first one's slot
     bool found;                   // false: a slot that is left over
@@ -70,15 +70,17 @@ __device__ __forceinline__ PagedShare paged_share(const PagedDevHeader& ph, int 
     // (nothing here depends on the order of the sequences: a sequence's share, and so its result, is the same wherever it is listed)
     const PagedShare equal = {item, split, ph.nsplit, item * ph.nsplit, true, false};
     const int slots = ph.W * ph.nsplit, slot = item * ph.nsplit + split;
-    const int longest = wave_max(tiles);
+    // whether the longest sequence's workgroups would have more than `most_tiles` tiles each with equal shares
+    auto more_than = [&](int most_tiles) { return __ballot(tiles > ph.nsplit * most_tiles) != 0; };
+    // (on their own: sequences of one length and short steps leave here, 0.1 us sooner than behind the sum)
+    if (__ballot(lane < ph.W && tiles != __builtin_amdgcn_readlane(tiles, 0)) == 0 || !more_than(2 * NWAVES)) return equal;
     const int saved = NWAVES * (ph.flags >> PH_SAVED_SHIFT);   // (in tiles, like the bounds)
-    if (longest <= 2 * NWAVES * ph.nsplit) return equal;       // (on its own: short steps leave here, 0.1 us sooner than behind the sum)
     const int all = __builtin_amdgcn_readlane(wave_scan_inclusive(tiles), 63);
     const int least = max(1, (int)((float)all * __builtin_amdgcn_rcpf((float)(NWAVES * slots))));          // steps with even shares, less what is left over
     int even = NWAVES * (least + (least * NWAVES * slots < all ? 1 : 0));
     // (with many sequences the search is long; what half a workgroup of each leaves over is estimated instead)
     if (saved > 0) even = (int)((float)all * __builtin_amdgcn_rcpf((float)(slots - (ph.W >> 1)))) + saved;
-    if (longest <= ph.nsplit * even) return equal;
+    if (!more_than(even)) return equal;
     // lane = a bound on the tiles of a workgroup, multiples of the four waves: does every sequence get its workgroups?
     const float mine = (float)tiles;
     const int bound = NWAVES * (least + lane * (1 + (least >> 5)));
@@ -88,7 +90,7 @@ __device__ __forceinline__ PagedShare paged_share(const PagedDevHeader& ph, int 
     for (int sq = 0; sq < ph.W; ++sq) need += groups(__int_as_float(__builtin_amdgcn_readlane(__float_as_int(mine), sq)), per);
     const unsigned long long fits = __ballot(need <= slots);
     const int fit = fits != 0 ? __builtin_ctzll(fits) : 0;
-    if (fits == 0 || longest <= ph.nsplit * __builtin_amdgcn_readlane(bound, fit)) return equal;
+    if (fits == 0 || !more_than(__builtin_amdgcn_readlane(bound, fit))) return equal;
     const float best = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(per), fit));
     const int n = lane < ph.W ? groups(mine, best) : 0;
     const int slot0 = wave_scan_inclusive(n) - n;
@@ -234,7 +236,7 @@ __global__ __launch_bounds__(NTHREADS, MINW) void paged_attention_kernel(const P
     }
     if (r0 >= rend) return;                 // uniform over the workgroup
     int loc0 = 0, len0 = 0, first_slot = 0;
-    bool other_shares = false;              // than equal ones
+    bool follow = false;                    // the reference of the exponentials follows the tiles: fewer workgroups than with equal shares
     if (shared) {
         loc0 = ph.loc[min(lane, ph.W - 1) * ph.LS];
         len0 = ph.frag_len[0];
@@ -245,7 +247,7 @@ __global__ __launch_bounds__(NTHREADS, MINW) void paged_attention_kernel(const P
         const PagedShare sh = paged_share(ph, item, split, lane, loc0, len0);
         if (!sh.found) return;              // uniform over the workgroup
         first_slot = sh.slot0;
-        other_shares = sh.other;
+        follow = sh.other && sh.ns < ns;
         if (sh.w != item || sh.split != split || sh.ns != ns) {
             item = sh.w;
             split = sh.split;
@@ -349,14 +351,14 @@ __global__ __launch_bounds__(NTHREADS, MINW) void paged_attention_kernel(const P
                     const int bt_n = bt_load(t + 2 * NW);
                     issue_tile(tr[1], kslots[1], bt_b, t + NW);
                     if constexpr (STATED) wait_k_landed<G, 1>();   // (see wait_k_landed: the table load in between only adds to what is behind)
-                    compute_tile<DT, E, EV, RB, false, QREG, false, false, G::SZ == 2>(tr[0], q_lds, qreg, lim, st, t * TILE, n, q, ph.sc, kslots[0], nullptr, nullptr, other_shares);
+                    compute_tile<DT, E, EV, RB, false, QREG, false, false, G::SZ == 2>(tr[0], q_lds, qreg, lim, st, t * TILE, n, q, ph.sc, kslots[0], nullptr, nullptr, follow);
                     bt_a = bt_n;
                 }
                 {
                     const int bt_n = bt_load(t + 3 * NW);
                     issue_tile(tr[0], kslots[0], bt_a, t + 2 * NW);
                     if constexpr (STATED) wait_k_landed<G, 1>();
-                    compute_tile<DT, E, EV, RB, false, QREG, false, false, G::SZ == 2>(tr[1], q_lds, qreg, lim, st, (t + NW) * TILE, n, q, ph.sc, kslots[1], nullptr, nullptr, other_shares);
+                    compute_tile<DT, E, EV, RB, false, QREG, false, false, G::SZ == 2>(tr[1], q_lds, qreg, lim, st, (t + NW) * TILE, n, q, ph.sc, kslots[1], nullptr, nullptr, follow);
                     bt_b = bt_n;
                 }
             }
@@ -366,8 +368,8 @@ __global__ __launch_bounds__(NTHREADS, MINW) void paged_attention_kernel(const P
                     issue_tile(tr[1], kslots[1], bt_b, t + NW);
                     if constexpr (STATED) wait_k_landed<G, 1>();
                     const int t0 = t * TILE;
-                    if (G::SZ == 4 && t0 + TILE <= minlim) compute_tile<DT, E, EV, RB, false, QREG, false, false, G::SZ == 2>(tr[0], q_lds, qreg, lim, st, t0, n, q, ph.sc, kslots[0], nullptr, nullptr, other_shares);
-                    else compute_tile<DT, E, EV, RB, true, QREG, false, false, G::SZ == 2>(tr[0], q_lds, qreg, lim, st, t0, n, q, ph.sc, kslots[0], nullptr, nullptr, other_shares);
+                    if (G::SZ == 4 && t0 + TILE <= minlim) compute_tile<DT, E, EV, RB, false, QREG, false, false, G::SZ == 2>(tr[0], q_lds, qreg, lim, st, t0, n, q, ph.sc, kslots[0], nullptr, nullptr, follow);
+                    else compute_tile<DT, E, EV, RB, true, QREG, false, false, G::SZ == 2>(tr[0], q_lds, qreg, lim, st, t0, n, q, ph.sc, kslots[0], nullptr, nullptr, follow);
                     bt_a = bt_n;
                 }
                 {
@@ -375,8 +377,8 @@ __global__ __launch_bounds__(NTHREADS, MINW) void paged_attention_kernel(const P
                     issue_tile(tr[0], kslots[0], bt_a, t + 2 * NW);
                     if constexpr (STATED) wait_k_landed<G, 1>();
                     const int t0 = (t + NW) * TILE;
-                    if (G::SZ == 4 && t0 + TILE <= minlim) compute_tile<DT, E, EV, RB, false, QREG, false, false, G::SZ == 2>(tr[1], q_lds, qreg, lim, st, t0, n, q, ph.sc, kslots[1], nullptr, nullptr, other_shares);
-                    else if (t0 < maxlim) compute_tile<DT, E, EV, RB, true, QREG, false, false, G::SZ == 2>(tr[1], q_lds, qreg, lim, st, t0, n, q, ph.sc, kslots[1], nullptr, nullptr, other_shares);
+                    if (G::SZ == 4 && t0 + TILE <= minlim) compute_tile<DT, E, EV, RB, false, QREG, false, false, G::SZ == 2>(tr[1], q_lds, qreg, lim, st, t0, n, q, ph.sc, kslots[1], nullptr, nullptr, follow);
+                    else if (t0 < maxlim) compute_tile<DT, E, EV, RB, true, QREG, false, false, G::SZ == 2>(tr[1], q_lds, qreg, lim, st, t0, n, q, ph.sc, kslots[1], nullptr, nullptr, follow);
                     bt_b = bt_n;
                 }
             }
