@@ -254,7 +254,9 @@ typedef struct hw_paged_plan {
     int32_t row_groups;        /* over all workers; an upper bound for the variable-length operator */
     int32_t splits;            /* workgroups per (kv head, row group); tile t of a sequence goes to wave t mod (4 * splits).  Decode
                                   steps of several sequences in a workspace of hw_paged_workspace_bytes: on average, each
-                                  sequence gets its share of them by its length, which the device knows */
+                                  sequence gets its share of them by its length, which the device knows.  Its result then
+                                  depends on the other lengths by rounding (not on the order of the sequences); with
+                                  hw_paged_problem.splits > 0 it does not */
     int32_t workgroups;
     int32_t device_planned;    /* packed queries in 128-row workgroups: the split is decided on the device from the query and KV
                                   lengths, in the prologue of the attention kernel.  row_groups is then the number

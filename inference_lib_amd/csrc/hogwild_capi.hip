@@ -188,7 +188,6 @@ int run(const hw_problem* p, void* stream_, int fused, int stages = HW_STAGE_ATT
     ma.pslots = ma.slot_rows = ma.guess = 0;
     ma.magic_rows = 0;
     if (stream_runs) {
-        ma.slot_rows = hw::PLAN_SLOT_ROWS;
         // (A row group with more pieces takes another batch of loads.  By the most pieces, one row group with five had all rows merged
         // four to a workgroup instead of eight: 37 prompt chunks with more than four at most 0.991 to 1.045 times as fast, 1.006 in the
         // mean, 1879 tokens behind 208 at 28/4 heads 64.3 -> 61.8 us a layer.)
@@ -276,7 +275,7 @@ int paged_run(const hw_paged_problem* p, void* stream_, int stages) {
     ma.xcd_local = ((!varlen || planned) && plan.workgroups % 8 == 0 && p->Hkv % 8 == 0) ? 1 : 0;
     ma.row_tab = planned || shared ? row_tab : nullptr;
     ma.pslots = planned ? plan.row_groups : shared ? plan.row_groups * plan.splits : 0;
-    ma.slot_rows = planned ? hw::PLAN_SLOT_ROWS : shared ? plan.rows / p->W : 0;
+    ma.slot_rows = shared ? plan.rows / p->W : 0;
     ma.guess = shared ? plan.splits : 0;
     ma.magic_rows = magic(shared ? ma.slot_rows : 1);
     if (planned) ma.wgs_per_head = 8;       // a row's slots are device data: the merge shape that suits a handful of them

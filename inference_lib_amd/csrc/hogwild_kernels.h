@@ -74,10 +74,11 @@ struct MergeArgs {
     int rows;           // rows 0 .. rows - 1 of every kv head are merged
     int xcd_local;      // kv head h was computed on XCD h / (Hkv/8): merge it there
     // Partials laid out by workgroup slot instead of by row (KH_STREAM, and the paged launches that are dealt on the device,
-    // see PagedHeader): row_tab[kv head][r] = {first slot | slots << 16, row within the slot}, a slot holds slot_rows rows (PLAN_SLOT_ROWS without guess), pslots
-    // slots per kv head; wgs_per_head then is what most rows have (for the choice of the merge kernel's shape).
+    // see PagedHeader): row_tab[kv head][r] = {first slot | slots << 16, row within the slot}, pslots slots per kv head, of PLAN_SLOT_ROWS rows
+    // or, with guess, slot_rows; wgs_per_head then is what most rows have (for the choice of the merge kernel's shape).
     const int* row_tab;
-    int pslots, slot_rows;
+    int pslots;
+    int slot_rows;      // (with guess)
     int guess;          // > 0: slots of a row where every slot_rows rows have the same number, one behind the other; requested ahead of the table
     unsigned magic_rows;   // ceil(2^32 / slot_rows), for guess
 };
@@ -118,11 +119,11 @@ struct alignas(64) PagedHeader {
 };
 static_assert(sizeof(PagedHeader) == 192, "PagedHeader must be 48 dwords");
 constexpr int PH_XCD_REMAP = 1;    // consecutive logical workgroup ids share an XCD
+constexpr int PH_KEEP = 4;         // K/V tiles stay in the L2 for the other row groups of a sequence (read by launch_paged_attention only)
 // The launch is planned on the device (packed queries in 128-row workgroups): nsplit = 1, nitems = workgroup slots per
 // kv head, and what slot j of a head does -- which row group of which sequence, which share of its tiles -- every
 // workgroup works out for itself from the query and KV lengths (plan_slot).  Behind part_ml the workgroups leave the
 // merge kernel a table per kv head of where each row's partial sums lie (MergeArgs::row_tab).
-constexpr int PH_KEEP = 4;         // K/V tiles stay in the L2 for the other row groups of a sequence (read by launch_paged_attention only)
 constexpr int PH_PLANNED = 2;
 constexpr int PH_GROUPS_SHIFT = 8;   // from this bit on, planned: the most row groups that the query tokens may come to
 // One row group per sequence (the fixed-length operator): the nitems * nsplit workgroups of a kv head are shared out by the

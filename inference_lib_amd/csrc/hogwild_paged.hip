@@ -41,16 +41,15 @@ namespace hw {
 // 31.7 -> 22.3 us, eight of 210 to 9000 at 32/8 37 -> 24, four of 300 to 11 000 at 16/8 and D = 256 41 -> 28.6, five of 844 to 5868 23.8 -> 22.2.
 // The shares are the smallest bound on the tiles of a workgroup (in steps of the four waves) at which the sequences' workgroups
 // are no more than there are, found by trying one bound in every lane.  Working that out and requesting the queries again takes 0.9 us,
-// a step of the four waves 1.1 to 1.2 (fit over 63 decode steps of 2 to 12 sequences, all head layouts): nsplit each wherever the longest sequence needs two
-// steps at most, or no more than it would need with even shares (more workgroups than CUs: paged_shares_save).  The lengths are read ahead of the queries, which are requested for
-// equal shares, as are the partial sums in the merge.
+// a step of the four waves 1.1 to 1.2 (fit over 63 decode steps of 2 to 12 sequences, all head layouts): nsplit each wherever the longest
+// sequence needs two steps at most, or no more than it would need with even shares (more workgroups than CUs: paged_shares_save).  The
+// lengths are read ahead of the queries, which are requested for equal shares, as are the partial sums in the merge.
 // A sequence with fewer workgroups has fewer tiles that are a wave's first, whose largest weight the storage type holds exactly: 1.04 to
-// 1.09 times the error against float64 (nine ragged steps x 6 seeds, bf16 and fp16).  With other than equal shares the reference of the
-// exponentials therefore follows the tiles of such a sequence (compute_tile's FOLLOW), 0.94 to 0.99 times the error of equal shares.
+// 1.09 times the error against float64 (seven ragged steps x 6 seeds, bf16 and fp16).  The reference of the exponentials therefore follows
+// the tiles of such a sequence (compute_tile's FOLLOW): 0.96 to 1.00 times the error of equal shares.
 struct PagedShare {
     int w, split, ns, slot0;      // sequence, which of its ns workgroups, the first one's slot
     bool found;                   // false: a slot that is left over
-    bool other;                   // not equal shares (the same for every workgroup of the launch)
 };
 // (loc0, len0: the first location of sequence min(lane, W - 1) and the first fragment's length, requested ahead of what the workgroup
 // needs besides, so that this is worked out while the rest is on its way)
@@ -68,7 +67,7 @@ __device__ __forceinline__ PagedShare paged_share(const PagedDevHeader& ph, int 
     }
     if (lane >= ph.W) tiles = 0;
     // (nothing here depends on the order of the sequences: a sequence's share, and so its result, is the same wherever it is listed)
-    const PagedShare equal = {item, split, ph.nsplit, item * ph.nsplit, true, false};
+    const PagedShare equal = {item, split, ph.nsplit, item * ph.nsplit, true};
     const int slots = ph.W * ph.nsplit, slot = item * ph.nsplit + split;
     // whether the longest sequence's workgroups would have more than `most_tiles` tiles each with equal shares
     auto more_than = [&](int most_tiles) { return __ballot(tiles > ph.nsplit * most_tiles) != 0; };
@@ -96,7 +95,6 @@ __device__ __forceinline__ PagedShare paged_share(const PagedDevHeader& ph, int 
     const int slot0 = wave_scan_inclusive(n) - n;
     const unsigned long long owner = __ballot(slot >= slot0 && slot < slot0 + n);
     PagedShare r;
-    r.other = true;
     r.found = owner != 0;
     r.w = r.found ? __builtin_ctzll(owner) : 0;
     r.slot0 = __builtin_amdgcn_readlane(slot0, r.w);
@@ -108,7 +106,7 @@ __device__ __forceinline__ PagedShare paged_share(const PagedDevHeader& ph, int 
 // SMALL: below 4 GB the K cache is reached through one buffer descriptor, and its transfers are buffer loads.  A transfer by 64-bit address
 // is a flat-encoded instruction with an LDS operand, for which the compiler waits until nothing is outstanding: it emptied the
 // look-ahead at every tile (vmcnt(0) in front of each request, where 16 and 17 operations may be in flight).  Four sequences of 12 528
-// tokens, append and attention 41.2 -> 39.3 us (6.3 TB/s in the attention), 2500 to 3600 tokens 18.2 -> 17.1, five of 296 to 10 543 22.3 -> 20.4;
+// tokens, append and attention 41.2 -> 39.3 us (6.0 TB/s in the attention), 2500 to 3600 tokens 18.2 -> 17.1, five of 296 to 10 543 22.3 -> 20.4;
 // bit-identical.
 struct CacheView {
     __amdgpu_buffer_rsrc_t k;
@@ -247,7 +245,7 @@ __global__ __launch_bounds__(NTHREADS, MINW) void paged_attention_kernel(const P
         const PagedShare sh = paged_share(ph, item, split, lane, loc0, len0);
         if (!sh.found) return;              // uniform over the workgroup
         first_slot = sh.slot0;
-        follow = sh.other && sh.ns < ns;
+        follow = sh.ns < ns;
         if (sh.w != item || sh.split != split || sh.ns != ns) {
             item = sh.w;
             split = sh.split;

@@ -441,8 +441,9 @@ static bool causal_chunk(const hw_problem* p) {
 //     this form);
 //   runs alone: 0.970 to 1.038 with up to three fragments, 0.992 in the mean of 49 calls, 0.997 in the mean of 21 with four and five,
 //     0.982 to 1.054 with six and more, 1.007 in the mean of 40.
-// Pre-rotated queries have no rotation to wait for: 1.007 to 1.22 in whole row groups and in runs; in rounds 1.00 to 1.11 with three
-// fragments or a workgroup to a row group, but for two calls of 0.98; with one opening a workgroup 0.974 to 1.03, 0.997 in the mean of ten.
+// Pre-rotated queries have no rotation to wait for: 1.007 to 1.22 in whole row groups and in runs; in rounds 0.98 to 1.11 with three
+// fragments or a workgroup to a row group, 1.012 in the mean of the 51 with least to do; with one opening a workgroup 0.974 to 1.03, 0.997
+// in the mean of ten.
 bool openings_ahead(const hw_problem* p, const hw_plan& plan, bool prerotated, bool stream_runs, const WholePlan* whole) {
     if (p->E != 128) return false;
     int nf = 0;
@@ -460,9 +461,10 @@ bool openings_ahead(const hw_problem* p, const hw_plan& plan, bool prerotated, b
 // and the workgroups with the later row groups, which see most, get less of the remainder or none of it.  (Taking in fewer tiles alone
 // gave nothing, the last row group's workgroup having as many as before; nor did unequal shares while unseen tiles cost as much as
 // others.)  us a layer: 938 tokens behind 577 at 40/8 heads 51 -> 44, 1088 behind 527 at 32/8 48 -> 40, 1112 behind 62 46 -> 41.5, 1024
-// behind 4096 117 -> 115; 70 calls of four head layouts 0.96 to 1.20 times as fast, 1.068 in the mean, two of them below 0.98.  The
-// costs of a piece and a fragment are from the same calls: at 8 and 2 tiles 1.046 in the mean, at 5 and 1 1.027, 12 and 2 1.063, 16 and 4
-// 1.065, 24 and 4 1.069; of several workers, dealt by all tiles, 1.015 at 8 and 2, 1.017 at 12 and 2, 1.016 at 24 and 4.
+// behind 4096 117 -> 115; of 86 calls of six head layouts, timed in turn with the form before, all are faster, 1.008 to 1.27 times, 1.095 in the
+// mean; with the lines of deal_by_seen in front of it they would be 0.97 to 1.15 times slower, 1.022 in the mean.  The costs of a piece and
+// a fragment are from the same calls: against 20 and 4 tiles 0.989 in the mean with 8 and 2 (0.86 at worst), 0.995 with 12 and 2, 0.999 with
+// 16 and 4, 1.001 with 24 and 4; of several workers, dealt by all tiles, 1.015 with 8 and 2, 1.017 with 12 and 2, 1.016 with 24 and 4.
 void whole_deal(const hw_problem* p, const CallPlan& cp, WholePlan* wp) {
     const hw_plan& plan = cp.plan[0];
     const int T = plan.tiles_per_head, wgs = wp->wgs, split = wp->split;

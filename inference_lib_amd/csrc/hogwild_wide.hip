@@ -1035,9 +1035,10 @@ __global__ __launch_bounds__(NW * 64, 1) void attention_wide_kernel(const Kernel
 // One thread per sequence and then per row group (at most PLAN_MAX_GROUPS of either; the host sends larger batches
 // down the unplanned path).  Every kv head has `pslots` workgroup slots.  A row group = up to 128 rows of one sequence;
 // its work is its sequence's tiles times the cost of a tile (a group of at most 64 rows keeps one wave per SIMD busy
-// instead of two: 0.67 against 0.88 us per tile measured, 3 : 4).  Every group takes one slot and a share of the others in
-// proportion to its work (what the rounding leaves over goes to the groups with the most work per slot), four tiles per
-// slot at least; slots are numbered through the groups in order.  Returns what slot `item` does
+// instead of two: 0.67 against 0.88 us per tile measured, 3 : 4).  Every group takes one slot at least, of four tiles or more; slots are
+// numbered through the groups in order.  Up to 64 sequences and row groups (plan_slot_wave) the slots are as many as the shorter of one
+// and two rounds of workgroups needs, each bounded alike; beyond (plan_slot) all of them are dealt, in proportion to the work, what the
+// rounding leaves over to the groups with the most work per slot.  Returns what slot `item` does
 // (found = false: nothing), and -- for the workgroup that holds a group's first slot -- tells the merge kernel through
 // the kv head's row table where the partial sums of the group's rows lie (a table per kv head, although they are all the
 // same: the merge of a head runs on the XCD whose workgroups wrote the head's partial sums and table, and finds both in
