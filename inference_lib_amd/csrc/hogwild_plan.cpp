@@ -605,12 +605,13 @@ bool paged_shared(const hw_paged_problem* p, const hw_paged_plan& plan) {
 // A launch of more workgroups than CUs evens itself out, as the workgroups of short sequences make room, and shares of one size only bring
 // its last round into step.  10 to 64 sequences at 4 to 16 kv heads, bf16, against equal shares: where up to six steps are saved 0.77 to
 // 1.16 times as fast, 0.957 in the mean of 83 steps; with more 0.95 to 1.45, 1.14 in the mean of 61; at head dimension 256 0.88 to 1.06,
-// 0.947 in the mean of six, with seven to nine, 1.10 in the mean of eight with more.  With several tokens or fragments looking the
+// 0.947 in the mean of six, with seven to nine, 1.10 in the mean of eight with more.  At 64, where the opening of a workgroup is shorter, 1.01
+// to 1.22 with six, 0.80 to 1.18 with less, 0.979 in the mean of 45.  With several tokens or fragments looking the
 // lengths up takes longer than that is worth in every round (60 sequences of 8 tokens at 8/4 heads, D = 64 17.4 -> 20.7 us).
 int paged_shares_save(const hw_paged_problem* p, const hw_paged_plan& plan, int num_cus) {
     if (plan.workgroups <= num_cus) return 0;
     if ((long long)p->F * p->S > 1) return -1;
-    return p->E > 128 ? 9 : 6;
+    return p->E > 128 ? 9 : p->E == 128 ? 6 : 5;
 }
 
 size_t paged_call_bytes(const hw_paged_problem* p, const hw_paged_plan& plan) {

@@ -139,8 +139,28 @@ static int kept_tiles() {
     return ok ? 0 : 1;
 }
 
+// Decode steps of sequences of different length: any step saved is worth other shares while there is a CU for every workgroup, many have to be
+// saved where there are more workgroups, and none is with several tokens or fragments then.
+static int shares_save() {
+    auto save = [](int D, int W, int Hq, int Hkv, int S, int F) {
+        hw_paged_problem p{};
+        p.dtype = HW_BF16;
+        p.F = F; p.W = W; p.Hq = Hq; p.Hkv = Hkv; p.E = p.Ev = D; p.S = S;
+        p.block_size = 16;
+        p.max_blocks = 400;
+        hw_paged_plan plan;
+        return hw::host::paged_plan(&p, 256, &plan) == HW_OK && hw::host::paged_shared(&p, plan) ? hw::host::paged_shares_save(&p, plan, 256) : -2;
+    };
+    const bool ok = save(128, 4, 40, 8, 1, 1) == 0 && save(128, 16, 40, 8, 2, 2) == 0 && save(128, 17, 40, 8, 1, 1) == 6 && save(64, 17, 40, 8, 1, 1) == 5 &&
+                    save(256, 17, 16, 8, 1, 1) == 9 && save(128, 17, 16, 8, 2, 1) == -1 && save(128, 17, 40, 8, 1, 2) == -1 && save(64, 64, 8, 2, 1, 1) == 0 &&
+                    save(64, 65, 8, 2, 1, 1) == -2 && save(128, 4, 40, 8, 3, 3) == -2;
+    if (!ok) std::printf("failed: steps that shares have to save\n");
+    return ok ? 0 : 1;
+}
+
 int main() {
     if (kept_tiles() != 0) return 1;
+    if (shares_save() != 0) return 1;
     if (seen_tiles() != 0) return 1;
     if (openings() != 0) return 1;
     if (usual_pieces() != 0) return 1;
