@@ -158,8 +158,30 @@ static int shares_save() {
     return ok ? 0 : 1;
 }
 
+// The kernel whose tiles are kept leaves the reference of the exponentials where it is, so none of its sequences may be shared out by length.
+static int kept_or_shared() {
+    for (int W = 2; W <= 64; W += 3)
+        for (int S = 1; S <= 40; ++S)
+            for (int group = 1; group <= 40; ++group) {
+                hw_paged_problem p{};
+                p.dtype = HW_BF16;
+                p.F = 1; p.W = W; p.Hkv = 2; p.Hq = 2 * group; p.E = p.Ev = 256; p.S = S;
+                p.block_size = 16;
+                p.max_blocks = 400;
+                for (p.row_blocks = 0; p.row_blocks <= 4; ++p.row_blocks) {
+                    hw_paged_plan plan;
+                    if (hw::host::paged_plan(&p, 256, &plan) == HW_OK && hw::host::paged_shared(&p, plan) && hw::host::paged_keep_in_l2(&p, plan)) {
+                        std::printf("failed: kept and shared: %d sequences, %d tokens, %d heads a group\n", W, S, group);
+                        return 1;
+                    }
+                }
+            }
+    return 0;
+}
+
 int main() {
     if (kept_tiles() != 0) return 1;
+    if (kept_or_shared() != 0) return 1;
     if (shares_save() != 0) return 1;
     if (seen_tiles() != 0) return 1;
     if (openings() != 0) return 1;
